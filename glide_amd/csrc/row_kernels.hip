@@ -1,0 +1,291 @@
+// gfx950 kernels of the transpose operator and the cached adjoint smoothing
+// passes on whole rows (row_ops.hpp): one wavefront per row segment of 64
+// columns, halo lanes and rows recomputed, no intermediate in global memory.
+//
+// k_adjoint_rows: one cached adjoint pass in one launch.  The transpose
+// operator minus the forcing for the rows of the workgroup, the cached 5x5
+// patch solves, and the multipliers' update into the other of two buffers
+// (neighbouring workgroups read the old ones).  MC: one colour phase of the
+// red-black pass, where every facet belongs to exactly one solving cell, so the
+// halo is one row above and below; otherwise the additive pass, whose facets
+// also take the increments of the cells left of and above the workgroup.
+// k_vjp_rows: the transpose operator alone.
+//
+// Workgroup height: a workgroup of NW wavefronts gives NW - 2 rows (MC), so 8
+// wavefronts redo 1.33 rows of the cell work per row and 16 redo 1.14.  Small
+// levels are bound by the length of one wavefront's chain and take 8 (more
+// workgroups, fewer wavefronts at each barrier).
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+#include "row_ops.hpp"
+#include "ssa_device.hpp"
+#include "ssa_kernels.hpp"
+#include "tab.hpp"
+
+namespace glide {
+
+namespace {
+
+// Increments of a patch from its 25 cached factors (J^T d = b).
+template <typename T>
+__device__ __forceinline__ void solve_cached(const T A[25], const T b[5], T d[5]) {
+    T y[5];
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+        T s = b[q];
+#pragma unroll
+        for (int k = 0; k < q; ++k) s -= A[q * 5 + k] * y[k];
+        y[q] = s;
+    }
+#pragma unroll
+    for (int q = 4; q >= 0; --q) {
+        T s = y[q];
+#pragma unroll
+        for (int k = q + 1; k < 5; ++k) s -= A[q * 5 + k] * d[k];
+        d[q] = s * A[q * 6];
+    }
+}
+
+template <typename T, int NW, bool MC>
+struct AdjointRows {
+    static constexpr int kHaloL = MC ? 2 : 3, kHaloR = 2;
+    static constexpr int kCols = kRowLanes - kHaloL - kHaloR;
+    static constexpr int kAbove = MC ? 1 : 2;  // rows above the first one the workgroup updates
+    static constexpr int kRows = NW - 1 - kAbove;
+
+    // omega: the signed weight of the increments
+    static __device__ __forceinline__ void pass(int bx, int by, const SsaArgs<T>& a, const T* __restrict__ cache,
+                                                const T* __restrict__ lu, const T* __restrict__ lv,
+                                                const T* __restrict__ lH, T* __restrict__ lu_dst,
+                                                T* __restrict__ lv_dst, T* __restrict__ lH_dst,
+                                                const T* __restrict__ fu, const T* __restrict__ fv,
+                                                const T* __restrict__ fH, T calving_rate, T omega, int colour) {
+        __shared__ typename TransposeRows<T, NW, false>::Lds s;
+        const int ny = a.ny, nx = a.nx;
+        const long n = (long)ny * nx;
+        const int lane = threadIdx.x, w = wave_row(threadIdx.y);
+        const int i = by * kRows - kAbove + w, j = bx * kCols - kHaloL + lane;
+        const bool cell = i >= 0 && i < ny && j >= 0 && j < nx;
+        // the wavefronts and lanes whose patches this workgroup solves
+        const bool solves = cell && w > 0 && w < NW - 1 && lane >= (MC ? kHaloL : kHaloL - 1) &&
+                            lane < kRowLanes - kHaloR && (!MC || ((i + j) & 1) == colour);
+        // the factors are loaded ahead of the operator, whose chain hides them
+        T A[25];
+        if (solves) {
+            const T* __restrict__ row = cache + (long)i * nx;
+            const unsigned k = cache_column(j, nx, MC);
+#pragma unroll
+            for (int q = 0; q < 25; ++q) A[q] = (row + q * n)[k];
+        }
+        TransposeRows<T, NW, false> t;
+        t.run(s, a, lu, lv, lH, fu, fv, fH, calving_rate, cache + (long)kAdjointCacheEta * n, w, lane, i, j);
+        const T rur = lane_right(t.ru);
+        T d[5] = {T(0), T(0), T(0), T(0), T(0)};
+        if (solves) {
+            const T b[5] = {t.ru, rur, t.rv, t.rvb, t.rH};
+            solve_cached(A, b, d);
+        }
+        const bool own = cell && w >= kAbove && w < NW - 1 && lane >= kHaloL && lane < kRowLanes - kHaloR;
+        const T lur = lane_right(t.lu), d1l = lane_left(d[1]);
+        T* __restrict__ urow = lu_dst + (long)i * (nx + 1);
+        T* __restrict__ vrow = lv_dst + (long)i * nx;
+        if constexpr (MC) {
+            // a facet is written by the cell that solves it; the domain-edge
+            // facets of the other colour's cells are copied
+            const bool left = lane > kHaloL && j >= 1 && j <= nx && i >= 0 && i < ny && w > 0 && w < NW - 1 &&
+                              lane <= kRowLanes - kHaloR && ((i + j - 1) & 1) == colour;
+            const bool act = solves;
+            if (act || left) urow[j] = t.lu + omega * (act ? d[0] : d1l);
+            if (act) {
+                vrow[j] = t.lv + omega * d[2];
+                (vrow + nx)[j] = t.lvb + omega * d[3];
+            }
+            if (own) {
+                (lH_dst + (long)i * nx)[j] = t.lH + omega * d[4];
+                if (!act) {
+                    if (j == 0) urow[0] = t.lu;
+                    if (j == nx - 1) urow[nx] = lur;
+                    if (i == 0) vrow[j] = t.lv;
+                    if (i == ny - 1) (vrow + nx)[j] = t.lvb;
+                }
+            }
+        } else {
+            // the increments of the bottom facets go to the row below
+            __syncthreads();
+            s.down[w][0][lane] = d[3];
+            __syncthreads();
+            if (own) {
+                const T h = T(0.5);
+                T x = h * d[0];
+                if (j > 0) x += h * d1l;
+                urow[j] = t.lu + omega * x;
+                if (j == nx - 1) urow[nx] = lur + omega * (h * d[1]);
+                x = h * d[2];
+                if (i > 0) x += h * s.down[w - 1][0][lane];
+                vrow[j] = t.lv + omega * x;
+                if (i == ny - 1) (vrow + nx)[j] = t.lvb + omega * (h * d[3]);
+                (lH_dst + (long)i * nx)[j] = t.lH + omega * d[4];
+            }
+        }
+    }
+};
+
+template <typename T, int NW, bool MC>
+__global__ __launch_bounds__(kRowLanes* NW) void k_adjoint_rows(SsaArgs<T> a, const T* __restrict__ cache,
+                                                                const T* __restrict__ lu, const T* __restrict__ lv,
+                                                                const T* __restrict__ lH, T* __restrict__ lu_dst,
+                                                                T* __restrict__ lv_dst, T* __restrict__ lH_dst,
+                                                                const T* __restrict__ fu, const T* __restrict__ fv,
+                                                                const T* __restrict__ fH, T calving_rate, T omega,
+                                                                int colour) {
+    AdjointRows<T, NW, MC>::pass(blockIdx.x, blockIdx.y, a, cache, lu, lv, lH, lu_dst, lv_dst, lH_dst, fu, fv, fH,
+                                 calving_rate, omega, colour);
+}
+
+template <typename T, int NW>
+__global__ __launch_bounds__(kRowLanes* NW) void k_tab_adj_pass(const TabAdjPass<T>* __restrict__ jobs,
+                                                                const int* __restrict__ start, int n, int colour) {
+    const int e = tab_find(start, n, blockIdx.x);
+    const TabAdjPass<T> J = jobs[e];
+    const int lb = blockIdx.x - start[e];
+    AdjointRows<T, NW, true>::pass(lb % J.gx, lb / J.gx, J.a, J.cache, J.lu, J.lv, J.lH, J.lu_dst, J.lv_dst, J.lH_dst,
+                                   J.fu, J.fv, J.fH, J.cr, J.omega, colour);
+}
+
+constexpr int kVjpWaves = 8;
+constexpr int kVjpCols = kRowLanes - 4, kVjpOutRows = kVjpWaves - 2;
+
+// The transpose operator for the facets and cells of 60 columns and 6 rows.
+template <typename T, bool DRAG>
+__device__ __forceinline__ void vjp_rows(int bx, int by, const SsaArgs<T>& a, const T* __restrict__ lu,
+                                         const T* __restrict__ lv, const T* __restrict__ lH,
+                                         const T* __restrict__ fu, const T* __restrict__ fv,
+                                         const T* __restrict__ fH, T* __restrict__ ou, T* __restrict__ ov,
+                                         T* __restrict__ oH, T calving_rate, const T* __restrict__ eta_cache) {
+    __shared__ typename TransposeRows<T, kVjpWaves, DRAG>::Lds s;
+    const int ny = a.ny, nx = a.nx;
+    const int lane = threadIdx.x, w = wave_row(threadIdx.y);
+    const int i = by * kVjpOutRows - 1 + w, j = bx * kVjpCols - 2 + lane;
+    TransposeRows<T, kVjpWaves, DRAG> t;
+    t.run(s, a, lu, lv, lH, fu, fv, fH, calving_rate, eta_cache, w, lane, i, j);
+    if (w < 1 || w > kVjpWaves - 2 || lane < 2 || lane >= kRowLanes - 2 || i > ny || j > nx) return;
+    if (i < ny) (ou + (long)i * (nx + 1))[j] = t.ru;
+    if (j < nx) (ov + (long)i * nx)[j] = t.rv;
+    if (i < ny && j < nx) (oH + (long)i * nx)[j] = t.rH;
+}
+
+template <typename T, bool DRAG>
+__global__ __launch_bounds__(kRowLanes* kVjpWaves) void k_vjp_rows(SsaArgs<T> a, const T* __restrict__ lu,
+                                                                   const T* __restrict__ lv,
+                                                                   const T* __restrict__ lH,
+                                                                   const T* __restrict__ fu,
+                                                                   const T* __restrict__ fv,
+                                                                   const T* __restrict__ fH, T* __restrict__ ou,
+                                                                   T* __restrict__ ov, T* __restrict__ oH,
+                                                                   T calving_rate, const T* __restrict__ eta_cache) {
+    vjp_rows<T, DRAG>(blockIdx.x, blockIdx.y, a, lu, lv, lH, fu, fv, fH, ou, ov, oH, calving_rate, eta_cache);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kRowLanes* kVjpWaves) void k_tab_vjp(const TabVjp<T>* __restrict__ jobs,
+                                                                  const int* __restrict__ start, int n) {
+    const int e = tab_find(start, n, blockIdx.x);
+    const TabVjp<T> J = jobs[e];
+    const int lb = blockIdx.x - start[e];
+    vjp_rows<T, false>(lb % J.gx, lb / J.gx, J.a, J.lu, J.lv, J.lH, J.fu, J.fv, J.fH, J.ou, J.ov, J.oH, J.cr,
+                       J.eta_cache);
+}
+
+// Wavefronts of a workgroup of the red-black adjoint phase.
+#ifndef GLIDE_ADJ_WAVES32
+#define GLIDE_ADJ_WAVES32 8
+#endif
+template <typename T>
+constexpr int adj_waves() { return std::is_same<T, float>::value ? GLIDE_ADJ_WAVES32 : 8; }
+
+template <typename T, int NW, bool MC>
+dim3 adjoint_grid(int ny, int nx) {
+    using P = AdjointRows<T, NW, MC>;
+    return dim3((nx + P::kCols - 1) / P::kCols, (ny + P::kRows - 1) / P::kRows);
+}
+
+}  // namespace
+
+template <typename T>
+hipError_t launch_adjoint_pass_fused(const SsaArgs<T>& a, const T* cache, const T* lu, const T* lv, const T* lH,
+                                     T* lu_dst, T* lv_dst, T* lH_dst, const T* fu, const T* fv, const T* fH,
+                                     T calving_rate, T omega, hipStream_t st) {
+    if (!a.P.linear_drag) return hipErrorInvalidValue;
+    TimedLaunch tl(kTimeAdjointCell, (long)a.ny * a.nx, st);
+    k_adjoint_rows<T, 8, false><<<adjoint_grid<T, 8, false>(a.ny, a.nx), dim3(kRowLanes, 8), 0, st>>>(
+        a, cache, lu, lv, lH, lu_dst, lv_dst, lH_dst, fu, fv, fH, calving_rate, -omega, -1);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_adjoint_pass_mc(const SsaArgs<T>& a, const T* cache, const T* lu, const T* lv, const T* lH,
+                                  T* lu_dst, T* lv_dst, T* lH_dst, const T* fu, const T* fv, const T* fH,
+                                  T calving_rate, T omega, int colour, hipStream_t st) {
+    if (!a.P.linear_drag) return hipErrorInvalidValue;
+    TimedLaunch tl(std::is_same<T, float>::value ? kTimeAdjointMc32 : kTimeAdjointMc64, (long)a.ny * a.nx, st);
+    constexpr int NW = adj_waves<T>();
+    k_adjoint_rows<T, NW, true><<<adjoint_grid<T, NW, true>(a.ny, a.nx), dim3(kRowLanes, NW), 0, st>>>(
+        a, cache, lu, lv, lH, lu_dst, lv_dst, lH_dst, fu, fv, fH, calving_rate, -omega, colour & 1);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_vjp(const SsaArgs<T>& a, const T* lu, const T* lv, const T* lH, const T* fu, const T* fv,
+                      const T* fH, T* ou, T* ov, T* oH, T calving_rate, const T* eta_cache, hipStream_t st) {
+    TimedLaunch tl(kTimeVjp, (long)a.ny * a.nx, st);
+    const dim3 g((a.nx + kVjpCols) / kVjpCols, (a.ny + kVjpOutRows) / kVjpOutRows), b(kRowLanes, kVjpWaves);
+    if (a.P.linear_drag)
+        k_vjp_rows<T, false><<<g, b, 0, st>>>(a, lu, lv, lH, fu, fv, fH, ou, ov, oH, calving_rate, eta_cache);
+    else
+        k_vjp_rows<T, true><<<g, b, 0, st>>>(a, lu, lv, lH, fu, fv, fH, ou, ov, oH, calving_rate, eta_cache);
+    return hipGetLastError();
+}
+
+// ------------------------------------------------------------ domain tables
+int tab_blocks_adj_pass(int ny, int nx, bool fp32, int* gx) {
+    const dim3 g = fp32 ? adjoint_grid<float, adj_waves<float>(), true>(ny, nx)
+                        : adjoint_grid<double, adj_waves<double>(), true>(ny, nx);
+    *gx = (int)g.x;
+    return (int)(g.x * g.y);
+}
+int tab_blocks_vjp(int ny, int nx, int* gx) {
+    *gx = (nx + kVjpCols) / kVjpCols;
+    return *gx * ((ny + kVjpOutRows) / kVjpOutRows);
+}
+
+template <typename T>
+hipError_t launch_tab_adj_pass(const TabAdjPass<T>* jobs, const int* start, int n, int blocks, int colour,
+                               hipStream_t st) {
+    if (n <= 0 || blocks <= 0) return hipSuccess;
+    constexpr int NW = adj_waves<T>();
+    k_tab_adj_pass<T, NW><<<blocks, dim3(kRowLanes, NW), 0, st>>>(jobs, start, n, colour & 1);
+    return hipGetLastError();
+}
+template <typename T>
+hipError_t launch_tab_vjp(const TabVjp<T>* jobs, const int* start, int n, int blocks, hipStream_t st) {
+    if (n <= 0 || blocks <= 0) return hipSuccess;
+    k_tab_vjp<T><<<blocks, dim3(kRowLanes, kVjpWaves), 0, st>>>(jobs, start, n);
+    return hipGetLastError();
+}
+
+#define GLIDE_ROWS_INST(T)                                                                                            \
+    template hipError_t launch_adjoint_pass_fused<T>(const SsaArgs<T>&, const T*, const T*, const T*, const T*, T*,   \
+                                                     T*, T*, const T*, const T*, const T*, T, T, hipStream_t);        \
+    template hipError_t launch_adjoint_pass_mc<T>(const SsaArgs<T>&, const T*, const T*, const T*, const T*, T*, T*,  \
+                                                  T*, const T*, const T*, const T*, T, T, int, hipStream_t);          \
+    template hipError_t launch_vjp<T>(const SsaArgs<T>&, const T*, const T*, const T*, const T*, const T*, const T*,  \
+                                      T*, T*, T*, T, const T*, hipStream_t);                                          \
+    template hipError_t launch_tab_adj_pass<T>(const TabAdjPass<T>*, const int*, int, int, int, hipStream_t);         \
+    template hipError_t launch_tab_vjp<T>(const TabVjp<T>*, const int*, int, int, hipStream_t);
+GLIDE_ROWS_INST(double)
+GLIDE_ROWS_INST(float)
+#undef GLIDE_ROWS_INST
+
+}  // namespace glide

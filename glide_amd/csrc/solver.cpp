@@ -339,7 +339,7 @@ VankaArgs<R> adjoint_vanka_args(const glide_level& L, const glide_vanka_config& 
 int adjoint_prepare(const glide_level& L, double dt, const glide_vanka_config& vc, int flags, hipStream_t st) {
     if (!L.adj_cache) return GLIDE_OK;
     SsaArgs<R> a = make_args(L, dt, true);
-    HIP_TRY(launch_adjoint_factor<R>(a, P(L.adj_cache), adjoint_vanka_args(L, vc, flags), st), "adjoint factor");
+    HIP_TRY(launch_adjoint_factor<R>(a, P(L.adj_cache), adjoint_vanka_args(L, vc, flags), false, st), "adjoint factor");
     return GLIDE_OK;
 }
 
@@ -1469,7 +1469,7 @@ VankaArgs<T> adjoint_args_t(const glide_level& L, const glide_vanka_config& vc) 
 template <typename T>
 int adjoint_prepare_t(const glide_level& L, double dt, const glide_vanka_config& vc, hipStream_t st) {
     SsaArgs<T> a = make_args_t<T>(L, dt, true);
-    HIP_TRY(launch_adjoint_factor<T>(a, PT<T>(L.adj_cache), adjoint_args_t<T>(L, vc), st), "adjoint factor");
+    HIP_TRY(launch_adjoint_factor<T>(a, PT<T>(L.adj_cache), adjoint_args_t<T>(L, vc), true, st), "adjoint factor");
     return GLIDE_OK;
 }
 
@@ -2168,7 +2168,7 @@ struct EnsRec {
             R.fu = CPT<T>(L.af_u); R.fv = CPT<T>(L.af_v); R.fH = CPT<T>(L.af_H);
             R.cr = T(L.phys.calving_rate);
             R.omega = -T(va.omega);
-            blocks.push_back(tab_blocks_adj_pass(L.ny, L.nx, tab_adj_pass_rows(sizeof(T) == 4), &R.gx));
+            blocks.push_back(tab_blocks_adj_pass(L.ny, L.nx, sizeof(T) == 4, &R.gx));
             red.push_back(R);
             TabAdjPass<T> B = R;
             B.lu = alt_u; B.lv = alt_v; B.lH = alt_H;

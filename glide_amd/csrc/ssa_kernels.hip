@@ -18,6 +18,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "row_ops.hpp"
 #include "ssa_device.hpp"
 #include "ssa_kernels.hpp"
 #include "tab.hpp"
@@ -32,12 +33,6 @@ constexpr int NT = TX * TY;
 #define GLIDE_VANKA_ROWS 1
 #endif
 constexpr int kVankaRows = GLIDE_VANKA_ROWS;
-// Tile height of the transpose operator
-#ifndef GLIDE_VJP_ROWS
-#define GLIDE_VJP_ROWS 4
-#endif
-constexpr int kVjpRows = GLIDE_VJP_ROWS;
-
 template <typename T, class Ld = LdPlain>
 __device__ __forceinline__ T cell_viscosity(const T* __restrict__ u, const T* __restrict__ v, const T* __restrict__ B,
                                             int ci, int cj, int ny, int nx, T dxi, const Phys<T>& P) {
@@ -817,9 +812,12 @@ __global__ __launch_bounds__(NT) void k_vanka_adjoint_cell(SsaArgs<T> a, const T
 // the diagonal, 0 for a pinned row (boundary facet or active-set cell), so
 // that its increment is exactly zero as when its right-hand side is cleared;
 // cache[25 * n + c] the cell viscosity, reused by the transpose operator.
+// split (the red-black passes): within a row of planes 0..24 the even columns
+// come first, then the odd ones, so that a colour phase reads only the factors
+// of the cells it solves (12.5 instead of 25 values per cell of the level).
 template <typename T>
 __device__ __forceinline__ void adjoint_factor_body(int bx, int by, const SsaArgs<T>& a, T* __restrict__ cache,
-                                                    const VankaArgs<T>& vk) {
+                                                    const VankaArgs<T>& vk, bool split) {
     __shared__ T s_eta[TY + 2][TX + 2];
     const int i0 = by * TY, j0 = bx * TX;
     const int tid = threadIdx.y * TX + threadIdx.x;
@@ -861,13 +859,14 @@ __device__ __forceinline__ void adjoint_factor_body(int bx, int by, const SsaArg
 #pragma unroll
     for (int k = 0; k < 5; ++k) A[k * 6] = pin[k] ? T(0) : inv[k];
 #pragma unroll
-    for (int q = 0; q < 25; ++q) cache[q * n + c] = A[q];
+    for (int q = 0; q < 25; ++q) (cache + q * n + (long)i * nx)[cache_column(j, nx, split)] = A[q];
     cache[25 * n + c] = s_eta[threadIdx.y + 1][threadIdx.x + 1];
 }
 
 template <typename T>
-__global__ __launch_bounds__(NT) void k_adjoint_factor(SsaArgs<T> a, T* __restrict__ cache, VankaArgs<T> vk) {
-    adjoint_factor_body<T>(blockIdx.x, blockIdx.y, a, cache, vk);
+__global__ __launch_bounds__(NT) void k_adjoint_factor(SsaArgs<T> a, T* __restrict__ cache, VankaArgs<T> vk,
+                                                       bool split) {
+    adjoint_factor_body<T>(blockIdx.x, blockIdx.y, a, cache, vk, split);
 }
 
 // Increments of a cell from its 25 cached factors A (in registers) and the
@@ -995,33 +994,15 @@ __global__ __launch_bounds__(NT) void k_vanka_adjoint_fused(const T* __restrict_
 // Jᵀλ (minus the adjoint forcing when use_forcing) as a gather.  Phase 1
 // computes, for the cells of the tile plus a one-cell ring, the masked
 // thickness multiplier, viscosity, its derivative along λ and the normal
-// stress rows applied to λ; phase 2 the shear-stress rows of the vertices and
-// the drag cross-terms of the facets; phase 3 gives every output its sum in a
-// fixed order.  Velocity rows use the symmetry of the velocity block as the
+// stress rows applied to λ; phase 2 the shear-stress rows of the vertices;
+// phase 3 gives every output its sum in a fixed order.  Velocity rows use the symmetry of the velocity block as the
 // reference does (glide/cuda/residuals.cu:797-817); Dirichlet facets and
 // masked cells return zero (residuals.cu:1122-1160).
-template <typename T, int ROWS>
-struct VjpTile {
-    T lHm[ROWS + 2][TX + 2];
-    T eta[ROWS + 2][TX + 2];
-    T etad[ROWS + 2][TX + 2];
-    T Hs[ROWS + 2][TX + 2];
-    T Lxx[ROWS + 2][TX + 2];
-    T Lyy[ROWS + 2][TX + 2];
-    T Kxx[ROWS + 2][TX + 2];   // d sigma_xx / d(eta H) at the cell
-    T Kyy[ROWS + 2][TX + 2];
-    T Lxy[ROWS + 1][TX + 1];   // vertices [i0, i0+ROWS] x [j0, j0+TX]
-    T Gxy[ROWS + 1][TX + 1];   // d sigma_xy / d(eta H) * 0.25 * (λ combination) * dxi
-    T Pu[4][ROWS + 1][TX + 1]; // λu * drag cross-derivatives, u facets rows [i0-1, i0+ROWS-1], cols [j0, j0+TX]
-    T Pv[4][ROWS + 1][TX + 1]; // λv * drag cross-derivatives, v facets rows [i0, i0+ROWS], cols [j0-1, j0+TX-1]
-};
-
 // The transpose operator for the outputs (facets and cells) i0 <= i < i0 +
 // rows, j0 <= j < j0 + cols inside the grid, by nthr threads (tid = 0 ..
 // nthr - 1) of one block, through the block storage S (cell arrays over the
-// one-cell ring, vertex arrays, and with S::kDrag the drag cross-terms;
-// without it the drag must be linear, whose cross-terms vanish), each output
-// handed to Out with its tile position and global index.
+// one-cell ring, vertex arrays), each output handed to Out with its tile
+// position and global index.  Linear drag only, whose cross-terms vanish.
 template <typename T, typename S, typename Out, class Ld = LdPlain>
 __device__ __forceinline__ void vjp_body(const SsaArgs<T>& a, const T* __restrict__ lu, const T* __restrict__ lv,
                                          const T* __restrict__ lH, const T* __restrict__ fu, const T* __restrict__ fv,
@@ -1060,7 +1041,7 @@ __device__ __forceinline__ void vjp_body(const SsaArgs<T>& a, const T* __restric
         s.Lxx(ri, rj) = Lx; s.Lyy(ri, rj) = Ly; s.Kxx(ri, rj) = Kx; s.Kyy(ri, rj) = Ky;
     }
     __syncthreads();
-    // phase 2a: vertices (vi, vj) in [i0, i0+rows] x [j0, j0+cols]
+    // phase 2: vertices (vi, vj) in [i0, i0+rows] x [j0, j0+cols]
     for (int k = tid; k < (rows + 1) * (cols + 1); k += nthr) {
         const int ri = k / (cols + 1), rj = k % (cols + 1);
         const int vi = i0 + ri, vj = j0 + rj;
@@ -1079,36 +1060,6 @@ __device__ __forceinline__ void vjp_body(const SsaArgs<T>& a, const T* __restric
             G = q.d_eH * T(0.25) * (lub - lut + lvl - lvr) * dxi;
         }
         s.Lxy(ri, rj) = L; s.Gxy(ri, rj) = G;
-    }
-    // phase 2b: drag cross-terms of u facets (rows i0-1.., cols j0..) and v facets (rows i0.., cols j0-1..)
-    for (int k = tid; S::kDrag && k < (rows + 1) * (cols + 1); k += nthr) {
-        const int ri = k / (cols + 1), rj = k % (cols + 1);
-        {
-            const int fi = i0 - 1 + ri, fj = j0 + rj;
-            T q0 = 0, q1 = 0, q2 = 0, q3 = 0;
-            if (fi >= 0 && fi < ny && fj >= 0 && fj <= nx && !a.P.linear_drag) {
-                Drag<T> t = basal_drag(u[(long)fi * (nx + 1) + fj], v[offV(fi, fj - 1, ny, nx)], v[offV(fi, fj, ny, nx)],
-                                       v[offV(fi + 1, fj - 1, ny, nx)], v[offV(fi + 1, fj, ny, nx)],
-                                       a.phi[offC(fi, fj - 1, ny, nx)], a.phi[offC(fi, fj, ny, nx)],
-                                       a.beta[offC(fi, fj - 1, ny, nx)], a.beta[offC(fi, fj, ny, nx)], a.P);
-                T l = Ld::get(lu + (long)fi * (nx + 1) + fj);
-                q0 = l * t.c0; q1 = l * t.c1; q2 = l * t.c2; q3 = l * t.c3;
-            }
-            s.Pu(0, ri, rj) = q0; s.Pu(1, ri, rj) = q1; s.Pu(2, ri, rj) = q2; s.Pu(3, ri, rj) = q3;
-        }
-        {
-            const int fi = i0 + ri, fj = j0 - 1 + rj;
-            T q0 = 0, q1 = 0, q2 = 0, q3 = 0;
-            if (fi >= 0 && fi <= ny && fj >= 0 && fj < nx && !a.P.linear_drag) {
-                Drag<T> t = basal_drag(v[(long)fi * nx + fj], u[offU(fi - 1, fj, ny, nx)], u[offU(fi - 1, fj + 1, ny, nx)],
-                                       u[offU(fi, fj, ny, nx)], u[offU(fi, fj + 1, ny, nx)],
-                                       a.phi[offC(fi - 1, fj, ny, nx)], a.phi[offC(fi, fj, ny, nx)],
-                                       a.beta[offC(fi - 1, fj, ny, nx)], a.beta[offC(fi, fj, ny, nx)], a.P);
-                T l = Ld::get(lv + (long)fi * nx + fj);
-                q0 = l * t.c0; q1 = l * t.c1; q2 = l * t.c2; q3 = l * t.c3;
-            }
-            s.Pv(0, ri, rj) = q0; s.Pv(1, ri, rj) = q1; s.Pv(2, ri, rj) = q2; s.Pv(3, ri, rj) = q3;
-        }
     }
     __syncthreads();
 
@@ -1129,9 +1080,6 @@ __device__ __forceinline__ void vjp_body(const SsaArgs<T>& a, const T* __restric
                 Drag<T> t = basal_drag(u[o], v[cc - 1], v[cc], v[cc + nx - 1], v[cc + nx], pl, pc, a.beta[cc - 1],
                                        a.beta[cc], a.P);
                 acc += Ld::get(lu + o) * t.d_w;
-                // cross terms from v facets (i,j) [ubl], (i,j-1) [ubr], (i+1,j) [utl], (i+1,j-1) [utr]
-                if (S::kDrag)
-                    acc += s.Pv(2, vi, cj) + s.Pv(3, vi, cj - 1) + s.Pv(0, vi + 1, cj) + s.Pv(1, vi + 1, cj - 1);
                 Flux<T> f = flux_x(u[o], H[cc - 1], H[cc], true);
                 acc += f.d_w * (s.lHm(ci, cj - 1) - s.lHm(ci, cj)) * dxi;
                 if (fu) acc -= fu[o];
@@ -1147,9 +1095,6 @@ __device__ __forceinline__ void vjp_body(const SsaArgs<T>& a, const T* __restric
                 T pt = a.phi[o - nx], pc = a.phi[o];
                 Drag<T> t = basal_drag(v[o], u[utl], u[utl + 1], u[ul], u[ul + 1], pt, pc, a.beta[o - nx], a.beta[o], a.P);
                 acc += Ld::get(lv + o) * t.d_w;
-                // cross terms from u facets (i,j) [vtr], (i,j+1) [vtl], (i-1,j) [vbr], (i-1,j+1) [vbl]
-                if (S::kDrag)
-                    acc += s.Pu(1, vi + 1, vj) + s.Pu(0, vi + 1, vj + 1) + s.Pu(3, vi, vj) + s.Pu(2, vi, vj + 1);
                 Flux<T> f = flux_y(v[o], H[o - nx], H[o], true);
                 acc += f.d_w * (s.lHm(ci, cj) - s.lHm(ci - 1, cj)) * dxi;
                 if (fv) acc -= fv[o];
@@ -1219,28 +1164,10 @@ __device__ __forceinline__ void vjp_body(const SsaArgs<T>& a, const T* __restric
     }
 }
 
-// Block storage of the transpose operator: a static tile of k_vjp, and a
-// whole level carved from dynamic LDS (linear drag only).
-template <typename T, int ROWS>
-struct VjpTileStore {
-    static constexpr bool kDrag = true;
-    VjpTile<T, ROWS>& t;
-    __device__ T& lHm(int r, int c) { return t.lHm[r][c]; }
-    __device__ T& eta(int r, int c) { return t.eta[r][c]; }
-    __device__ T& etad(int r, int c) { return t.etad[r][c]; }
-    __device__ T& Hs(int r, int c) { return t.Hs[r][c]; }
-    __device__ T& Lxx(int r, int c) { return t.Lxx[r][c]; }
-    __device__ T& Lyy(int r, int c) { return t.Lyy[r][c]; }
-    __device__ T& Kxx(int r, int c) { return t.Kxx[r][c]; }
-    __device__ T& Kyy(int r, int c) { return t.Kyy[r][c]; }
-    __device__ T& Lxy(int r, int c) { return t.Lxy[r][c]; }
-    __device__ T& Gxy(int r, int c) { return t.Gxy[r][c]; }
-    __device__ T& Pu(int q, int r, int c) { return t.Pu[q][r][c]; }
-    __device__ T& Pv(int q, int r, int c) { return t.Pv[q][r][c]; }
-};
+// Block storage of the transpose operator: a tile or a whole level carved
+// from one LDS array.
 template <typename T>
 struct VjpLevelStore {
-    static constexpr bool kDrag = false;
     T* cell;  // 8 arrays of (rows + 2) x (cols + 2)
     T* vert;  // 2 arrays of (rows + 1) x (cols + 1)
     int cw, nc, vw, nv;
@@ -1254,8 +1181,6 @@ struct VjpLevelStore {
     __device__ T& Kyy(int r, int c) { return cell[7 * nc + r * cw + c]; }
     __device__ T& Lxy(int r, int c) { return vert[r * vw + c]; }
     __device__ T& Gxy(int r, int c) { return vert[nv + r * vw + c]; }
-    __device__ T& Pu(int, int, int) { return cell[0]; }  // never used without kDrag
-    __device__ T& Pv(int, int, int) { return cell[0]; }
 };
 
 // Output sinks of vjp_body: arrays in the grid's own layouts, or tile-local
@@ -1277,54 +1202,20 @@ struct VjpTileOut {
     __device__ void put_h(int ti, int tj, long, T x) { h[ti][tj] = x; }
 };
 
-template <typename T, int ROWS>
-__global__ __launch_bounds__(TX * ROWS) void k_vjp(SsaArgs<T> a, const T* __restrict__ lu, const T* __restrict__ lv,
-                                            const T* __restrict__ lH, const T* __restrict__ fu,
-                                            const T* __restrict__ fv, const T* __restrict__ fH, T* __restrict__ out_u,
-                                            T* __restrict__ out_v, T* __restrict__ out_H, T calving_rate,
-                                            const T* __restrict__ eta_cache) {
-    __shared__ VjpTile<T, ROWS> t;
-    VjpTileStore<T, ROWS> s{t};
-    VjpGridOut<T> o{out_u, out_v, out_H};
-    vjp_body(a, lu, lv, lH, fu, fv, fH, o, calving_rate, eta_cache, (int)blockIdx.y * ROWS, (int)blockIdx.x * TX,
-             ROWS, TX, (int)(threadIdx.y * TX + threadIdx.x), TX * ROWS, s);
-}
-
-// A whole cached adjoint pass in one launch (linear drag): the transpose
-// operator minus the forcing for the facets and cells of the tile and of its
-// left column and top row (vjp_body over rows i0 - 1 .. i0 + TY and columns
-// j0 - 1 .. j0 + TX, into LDS), the cached patch solves of the tile's cells
-// and of the cells left of and above it, then the in-place update of
-// k_vanka_adjoint_fused, written to the other of two multiplier buffers:
-// the transpose operator reads the multipliers of neighbouring tiles, which
-// their blocks update during the same pass.  The same arithmetic as k_vjp
-// followed by k_vanka_adjoint_fused; it recomputes the ring's residuals (1.4x the
-// transpose operator's work) and saves a launch, the residual planes' round
-// trip through HBM and the second kernel's ramp: 9.7 against 12.6 us per
-// pass at 32², 14.6 against 19.8 us at 256², and still ahead at 512².
-// The one-launch adjoint pass uses TY-row tiles (2 TY thread rows, so that the
-// ring's patch solves run beside the tile's).  Each tile recomputes the
-// transpose operator on its top row and left column, (TY + 2) / TY of the
-// work; 8-row tiles (1024 threads, 88 KB of LDS) measured 35.2 against
-// 38.6 us per pass at 512² alone, but the coupled step, whose enthalpy
-// kernels share the GPU with these passes, ran 0.75 ms slower with them.
-
-// One adjoint pass over the TR x TX tile at (i0, j0) with TX x 2 TR threads:
-// k_vjp's body over the tile plus its left column and top row (into LDS), the
+// One cached adjoint pass over the TR x TX tile at (i0, j0) with TX x 2 TR
+// threads (linear drag), for k_adjoint_persistent: the transpose operator minus
+// the forcing over the tile plus its left column and top row (into LDS), the
 // cached patch solves of the tile (thread rows < TR) and of the ring (the
 // other threads), then the update of the tile's multipliers into the
-// destination buffers.
-// MC: one colour phase of the multicolour adjoint pass instead: only cells
-// with (i + j) % 2 == colour solve, and each unknown receives its (single)
-// solving cell's full increment times omega.
-template <typename T, class Ld, int TR, bool MC = false>
+// destination buffers (neighbouring tiles read the old ones in the same pass).
+template <typename T, class Ld, int TR>
 __device__ __forceinline__ void adjoint_pass_tile(const SsaArgs<T>& a, const T* __restrict__ cache,
                                                   const T* __restrict__ lu, const T* __restrict__ lv,
                                                   const T* __restrict__ lH, T* __restrict__ lu_dst,
                                                   T* __restrict__ lv_dst, T* __restrict__ lH_dst,
                                                   const T* __restrict__ fu, const T* __restrict__ fv,
                                                   const T* __restrict__ fH, T calving_rate, T omega, int i0, int j0,
-                                                  int ty, int tx, int colour = -1) {
+                                                  int ty, int tx) {
     constexpr int RR = TR + 2, RC = TX + 2;
     constexpr int CW = RC + 2, NCELL = (RR + 2) * CW, VW = RC + 1, NVERT = (RR + 1) * VW;
     __shared__ T s_cell[8 * NCELL];
@@ -1349,20 +1240,9 @@ __device__ __forceinline__ void adjoint_pass_tile(const SsaArgs<T>& a, const T* 
                                                           tid, NTF, store);
     __syncthreads();
     auto increments = [&](int ci, int cj, T w[5]) {
-        if constexpr (MC) {
-            if (((ci + cj) & 1) != colour) {
-#pragma unroll
-                for (int q = 0; q < 5; ++q) w[q] = T(0);
-                return;
-            }
-        }
         const int ti = ci - i0 + 1, tj = cj - j0 + 1;
         const T b[5] = {r_u[ti][tj], r_u[ti][tj + 1], r_v[ti][tj], r_v[ti + 1][tj], r_h[ti][tj]};
         adjoint_cached_solve(cache, n, (long)ci * nx + cj, b, w);
-        if constexpr (MC) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) w[q] = T(2) * w[q];  // full facet weight
-        }
     };
     // thread rows 0 .. TR-1 own the tile's cells, the rest solve the ring
     const int i = i0 + ty, j = j0 + tx;
@@ -1414,24 +1294,8 @@ __device__ __forceinline__ void adjoint_pass_tile(const SsaArgs<T>& a, const T* 
     lH_dst[c] = Ld::get(lH + c) + omega * w[4];
 }
 
-template <typename T, int TR, bool MC = false>
-__global__ __launch_bounds__(TX * 2 * TR) void k_adjoint_pass_fused(SsaArgs<T> a, const T* __restrict__ cache,
-                                                                           const T* __restrict__ lu,
-                                                                           const T* __restrict__ lv,
-                                                                           const T* __restrict__ lH,
-                                                                           T* __restrict__ lu_dst,
-                                                                           T* __restrict__ lv_dst,
-                                                                           T* __restrict__ lH_dst,
-                                                                           const T* __restrict__ fu,
-                                                                           const T* __restrict__ fv,
-                                                                           const T* __restrict__ fH, T calving_rate,
-                                                                           T omega, int colour) {
-    adjoint_pass_tile<T, LdPlain, TR, MC>(a, cache, lu, lv, lH, lu_dst, lv_dst, lH_dst, fu, fv, fH, calving_rate,
-                                          omega, blockIdx.y * TR, blockIdx.x * TX, threadIdx.y, threadIdx.x, colour);
-}
-
 // n_iter adjoint passes of a level at most TX cells wide in one launch
-// (bitwise what n_iter k_adjoint_pass_fused launches give): working workgroup
+// (what n_iter one-launch passes give, to rounding): working workgroup
 // b runs the pass of tile row b; pass p reads the multipliers from lu/lv/lH
 // (p even) or the alternate buffers (p odd) and writes the other set, with the
 // barriers and the one-XCD placement of k_vanka_persistent.  If a barrier
@@ -1747,51 +1611,6 @@ hipError_t launch_vanka_adjoint_pass(const SsaArgs<T>& a, const T* ru, const T* 
     return hipGetLastError();
 }
 
-template <typename T>
-hipError_t launch_vjp(const SsaArgs<T>& a, const T* lu, const T* lv, const T* lH, const T* fu, const T* fv,
-                      const T* fH, T* ou, T* ov, T* oH, T calving_rate, const T* eta_cache, hipStream_t st) {
-    TimedLaunch tl(kTimeVjp, (long)a.ny * a.nx, st);
-    constexpr int R = kVjpRows;
-    const dim3 g((a.nx + 1 + TX - 1) / TX, (a.ny + 1 + R - 1) / R);
-    k_vjp<T, R><<<g, dim3(TX, R), 0, st>>>(a, lu, lv, lH, fu, fv, fH, ou, ov, oH, calving_rate, eta_cache);
-    return hipGetLastError();
-}
-
-template <typename T>
-hipError_t launch_adjoint_pass_fused(const SsaArgs<T>& a, const T* cache, const T* lu, const T* lv, const T* lH,
-                                     T* lu_dst, T* lv_dst, T* lH_dst, const T* fu, const T* fv, const T* fH,
-                                     T calving_rate, T omega, hipStream_t st) {
-    if (!a.P.linear_drag) return hipErrorInvalidValue;
-    TimedLaunch tl(kTimeAdjointCell, (long)a.ny * a.nx, st);
-    k_adjoint_pass_fused<T, TY><<<tile_grid(a.ny, a.nx, false), dim3(TX, 2 * TY), 0, st>>>(
-        a, cache, lu, lv, lH, lu_dst, lv_dst, lH_dst, fu, fv, fH, calving_rate, -omega, -1);
-    return hipGetLastError();
-}
-
-// Tile rows of the multicolour adjoint phase: TY, or GLIDE_MC_ADJ_ROWS32 rows
-// in FP32 (the FP64 tile keeps TY rows, whose LDS would double).  8 rows
-// halve the ring's share of the transpose operator but measured no faster:
-// 25.4 against 26.8 us per phase at 512², 75.3 against 73.5 ms per batched
-// 96-domain ensemble step.
-#ifndef GLIDE_MC_ADJ_ROWS32
-#define GLIDE_MC_ADJ_ROWS32 4
-#endif
-template <typename T>
-constexpr int mc_adj_rows() { return std::is_same<T, float>::value ? GLIDE_MC_ADJ_ROWS32 : TY; }
-int tab_adj_pass_rows(bool fp32) { return fp32 ? mc_adj_rows<float>() : mc_adj_rows<double>(); }
-
-template <typename T>
-hipError_t launch_adjoint_pass_mc(const SsaArgs<T>& a, const T* cache, const T* lu, const T* lv, const T* lH,
-                                  T* lu_dst, T* lv_dst, T* lH_dst, const T* fu, const T* fv, const T* fH,
-                                  T calving_rate, T omega, int colour, hipStream_t st) {
-    if (!a.P.linear_drag) return hipErrorInvalidValue;
-    TimedLaunch tl(std::is_same<T, float>::value ? kTimeAdjointMc32 : kTimeAdjointMc64, (long)a.ny * a.nx, st);
-    constexpr int R = mc_adj_rows<T>();
-    const dim3 g((a.nx + TX - 1) / TX, (a.ny + R - 1) / R);
-    k_adjoint_pass_fused<T, R, true><<<g, dim3(TX, 2 * R), 0, st>>>(a, cache, lu, lv, lH, lu_dst, lv_dst, lH_dst, fu,
-                                                                   fv, fH, calving_rate, -omega, colour & 1);
-    return hipGetLastError();
-}
 bool adjoint_persistent_fits(int ny, int nx) {
     // the three sync words sit behind the alternating multipliers in the 5 ny nx workspace
     return nx >= 1 && nx <= TX && ny >= 1 && (ny + TY - 1) / TY <= kAdjointPersistentMaxBlocks &&
@@ -1834,9 +1653,9 @@ hipError_t launch_adjoint_coarse(const SsaArgs<T>& a, const T* cache, T* lu, T* 
 }
 
 template <typename T>
-hipError_t launch_adjoint_factor(const SsaArgs<T>& a, T* cache, const VankaArgs<T>& vk, hipStream_t st) {
+hipError_t launch_adjoint_factor(const SsaArgs<T>& a, T* cache, const VankaArgs<T>& vk, bool split, hipStream_t st) {
     TimedLaunch tl(kTimeAdjointFactor, (long)a.ny * a.nx, st);
-    k_adjoint_factor<T><<<tile_grid(a.ny, a.nx, false), dim3(TX, TY), 0, st>>>(a, cache, vk);
+    k_adjoint_factor<T><<<tile_grid(a.ny, a.nx, false), dim3(TX, TY), 0, st>>>(a, cache, vk, split);
     return hipGetLastError();
 }
 
@@ -1944,33 +1763,7 @@ __global__ __launch_bounds__(NT) void k_tab_adj_factor(const TabAdjFactor<T>* __
     const int e = tab_find(start, n, blockIdx.x);
     const TabAdjFactor<T> J = jobs[e];
     const int lb = blockIdx.x - start[e];
-    adjoint_factor_body<T>(lb % J.gx, lb / J.gx, J.a, J.cache, J.vk);
-}
-
-template <typename T, int TR>
-__global__ __launch_bounds__(TX * 2 * TR) void k_tab_adj_pass(const TabAdjPass<T>* __restrict__ jobs,
-                                                              const int* __restrict__ start, int n, int colour) {
-    const int e = tab_find(start, n, blockIdx.x);
-    const TabAdjPass<T> J = jobs[e];
-    const int lb = blockIdx.x - start[e];
-    const int bx = lb % J.gx, by = lb / J.gx;
-    adjoint_pass_tile<T, LdPlain, TR, true>(J.a, J.cache, J.lu, J.lv, J.lH, J.lu_dst, J.lv_dst, J.lH_dst, J.fu, J.fv,
-                                            J.fH, J.cr, J.omega, by * TR, bx * TX, threadIdx.y, threadIdx.x, colour);
-}
-
-template <typename T>
-__global__ __launch_bounds__(TX * kVjpRows) void k_tab_vjp(const TabVjp<T>* __restrict__ jobs,
-                                                           const int* __restrict__ start, int n) {
-    constexpr int ROWS = kVjpRows;
-    __shared__ VjpTile<T, ROWS> t;
-    const int e = tab_find(start, n, blockIdx.x);
-    const TabVjp<T> J = jobs[e];
-    const int lb = blockIdx.x - start[e];
-    const int bx = lb % J.gx, by = lb / J.gx;
-    VjpTileStore<T, ROWS> s{t};
-    VjpGridOut<T> o{J.ou, J.ov, J.oH};
-    vjp_body(J.a, J.lu, J.lv, J.lH, J.fu, J.fv, J.fH, o, J.cr, J.eta_cache, by * ROWS, bx * TX, ROWS, TX,
-             (int)(threadIdx.y * TX + threadIdx.x), TX * ROWS, s);
+    adjoint_factor_body<T>(lb % J.gx, lb / J.gx, J.a, J.cache, J.vk, true);
 }
 
 template <typename T>
@@ -1992,14 +1785,6 @@ int tab_blocks_adj_factor(int ny, int nx, int* gx) {
     *gx = (int)g.x;
     return (int)(g.x * g.y);
 }
-int tab_blocks_adj_pass(int ny, int nx, int rows, int* gx) {
-    *gx = (nx + TX - 1) / TX;
-    return *gx * ((ny + rows - 1) / rows);
-}
-int tab_blocks_vjp(int ny, int nx, int* gx) {
-    *gx = (nx + 1 + TX - 1) / TX;
-    return *gx * ((ny + 1 + kVjpRows - 1) / kVjpRows);
-}
 int tab_blocks_grad(int ny, int nx, int* gx) {
     *gx = (nx + 255) / 256;
     return *gx * ny;
@@ -2018,20 +1803,6 @@ hipError_t launch_tab_adj_factor(const TabAdjFactor<T>* jobs, const int* start, 
     return hipGetLastError();
 }
 template <typename T>
-hipError_t launch_tab_adj_pass(const TabAdjPass<T>* jobs, const int* start, int n, int blocks, int colour,
-                               hipStream_t st) {
-    if (n <= 0 || blocks <= 0) return hipSuccess;
-    constexpr int R = mc_adj_rows<T>();
-    k_tab_adj_pass<T, R><<<blocks, dim3(TX, 2 * R), 0, st>>>(jobs, start, n, colour & 1);
-    return hipGetLastError();
-}
-template <typename T>
-hipError_t launch_tab_vjp(const TabVjp<T>* jobs, const int* start, int n, int blocks, hipStream_t st) {
-    if (n <= 0 || blocks <= 0) return hipSuccess;
-    k_tab_vjp<T><<<blocks, dim3(TX, kVjpRows), 0, st>>>(jobs, start, n);
-    return hipGetLastError();
-}
-template <typename T>
 hipError_t launch_tab_grad(const TabGrad<T>* jobs, const int* start, int n, int blocks, hipStream_t st) {
     if (n <= 0 || blocks <= 0) return hipSuccess;
     k_tab_grad<T><<<blocks, 256, 0, st>>>(jobs, start, n);
@@ -2041,8 +1812,6 @@ hipError_t launch_tab_grad(const TabGrad<T>* jobs, const int* start, int n, int 
 #define GLIDE_TAB_INSTANTIATE(T)                                                                                     \
     template hipError_t launch_tab_residual<T>(const TabResidual<T>*, const int*, int, int, hipStream_t);            \
     template hipError_t launch_tab_adj_factor<T>(const TabAdjFactor<T>*, const int*, int, int, hipStream_t);         \
-    template hipError_t launch_tab_adj_pass<T>(const TabAdjPass<T>*, const int*, int, int, int, hipStream_t);        \
-    template hipError_t launch_tab_vjp<T>(const TabVjp<T>*, const int*, int, int, hipStream_t);                      \
     template hipError_t launch_tab_grad<T>(const TabGrad<T>*, const int*, int, int, hipStream_t);
 
 GLIDE_TAB_INSTANTIATE(double)
@@ -2061,19 +1830,13 @@ GLIDE_TAB_INSTANTIATE(float)
                                                   const PersistentCtl&, hipStream_t);                             \
     template hipError_t launch_vanka_adjoint_pass<T>(const SsaArgs<T>&, const T*, const T*, const T*, T*, T*, T*, T*, \
                                                      const VankaArgs<T>&, T, hipStream_t);                           \
-    template hipError_t launch_adjoint_pass_fused<T>(const SsaArgs<T>&, const T*, const T*, const T*, const T*, T*,   \
-                                                     T*, T*, const T*, const T*, const T*, T, T, hipStream_t);       \
-    template hipError_t launch_adjoint_pass_mc<T>(const SsaArgs<T>&, const T*, const T*, const T*, const T*, T*, T*, \
-                                                  T*, const T*, const T*, const T*, T, T, int, hipStream_t);         \
     template bool adjoint_coarse_fits<T>(const SsaArgs<T>&);                                                         \
     template hipError_t launch_adjoint_persistent<T>(const SsaArgs<T>&, const T*, T*, T*, T*, T*, T*, T*, const T*,  \
                                                      const T*, const T*, T, T, int, const PersistentCtl&,            \
                                                      hipStream_t);                                                    \
     template hipError_t launch_adjoint_coarse<T>(const SsaArgs<T>&, const T*, T*, T*, T*, const T*, const T*,          \
                                                  const T*, T, T, int, hipStream_t);                                  \
-    template hipError_t launch_vjp<T>(const SsaArgs<T>&, const T*, const T*, const T*, const T*, const T*, const T*, \
-                                      T*, T*, T*, T, const T*, hipStream_t);                                         \
-    template hipError_t launch_adjoint_factor<T>(const SsaArgs<T>&, T*, const VankaArgs<T>&, hipStream_t);          \
+    template hipError_t launch_adjoint_factor<T>(const SsaArgs<T>&, T*, const VankaArgs<T>&, bool, hipStream_t);          \
     template hipError_t launch_vanka_adjoint_pass_cached<T>(int, int, const T*, const T*, const T*, const T*, T*, T*, \
                                                             T*, T*, T, bool, hipStream_t);                           \
     template hipError_t launch_grad_beta_bed<T>(const SsaArgs<T>&, const T*, const T*, T*, T*, int, hipStream_t); \

@@ -189,7 +189,7 @@ hipError_t launch_vjp(const SsaArgs<T>& a, const T* lu, const T* lv, const T* lH
 constexpr int kAdjointCacheValues = 26;
 constexpr int kAdjointCacheEta = 25;  // plane of the cell viscosity
 template <typename T>
-hipError_t launch_adjoint_factor(const SsaArgs<T>& a, T* cache, const VankaArgs<T>& vk, hipStream_t st);
+hipError_t launch_adjoint_factor(const SsaArgs<T>& a, T* cache, const VankaArgs<T>& vk, bool split, hipStream_t st);
 // fused: one launch (patch solves of the tile and its left/top neighbours,
 // then the in-place multiplier update); otherwise solve into work + apply.
 template <typename T>
