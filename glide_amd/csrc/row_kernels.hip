@@ -12,9 +12,15 @@
 // k_vjp_rows: the transpose operator alone.
 //
 // Workgroup height: a workgroup of NW wavefronts gives NW - 2 rows (MC), so 8
-// wavefronts redo 1.33 rows of the cell work per row and 16 redo 1.14.  Small
-// levels are bound by the length of one wavefront's chain and take 8 (more
-// workgroups, fewer wavefronts at each barrier).
+// wavefronts do the cell work of 1.33 rows per row and 16 of 1.14; 16 measured
+// slower all the same (FP32 phase at 512 x 512 12.1 against 10.4 us, at the
+// finest levels of 48 domains of 48 to 384 cells a side 69 against 62 us): a
+// barrier then holds up twice the wavefronts.  Against the tile kernels (4 x 64
+// cells, 512 threads, bound by VALU issue) the FP32 phase at 512 x 512 went from
+// 24.8 to 10.4 us (33.0 MB of state, multipliers and the colour's factors: 3.2
+// TB/s), the 48 domains' finest level from 232 to 62 us (3.8 TB/s, of 4.9 TB/s
+// a large copy reaches: bound by memory), the FP64 transpose operator at 1536 x
+// 2048 from 268 to 104 us (4.3 TB/s).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -198,12 +204,7 @@ __global__ __launch_bounds__(kRowLanes* kVjpWaves) void k_tab_vjp(const TabVjp<T
                        J.eta_cache);
 }
 
-// Wavefronts of a workgroup of the red-black adjoint phase.
-#ifndef GLIDE_ADJ_WAVES32
-#define GLIDE_ADJ_WAVES32 8
-#endif
-template <typename T>
-constexpr int adj_waves() { return std::is_same<T, float>::value ? GLIDE_ADJ_WAVES32 : 8; }
+constexpr int kAdjWaves = 8;
 
 template <typename T, int NW, bool MC>
 dim3 adjoint_grid(int ny, int nx) {
@@ -219,7 +220,7 @@ hipError_t launch_adjoint_pass_fused(const SsaArgs<T>& a, const T* cache, const 
                                      T calving_rate, T omega, hipStream_t st) {
     if (!a.P.linear_drag) return hipErrorInvalidValue;
     TimedLaunch tl(kTimeAdjointCell, (long)a.ny * a.nx, st);
-    k_adjoint_rows<T, 8, false><<<adjoint_grid<T, 8, false>(a.ny, a.nx), dim3(kRowLanes, 8), 0, st>>>(
+    k_adjoint_rows<T, kAdjWaves, false><<<adjoint_grid<T, kAdjWaves, false>(a.ny, a.nx), dim3(kRowLanes, kAdjWaves), 0, st>>>(
         a, cache, lu, lv, lH, lu_dst, lv_dst, lH_dst, fu, fv, fH, calving_rate, -omega, -1);
     return hipGetLastError();
 }
@@ -230,8 +231,7 @@ hipError_t launch_adjoint_pass_mc(const SsaArgs<T>& a, const T* cache, const T* 
                                   T calving_rate, T omega, int colour, hipStream_t st) {
     if (!a.P.linear_drag) return hipErrorInvalidValue;
     TimedLaunch tl(std::is_same<T, float>::value ? kTimeAdjointMc32 : kTimeAdjointMc64, (long)a.ny * a.nx, st);
-    constexpr int NW = adj_waves<T>();
-    k_adjoint_rows<T, NW, true><<<adjoint_grid<T, NW, true>(a.ny, a.nx), dim3(kRowLanes, NW), 0, st>>>(
+    k_adjoint_rows<T, kAdjWaves, true><<<adjoint_grid<T, kAdjWaves, true>(a.ny, a.nx), dim3(kRowLanes, kAdjWaves), 0, st>>>(
         a, cache, lu, lv, lH, lu_dst, lv_dst, lH_dst, fu, fv, fH, calving_rate, -omega, colour & 1);
     return hipGetLastError();
 }
@@ -250,8 +250,8 @@ hipError_t launch_vjp(const SsaArgs<T>& a, const T* lu, const T* lv, const T* lH
 
 // ------------------------------------------------------------ domain tables
 int tab_blocks_adj_pass(int ny, int nx, bool fp32, int* gx) {
-    const dim3 g = fp32 ? adjoint_grid<float, adj_waves<float>(), true>(ny, nx)
-                        : adjoint_grid<double, adj_waves<double>(), true>(ny, nx);
+    const dim3 g = fp32 ? adjoint_grid<float, kAdjWaves, true>(ny, nx)
+                        : adjoint_grid<double, kAdjWaves, true>(ny, nx);
     *gx = (int)g.x;
     return (int)(g.x * g.y);
 }
@@ -264,8 +264,7 @@ template <typename T>
 hipError_t launch_tab_adj_pass(const TabAdjPass<T>* jobs, const int* start, int n, int blocks, int colour,
                                hipStream_t st) {
     if (n <= 0 || blocks <= 0) return hipSuccess;
-    constexpr int NW = adj_waves<T>();
-    k_tab_adj_pass<T, NW><<<blocks, dim3(kRowLanes, NW), 0, st>>>(jobs, start, n, colour & 1);
+    k_tab_adj_pass<T, kAdjWaves><<<blocks, dim3(kRowLanes, kAdjWaves), 0, st>>>(jobs, start, n, colour & 1);
     return hipGetLastError();
 }
 template <typename T>
