@@ -81,16 +81,14 @@ VERIFY_ROUNDS = 4  # timed runs at most, each tightening the stages whose quanti
 
 # Algorithmic bytes of one launch per cell of its level, in values of the
 # launch's precision (each plane counted once):
-#   red-black colour phase: reads u, v, H, the frozen viscosity, phi, beta,
-#     bed, f_u, f_v (every cell), f_H, gamma and the active-set flag (the
-#     solving half); writes u, v, H (every cell) and the flag (the solving
-#     half): 10.5 + 3.5
+#   red-black pass: reads u, v, H, phi, beta, bed, B, f_u, f_v, f_H and gamma;
+#     writes u, v, H and the active-set flag: 11 + 4
 #   red-black adjoint colour phase: the transpose operator reads the three
 #     multiplier planes, the three right-hand sides, the cached viscosity and
 #     u, v, H, phi, beta, bed and the flag; the solving half reads its 25 LU
 #     values; writes the three multiplier planes: 16 + 12.5 + 3
 #   FP64 residual: 12 inputs + 3 outputs
-ALG_VALUES = {"vanka_mc32": 14.0, "vanka_mc64": 14.0, "adjoint_mc32": 31.5, "adjoint_mc64": 31.5,
+ALG_VALUES = {"vanka_mc32": 15.0, "vanka_mc64": 15.0, "adjoint_mc32": 31.5, "adjoint_mc64": 31.5,
               "residual": 15.0, "vjp": 18.0}
 # bytes per value; at the finest level the transpose operator runs in FP64
 # (the mixed adjoint's Krylov products and residuals)

@@ -2,27 +2,28 @@
 // of the mixed-precision solver (no counterpart in the reference, whose Vanka
 // pass is additive: glide/cuda/vanka.cu:477-660).
 //
-// A pass is three launches: the cell viscosity of the state the pass starts
-// from (frozen for the pass, as in the reference), then the red cells
-// ((i + j) even) and the black cells.  A colour phase reads the state from one
-// buffer set and writes the complete new state to the other: each facet
-// belongs to exactly one cell of a colour, which writes it; the cells of the
-// other colour copy their thickness and the domain-edge facets nobody of the
-// colour owns.  Cells of one colour read each other's old values, so a phase
-// is a block-Jacobi step over non-overlapping patches and its result does not
-// depend on scheduling (run-to-run bitwise identical).
+// A pass takes the cell viscosity of the state it starts from (frozen for the
+// pass, as in the reference), solves the red cells ((i + j) even) and then the
+// black ones; each facet belongs to exactly one cell of a colour.  Cells of one
+// colour read each other's old values, so a colour is a block-Jacobi step over
+// non-overlapping patches and the result does not depend on scheduling
+// (run-to-run bitwise identical).
 //
-// Work mapping: a lane owns one cell of the active colour and the inactive
-// cell beside it in the same row, so a wavefront covers 128 columns and no
-// lane idles on the other colour; the active cells' loads are stride-2 and the
-// other colour's phase reads the other half of the same lines.  The local
+// k_mc_pass: the whole pass in one launch, from one buffer set into another.
+// A workgroup updates 58 columns and 2 NW - 2 rows (NW wavefronts).  It loads
+// the state three cells around them into LDS, one wavefront per row, and forms
+// the viscosity; then a half wavefront owns a row and a lane a cell pair: it
+// solves the red cells of the tile and of a ring of one cell around it (what a
+// black cell reads of another cell was written by the red cells beside it, or
+// is old), puts them back into LDS, and solves the black cells.  The local
 // Newton iteration runs the folded cell system of the additive smoother
-// (cell_system, refined hardware reciprocals), without compensated updates
-// and with the caller's relaxation and stopping threshold.
+// (cell_system, refined hardware reciprocals), without compensated updates and
+// with the caller's relaxation and stopping threshold.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
 
+#include "row_ops.hpp"
 #include "ssa_device.hpp"
 #include "ssa_kernels.hpp"
 #include "tab.hpp"
@@ -31,50 +32,122 @@ namespace glide {
 
 namespace {
 
-constexpr int kMcLanes = 64;  // cell pairs per wavefront row segment
-constexpr int kMcRows = 4;    // rows per block
+constexpr int kMcCols = kRowLanes - 6;  // columns a workgroup updates
 
-// Kernel bodies take their block index (bx, by) as arguments, so that the
-// domain-table launches (one launch over many domains) run them unchanged.
+// rows rr = 0 .. kF - 1 of u and v are the tile's rows -3 .. kRows + 2, rows
+// 0 .. kC - 1 of the cell planes its rows -2 .. kRows + 1; column l is the
+// tile's column l - 3.
+template <typename T, int NW>
+struct McLds {
+    static constexpr int kRows = 2 * NW - 2, kF = kRows + 6, kC = kRows + 4;
+    T u[kF][kRowLanes], v[kF][kRowLanes];
+    T H[kC][kRowLanes], eH[kC][kRowLanes], eta[kC][kRowLanes];
+    T S[kC][kRowLanes], bp[kC][kRowLanes], phi[kC][kRowLanes];  // flotation surface, beta * phi
+};
+
+// What a cell's solve reads of its own cell only.
 template <typename T>
-__device__ __forceinline__ void cell_eta_body(int bx, int by, const SsaArgs<T>& a, T* __restrict__ eta) {
-    const int j = bx * 256 + threadIdx.x, i = by;
-    if (j >= a.nx) return;
-    CellVel<T> c = load_cell_vel<T>(a.u, a.v, i, j, a.ny, a.nx);
-    const T e2 = strain_invariant(c, i, j, a.ny, a.nx, a.dxi, a.P.eps_reg);
-    eta[(long)i * a.nx + j] = T(0.5) * a.B[(long)i * a.nx + j] * glen_power(e2, a.P);
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_cell_eta(SsaArgs<T> a, T* __restrict__ eta) {
-    cell_eta_body<T>(blockIdx.x, blockIdx.y, a, eta);
-}
-
-// Local Newton iteration of cell (i, j) against the state in a; returns the
-// new unknowns x and the active-set flag.  EDGE: the cell may lie on the
-// domain edge (the Dirichlet pins are tested).
-template <typename T, bool LINEAR, bool EDGE>
-__device__ __forceinline__ void mc_newton(const SsaArgs<T>& a, const T* __restrict__ eta, int i, int j,
-                                          const VankaArgs<T>& vk, T x[5], T& masked) {
-    const int ny = a.ny, nx = a.nx;
-    CellSys<T> cs;
-    T thk;
-    {
-        Patch<T> p;
-        load_patch_with<T>(p, a, [&](int di, int dj) { return eta[offC(i + di, j + dj, ny, nx)]; }, i, j, a.f_u, a.f_v,
-                           a.f_H, a.phi);
-        make_cell_sys(cs, p, a.P, vk.calving_rate, a.dxi, a.dt, vk.ssa_damping, vk.mc_damping);
-        thk = p.gam;
+struct McCentre {
+    T f[5], bed, thk;
+    __device__ __forceinline__ void load(const SsaArgs<T>& a, int i, int j) {
+        const long c = (long)i * a.nx + j, ou = c + i;
+        if (a.f_u) {
+            f[0] = a.f_u[ou]; f[1] = a.f_u[ou + 1];
+            f[2] = a.f_v[c]; f[3] = a.f_v[c + a.nx];
+            f[4] = a.f_H[c];
+        } else {
+            f[0] = f[1] = f[2] = f[3] = f[4] = T(0);
+        }
+        bed = a.bed[c];
+        thk = a.gamma ? a.gamma[c] : T(0);
     }
-    const long c = (long)i * nx + j;
-    x[0] = a.u[(long)i * (nx + 1) + j];
-    x[1] = a.u[(long)i * (nx + 1) + j + 1];
-    x[2] = a.v[c];
-    x[3] = a.v[c + nx];
-    x[4] = a.H[c];
-    const bool pin0 = j == 0, pin1 = j == nx - 1, pin2 = i == 0, pin3 = i == ny - 1;
-    T rnorm = T(1e30);
-    for (int it = 0; it < vk.newton_steps && rnorm > vk.tol; ++it) {
+};
+
+// Local Newton iteration of the cell at LDS row rr, column c (grid cell (i, j))
+// against the state in LDS: the new unknowns x, the active-set flag, and the
+// cell's viscosity and surface coefficients.  EDGE: the cell may lie on the
+// domain edge (the Dirichlet pins are tested).
+template <typename T, int NW, bool LINEAR, bool EDGE>
+__device__ __forceinline__ void mc_newton(const McLds<T, NW>& s, const SsaArgs<T>& a, const McCentre<T>& q,
+                                          const VankaArgs<T>& vk, bool solves, int rr, int c, int i, int j, T x[5],
+                                          T& masked, T& e_c, T& Zc, T& gc) {
+    const int ny = a.ny, nx = a.nx, k = rr - 1;
+    const bool il = !EDGE || j > 0, ir = !EDGE || j + 1 < nx, it_ = !EDGE || i > 0, ib = !EDGE || i + 1 < ny;
+    const T D = a.dxi, D2 = D * D;
+    CellSys<T> cs;
+    {
+        const T e_l = s.eH[k][c - 1], e_r = s.eH[k][c + 1], e_t = s.eH[k - 1][c], e_b = s.eH[k + 1][c];
+        e_c = s.eta[k][c];
+        cs.D = D;
+        cs.hD = T(0.5) * D;
+        cs.H_l = s.H[k][c - 1]; cs.H_r = s.H[k][c + 1]; cs.H_t = s.H[k - 1][c]; cs.H_b = s.H[k + 1][c];
+        cs.dL = il ? D : T(0); cs.dR = ir ? D : T(0); cs.dT = it_ ? D : T(0); cs.dB = ib ? D : T(0);
+        const T p_c = s.phi[k][c];
+        T kcal = T(0);
+        if (vk.calving_rate != T(0))
+            kcal = (T(1) - p_c) * vk.calving_rate *
+                   ((T(1) - s.phi[k][c - 1]) + (T(1) - s.phi[k][c + 1]) + (T(1) - s.phi[k - 1][c]) +
+                    (T(1) - s.phi[k + 1][c]));
+        cs.r4h = T(1) / a.dt + kcal * D;
+        cs.j24c = cs.r4h + vk.mc_damping;
+        cs.f4 = q.f[4];
+        cs.kH = T(2) * e_c * D2;
+        const T qc = T(0.25) * e_c;
+        const bool vtl = it_ && il, vtr = it_ && ir, vbl = ib && il, vbr = ib && ir;
+        cs.C_tl = vtl ? T(0.25) * (s.eH[k - 1][c - 1] + e_t + e_l) : T(0);
+        cs.C_tr = vtr ? T(0.25) * (e_t + s.eH[k - 1][c + 1] + e_r) : T(0);
+        cs.C_bl = vbl ? T(0.25) * (e_l + s.eH[k + 1][c - 1] + e_b) : T(0);
+        cs.C_br = vbr ? T(0.25) * (e_r + e_b + s.eH[k + 1][c + 1]) : T(0);
+        cs.q_tl = vtl ? qc : T(0); cs.q_tr = vtr ? qc : T(0); cs.q_bl = vbl ? qc : T(0); cs.q_br = vbr ? qc : T(0);
+        cs.u_tl = s.u[rr - 1][c]; cs.u_tr = s.u[rr - 1][c + 1];
+        cs.u_bl = s.u[rr + 1][c]; cs.u_br = s.u[rr + 1][c + 1];
+        cs.v_lt = s.v[rr][c - 1]; cs.v_lb = s.v[rr + 1][c - 1];
+        cs.v_rt = s.v[rr][c + 1]; cs.v_rb = s.v[rr + 1][c + 1];
+        cs.s_tl = cs.hD * (cs.u_tl - cs.v_lt);
+        cs.s_tr = cs.hD * (cs.u_tr + cs.v_rt);
+        cs.s_bl = -cs.hD * (cs.u_bl + cs.v_lb);
+        cs.s_br = cs.hD * (cs.v_rb - cs.u_br);
+        const T nl = il ? T(2) * e_l * D2 : T(0), nr = ir ? T(2) * e_r * D2 : T(0);
+        const T nt = it_ ? T(2) * e_t * D2 : T(0), nb = ib ? T(2) * e_b * D2 : T(0);
+        cs.c0 = -nl * (cs.v_lt - cs.v_lb - T(2) * s.u[rr][c - 1]) - q.f[0];
+        cs.c1 = nr * (T(2) * s.u[rr][c + 2] + cs.v_rt - cs.v_rb) - q.f[1];
+        cs.c2 = nt * (cs.u_tr - cs.u_tl + T(2) * s.v[rr - 1][c]) - q.f[2];
+        cs.c3 = -nb * (cs.u_br - cs.u_bl - T(2) * s.v[rr + 2][c]) - q.f[3];
+        const T b_c = s.bp[k][c];
+        cs.be_l = T(0.5) * (s.bp[k][c - 1] + b_c);
+        cs.be_r = T(0.5) * (b_c + s.bp[k][c + 1]);
+        cs.be_t = T(0.5) * (s.bp[k - 1][c] + b_c);
+        cs.be_b = T(0.5) * (b_c + s.bp[k + 1][c]);
+        const T lin = LINEAR ? T(1) : T(0), wd = a.P.water_drag;
+        cs.o0 = -T(2) * nl - lin * (cs.be_l + wd);
+        cs.o1 = -T(2) * nr - lin * (cs.be_r + wd);
+        cs.o2 = -T(2) * nt - lin * (cs.be_t + wd);
+        cs.o3 = -T(2) * nb - lin * (cs.be_b + wd);
+        cs.a0 = cs.o0 - (cs.C_tl + cs.C_bl) * D2 - vk.ssa_damping;
+        cs.a1 = cs.o1 - (cs.C_tr + cs.C_br) * D2 - vk.ssa_damping;
+        cs.a2 = cs.o2 - (cs.C_tl + cs.C_tr) * D2 - vk.ssa_damping;
+        cs.a3 = cs.o3 - (cs.C_bl + cs.C_br) * D2 - vk.ssa_damping;
+        cs.h0 = -(cs.q_tl + cs.q_bl) * D2;
+        cs.h1 = -(cs.q_tr + cs.q_br) * D2;
+        cs.h2 = -(cs.q_tl + cs.q_tr) * D2;
+        cs.h3 = -(cs.q_bl + cs.q_br) * D2;
+        cs.eD = T(2) * e_c * D;
+        cs.S_l = s.S[k][c - 1]; cs.S_r = s.S[k][c + 1]; cs.S_t = s.S[k - 1][c]; cs.S_b = s.S[k + 1][c];
+        cs.Zc = Zc = p_c * q.bed;
+        cs.gc = gc = T(1) - (T(1) - p_c) * T(0.917);
+    }
+    const T thk = q.thk;
+    x[0] = s.u[rr][c];
+    x[1] = s.u[rr][c + 1];
+    x[2] = s.v[rr][c];
+    x[3] = s.v[rr + 1][c];
+    x[4] = s.H[k][c];
+    const bool pin0 = EDGE && j == 0, pin1 = EDGE && j == nx - 1, pin2 = EDGE && i == 0, pin3 = EDGE && i == ny - 1;
+    // every lane iterates as long as one of the wavefront does: a wavefront with
+    // few lanes left in its execution mask issues the same instructions at a
+    // third of the rate (12 steps at 12 x 59 cells: 61 us against 24 us)
+    bool go = solves && vk.newton_steps > 0 && T(1e30) > vk.tol;
+    for (int it = 1; __any(go); ++it) {
         T J[25], r[5];
         cell_system<T, T, LINEAR>(cs, cs, x, J, r, a.P);
         if constexpr (EDGE) {
@@ -83,66 +156,165 @@ __device__ __forceinline__ void mc_newton(const SsaArgs<T>& a, const T* __restri
             if (pin2) { pin_row(J, 2); r[2] = x[2]; }
             if (pin3) { pin_row(J, 3); r[3] = x[3]; }
         }
-        if ((x[4] - a.dt * r[4]) <= thk) {
-            masked = T(1);
+        const bool pin4 = (x[4] - a.dt * r[4]) <= thk;
+        if (pin4) {
             pin_row(J, 4);
             r[4] = x[4] - thk;
-        } else {
-            masked = T(0);
         }
         T d[5];
         lu5_solve_rcp(J, r, d);
-        rnorm = r[0] * r[0] + r[1] * r[1] + r[2] * r[2] + r[3] * r[3] + r[4] * r[4];
+        const T rnorm = r[0] * r[0] + r[1] * r[1] + r[2] * r[2] + r[3] * r[3] + r[4] * r[4];
 #pragma unroll
-        for (int k = 0; k < 5; ++k) x[k] -= vk.relax * d[k];
-        x[4] = fmax(x[4], thk);
+        for (int k2 = 0; k2 < 5; ++k2) {
+            const T y = x[k2] - vk.relax * d[k2];
+            x[k2] = go ? (k2 == 4 ? fmax(y, thk) : y) : x[k2];
+        }
+        masked = go ? (pin4 ? T(1) : T(0)) : masked;
+        go = go && it < vk.newton_steps && rnorm > vk.tol;
     }
 }
 
-// ROWS rows of cell pairs per block (kMcLanes pairs each); the arithmetic of
-// a cell does not depend on ROWS.
-template <typename T, bool LINEAR, int ROWS = kMcRows>
-__device__ __forceinline__ void vanka_mc_body(int bx, int by, const SsaArgs<T>& a, const T* __restrict__ eta,
-                                              T* __restrict__ u_dst, T* __restrict__ v_dst, T* __restrict__ H_dst,
-                                              T* __restrict__ mask, const VankaArgs<T>& vk, int colour) {
+template <typename T, int NW, bool LINEAR>
+__device__ __forceinline__ void mc_pass_body(int bx, int by, const SsaArgs<T>& a, T* __restrict__ u_dst,
+                                             T* __restrict__ v_dst, T* __restrict__ H_dst, T* __restrict__ mask,
+                                             T* __restrict__ phi_dst, const VankaArgs<T>& vk) {
+    using L = McLds<T, NW>;
+    __shared__ L s;
     const int ny = a.ny, nx = a.nx;
-    const int i = by * ROWS + threadIdx.y;
-    if (i >= ny) return;
-    const int pair = bx * kMcLanes + threadIdx.x;
-    const int p = (i + colour) & 1;
-    const int j = 2 * pair + p;        // the lane's cell of the active colour
-    const int jo = 2 * pair + 1 - p;   // and the other colour's cell beside it
-    if (j < nx) {
-        const long c = (long)i * nx + j;
-        T x[5], masked = mask[c];
-        // waves holding a row on the domain edge or the first / last column
-        // test the Dirichlet pins; the others run a loop copy without them
-        const bool edge = i == 0 || i == ny - 1 || bx == 0 || 2 * (bx + 1) * kMcLanes >= nx;
-        if (edge) mc_newton<T, LINEAR, true>(a, eta, i, j, vk, x, masked);
-        else mc_newton<T, LINEAR, false>(a, eta, i, j, vk, x, masked);
-        u_dst[(long)i * (nx + 1) + j] = x[0];
-        u_dst[(long)i * (nx + 1) + j + 1] = x[1];
-        v_dst[c] = x[2];
-        v_dst[c + nx] = x[3];
-        H_dst[c] = x[4];
-        mask[c] = masked;
+    const int lane = threadIdx.x, w = wave_row(threadIdx.y);
+    const int i0 = by * L::kRows, j0 = bx * kMcCols;
+
+    // this thread's cell of a colour: its tile row r (red: also the rows -1 and
+    // kRows of the ring) and column c; the last wavefront has no black row
+    auto place = [&](int colour, int& r, int& c) -> bool {
+        r = 2 * w + (lane >> 5) - 1 + colour;
+        const int i = i0 + r, lo = colour ? 0 : -1, hi = kMcCols - lo;
+        c = lo + 2 * (lane & 31) + ((i + lo + colour) & 1);  // j0 is even
+        return i >= 0 && i < ny && r < L::kRows - lo && c < hi && j0 + c >= 0 && j0 + c < nx;
+    };
+    int r, c;
+    bool solves = place(0, r, c);
+    McCentre<T> q{};
+    if (solves) q.load(a, i0 + r, j0 + c);
+
+    // the tile's rows, one wavefront each: state, surface, drag, viscosity; all
+    // loads are issued before the first is used
+    constexpr int kIt = (L::kF + NW - 1) / NW;
+    T u_[kIt], v_[kIt], H_[kIt], B_[kIt], z_[kIt], b_[kIt], p_[kIt];
+    const int j = j0 - 3 + lane, jc = clampi(j, 0, nx - 1), ju = clampi(j, 0, nx);
+#pragma unroll
+    for (int t = 0; t < kIt; ++t) {
+        const int ir = i0 - 3 + w + t * NW, ic = clampi(ir, 0, ny - 1);
+        const long rc = (long)ic * nx;
+        u_[t] = (a.u + rc + ic)[ju];
+        v_[t] = (a.v + (long)clampi(ir, 0, ny) * nx)[jc];
+        H_[t] = (a.H + rc)[jc];
+        B_[t] = (a.B + rc)[jc];
+        z_[t] = (a.bed + rc)[jc];
+        b_[t] = (a.beta + rc)[jc];
+        p_[t] = phi_dst ? T(0) : (a.phi + rc)[jc];
     }
-    if (jo < nx) {
-        const long c = (long)i * nx + jo;
-        H_dst[c] = a.H[c];
-        if (jo == 0) u_dst[(long)i * (nx + 1)] = a.u[(long)i * (nx + 1)];
-        if (jo == nx - 1) u_dst[(long)i * (nx + 1) + nx] = a.u[(long)i * (nx + 1) + nx];
-        if (i == 0) v_dst[jo] = a.v[jo];
-        if (i == ny - 1) v_dst[(long)ny * nx + jo] = a.v[(long)ny * nx + jo];
+#pragma unroll
+    for (int t = 0; t < kIt; ++t) {
+        const int rr = w + t * NW;
+        if (rr < L::kF) {
+            s.u[rr][lane] = u_[t];
+            s.v[rr][lane] = v_[t];
+        }
+        if (rr >= 1 && rr <= L::kC) {
+            const int ir = i0 - 3 + rr;
+            const T H = H_[t];
+            T p = p_[t];
+            if (phi_dst) {
+                p = grounded_fraction(H, z_[t], a.P.frd);
+                if (ir >= 0 && ir < ny && rr >= 3 && rr < 3 + L::kRows && lane >= 3 && lane < 3 + kMcCols && j < nx)
+                    (phi_dst + (long)ir * nx)[j] = p;
+            }
+            s.H[rr - 1][lane] = H;
+            s.phi[rr - 1][lane] = p;
+            s.S[rr - 1][lane] = p * z_[t] - (T(1) - p) * T(0.917) * H + H;
+            s.bp[rr - 1][lane] = b_[t] * p;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < kIt; ++t) {
+        const int rr = w + t * NW;
+        if (rr >= 1 && rr <= L::kC) {
+            const int ir = i0 - 3 + rr;
+            const bool jin = j > 0 && j < nx;
+            const bool vt_in = jin && ir > 0 && ir < ny, vb_in = jin && ir + 1 > 0 && ir + 1 < ny;
+            const T u = u_[t], v = v_[t], vb = s.v[rr + 1][lane];
+            const T hD = T(0.5) * a.dxi;
+            const T vl = lane_left(v), vbl = lane_left(vb);
+            const T et = vt_in ? hD * ((s.u[rr - 1][lane] - u) + (v - vl)) : T(0);
+            const T eb = vb_in ? hD * ((u - s.u[rr + 1][lane]) + (vb - vbl)) : T(0);
+            const T qs = et * et + eb * eb;
+            const T exx = (lane_right(u) - u) * a.dxi, eyy = (v - vb) * a.dxi;
+            const T e2 = exx * exx + eyy * eyy + exx * eyy + T(0.25) * (qs + lane_right(qs)) + a.P.eps_reg;
+            const T eta = T(0.5) * B_[t] * glen_power(e2, a.P);
+            s.eta[rr - 1][lane] = eta;
+            s.eH[rr - 1][lane] = eta * H_[t];
+        }
+    }
+    __syncthreads();
+
+    const bool stepped = vk.newton_steps > 0 && T(1e30) > vk.tol;
+#pragma unroll 1
+    for (int colour = 0; colour < 2; ++colour) {
+        // the black cell's own values are loaded ahead of the red solve
+        int rn = 0, cn = 0;
+        const bool next = colour == 0 && place(1, rn, cn);
+        McCentre<T> qn{};
+        if (next) qn.load(a, i0 + rn, j0 + cn);
+        // wavefronts whose rows or columns touch the domain edge test the pins
+        const int it = i0 + 2 * w - 1 + colour;
+        const bool edge = it <= 0 || it + 1 >= ny - 1 || bx == 0 || j0 + kMcCols >= nx - 1;
+        // lanes without a cell compute along inside the tile
+        const int i = i0 + r, j = j0 + c, rr = min(r, L::kRows) + 3, l = min(c, kMcCols) + 3;
+        T x[5], masked = T(0), e_c = T(0), Zc = T(0), gc = T(0);
+        if (__any(solves)) {
+            if (edge) mc_newton<T, NW, LINEAR, true>(s, a, q, vk, solves, rr, l, i, j, x, masked, e_c, Zc, gc);
+            else mc_newton<T, NW, LINEAR, false>(s, a, q, vk, solves, rr, l, i, j, x, masked, e_c, Zc, gc);
+        }
+        const long o = (long)i * nx + j, ou = o + i;
+        const bool own = solves && r >= 0 && r < L::kRows && c >= 0 && c < kMcCols;
+        if (own) {
+            H_dst[o] = x[4];
+            if (stepped) mask[o] = masked;
+            // black cells write the facets; the domain's edge facets of a red
+            // cell have no black cell
+            if (colour == 1 || j == 0) u_dst[ou] = x[0];
+            if (colour == 1 || j == nx - 1) u_dst[ou + 1] = x[1];
+            if (colour == 1 || i == 0) v_dst[o] = x[2];
+            if (colour == 1 || i == ny - 1) v_dst[o + nx] = x[3];
+        }
+        if (colour == 1) break;
+        __syncthreads();
+        if (solves) {
+            s.u[rr][l] = x[0];
+            s.u[rr][l + 1] = x[1];
+            s.v[rr][l] = x[2];
+            s.v[rr + 1][l] = x[3];
+            s.H[rr - 1][l] = x[4];
+            s.eH[rr - 1][l] = e_c * x[4];
+            s.S[rr - 1][l] = Zc + gc * x[4];
+        }
+        __syncthreads();
+        r = rn; c = cn;
+        solves = next;
+        q = qn;
     }
 }
 
-template <typename T, bool LINEAR>
-__global__ __launch_bounds__(kMcLanes* kMcRows) void k_vanka_mc(SsaArgs<T> a, const T* __restrict__ eta,
-                                                                T* __restrict__ u_dst, T* __restrict__ v_dst,
-                                                                T* __restrict__ H_dst, T* __restrict__ mask,
-                                                                VankaArgs<T> vk, int colour) {
-    vanka_mc_body<T, LINEAR>(blockIdx.x, blockIdx.y, a, eta, u_dst, v_dst, H_dst, mask, vk, colour);
+template <typename T, int NW, bool LINEAR>
+__global__ __launch_bounds__(kRowLanes* NW) void k_mc_pass(SsaArgs<T> a, T* __restrict__ u_dst,
+                                                           T* __restrict__ v_dst, T* __restrict__ H_dst,
+                                                           T* __restrict__ mask, T* __restrict__ phi_dst,
+                                                           VankaArgs<T> vk, int gx, int blocks) {
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    if (b >= blocks) return;
+    mc_pass_body<T, NW, LINEAR>(b % gx, b / gx, a, u_dst, v_dst, H_dst, mask, phi_dst, vk);
 }
 
 template <typename T>
@@ -165,77 +337,65 @@ hipError_t launch_pin_rows(T* du, T* dv, T* dH, const T* mask, int ny, int nx, h
     return hipGetLastError();
 }
 
-template <typename T>
-hipError_t launch_cell_eta(const SsaArgs<T>& a, T* eta, hipStream_t st) {
-    k_cell_eta<T><<<dim3((a.nx + 255) / 256, a.ny), 256, 0, st>>>(a, eta);
-    return hipGetLastError();
+namespace {
+int mc_blocks(int ny, int nx, int waves, int* gx) {
+    const int rows = 2 * waves - 2;
+    *gx = (nx + kMcCols - 1) / kMcCols;
+    return *gx * ((ny + rows - 1) / rows);
 }
+}  // namespace
+
+// Wavefronts of a workgroup, i.e. 2 kMcWaves - 2 rows: the ring costs (2 NW) /
+// (2 NW - 2) of the red solves.  Per pass FP32 256 x 256 / FP64 2048 x 2048 with
+// 2, 4 and 8 wavefronts: 11.6 / 9.3 / 11.5 us and 293 / 209 / 244 us; 8 hold
+// one workgroup of FP64 per CU, whose loads then overlap with nothing.
+constexpr int kMcWaves = 4;
 
 template <typename T>
-hipError_t launch_vanka_mc(const SsaArgs<T>& a, const T* eta, T* u_dst, T* v_dst, T* H_dst, T* mask,
-                           const VankaArgs<T>& vk, int colour, hipStream_t st) {
-    const int pairs = (a.nx + 1) / 2;
-    const dim3 g((pairs + kMcLanes - 1) / kMcLanes, (a.ny + kMcRows - 1) / kMcRows), b(kMcLanes, kMcRows);
+hipError_t launch_vanka_mc(const SsaArgs<T>& a, T* u_dst, T* v_dst, T* H_dst, T* mask, T* phi_dst,
+                           const VankaArgs<T>& vk, hipStream_t st) {
     TimedLaunch tl(std::is_same<T, float>::value ? kTimeVankaMc32 : kTimeVankaMc64, (long)a.ny * a.nx, st);
+    constexpr int NW = kMcWaves;
+    int gx;
+    const int blocks = mc_blocks(a.ny, a.nx, NW, &gx);
+    const dim3 b(kRowLanes, NW);
+    const int g = (blocks + kXcdCount - 1) / kXcdCount * kXcdCount;
     if (a.P.linear_drag)
-        k_vanka_mc<T, true><<<g, b, 0, st>>>(a, eta, u_dst, v_dst, H_dst, mask, vk, colour & 1);
+        k_mc_pass<T, NW, true><<<g, b, 0, st>>>(a, u_dst, v_dst, H_dst, mask, phi_dst, vk, gx, blocks);
     else
-        k_vanka_mc<T, false><<<g, b, 0, st>>>(a, eta, u_dst, v_dst, H_dst, mask, vk, colour & 1);
+        k_mc_pass<T, NW, false><<<g, b, 0, st>>>(a, u_dst, v_dst, H_dst, mask, phi_dst, vk, gx, blocks);
     return hipGetLastError();
 }
 
 // ------------------------------------------------------------ domain tables
 namespace {
-template <typename T>
-__global__ __launch_bounds__(256) void k_tab_eta(const TabEta<T>* __restrict__ jobs, const int* __restrict__ start,
-                                                 int n) {
-    const int e = tab_find(start, n, blockIdx.x);
-    const TabEta<T> J = jobs[e];
-    const int lb = blockIdx.x - start[e];
-    cell_eta_body<T>(lb % J.gx, lb / J.gx, J.a, J.eta);
-}
-
-template <typename T, bool LINEAR, int ROWS>
-__global__ __launch_bounds__(kMcLanes* ROWS) void k_tab_vanka_mc(const TabVankaMc<T>* __restrict__ jobs,
-                                                                 const int* __restrict__ start, int n, int colour) {
+template <typename T, int NW, bool LINEAR>
+__global__ __launch_bounds__(kRowLanes* NW) void k_tab_mc_pass(const TabVankaMc<T>* __restrict__ jobs,
+                                                               const int* __restrict__ start, int n) {
     const int e = tab_find(start, n, blockIdx.x);
     const TabVankaMc<T> J = jobs[e];
     const int lb = blockIdx.x - start[e];
-    vanka_mc_body<T, LINEAR, ROWS>(lb % J.gx, lb / J.gx, J.a, J.eta, J.u_dst, J.v_dst, J.H_dst, J.mask, J.vk,
-                                   colour);
+    mc_pass_body<T, NW, LINEAR>(lb % J.gx, lb / J.gx, J.a, J.u_dst, J.v_dst, J.H_dst, J.mask, J.phi_dst, J.vk);
 }
+// wavefronts of a workgroup for a tile setting of 1, 2, 4 or 8
+int mc_tile_waves(int rows) { return rows < 2 ? 2 : rows; }
 }  // namespace
 
-int tab_blocks_eta(int ny, int nx, int* gx) {
-    *gx = (nx + 255) / 256;
-    return *gx * ny;
-}
 bool tab_vanka_mc_rows_ok(int rows) { return rows == 1 || rows == 2 || rows == 4 || rows == 8; }
-int tab_blocks_vanka_mc(int ny, int nx, int rows, int* gx) {
-    const int pairs = (nx + 1) / 2;
-    *gx = (pairs + kMcLanes - 1) / kMcLanes;
-    return *gx * ((ny + rows - 1) / rows);
-}
+int tab_blocks_vanka_mc(int ny, int nx, int rows, int* gx) { return mc_blocks(ny, nx, mc_tile_waves(rows), gx); }
 
 template <typename T>
-hipError_t launch_tab_eta(const TabEta<T>* jobs, const int* start, int n, int blocks, hipStream_t st) {
+hipError_t launch_tab_vanka_mc(const TabVankaMc<T>* jobs, const int* start, int n, int blocks, bool linear, int rows,
+                               hipStream_t st) {
     if (n <= 0 || blocks <= 0) return hipSuccess;
-    k_tab_eta<T><<<blocks, 256, 0, st>>>(jobs, start, n);
-    return hipGetLastError();
-}
-template <typename T>
-hipError_t launch_tab_vanka_mc(const TabVankaMc<T>* jobs, const int* start, int n, int blocks, int colour,
-                               bool linear, int rows, hipStream_t st) {
-    if (n <= 0 || blocks <= 0) return hipSuccess;
-    const dim3 b(kMcLanes, rows);
-    const int c = colour & 1;
-#define GLIDE_TAB_MC(R)                                                                        \
-    if (rows == R) {                                                                           \
-        if (linear) k_tab_vanka_mc<T, true, R><<<blocks, b, 0, st>>>(jobs, start, n, c);      \
-        else k_tab_vanka_mc<T, false, R><<<blocks, b, 0, st>>>(jobs, start, n, c);            \
-        return hipGetLastError();                                                              \
+    const int nw = mc_tile_waves(rows);
+    const dim3 b(kRowLanes, nw);
+#define GLIDE_TAB_MC(W)                                                                     \
+    if (nw == W) {                                                                          \
+        if (linear) k_tab_mc_pass<T, W, true><<<blocks, b, 0, st>>>(jobs, start, n);       \
+        else k_tab_mc_pass<T, W, false><<<blocks, b, 0, st>>>(jobs, start, n);             \
+        return hipGetLastError();                                                           \
     }
-    GLIDE_TAB_MC(1)
     GLIDE_TAB_MC(2)
     GLIDE_TAB_MC(4)
     GLIDE_TAB_MC(8)
@@ -367,17 +527,13 @@ hipError_t launch_krylov_axpy(double* out, const double* V, long ld, long n, int
 
 #define GLIDE_MC_INSTANTIATE(T)                                                                                     \
     template hipError_t launch_pin_rows<T>(T*, T*, T*, const T*, int, int, hipStream_t);                           \
-    template hipError_t launch_cell_eta<T>(const SsaArgs<T>&, T*, hipStream_t);                                    \
-    template hipError_t launch_vanka_mc<T>(const SsaArgs<T>&, const T*, T*, T*, T*, T*, const VankaArgs<T>&, int,  \
-                                           hipStream_t);
+    template hipError_t launch_vanka_mc<T>(const SsaArgs<T>&, T*, T*, T*, T*, T*, const VankaArgs<T>&, hipStream_t);
 
 GLIDE_MC_INSTANTIATE(double)
 GLIDE_MC_INSTANTIATE(float)
 
 #define GLIDE_MC_TAB_INSTANTIATE(T)                                                                                 \
-    template hipError_t launch_tab_eta<T>(const TabEta<T>*, const int*, int, int, hipStream_t);                    \
-    template hipError_t launch_tab_vanka_mc<T>(const TabVankaMc<T>*, const int*, int, int, int, bool, int,   \
-                                               hipStream_t);
+    template hipError_t launch_tab_vanka_mc<T>(const TabVankaMc<T>*, const int*, int, int, bool, int, hipStream_t);
 
 GLIDE_MC_TAB_INSTANTIATE(double)
 GLIDE_MC_TAB_INSTANTIATE(float)

@@ -222,31 +222,12 @@ int persistent_ctl(const glide_level& L, PersistentCtl* ctl) {
     return GLIDE_OK;
 }
 
-// Multicolour passes (glide_vanka_config.multicolour): per pass the cell
-// viscosity of the current state into the workspace (behind the alternate
-// state), then the red phase into the alternate buffers and the black phase
-// back into the level's own; the grounded fraction is refreshed before each
-// pass unless frozen.
-int vanka_sweeps_mc(const glide_level& L, double dt, int n_iter, const VankaArgs<R>& vk, double relax_phi,
-                    bool freeze_phi, hipStream_t st) {
-    R* alt_u = P(L.work);
-    R* alt_v = alt_u + nU(L);
-    R* alt_H = alt_v + nV(L);
-    R* eta = alt_H + nC(L);
-    for (int it = 0; it < n_iter; ++it) {
-        if (!freeze_phi) GLIDE_TRY(grounded(L, relax_phi, st));
-        SsaArgs<R> a = make_args(L, dt, false);
-        HIP_TRY(launch_cell_eta<R>(a, eta, st), "cell viscosity");
-        HIP_TRY(launch_vanka_mc<R>(a, eta, alt_u, alt_v, alt_H, P(L.mask), vk, 0, st), "vanka red phase");
-        SsaArgs<R> b = a;
-        b.u = alt_u; b.v = alt_v; b.H = alt_H;
-        HIP_TRY(launch_vanka_mc<R>(b, eta, P(L.u), P(L.v), P(L.H), P(L.mask), vk, 1, st), "vanka black phase");
-    }
-    return GLIDE_OK;
-}
+template <typename T>
+int mc_sweeps_t(const glide_level& L, double dt, int n_iter, const glide_vanka_config& vc, int flags, hipStream_t st);
 
 int vanka_sweeps(const glide_level& L, double dt, int n_iter, const glide_vanka_config& vc, int flags,
                  hipStream_t st) {
+    if (vc.multicolour) return mc_sweeps_t<R>(L, dt, n_iter, vc, flags, st);
     const bool freeze_phi = (flags & GLIDE_FREEZE_PHI) != 0;
     VankaArgs<R> vk;
     vk.newton_steps = vc.newton_steps;
@@ -257,7 +238,6 @@ int vanka_sweeps(const glide_level& L, double dt, int n_iter, const glide_vanka_
     vk.local_fp32 = vc.local_fp32;
     vk.relax = vc.relaxation;
     vk.tol = vc.newton_tol;
-    if (vc.multicolour) return vanka_sweeps_mc(L, dt, n_iter, vk, vc.relax_phi, freeze_phi, st);
     // small levels with a frozen grounded fraction: one fused launch per pass,
     // the state alternating between the level's buffers and the workspace
     // (5 planes hold u, v and H); an odd pass count copies it back at the end
@@ -419,10 +399,6 @@ int restrict_c(const void* f, void* c, const glide_level& C, int use_max, hipStr
 }
 int axpby(void* out, double a, const void* x, double b, const void* y, size_t n, hipStream_t st) {
     HIP_TRY(launch_axpby<R>(P(out), a, CP(x), b, CP(y), 0.0, nullptr, (long)n, st), "axpby");
-    return GLIDE_OK;
-}
-int copy(void* dst, const void* src, size_t n, hipStream_t st) {
-    HIP_TRY(launch_copy<R>(P(dst), CP(src), (long)n, st), "copy");
     return GLIDE_OK;
 }
 int fill(void* dst, double val, size_t n, hipStream_t st) {
@@ -881,11 +857,15 @@ int residual_t(const glide_level& L, double dt, int flags, T* ou, T* ov, T* oH, 
     return GLIDE_OK;
 }
 
-// Multicolour passes on a level of element type T (see vanka_sweeps_mc).
+// Multicolour passes (glide_vanka_config.multicolour) on a level of element
+// type T, one launch each, alternating between the level's state and the
+// workspace; an odd count copies the state back at the end.  The pass itself
+// refreshes the grounded fraction unless frozen or relaxed (a workgroup would
+// then read the old fraction of cells that another one rewrites).
 template <typename T>
 int mc_sweeps_t(const glide_level& L, double dt, int n_iter, const glide_vanka_config& vc, int flags,
                 hipStream_t st) {
-    const bool freeze_phi = (flags & GLIDE_FREEZE_PHI) != 0;
+    const bool freeze_phi = (flags & GLIDE_FREEZE_PHI) != 0, relaxed = T(vc.relax_phi) != T(0);
     VankaArgs<T> vk;
     vk.newton_steps = vc.newton_steps;
     vk.ssa_damping = T(vc.ssa_damping);
@@ -895,22 +875,27 @@ int mc_sweeps_t(const glide_level& L, double dt, int n_iter, const glide_vanka_c
     vk.local_fp32 = 0;
     vk.relax = T(vc.relaxation);
     vk.tol = T(vc.newton_tol);
-    T* alt_u = PT<T>(L.work);
-    T* alt_v = alt_u + nU(L);
-    T* alt_H = alt_v + nV(L);
-    T* eta = alt_H + nC(L);
+    T* own[3] = {PT<T>(L.u), PT<T>(L.v), PT<T>(L.H)};
+    T* alt[3] = {PT<T>(L.work), PT<T>(L.work) + nU(L), PT<T>(L.work) + nU(L) + nV(L)};
     for (int it = 0; it < n_iter; ++it) {
-        if (!freeze_phi)
-            HIP_TRY(launch_grounded<T>(PT<T>(L.phi), CPT<T>(L.H), CPT<T>(L.bed), T(L.phys.flotation_reg_driving),
+        T* const* src = (it & 1) ? alt : own;
+        T* const* dst = (it & 1) ? own : alt;
+        SsaArgs<T> a = make_args_t<T>(L, dt, false);
+        a.u = src[0]; a.v = src[1]; a.H = src[2];
+        if (!freeze_phi && relaxed)
+            HIP_TRY(launch_grounded<T>(PT<T>(L.phi), a.H, CPT<T>(L.bed), T(L.phys.flotation_reg_driving),
                                        T(vc.relax_phi), (long)nC(L), st),
                     "grounded");
-        SsaArgs<T> a = make_args_t<T>(L, dt, false);
-        HIP_TRY(launch_cell_eta<T>(a, eta, st), "cell viscosity");
-        HIP_TRY(launch_vanka_mc<T>(a, eta, alt_u, alt_v, alt_H, PT<T>(L.mask), vk, 0, st), "vanka red phase");
-        SsaArgs<T> b = a;
-        b.u = alt_u; b.v = alt_v; b.H = alt_H;
-        HIP_TRY(launch_vanka_mc<T>(b, eta, PT<T>(L.u), PT<T>(L.v), PT<T>(L.H), PT<T>(L.mask), vk, 1, st),
-                "vanka black phase");
+        HIP_TRY(launch_vanka_mc<T>(a, dst[0], dst[1], dst[2], PT<T>(L.mask),
+                                   freeze_phi || relaxed ? nullptr : PT<T>(L.phi), vk, st),
+                "red-black pass");
+    }
+    if (n_iter > 0 && (n_iter & 1)) {
+        EwBatch<T> b;
+        b.copy(own[0], alt[0], (long)nU(L));
+        b.copy(own[1], alt[1], (long)nV(L));
+        b.copy(own[2], alt[2], (long)nC(L));
+        HIP_TRY(launch_ew_batch<T>(b, st), "state back");
     }
     return GLIDE_OK;
 }
@@ -1637,7 +1622,7 @@ int mixed_adj_vcycle(MixedCtx& X, int l, bool finest) {
 // table arena and replayed as one HIP graph.
 
 enum TabKind {
-    kKEw, kKXfer, kKRes32, kKRes64, kKEta32, kKEta64, kKMc32, kKMc64, kKFac32, kKFac64, kKPass32, kKPass64,
+    kKEw, kKXfer, kKRes32, kKRes64, kKMc32, kKMc64, kKFac32, kKFac64, kKPass32, kKPass64,
     kKVjp32, kKVjp64, kKGrad64
 };
 
@@ -1790,10 +1775,10 @@ struct EnsRec {
         if (Ls.empty() || n_iter <= 0) return GLIDE_OK;
         const int linear = make_phys(Ls[0]->phys).linear_drag;
         const int tile = rows[slot];
-        std::vector<TabEta<T>> eta;
-        std::vector<TabVankaMc<T>> red, black;
-        std::vector<int> be, bm;
-        EwList g;
+        std::vector<TabVankaMc<T>> out, back;
+        std::vector<int> bm;
+        EwList gout, gback, copy;
+        const bool f32 = sizeof(T) == 4, relaxed = T(vf.relax_phi) != T(0);
         for (size_t q = 0; q < Ls.size(); ++q) {
             const glide_level& L = *Ls[q];
             if (make_phys(L.phys).linear_drag != linear)
@@ -1807,38 +1792,37 @@ struct EnsRec {
             vk.local_fp32 = 0;
             vk.relax = T(vf.relaxation);
             vk.tol = T(vf.newton_tol);
-            T* alt_u = PT<T>(L.work);
-            T* alt_v = alt_u + nU(L);
-            T* alt_H = alt_v + nV(L);
-            T* e = alt_H + nC(L);
-            if (!(flags[q] & GLIDE_FREEZE_PHI))
-                g.add(sizeof(T) == 4 ? kTabGrounded32 : kTabGrounded64, L.phi, L.H, L.bed, nullptr,
-                      (double)T(L.phys.flotation_reg_driving), (double)T(vf.relax_phi), 0.0, (long)nC(L));
-            TabEta<T> E{};
-            E.a = make_args_t<T>(L, dt, false);
-            E.eta = e;
-            be.push_back(tab_blocks_eta(L.ny, L.nx, &E.gx));
-            eta.push_back(E);
-            TabVankaMc<T> R{};
-            R.a = E.a;
-            R.eta = e;
-            R.u_dst = alt_u; R.v_dst = alt_v; R.H_dst = alt_H;
-            R.mask = PT<T>(L.mask);
-            R.vk = vk;
-            bm.push_back(tab_blocks_vanka_mc(L.ny, L.nx, tile, &R.gx));
-            red.push_back(R);
-            TabVankaMc<T> B = R;
-            B.a.u = alt_u; B.a.v = alt_v; B.a.H = alt_H;
-            B.u_dst = PT<T>(L.u); B.v_dst = PT<T>(L.v); B.H_dst = PT<T>(L.H);
-            black.push_back(B);
+            T* own[3] = {PT<T>(L.u), PT<T>(L.v), PT<T>(L.H)};
+            T* alt[3] = {PT<T>(L.work), PT<T>(L.work) + nU(L), PT<T>(L.work) + nU(L) + nV(L)};
+            const bool refresh = !(flags[q] & GLIDE_FREEZE_PHI);
+            if (refresh && relaxed) {
+                const int op = f32 ? kTabGrounded32 : kTabGrounded64;
+                const double c = (double)T(L.phys.flotation_reg_driving), rx = (double)T(vf.relax_phi);
+                gout.add(op, L.phi, own[2], L.bed, nullptr, c, rx, 0.0, (long)nC(L));
+                gback.add(op, L.phi, alt[2], L.bed, nullptr, c, rx, 0.0, (long)nC(L));
+            }
+            TabVankaMc<T> J{};
+            J.a = make_args_t<T>(L, dt, false);
+            J.u_dst = alt[0]; J.v_dst = alt[1]; J.H_dst = alt[2];
+            J.mask = PT<T>(L.mask);
+            J.phi_dst = refresh && !relaxed ? PT<T>(L.phi) : nullptr;
+            J.vk = vk;
+            bm.push_back(tab_blocks_vanka_mc(L.ny, L.nx, tile, &J.gx));
+            out.push_back(J);
+            J.a.u = alt[0]; J.a.v = alt[1]; J.a.H = alt[2];
+            J.u_dst = own[0]; J.v_dst = own[1]; J.H_dst = own[2];
+            back.push_back(J);
+            const size_t n3[3] = {nU(L), nV(L), nC(L)};
+            for (int k = 0; k < 3; ++k) {
+                if (f32) copy.copy32(own[k], alt[k], n3[k]);
+                else copy.copy64(own[k], alt[k], n3[k]);
+            }
         }
-        const bool f32 = sizeof(T) == 4;
         for (int it = 0; it < n_iter; ++it) {
-            ew(g);
-            prog.add(f32 ? kKEta32 : kKEta64, eta, be);
-            prog.add(f32 ? kKMc32 : kKMc64, red, bm, 0, linear, tile);
-            prog.add(f32 ? kKMc32 : kKMc64, black, bm, 1, linear, tile);
+            ew((it & 1) ? gback : gout);
+            prog.add(f32 ? kKMc32 : kKMc64, (it & 1) ? back : out, bm, 0, linear, tile);
         }
+        if (n_iter & 1) ew(copy);
         return GLIDE_OK;
     }
 
@@ -2495,15 +2479,13 @@ int run_tab_op(const TabOp& op, const unsigned char* dev, hipStream_t st) {
         case kKRes64:
             e = launch_tab_residual<double>(static_cast<const TabResidual<double>*>(jobs), start, op.n, op.blocks, st);
             break;
-        case kKEta32: e = launch_tab_eta<float>(static_cast<const TabEta<float>*>(jobs), start, op.n, op.blocks, st); break;
-        case kKEta64: e = launch_tab_eta<double>(static_cast<const TabEta<double>*>(jobs), start, op.n, op.blocks, st); break;
         case kKMc32:
             e = launch_tab_vanka_mc<float>(static_cast<const TabVankaMc<float>*>(jobs), start, op.n, op.blocks,
-                                           op.colour, op.linear != 0, op.rows, st);
+                                           op.linear != 0, op.rows, st);
             break;
         case kKMc64:
             e = launch_tab_vanka_mc<double>(static_cast<const TabVankaMc<double>*>(jobs), start, op.n, op.blocks,
-                                            op.colour, op.linear != 0, op.rows, st);
+                                            op.linear != 0, op.rows, st);
             break;
         case kKFac32:
             e = launch_tab_adj_factor<float>(static_cast<const TabAdjFactor<float>*>(jobs), start, op.n, op.blocks, st);

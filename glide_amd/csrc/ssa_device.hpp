@@ -34,7 +34,12 @@ __device__ __forceinline__ double inv_cbrt(double x) {
     y = y * (4.0 - x * (y * y * y)) * (1.0 / 3.0);
     return y;
 }
-__device__ __forceinline__ float inv_cbrt(float x) { return pow(x, -1.0f / 3.0f); }
+// FP32: the same estimate, one of the steps in FP64, rounded once.
+__device__ __forceinline__ float inv_cbrt(float x) {
+    if (!(x > 1e-30f && x < 1e30f)) return pow(x, -1.0f / 3.0f);
+    const double y = (double)__builtin_amdgcn_exp2f(__builtin_amdgcn_logf(x) * (-1.0f / 3.0f));
+    return (float)(y * (4.0 - (double)x * (y * y * y)) * (1.0 / 3.0));
+}
 
 // The Glen-law viscosity power e2^((1-n)/(2n)).
 template <typename T>

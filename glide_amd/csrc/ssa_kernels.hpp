@@ -209,23 +209,19 @@ hipError_t launch_grad_B(const SsaArgs<T>& a, const T* lu, const T* lv, T* gB, h
 
 
 // Multicolour (red-black) Vanka smoothing (mc_kernels.hip; no counterpart in
-// the reference).  launch_cell_eta fills eta (ny, nx) with the cell viscosity
-// of the state in a.  launch_vanka_mc runs one colour phase: every cell with
-// (i + j) % 2 == colour solves its 5x5 patch (local Newton with vk.relax,
-// vk.tol, the Vanka dampings, viscosity from eta) against the state in a and
-// writes its five unknowns to u_dst / v_dst / H_dst; the other cells copy their
-// thickness and the domain-edge facets no cell of the colour owns, so the
-// destination holds the complete new state; the active-set flag is written in
-// place.  The destination buffers must differ from a's state.
-template <typename T>
-hipError_t launch_cell_eta(const SsaArgs<T>& a, T* eta, hipStream_t st);
+// the reference).  launch_vanka_mc runs one pass: with the viscosity of the
+// state in a, every red cell, then every black one solves its 5x5 patch (local
+// Newton with vk.relax, vk.tol and the Vanka dampings).  The complete new state
+// goes to u_dst / v_dst / H_dst, which must differ from a's buffers, the
+// active-set flag in place.  phi_dst != nullptr: the pass takes the grounded
+// fraction of the state in a (not a.phi) and writes it there.
 // Zero the multipliers / corrections of the rows the patch solves pin: the
 // domain-edge facets and the cells of the active set (mask > 0.5).
 template <typename T>
 hipError_t launch_pin_rows(T* du, T* dv, T* dH, const T* mask, int ny, int nx, hipStream_t st);
 template <typename T>
-hipError_t launch_vanka_mc(const SsaArgs<T>& a, const T* eta, T* u_dst, T* v_dst, T* H_dst, T* mask,
-                           const VankaArgs<T>& vk, int colour, hipStream_t st);
+hipError_t launch_vanka_mc(const SsaArgs<T>& a, T* u_dst, T* v_dst, T* H_dst, T* mask, T* phi_dst,
+                           const VankaArgs<T>& vk, hipStream_t st);
 
 // Element-wise jobs between FP64 and FP32 buffers of the mixed-precision
 // solver (mc_kernels.hip), batched into one launch (the jobs must not read

@@ -34,17 +34,11 @@ struct TabResidual {
     T cr;
     int gx;
 };
-template <typename T>
-struct TabEta {
-    SsaArgs<T> a;
-    T* eta;
-    int gx;
-};
+// one red-black pass; phi_dst != nullptr: from the refreshed grounded fraction
 template <typename T>
 struct TabVankaMc {
     SsaArgs<T> a;
-    const T* eta;
-    T *u_dst, *v_dst, *H_dst, *mask;
+    T *u_dst, *v_dst, *H_dst, *mask, *phi_dst;
     VankaArgs<T> vk;
     int gx;
 };
@@ -128,8 +122,7 @@ struct TabXfer {
 // Blocks of one job (its single-domain grid) and the launchers: jobs and
 // start in device memory (start with n entries), `blocks` the total.
 int tab_blocks_residual(int ny, int nx, int* gx);
-int tab_blocks_eta(int ny, int nx, int* gx);
-// the red-black phase's blocks hold `rows` rows of cell pairs (1, 2, 4 or 8)
+// the red-black pass's tile setting (1, 2, 4 or 8: 2, 2, 6 or 14 rows a block)
 bool tab_vanka_mc_rows_ok(int rows);
 int tab_blocks_vanka_mc(int ny, int nx, int rows, int* gx);
 int tab_blocks_adj_factor(int ny, int nx, int* gx);
@@ -142,10 +135,8 @@ inline int tab_blocks_ew(long n) { return (int)((n + kTabEwPerBlock - 1) / kTabE
 template <typename T>
 hipError_t launch_tab_residual(const TabResidual<T>* jobs, const int* start, int n, int blocks, hipStream_t st);
 template <typename T>
-hipError_t launch_tab_eta(const TabEta<T>* jobs, const int* start, int n, int blocks, hipStream_t st);
-template <typename T>
-hipError_t launch_tab_vanka_mc(const TabVankaMc<T>* jobs, const int* start, int n, int blocks, int colour,
-                               bool linear, int rows, hipStream_t st);
+hipError_t launch_tab_vanka_mc(const TabVankaMc<T>* jobs, const int* start, int n, int blocks, bool linear, int rows,
+                               hipStream_t st);
 template <typename T>
 hipError_t launch_tab_adj_factor(const TabAdjFactor<T>* jobs, const int* start, int n, int blocks, hipStream_t st);
 template <typename T>

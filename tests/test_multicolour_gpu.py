@@ -66,6 +66,40 @@ def test_mc_passes_match_oracle(orc, shape, mode, m):
         assert np.array_equal(N(g.state.mask.data), mask), k
 
 
+@pytest.mark.parametrize("shape", [(6, 58), (7, 59), (13, 117), (12, 64), (2, 122)])
+@pytest.mark.parametrize("relax_phi", [0.0, 0.3])
+def test_mc_pass_tiles_and_grounded_refresh(orc, shape, relax_phi):
+    """Sizes at the edges of the passes' tiles (6 rows, 58 columns): three
+    passes that refresh the grounded fraction themselves (or relax it) equal,
+    bitwise, the fraction's own launch and a frozen pass three times, and the
+    first pass the oracle's (the pass bar 1e-12)."""
+    ny, nx = shape
+    print(f"mc tiles shape={shape} relax_phi={relax_phi}", flush=True)
+    F = dome_fields(ny=ny, nx=nx, seed=5, mask_frac=0.1)
+    out = []
+    for split in (False, True):
+        g = grid_from(F)
+        fo = g.forward_operators
+        _configure(fo.vanka_config, MIXED)
+        fo.vanka_config.relax_phi = relax_phi
+        if split:
+            for k in range(3):
+                fo.compute_phi(relax_phi)
+                if k == 0:
+                    Fo = dict(F, phi=N(g.state.phi.data))
+                fo.vanka_sweep(10.0, 1, freeze_phi=True)
+                if k == 0:
+                    u, v, H, mask, _ = orc.mc_sweep(Fo, orc.phys(), 1500.0, 10.0, **_oracle_kw(MIXED))
+                    for a, b in ((g.state.u, u), (g.state.v, v), (g.state.H, H)):
+                        assert rel_err(N(a.data), b) < 1e-12
+        else:
+            fo.vanka_sweep(10.0, 3)
+        torch.cuda.synchronize()
+        out.append([N(t.data) for t in (g.state.u, g.state.v, g.state.H, g.state.mask)])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
 def _warm_models(orc, n, L, warm=2, ny=None, compat=True):
     """GPU model and oracle hierarchy after `warm` additive V-cycles (matching
     to 1e-10), then H_prev = H (the start of a next time step)."""
