@@ -339,10 +339,16 @@ __device__ __forceinline__ void fill_eta_tile(T (*s_eta)[TX + 2], const SsaArgs<
 // returns the increments w = ((u_l, u_r, v_t, v_b) change / 2, H change) and
 // the active-set flag.  edge: the calling wave may hold cells on the domain's
 // edge (the loop then tests the Dirichlet pins; interior waves carry no pin
-// code).  The wave-uniform edge test keeps one loop copy per wave.
+// code).  The wave-uniform edge test keeps one loop copy per wave.  Every lane
+// of the wavefront calls it (those without a cell to solve with the indices of
+// another one and solves = false) and iterates as long as any of them does:
+// with about ten lanes or fewer in its execution mask a wavefront issues these
+// instructions at a third of the rate, and the last iterations of a pass belong
+// to a few cells.
 template <typename T, bool LINEAR, typename TJ, int W, class Ld = LdPlain>
 __device__ __forceinline__ void cell_newton(const SsaArgs<T>& a, const T (*s_eta)[W], int li, int lj, int i, int j,
-                                            const VankaArgs<T>& vk, bool edge, T w[5], T& masked, int& iters) {
+                                            const VankaArgs<T>& vk, bool solves, bool edge, T w[5], T& masked,
+                                            int& iters) {
     const int ny = a.ny, nx = a.nx;
     CellSys<T> cs;
     T thk;
@@ -364,13 +370,13 @@ __device__ __forceinline__ void cell_newton(const SsaArgs<T>& a, const T (*s_eta
     T cmp[5];
 #pragma unroll
     for (int k = 0; k < 5; ++k) cmp[k] = T(0);
-    T rnorm = T(1);
     const T tol = T(1e-6);
     const bool pin0 = j == 0, pin1 = j == nx - 1, pin2 = i == 0, pin3 = i == ny - 1;
     int it = 0;
+    bool go = solves && vk.newton_steps > 0;
     auto newton = [&](auto edge_tag) {
         constexpr bool EDGE = decltype(edge_tag)::value;
-        while (it < vk.newton_steps && rnorm > tol) {
+        while (__any(go)) {
             TJ J[25];
             T r[5];
             cell_system<T, TJ, LINEAR>(cs, *cq, x, J, r, a.P);
@@ -380,26 +386,27 @@ __device__ __forceinline__ void cell_newton(const SsaArgs<T>& a, const T (*s_eta
                 if (pin2) { pin_row(J, 2); r[2] = x[2]; }
                 if (pin3) { pin_row(J, 3); r[3] = x[3]; }
             }
-            if ((x[4] - a.dt * r[4]) <= thk) {
-                masked = T(1);
+            const bool pin4 = (x[4] - a.dt * r[4]) <= thk;
+            if (pin4) {
                 pin_row(J, 4);
                 r[4] = x[4] - thk;
-            } else {
-                masked = T(0);
             }
+            masked = go ? (pin4 ? T(1) : T(0)) : masked;
             TJ rj[5] = {TJ(r[0]), TJ(r[1]), TJ(r[2]), TJ(r[3]), TJ(r[4])};
             TJ d[5];
             lu5_solve_rcp(J, rj, d);
-            rnorm = r[0] * r[0] + r[1] * r[1] + r[2] * r[2] + r[3] * r[3] + r[4] * r[4];
+            const T rnorm = r[0] * r[0] + r[1] * r[1] + r[2] * r[2] + r[3] * r[3] + r[4] * r[4];
 #pragma unroll
             for (int k = 0; k < 5; ++k) {  // compensated relaxed update, local relaxation 0.5
-                T y = T(-0.5) * T(d[k]) - cmp[k];
+                const T y = T(-0.5) * T(d[k]) - cmp[k];
                 T t = x[k] + y;
-                cmp[k] = (t - x[k]) - y;
-                x[k] = t;
+                const T e = (t - x[k]) - y;
+                if (k == 4) t = fmax(t, thk);
+                cmp[k] = go ? e : cmp[k];
+                x[k] = go ? t : x[k];
             }
-            x[4] = fmax(x[4], thk);
-            ++it;
+            it += go ? 1 : 0;
+            go = go && it < vk.newton_steps && rnorm > tol;
         }
     };
     if (edge) newton(std::true_type{});
@@ -426,12 +433,15 @@ __global__ __launch_bounds__(TX * ROWS) void k_vanka_cell(SsaArgs<T> a, T* __res
     __syncthreads();
     const int i = i0 + threadIdx.y, j = j0 + threadIdx.x;
     const int ny = a.ny, nx = a.nx;
-    if (i >= ny || j >= nx) return;
-    const long c = (long)i * nx + j;
+    if (i >= ny) return;
+    const int jc = min(j, nx - 1);
+    const long c = (long)i * nx + jc;
     T w[5], masked = mask[c];
     int it = 0;
     const bool edge_wave = i == 0 || i == ny - 1 || j0 == 0 || j0 + TX >= nx;
-    cell_newton<T, LINEAR, TJ, TX + 2>(a, s_eta, threadIdx.y + 1, threadIdx.x + 1, i, j, vk, edge_wave, w, masked, it);
+    cell_newton<T, LINEAR, TJ, TX + 2>(a, s_eta, threadIdx.y + 1, jc - j0 + 1, i, jc, vk, j < nx, edge_wave, w, masked,
+                                       it);
+    if (j >= nx) return;
     const long n = (long)ny * nx;
 #pragma unroll
     for (int q = 0; q < 5; ++q) work[q * n + c] = w[q];
@@ -481,11 +491,15 @@ __global__ __launch_bounds__(3 * TX) void k_vanka_fused(SsaArgs<T> a, T* __restr
     T w[5] = {T(0), T(0), T(0), T(0), T(0)};
     T masked = (wv == 0 && active) ? mask[(long)i0 * nx + cj] : T(0);
     int it = 0;
-    if (active) {
-        cell_newton<T, LINEAR, TJ, W>(a, s_eta, ci - i0 + 2, cj - j0 + 2, ci, cj, vk, edge, w, masked, it);
-        if (wv == 0) s_w1[lane + 1] = w[1];
-        else if (wv == 1) s_w3[lane] = w[3];
-        else s_w1[0] = w[1];
+    if (__any(active)) {
+        // lanes without a cell compute along on the nearest one
+        const int cc = wv == 2 ? j0 - 1 : min(cj, nx - 1);
+        cell_newton<T, LINEAR, TJ, W>(a, s_eta, ci - i0 + 2, cc - j0 + 2, ci, cc, vk, active, edge, w, masked, it);
+        if (active) {
+            if (wv == 0) s_w1[lane + 1] = w[1];
+            else if (wv == 1) s_w3[lane] = w[3];
+            else s_w1[0] = w[1];
+        }
     }
     __syncthreads();
     if (wv != 0 || !active) return;
@@ -660,10 +674,13 @@ __global__ __launch_bounds__(TX * (RW + 1)) void k_vanka_persistent(SsaArgs<T> a
         T w[5] = {T(0), T(0), T(0), T(0), T(0)};
         T masked = own ? Ld::get(mask + (long)ci * nx + cj) : T(0);
         int it = 0;
-        if (active) {
-            cell_newton<T, LINEAR, TJ, W, Ld>(s, s_eta, ci - i0 + 2, cj + 2, ci, cj, vk, true, w, masked, it);
-            if (wv < RW) s_w1[wv][lane + 1] = w[1];
-            s_w3[wv][lane] = w[3];
+        if (__any(active)) {
+            const int cc = min(cj, nx - 1);  // lanes without a cell compute along on the last one
+            cell_newton<T, LINEAR, TJ, W, Ld>(s, s_eta, ci - i0 + 2, cc + 2, ci, cc, vk, active, true, w, masked, it);
+            if (active) {
+                if (wv < RW) s_w1[wv][lane + 1] = w[1];
+                s_w3[wv][lane] = w[3];
+            }
         }
         __syncthreads();
         if (own) {
