@@ -245,4 +245,162 @@ struct TransposeRows {
     }
 };
 
+// The coupled residual (JVP false) or its derivative along d = (du, dv, dH)
+// (JVP true; grounded fraction, mask, bed, B and beta frozen) on row segments,
+// without forcing, active set and Dirichlet rows.  Rows, lanes and halo as in
+// TransposeRows: the results are valid for wavefronts 1 .. NW - 2 and lanes
+// 2 .. 61.  A wavefront owns the cells, facets and top-left vertices of a row.
+template <typename T, int NW, bool DRAG, bool JVP>
+struct ForwardRows {
+    static constexpr int kUp = JVP ? 8 : 5;  // planes a row hands to the row below it
+    struct Lds {
+        T up[NW][kUp][kRowLanes];
+        T down[NW][2][kRowLanes];
+    };
+
+    T u, v, H, phi;    // this lane's facets and cell
+    T ru, rv, rH, dH;  // dH: the direction's thickness
+
+    // barrier 1 and 2 of the workgroup are inside; every wavefront calls it
+    __device__ __forceinline__ void run(Lds& s, const SsaArgs<T>& a, const T* __restrict__ pdu,
+                                        const T* __restrict__ pdv, const T* __restrict__ pdH, T calving_rate, int w,
+                                        int lane, int i, int j) {
+        const int ny = a.ny, nx = a.nx;
+        const T D = a.dxi, hD = T(0.5) * D;
+        const int jc = clampi(j, 0, nx - 1), ju = clampi(j, 0, nx);
+        const int ic = clampi(i, 0, ny - 1);
+        const long rc = (long)ic * nx, rf = (long)ic * (nx + 1);
+        const long rft = (long)clampi(i - 1, 0, ny - 1) * (nx + 1), rfb = (long)clampi(i + 1, 0, ny - 1) * (nx + 1);
+        const long rv0 = (long)clampi(i, 0, ny) * nx, rv1 = (long)clampi(i + 1, 0, ny) * nx;
+        u = (a.u + rf)[ju];
+        const T ut = (a.u + rft)[ju], ub = (a.u + rfb)[ju];
+        v = (a.v + rv0)[jc];
+        const T vb = (a.v + rv1)[jc];
+        H = (a.H + rc)[jc];
+        phi = (a.phi + rc)[jc];
+        const T bed = (a.bed + rc)[jc], beta = (a.beta + rc)[jc], B = (a.B + rc)[jc];
+        T du = T(0), dut = T(0), dub = T(0), dv = T(0), dvb = T(0);
+        dH = T(0);
+        if constexpr (JVP) {
+            du = (pdu + rf)[ju];
+            dut = (pdu + rft)[ju];
+            dub = (pdu + rfb)[ju];
+            dv = (pdv + rv0)[jc];
+            dvb = (pdv + rv1)[jc];
+            dH = (pdH + rc)[jc];
+        }
+        const bool jin = j > 0 && j < nx;
+        const bool vt_in = jin && i > 0 && i < ny, vb_in = jin && i + 1 > 0 && i + 1 < ny;
+        const T vl = lane_left(v), vbl = lane_left(vb), ur = lane_right(u);
+        const T et = vt_in ? hD * ((ut - u) + (v - vl)) : T(0);
+        const T eb = vb_in ? hD * ((u - ub) + (vb - vbl)) : T(0);
+        const T exx = (ur - u) * D, eyy = (v - vb) * D;
+        const T qs = et * et + eb * eb;
+        const T sx = T(2) * exx + eyy, sy = exx + T(2) * eyy;
+        const T e2 = exx * exx + eyy * eyy + exx * eyy + T(0.25) * (qs + lane_right(qs)) + a.P.eps_reg;
+        const T eta = T(0.5) * B * glen_power(e2, a.P);
+        const T eH = eta * H;
+        const T g = T(1) - (T(1) - phi) * T(0.917);
+        const T S = phi * bed + g * H, bp = beta * phi;
+        // normal stresses (JVP: their derivatives) and the derivative of eta H
+        T Sxx = T(2) * eH * sx, Syy = T(2) * eH * sy, dt_ = T(0), deH = T(0), dvl = T(0), dvbl = T(0), dur = T(0);
+        if constexpr (JVP) {
+            dvl = lane_left(dv);
+            dvbl = lane_left(dvb);
+            dur = lane_right(du);
+            dt_ = vt_in ? hD * ((dut - du) + (dv - dvl)) : T(0);
+            const T db = vb_in ? hD * ((du - dub) + (dvb - dvbl)) : T(0);
+            const T dxx = (dur - du) * D, dyy = (dv - dvb) * D;
+            const T ws = et * dt_ + eb * db;
+            const T de2 = sx * dxx + sy * dyy + T(0.5) * (ws + lane_right(ws));
+            deH = eH * (a.P.glen_p * de2) * row_rcp(e2) + eta * dH;
+            Sxx = T(2) * (eH * (T(2) * dxx + dyy) + sx * deH);
+            Syy = T(2) * (eH * (dxx + T(2) * dyy) + sy * deH);
+        }
+        {
+            T(*p)[kRowLanes] = s.up[w];
+            p[0][lane] = eH; p[1][lane] = Syy; p[2][lane] = H; p[3][lane] = S; p[4][lane] = bp;
+            if constexpr (JVP) { p[kUp - 3][lane] = deH; p[kUp - 2][lane] = dH; p[kUp - 1][lane] = g; }
+        }
+
+        // u facet (i, j) but for the shear of its vertices, and its mass flux
+        T Fx = T(0);
+        {
+            const T Hl = lane_left(H), Sl = lane_left(S), Sxl = lane_left(Sxx), be = T(0.5) * (lane_left(bp) + bp);
+            const T sp = u * u + T(10), rs = row_rsqrt(sp), al = sp * rs, Hm = T(0.5) * (Hl + H);
+            T pw = T(1), dpw = T(0);
+            if constexpr (DRAG) {
+                const T z = u * u + T(0.25) * (vl * vl + v * v + vbl * vbl + vb * vb) + a.P.u_reg;
+                pw = pow(z, a.P.drag_q);
+                if constexpr (JVP) dpw = a.P.drag_q * pow(z, a.P.drag_q - T(1));
+            }
+            if constexpr (JVP) {
+                const T dHl = lane_left(dH), gl = lane_left(g);
+                if (jin) Fx = (Hm - T(0.5) * (u * rs) * (H - Hl)) * du + T(0.5) * ((u + al) * dHl + (u - al) * dH);
+                ru = (Sxx - Sxl) * D - (be * (T(2) * dpw * u * u + pw) + a.P.water_drag) * du;
+                if constexpr (DRAG) ru -= be * T(0.5) * dpw * u * (vl * dvl + v * dv + vbl * dvbl + vb * dvb);
+                ru -= (T(0.5) * (dHl + dH) * (S - Sl) + Hm * (g * dH - gl * dHl)) * D;
+            } else {
+                if (jin) Fx = Hm * u - T(0.5) * al * (H - Hl);
+                ru = (Sxx - Sxl) * D - (be * pw + a.P.water_drag) * u - Hm * (S - Sl) * D;
+            }
+        }
+        __syncthreads();
+
+        // the top-left vertex and the v facet (i, j)
+        T Txy = T(0), Fy = T(0);
+        rv = T(0);
+        if (w > 0) {
+            const T(*p)[kRowLanes] = s.up[w - 1];
+            const T eHs = eH + p[0][lane], Syt = p[1][lane], Ht = p[2][lane], St = p[3][lane];
+            const T be = T(0.5) * (p[4][lane] + bp);
+            const T eHv = T(0.25) * (eHs + lane_left(eHs));
+            T deHs = T(0), dHt = T(0), gt = T(0);
+            if constexpr (JVP) { deHs = deH + p[kUp - 3][lane]; dHt = p[kUp - 2][lane]; gt = p[kUp - 1][lane]; }
+            if constexpr (JVP) Txy = T(2) * (eHv * dt_ + et * (T(0.25) * (deHs + lane_left(deHs))));
+            else Txy = T(2) * eHv * et;
+            const T Txr = lane_right(Txy);  // zero beyond the domain's vertices
+            const T sp = v * v + T(10), rs = row_rsqrt(sp), al = sp * rs, Hm = T(0.5) * (Ht + H);
+            const bool iin = i > 0 && i < ny;
+            T pw = T(1), dpw = T(0);
+            if constexpr (DRAG) {
+                const T utr = lane_right(ut);
+                const T z = v * v + T(0.25) * (ut * ut + utr * utr + u * u + ur * ur) + a.P.u_reg;
+                pw = pow(z, a.P.drag_q);
+                if constexpr (JVP) dpw = a.P.drag_q * pow(z, a.P.drag_q - T(1));
+            }
+            if constexpr (JVP) {
+                if (iin) Fy = (Hm - T(0.5) * (v * rs) * (Ht - H)) * dv + T(0.5) * ((v - al) * dHt + (v + al) * dH);
+                rv = (Syt - Syy) * D + (Txr - Txy) * D - (be * (T(2) * dpw * v * v + pw) + a.P.water_drag) * dv;
+                if constexpr (DRAG) {
+                    const T utr = lane_right(ut), dutr = lane_right(dut);
+                    rv -= be * T(0.5) * dpw * v * (ut * dut + utr * dutr + u * du + ur * dur);
+                }
+                rv -= (T(0.5) * (dHt + dH) * (St - S) + Hm * (gt * dHt - g * dH)) * D;
+            } else {
+                if (iin) Fy = Hm * v - T(0.5) * al * (Ht - H);
+                rv = (Syt - Syy) * D + (Txr - Txy) * D - (be * pw + a.P.water_drag) * v - Hm * (St - S) * D;
+            }
+            s.down[w][0][lane] = Txy;
+            s.down[w][1][lane] = Fy;
+        }
+        __syncthreads();
+
+        rH = T(0);
+        if (w > 0 && w < NW - 1) {
+            const T(*q)[kRowLanes] = s.down[w + 1];
+            ru += (Txy - q[0][lane]) * D;
+            const T Hq = JVP ? dH : H;
+            rH = Hq / a.dt + ((lane_right(Fx) - Fx) + (Fy - q[1][lane])) * D;
+            if (calving_rate != T(0)) {
+                const long rt = (long)clampi(ic - 1, 0, ny - 1) * nx, rb = (long)clampi(ic + 1, 0, ny - 1) * nx;
+                const int jl = clampi(jc - 1, 0, nx - 1), jr = clampi(jc + 1, 0, nx - 1);
+                const T k = (T(1) - phi) * ((T(1) - (a.phi + rc)[jl]) + (T(1) - (a.phi + rc)[jr]) +
+                                            (T(1) - (a.phi + rt)[jc]) + (T(1) - (a.phi + rb)[jc]));
+                rH += k * calving_rate * Hq * D;
+            }
+        }
+    }
+};
+
 }  // namespace glide

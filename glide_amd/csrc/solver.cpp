@@ -1750,10 +1750,14 @@ struct EnsRec {
     template <typename T>
     int residual(const std::vector<const glide_level*>& Ls, const std::vector<int>& flags, const std::vector<void*>& out,
                  int stride) {
+        if (Ls.empty()) return GLIDE_OK;
+        const int linear = make_phys(Ls[0]->phys).linear_drag;
         std::vector<TabResidual<T>> jobs;
         std::vector<int> blocks;
         for (size_t q = 0; q < Ls.size(); ++q) {
             const glide_level& L = *Ls[q];
+            if (make_phys(L.phys).linear_drag != linear)
+                return fail(GLIDE_ERR_INVALID_ARG, "the ensemble's domains must share the drag law");
             TabResidual<T> J{};
             J.a = make_args_t<T>(L, dt, false);
             J.ou = PT<T>(out[q * stride + 0]);
@@ -1765,7 +1769,7 @@ struct EnsRec {
             blocks.push_back(tab_blocks_residual(L.ny, L.nx, &J.gx));
             jobs.push_back(J);
         }
-        prog.add(sizeof(T) == 4 ? kKRes32 : kKRes64, jobs, blocks);
+        prog.add(sizeof(T) == 4 ? kKRes32 : kKRes64, jobs, blocks, 0, linear);
         return GLIDE_OK;
     }
 
@@ -2474,10 +2478,12 @@ int run_tab_op(const TabOp& op, const unsigned char* dev, hipStream_t st) {
         case kKEw: e = launch_tab_ew(static_cast<const TabEw*>(jobs), start, op.n, op.blocks, st); break;
         case kKXfer: e = launch_tab_xfer(static_cast<const TabXfer*>(jobs), start, op.n, op.blocks, st); break;
         case kKRes32:
-            e = launch_tab_residual<float>(static_cast<const TabResidual<float>*>(jobs), start, op.n, op.blocks, st);
+            e = launch_tab_residual<float>(static_cast<const TabResidual<float>*>(jobs), start, op.n, op.blocks,
+                                           op.linear != 0, st);
             break;
         case kKRes64:
-            e = launch_tab_residual<double>(static_cast<const TabResidual<double>*>(jobs), start, op.n, op.blocks, st);
+            e = launch_tab_residual<double>(static_cast<const TabResidual<double>*>(jobs), start, op.n, op.blocks,
+                                           op.linear != 0, st);
             break;
         case kKMc32:
             e = launch_tab_vanka_mc<float>(static_cast<const TabVankaMc<float>*>(jobs), start, op.n, op.blocks,

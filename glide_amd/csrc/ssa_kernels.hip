@@ -51,263 +51,6 @@ __global__ __launch_bounds__(256) void k_grounded(T* __restrict__ phi, const T* 
     phi[k] = relax == T(0) ? g : (T(1) - relax) * g + relax * phi[k];
 }
 
-// ------------------------------------------------------------------ residual
-// Kernel bodies take their block index (bx, by) as arguments, so that the
-// domain-table launches (one launch over many domains) run them unchanged.
-template <typename T>
-__device__ __forceinline__ void residual_body(int bx, int by, const SsaArgs<T>& a, T* __restrict__ out_u,
-                                              T* __restrict__ out_v, T* __restrict__ out_H, int use_forcing,
-                                              int use_mask, T calving_rate) {
-    __shared__ T s_eta[TY + 2][TX + 2];
-    const int ny = a.ny, nx = a.nx;
-    const T dxi = a.dxi;
-    const int i0 = by * TY, j0 = bx * TX;
-    const int tid = threadIdx.y * TX + threadIdx.x;
-    for (int k = tid; k < (TY + 2) * (TX + 2); k += NT) {
-        int ci = i0 - 1 + k / (TX + 2), cj = j0 - 1 + k % (TX + 2);
-        T e = T(0);
-        if (ci >= 0 && ci < ny && cj >= 0 && cj < nx) e = cell_viscosity(a.u, a.v, a.B, ci, cj, ny, nx, dxi, a.P);
-        s_eta[k / (TX + 2)][k % (TX + 2)] = e;
-    }
-    __syncthreads();
-    const int i = i0 + threadIdx.y, j = j0 + threadIdx.x;
-    if (i > ny || j > nx) return;
-    const int li = threadIdx.y + 1, lj = threadIdx.x + 1;
-    const T* __restrict__ u = a.u;
-    const T* __restrict__ v = a.v;
-    const T* __restrict__ H = a.H;
-    const T* __restrict__ ph = a.phi;
-
-    if (i < ny && j < nx) {
-        const long c = (long)i * nx + j;
-        T Hc = H[c], pc = ph[c];
-        T Hl = H[offC(i, j - 1, ny, nx)], Hr = H[offC(i, j + 1, ny, nx)];
-        T Ht = H[offC(i - 1, j, ny, nx)], Hb = H[offC(i + 1, j, ny, nx)];
-        T rH = Hc / a.dt;
-        if (use_forcing) rH -= a.f_H[c];
-        rH -= flux_x(u[offU(i, j, ny, nx)], Hl, Hc, j > 0).res * dxi;
-        rH += (T(1) - pc) * (T(1) - ph[offC(i, j - 1, ny, nx)]) * calving_rate * Hc * dxi;
-        rH += flux_x(u[offU(i, j + 1, ny, nx)], Hc, Hr, j + 1 < nx).res * dxi;
-        rH += (T(1) - pc) * (T(1) - ph[offC(i, j + 1, ny, nx)]) * calving_rate * Hc * dxi;
-        rH += flux_y(v[offV(i, j, ny, nx)], Ht, Hc, i > 0).res * dxi;
-        rH += (T(1) - pc) * (T(1) - ph[offC(i - 1, j, ny, nx)]) * calving_rate * Hc * dxi;
-        rH -= flux_y(v[offV(i + 1, j, ny, nx)], Hc, Hb, i + 1 < ny).res * dxi;
-        rH += (T(1) - pc) * (T(1) - ph[offC(i + 1, j, ny, nx)]) * calving_rate * Hc * dxi;
-        T mk = use_mask ? a.mask[c] : T(0);
-        out_H[c] = (T(1) - mk) * rH + mk * (Hc - a.gamma[c]);
-    }
-    if (i < ny) {
-        const long o = (long)i * (nx + 1) + j;
-        T ru;
-        if (j == 0 || j == nx) {
-            ru = u[o];
-        } else {
-            ru = use_forcing ? -a.f_u[o] : T(0);
-            T ul = u[o];
-            T Hc = H[(long)i * nx + j], Hl = H[(long)i * nx + j - 1];
-            T vt = v[(long)i * nx + j], vb = v[(long)(i + 1) * nx + j];
-            T vlt = v[(long)i * nx + j - 1], vlb = v[(long)(i + 1) * nx + j - 1];
-            ru += sxx(ul, u[o + 1], vt, vb, s_eta[li][lj] * Hc, dxi, true).res * dxi;
-            ru -= sxx(u[o - 1], ul, vlt, vlb, s_eta[li][lj - 1] * Hl, dxi, true).res * dxi;
-            if (i > 0) {
-                T eH = T(0.25) * (s_eta[li - 1][lj - 1] * H[(long)(i - 1) * nx + j - 1] +
-                                  s_eta[li - 1][lj] * H[(long)(i - 1) * nx + j] + s_eta[li][lj - 1] * Hl +
-                                  s_eta[li][lj] * Hc);
-                ru += sxy(u[o - (nx + 1)], ul, vlt, vt, eH, dxi, true).res * dxi;
-            }
-            if (i + 1 < ny) {
-                T eH = T(0.25) * (s_eta[li][lj - 1] * Hl + s_eta[li][lj] * Hc +
-                                  s_eta[li + 1][lj - 1] * H[(long)(i + 1) * nx + j - 1] +
-                                  s_eta[li + 1][lj] * H[(long)(i + 1) * nx + j]);
-                ru -= sxy(ul, u[o + (nx + 1)], vlb, vb, eH, dxi, true).res * dxi;
-            }
-            T pl = ph[(long)i * nx + j - 1], pc = ph[(long)i * nx + j];
-            ru += basal_drag(ul, vlt, vt, vlb, vb, pl, pc, a.beta[(long)i * nx + j - 1], a.beta[(long)i * nx + j], a.P)
-                      .res;
-            ru -= drive_x(Hl, Hc, a.bed[(long)i * nx + j - 1], a.bed[(long)i * nx + j], pl, pc, dxi, true).res;
-        }
-        out_u[o] = ru;
-    }
-    if (j < nx) {
-        const long o = (long)i * nx + j;
-        T rv;
-        if (i == 0 || i == ny) {
-            rv = v[o];
-        } else {
-            rv = use_forcing ? -a.f_v[o] : T(0);
-            T vt = v[o];
-            T Hc = H[o], Ht = H[o - nx];
-            T ul = u[(long)i * (nx + 1) + j], ur = u[(long)i * (nx + 1) + j + 1];
-            T utl = u[(long)(i - 1) * (nx + 1) + j], utr = u[(long)(i - 1) * (nx + 1) + j + 1];
-            rv += syy(utl, utr, v[o - nx], vt, s_eta[li - 1][lj] * Ht, dxi, true).res * dxi;
-            rv -= syy(ul, ur, vt, v[o + nx], s_eta[li][lj] * Hc, dxi, true).res * dxi;
-            if (j > 0) {
-                T eH = T(0.25) * (s_eta[li - 1][lj - 1] * H[o - nx - 1] + s_eta[li - 1][lj] * Ht +
-                                  s_eta[li][lj - 1] * H[o - 1] + s_eta[li][lj] * Hc);
-                rv -= sxy(utl, ul, v[o - 1], vt, eH, dxi, true).res * dxi;
-            }
-            if (j + 1 < nx) {
-                T eH = T(0.25) * (s_eta[li - 1][lj] * Ht + s_eta[li - 1][lj + 1] * H[o - nx + 1] +
-                                  s_eta[li][lj] * Hc + s_eta[li][lj + 1] * H[o + 1]);
-                rv += sxy(utr, ur, vt, v[o + 1], eH, dxi, true).res * dxi;
-            }
-            T pt = ph[o - nx], pc = ph[o];
-            rv += basal_drag(vt, utl, utr, ul, ur, pt, pc, a.beta[o - nx], a.beta[o], a.P).res;
-            rv -= drive_y(Ht, Hc, a.bed[o - nx], a.bed[o], pt, pc, dxi, true).res;
-        }
-        out_v[o] = rv;
-    }
-}
-
-template <typename T>
-__global__ __launch_bounds__(NT) void k_residual(SsaArgs<T> a, T* __restrict__ out_u, T* __restrict__ out_v,
-                                                 T* __restrict__ out_H, int use_forcing, int use_mask,
-                                                 T calving_rate) {
-    residual_body<T>(blockIdx.x, blockIdx.y, a, out_u, out_v, out_H, use_forcing, use_mask, calving_rate);
-}
-
-// ------------------------------------------------------------------ JVP
-// J(x) d of the coupled residual along d = (du, dv, dH) with the grounded
-// fraction, mask, bed, B and beta frozen (glide/cuda/residuals.cu:340-660):
-// the derivative of k_residual term by term.  Dirichlet facet rows are zero
-// and the thickness row is (1 - mask) times the mass-balance derivative, as
-// in the reference.  The tile holds each cell's viscosity and its derivative
-// along d.
-template <typename T>
-__global__ __launch_bounds__(NT) void k_jvp(SsaArgs<T> a, const T* __restrict__ du, const T* __restrict__ dv,
-                                            const T* __restrict__ dH, T* __restrict__ out_u, T* __restrict__ out_v,
-                                            T* __restrict__ out_H, int use_mask, T calving_rate) {
-    __shared__ T s_eta[TY + 2][TX + 2];
-    __shared__ T s_etd[TY + 2][TX + 2];
-    const int ny = a.ny, nx = a.nx;
-    const T dxi = a.dxi;
-    const int i0 = blockIdx.y * TY, j0 = blockIdx.x * TX;
-    const int tid = threadIdx.y * TX + threadIdx.x;
-    for (int k = tid; k < (TY + 2) * (TX + 2); k += NT) {
-        int ci = i0 - 1 + k / (TX + 2), cj = j0 - 1 + k % (TX + 2);
-        T e = T(0), ed = T(0);
-        if (ci >= 0 && ci < ny && cj >= 0 && cj < nx) {
-            CellVel<T> c = load_cell_vel(a.u, a.v, ci, cj, ny, nx);
-            CellVel<T> d = load_cell_vel(du, dv, ci, cj, ny, nx);
-            T e2 = strain_invariant(c, ci, cj, ny, nx, dxi, a.P.eps_reg);
-            T de2 = strain_invariant_dir(c, d, ci, cj, ny, nx, dxi);
-            e = T(0.5) * a.B[(long)ci * nx + cj] * glen_power(e2, a.P);
-            ed = e * a.P.glen_p * de2 / e2;
-        }
-        s_eta[k / (TX + 2)][k % (TX + 2)] = e;
-        s_etd[k / (TX + 2)][k % (TX + 2)] = ed;
-    }
-    __syncthreads();
-    const int i = i0 + threadIdx.y, j = j0 + threadIdx.x;
-    if (i > ny || j > nx) return;
-    const int li = threadIdx.y + 1, lj = threadIdx.x + 1;
-    const T* __restrict__ u = a.u;
-    const T* __restrict__ v = a.v;
-    const T* __restrict__ H = a.H;
-    const T* __restrict__ ph = a.phi;
-    // eta H of tile cell (ti, tj) at grid cell c and its derivative along d
-    auto eH = [&](int ti, int tj, long c) { return s_eta[ti][tj] * H[c]; };
-    auto deH = [&](int ti, int tj, long c) { return s_etd[ti][tj] * H[c] + s_eta[ti][tj] * dH[c]; };
-
-    if (i < ny && j < nx) {
-        const long c = (long)i * nx + j;
-        T Hc = H[c], pc = ph[c], dHc = dH[c];
-        const long cl = offC(i, j - 1, ny, nx), cr = offC(i, j + 1, ny, nx);
-        const long ct = offC(i - 1, j, ny, nx), cb = offC(i + 1, j, ny, nx);
-        T d = dHc / a.dt;
-        Flux<T> f = flux_x(u[offU(i, j, ny, nx)], H[cl], Hc, j > 0);
-        d -= (f.d_w * du[offU(i, j, ny, nx)] + f.d_HA * dH[cl] + f.d_HB * dHc) * dxi;
-        d += (T(1) - pc) * (T(1) - ph[cl]) * calving_rate * dHc * dxi;
-        f = flux_x(u[offU(i, j + 1, ny, nx)], Hc, H[cr], j + 1 < nx);
-        d += (f.d_w * du[offU(i, j + 1, ny, nx)] + f.d_HA * dHc + f.d_HB * dH[cr]) * dxi;
-        d += (T(1) - pc) * (T(1) - ph[cr]) * calving_rate * dHc * dxi;
-        f = flux_y(v[offV(i, j, ny, nx)], H[ct], Hc, i > 0);
-        d += (f.d_w * dv[offV(i, j, ny, nx)] + f.d_HA * dH[ct] + f.d_HB * dHc) * dxi;
-        d += (T(1) - pc) * (T(1) - ph[ct]) * calving_rate * dHc * dxi;
-        f = flux_y(v[offV(i + 1, j, ny, nx)], Hc, H[cb], i + 1 < ny);
-        d -= (f.d_w * dv[offV(i + 1, j, ny, nx)] + f.d_HA * dHc + f.d_HB * dH[cb]) * dxi;
-        d += (T(1) - pc) * (T(1) - ph[cb]) * calving_rate * dHc * dxi;
-        T mk = use_mask ? a.mask[c] : T(0);
-        out_H[c] = (T(1) - mk) * d;
-    }
-    if (i < ny) {
-        const long o = (long)i * (nx + 1) + j;
-        T d = T(0);
-        if (j > 0 && j < nx) {
-            const long c = (long)i * nx + j;
-            T ul = u[o], dul = du[o];
-            T vt = v[c], vb = v[c + nx], vlt = v[c - 1], vlb = v[c + nx - 1];
-            T dvt = dv[c], dvb = dv[c + nx], dvlt = dv[c - 1], dvlb = dv[c + nx - 1];
-            NormalStress<T> s = sxx(ul, u[o + 1], vt, vb, eH(li, lj, c), dxi, true);
-            d += (s.d_ul * dul + s.d_ur * du[o + 1] + s.d_vt * dvt + s.d_vb * dvb + s.d_eH * deH(li, lj, c)) * dxi;
-            s = sxx(u[o - 1], ul, vlt, vlb, eH(li, lj - 1, c - 1), dxi, true);
-            d -= (s.d_ul * du[o - 1] + s.d_ur * dul + s.d_vt * dvlt + s.d_vb * dvlb +
-                  s.d_eH * deH(li, lj - 1, c - 1)) * dxi;
-            if (i > 0) {
-                T e = T(0.25) * (eH(li - 1, lj - 1, c - nx - 1) + eH(li - 1, lj, c - nx) + eH(li, lj - 1, c - 1) +
-                                 eH(li, lj, c));
-                T de = T(0.25) * (deH(li - 1, lj - 1, c - nx - 1) + deH(li - 1, lj, c - nx) +
-                                  deH(li, lj - 1, c - 1) + deH(li, lj, c));
-                ShearStress<T> t = sxy(u[o - (nx + 1)], ul, vlt, vt, e, dxi, true);
-                d += (t.d_ut * du[o - (nx + 1)] + t.d_ub * dul + t.d_vl * dvlt + t.d_vr * dvt + t.d_eH * de) * dxi;
-            }
-            if (i + 1 < ny) {
-                T e = T(0.25) * (eH(li, lj - 1, c - 1) + eH(li, lj, c) + eH(li + 1, lj - 1, c + nx - 1) +
-                                 eH(li + 1, lj, c + nx));
-                T de = T(0.25) * (deH(li, lj - 1, c - 1) + deH(li, lj, c) + deH(li + 1, lj - 1, c + nx - 1) +
-                                  deH(li + 1, lj, c + nx));
-                ShearStress<T> t = sxy(ul, u[o + (nx + 1)], vlb, vb, e, dxi, true);
-                d -= (t.d_ut * dul + t.d_ub * du[o + (nx + 1)] + t.d_vl * dvlb + t.d_vr * dvb + t.d_eH * de) * dxi;
-            }
-            T pl = ph[c - 1], pc = ph[c];
-            Drag<T> g = basal_drag(ul, vlt, vt, vlb, vb, pl, pc, a.beta[c - 1], a.beta[c], a.P);
-            d += g.d_w * dul + g.c0 * dvlt + g.c1 * dvt + g.c2 * dvlb + g.c3 * dvb;
-            Drive<T> r = drive_x(H[c - 1], H[c], a.bed[c - 1], a.bed[c], pl, pc, dxi, true);
-            d -= r.d_HA * dH[c - 1] + r.d_HB * dH[c];
-
-        }
-        out_u[o] = d;
-    }
-    if (j < nx) {
-        const long o = (long)i * nx + j;
-        T d = T(0);
-        if (i > 0 && i < ny) {
-            const long ou = (long)i * (nx + 1) + j, ot = ou - (nx + 1);
-            T vt = v[o], dvt = dv[o];
-            T ul = u[ou], ur = u[ou + 1], utl = u[ot], utr = u[ot + 1];
-            T dul = du[ou], dur = du[ou + 1], dutl = du[ot], dutr = du[ot + 1];
-            NormalStress<T> s = syy(utl, utr, v[o - nx], vt, eH(li - 1, lj, o - nx), dxi, true);
-            d += (s.d_ul * dutl + s.d_ur * dutr + s.d_vt * dv[o - nx] + s.d_vb * dvt +
-                  s.d_eH * deH(li - 1, lj, o - nx)) * dxi;
-            s = syy(ul, ur, vt, v[o + nx], eH(li, lj, o), dxi, true);
-            d -= (s.d_ul * dul + s.d_ur * dur + s.d_vt * dvt + s.d_vb * dv[o + nx] + s.d_eH * deH(li, lj, o)) * dxi;
-            if (j > 0) {
-                T e = T(0.25) * (eH(li - 1, lj - 1, o - nx - 1) + eH(li - 1, lj, o - nx) + eH(li, lj - 1, o - 1) +
-                                 eH(li, lj, o));
-                T de = T(0.25) * (deH(li - 1, lj - 1, o - nx - 1) + deH(li - 1, lj, o - nx) +
-                                  deH(li, lj - 1, o - 1) + deH(li, lj, o));
-                ShearStress<T> t = sxy(utl, ul, v[o - 1], vt, e, dxi, true);
-                d -= (t.d_ut * dutl + t.d_ub * dul + t.d_vl * dv[o - 1] + t.d_vr * dvt + t.d_eH * de) * dxi;
-            }
-            if (j + 1 < nx) {
-                T e = T(0.25) * (eH(li - 1, lj, o - nx) + eH(li - 1, lj + 1, o - nx + 1) + eH(li, lj, o) +
-                                 eH(li, lj + 1, o + 1));
-                T de = T(0.25) * (deH(li - 1, lj, o - nx) + deH(li - 1, lj + 1, o - nx + 1) + deH(li, lj, o) +
-                                  deH(li, lj + 1, o + 1));
-                ShearStress<T> t = sxy(utr, ur, vt, v[o + 1], e, dxi, true);
-                d += (t.d_ut * dutr + t.d_ub * dur + t.d_vl * dvt + t.d_vr * dv[o + 1] + t.d_eH * de) * dxi;
-            }
-            T pt = ph[o - nx], pc = ph[o];
-            Drag<T> g = basal_drag(vt, utl, utr, ul, ur, pt, pc, a.beta[o - nx], a.beta[o], a.P);
-            d += g.d_w * dvt + g.c0 * dutl + g.c1 * dutr + g.c2 * dul + g.c3 * dur;
-            Drive<T> r = drive_y(H[o - nx], H[o], a.bed[o - nx], a.bed[o], pt, pc, dxi, true);
-            d -= r.d_HA * dH[o - nx] + r.d_HB * dH[o];
-
-        }
-        out_v[o] = d;
-    }
-}
-
 // ------------------------------------------------------------------ Vanka
 // Gather the patch of cell (i,j); viscosity from the LDS tile (li, lj are the
 // cell's tile coordinates including the one-cell ring).
@@ -1524,23 +1267,6 @@ hipError_t launch_grounded(T* phi, const T* H, const T* bed, T c, T relax, long 
 }
 
 template <typename T>
-hipError_t launch_residual(const SsaArgs<T>& a, T* ou, T* ov, T* oH, int use_forcing, int use_mask, T calving_rate,
-                           hipStream_t st) {
-    TimedLaunch tl(kTimeResidual, (long)a.ny * a.nx, st);
-    k_residual<T><<<tile_grid(a.ny, a.nx, true), dim3(TX, TY), 0, st>>>(a, ou, ov, oH, use_forcing, use_mask,
-                                                                         calving_rate);
-    return hipGetLastError();
-}
-
-template <typename T>
-hipError_t launch_jvp(const SsaArgs<T>& a, const T* du, const T* dv, const T* dH, T* ou, T* ov, T* oH, int use_mask,
-                      T calving_rate, hipStream_t st) {
-    k_jvp<T><<<tile_grid(a.ny, a.nx, true), dim3(TX, TY), 0, st>>>(a, du, dv, dH, ou, ov, oH, use_mask,
-                                                                     calving_rate);
-    return hipGetLastError();
-}
-
-template <typename T>
 hipError_t launch_vanka_pass(const SsaArgs<T>& a, T* u, T* v, T* H, T* work, T* mask, const VankaArgs<T>& vk, T omega,
                              T* phi_next, T relax_phi, hipStream_t st) {
     {
@@ -1765,14 +1491,6 @@ hipError_t launch_zero_masked(T* g, const T* mask, long n, hipStream_t st) {
 // ------------------------------------------------------------ domain tables
 // One launch over many domains (tab.hpp): each block runs the single-domain
 // body of its job with its block index inside the job's own grid.
-template <typename T>
-__global__ __launch_bounds__(NT) void k_tab_residual(const TabResidual<T>* __restrict__ jobs,
-                                                     const int* __restrict__ start, int n) {
-    const int e = tab_find(start, n, blockIdx.x);
-    const TabResidual<T> J = jobs[e];
-    const int lb = blockIdx.x - start[e];
-    residual_body<T>(lb % J.gx, lb / J.gx, J.a, J.ou, J.ov, J.oH, J.use_forcing, J.use_mask, J.cr);
-}
 
 template <typename T>
 __global__ __launch_bounds__(NT) void k_tab_adj_factor(const TabAdjFactor<T>* __restrict__ jobs,
@@ -1792,11 +1510,6 @@ __global__ __launch_bounds__(256) void k_tab_grad(const TabGrad<T>* __restrict__
     grad_beta_bed_body<T>(lb % J.gx, lb / J.gx, J.a, J.lu, J.lv, J.gbeta, J.gbed, J.exact);
 }
 
-int tab_blocks_residual(int ny, int nx, int* gx) {
-    const dim3 g = tile_grid(ny, nx, true);
-    *gx = (int)g.x;
-    return (int)(g.x * g.y);
-}
 int tab_blocks_adj_factor(int ny, int nx, int* gx) {
     const dim3 g = tile_grid(ny, nx, false);
     *gx = (int)g.x;
@@ -1807,12 +1520,6 @@ int tab_blocks_grad(int ny, int nx, int* gx) {
     return *gx * ny;
 }
 
-template <typename T>
-hipError_t launch_tab_residual(const TabResidual<T>* jobs, const int* start, int n, int blocks, hipStream_t st) {
-    if (n <= 0 || blocks <= 0) return hipSuccess;
-    k_tab_residual<T><<<blocks, dim3(TX, TY), 0, st>>>(jobs, start, n);
-    return hipGetLastError();
-}
 template <typename T>
 hipError_t launch_tab_adj_factor(const TabAdjFactor<T>* jobs, const int* start, int n, int blocks, hipStream_t st) {
     if (n <= 0 || blocks <= 0) return hipSuccess;
@@ -1827,7 +1534,6 @@ hipError_t launch_tab_grad(const TabGrad<T>* jobs, const int* start, int n, int 
 }
 
 #define GLIDE_TAB_INSTANTIATE(T)                                                                                     \
-    template hipError_t launch_tab_residual<T>(const TabResidual<T>*, const int*, int, int, hipStream_t);            \
     template hipError_t launch_tab_adj_factor<T>(const TabAdjFactor<T>*, const int*, int, int, hipStream_t);         \
     template hipError_t launch_tab_grad<T>(const TabGrad<T>*, const int*, int, int, hipStream_t);
 
@@ -1836,9 +1542,6 @@ GLIDE_TAB_INSTANTIATE(float)
 
 #define GLIDE_INSTANTIATE(T)                                                                                         \
     template hipError_t launch_grounded<T>(T*, const T*, const T*, T, T, long, hipStream_t);                          \
-    template hipError_t launch_residual<T>(const SsaArgs<T>&, T*, T*, T*, int, int, T, hipStream_t);                  \
-    template hipError_t launch_jvp<T>(const SsaArgs<T>&, const T*, const T*, const T*, T*, T*, T*, int, T,      \
-                                      hipStream_t);                                                           \
     template hipError_t launch_vanka_pass<T>(const SsaArgs<T>&, T*, T*, T*, T*, T*, const VankaArgs<T>&, T, T*, T,   \
                                              hipStream_t);                                                           \
     template hipError_t launch_vanka_dump<T>(const SsaArgs<T>&, T*, T*, T, hipStream_t);                              \

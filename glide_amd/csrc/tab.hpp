@@ -133,7 +133,8 @@ int tab_blocks_xfer(int op, int ny, int nx, int* gx);
 inline int tab_blocks_ew(long n) { return (int)((n + kTabEwPerBlock - 1) / kTabEwPerBlock); }
 
 template <typename T>
-hipError_t launch_tab_residual(const TabResidual<T>* jobs, const int* start, int n, int blocks, hipStream_t st);
+hipError_t launch_tab_residual(const TabResidual<T>* jobs, const int* start, int n, int blocks, bool linear,
+                               hipStream_t st);
 template <typename T>
 hipError_t launch_tab_vanka_mc(const TabVankaMc<T>* jobs, const int* start, int n, int blocks, bool linear, int rows,
                                hipStream_t st);

@@ -103,6 +103,37 @@ def test_jvp(orc, shape, m, calving, use_mask):
     assert np.all(N(fo.jvp_u)[:, [0, -1]] == 0) and np.all(N(fo.jvp_v)[[0, -1]] == 0)
 
 
+@pytest.mark.parametrize("shape", [(5, 59), (6, 60), (7, 61), (12, 119), (13, 121), (2, 2)])
+@pytest.mark.parametrize("m", [1.0, 1.0 / 3.0])
+def test_row_operators_at_tile_edges(orc, shape, m):
+    """Residual, J d and J^T lambda at the edges of the row kernels' tiles
+    (6 rows, 60 columns), with calving, against the oracle (the bar of the
+    other sizes)."""
+    ny, nx = shape
+    print(f"row operators shape={shape} m={m:.3f}", flush=True)
+    F = dome_fields(ny=ny, nx=nx, seed=35, mask_frac=0.2)
+    P = orc.phys(m=m, calving_rate=0.3)
+    g = grid_from(F)
+    g.sliding.m.set(m)
+    g.calving.calving_rate.set(0.3)
+    rng = np.random.default_rng(36)
+    d = (rng.standard_normal((ny, nx + 1)), rng.standard_normal((ny + 1, nx)), rng.standard_normal((ny, nx)))
+    fo, ao = g.forward_operators, g.adjoint_operators
+    for t, q in zip((fo.var_u, fo.var_v, fo.var_H), d):
+        t.copy_(T(q))
+    for t, q in zip((g.adjoint.lambda_u, g.adjoint.lambda_v, g.adjoint.lambda_H), d):
+        t.set(T(q))
+    fo.compute_residual(10.0, freeze_phi=True)
+    fo.compute_jvp(10.0, freeze_phi=True)
+    ao.compute_vjp(10.0)
+    torch.cuda.synchronize()
+    for got, ref in (((fo.r_u, fo.r_v, fo.r_H), orc.residual(F, P, 1500.0, 10.0)),
+                     ((fo.jvp_u, fo.jvp_v, fo.jvp_H), orc.jvp(F, *d, P, 1500.0, 10.0)),
+                     ((ao.vjp_u, ao.vjp_v, ao.vjp_H), orc.vjp(F, *d, P, 1500.0, 10.0))):
+        for a, b in zip(got, ref):
+            assert rel_err(N(a), b) < KTOL
+
+
 def test_jvp_freeze_calving_and_phi_refresh(orc):
     """freeze_calving drops the calving term; without freeze_phi the grounded
     fraction is recomputed from H and bed first."""
