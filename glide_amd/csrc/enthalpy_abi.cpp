@@ -148,6 +148,7 @@ int make_args(const glide_enth_column* C, double dt, bool needs_state, EnthArgs<
     a->u2d = nullptr;
     a->v2d = nullptr;
     a->vel_div = 1.0;
+    a->set_constants();
     return GLIDE_OK;
 }
 
@@ -173,21 +174,21 @@ int sweep_core(const glide_enth_column* C, double dt, int n_iter, const glide_en
     const double rtol = cfg->relative_tolerance, atol = cfg->absolute_tolerance;
     if (C->sweep_work && u2d && rmax && cfg->alternating && !cfg->multicolour && cfg->n_newton >= 1 && n_iter >= 1 &&
         enth_lm_supported(C->nz)) {
-        // The same sweep on level-major copies (sweep_work: E, E_prev, f_E,
+        // The same sweep on tiled copies (sweep_work: E, E_prev, f_E,
         // omega planes; E_work holds the column pass's output in that layout).
         const long ncol = (long)C->ny * C->nx, plane = ncol * C->nz;
         R* wk = P(C->sweep_work);
         R *Elm = wk, *Eplm = wk + plane, *fElm = wk + 2 * plane, *omlm = wk + 3 * plane, *Wlm = P(C->E_work);
         const int nz = C->nz;
-        HIP_TRY(launch_enth_lm_layout<R>(CP(C->E), Elm, ncol, nz, true, st), "enthalpy level-major copy");
-        HIP_TRY(launch_enth_lm_layout<R>(CP(C->E_prev), Eplm, ncol, nz, true, st), "enthalpy level-major copy");
-        HIP_TRY(launch_enth_lm_layout<R>(CP(C->f_E), fElm, ncol, nz, true, st), "enthalpy level-major copy");
+        HIP_TRY(launch_enth_lm_layout<R>(CP(C->E), Elm, ncol, nz, true, st), "enthalpy tiled copy");
+        HIP_TRY(launch_enth_lm_layout<R>(CP(C->E_prev), Eplm, ncol, nz, true, st), "enthalpy tiled copy");
+        HIP_TRY(launch_enth_lm_layout<R>(CP(C->f_E), fElm, ncol, nz, true, st), "enthalpy tiled copy");
         EnthArgs<R> L = A;
         L.E = Elm;
         L.E_prev = Eplm;
         L.f_E = fElm;
         if (A.omega) {
-            HIP_TRY(launch_enth_lm_layout<R>(A.omega, omlm, ncol, nz, true, st), "enthalpy level-major copy");
+            HIP_TRY(launch_enth_lm_layout<R>(A.omega, omlm, ncol, nz, true, st), "enthalpy tiled copy");
             L.omega = omlm;
         }
         HIP_TRY(launch_enth_residual_lm<R>(L, nullptr, partials, status, 0, rtol, atol, st), "enthalpy residual");

@@ -17,6 +17,8 @@
 // thread in a level-major checkerboard layout (see the adjoint layout below).
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+
 #include "enthalpy_kernels.hpp"
 #include "ssa_device.hpp"
 
@@ -102,9 +104,16 @@ __device__ __forceinline__ T e_pmp(T sigma, T H) {
     return (t_pmp(sigma, H) - T(kTRef)) * T(kCI / kEScale);
 }
 // glide/cuda/enthalpy.cu:48-98
-template <typename T>
-__device__ __forceinline__ T diffusivity(T E, T Ep) {
+//
+// COLD: ice more than about a kelvin below its melting point sits at the clamp
+// z = -20, most of a column; a wavefront whose lanes are all there takes the
+// value at the clamp (cold_values) instead of its exponential.
+template <typename T, bool COLD = false>
+__device__ __forceinline__ T diffusivity(T E, T Ep, T at_clamp = T(0)) {
     T z = (E - Ep) * T(kEScale) * T(0.01);
+    if constexpr (COLD) {
+        if (!__any(!(z <= T(-20)))) return at_clamp;
+    }
     z = fmin(fmax(z, T(-20)), T(20));
     T s = fast_rcp(T(1) + exp_rows(-z));
     return T(kKCold) * (T(1) - s + T(kKTempFactor) * s);
@@ -116,13 +125,31 @@ __device__ __forceinline__ T diffusivity(T E, T Ep) {
 // exp(a) / (1 + exp(a)) over the latent heat (the reference writes it as
 // 1 / (1 + exp(-a)), equal up to rounding; it only enters the Newton
 // Jacobian).  Both come from one exponential.
+// COLD as for the diffusivity: the clamp a = -20.
 template <typename T>
-__device__ __forceinline__ void water_and_slope(T E, T Ep, T& w, T& dw) {
+struct ColdValues {
+    T K, w, dw;
+};
+template <typename T, bool COLD = false>
+__device__ __forceinline__ void water_and_slope(T E, T Ep, T& w, T& dw, const ColdValues<T>* cold = nullptr) {
     const T x = (E - Ep) * T(kEScale);
+    if constexpr (COLD) {
+        if (!__any(!(T(kDrainSharpness) * x <= T(-20)))) {
+            w = cold->w;
+            dw = cold->dw;
+            return;
+        }
+    }
     const T ax = fmin(fmax(T(kDrainSharpness) * x, T(-20)), T(20));
     const T ez = exp_rows(ax);
     w = ((ax > T(10)) ? x : log_rows(T(1) + ez) * T(1.0 / kDrainSharpness)) * T(1.0 / kLHeat);
     dw = (ez * fast_rcp(T(1) + ez)) * T(1.0 / kLHeat);
+}
+template <typename T>
+ColdValues<T> cold_values() {  // on the host, as the functions above form them
+    const double e = std::exp(-20.0), q = 1.0 / (1.0 + std::exp(20.0));
+    return {T(kKCold * (1.0 - q + kKTempFactor * q)), T(std::log(1.0 + e) * (1.0 / kDrainSharpness) * (1.0 / kLHeat)),
+            T(e / (1.0 + e) * (1.0 / kLHeat))};
 }
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
@@ -233,8 +260,8 @@ __device__ __forceinline__ void interface_K(int k, int nz, T h, T Ek, T Ekp1, T&
     Kl = lane_get(Ku, max(k - 1, 0));
 }
 
-// Per-column constants of the rows: functions of nz, dt and the column's
-// thickness only, formed once per column so that the rows divide by nothing.
+// Per-column constants of the rows: functions of nz and dt (formed on the host)
+// and of the column's thickness, so that the rows divide by nothing.
 template <typename T>
 struct ColConst {
     T dsig, di, hdi, d2, idd;  // 1/(nz-1), 1/dsig, 1/(dsig/2), 1/dsig^2, 1/(dsig dsig/2)
@@ -242,23 +269,16 @@ struct ColConst {
 };
 template <typename T>
 __device__ __forceinline__ ColConst<T> col_const(const EnthArgs<T>& A, T h) {
-    ColConst<T> c;
-    c.dsig = T(1) / T(A.nz - 1);
-    c.di = T(1) / c.dsig;
-    c.hdi = T(1) / (T(0.5) * c.dsig);
-    c.d2 = T(1) / (c.dsig * c.dsig);
-    c.idd = T(1) / (c.dsig * (T(0.5) * c.dsig));
-    c.hinv = T(1) / h;
-    c.invdt = T(1) / A.dt;
-    return c;
+    return {A.dsig, A.di, A.hdi, A.d2, A.idd, T(1) / h, A.invdt};
 }
 
 // The column's own terms of level k's row (sigma advection, diffusion with
 // the interface diffusivities Ku / Kl from interface_K, drainage), added to
 // w, which holds the time and horizontal terms.
-template <typename T>
+template <typename T, bool COLD = false>
 __device__ __forceinline__ void column_terms(const EnthArgs<T>& A, const ColConst<T>& c, int k, T h, T Ek, T Ekm1,
-                                             T Ekp1, T om_m, T om_k, T om_p, T Ku, T Kl, Row<T>& w) {
+                                             T Ekp1, T om_m, T om_k, T om_p, T Ku, T Kl, Row<T>& w,
+                                             const ColdValues<T>* cold = nullptr) {
     const T Ep_k = e_pmp(T(k) * c.dsig, h);
     if (k == 0) {
         if (A.flags & 2) {
@@ -290,7 +310,7 @@ __device__ __forceinline__ void column_terms(const EnthArgs<T>& A, const ColCons
     }
     if (A.flags & 4) {
         T wc, dwc;
-        water_and_slope(Ek, Ep_k, wc, dwc);
+        water_and_slope<T, COLD>(Ek, Ep_k, wc, dwc, cold);
         w.r += h * T(kRhoW) * T(kLHeat) * (A.drain_rate * wc) * T(1.0 / kEScale);
         w.b += h * T(kRhoW) * T(kLHeat) * A.drain_rate * dwc;
     }
@@ -1532,20 +1552,20 @@ hipError_t launch_enth_elementary(const double* x, long n, double* e_out, double
     return hipGetLastError();
 }
 
-// ------------------------------------------------ level-major fused sweep
+// ------------------------------------------------ tiled fused sweep
 // (no counterpart in the reference, whose sweep works on the (ny, nx, nz)
 // arrays, glide/enthalpy.py:426-471).  The sweep of a thermal step runs on
-// (nz, ny * nx) copies of E, E_prev, f_E and omega, in which level k of a run
-// of columns is contiguous.  The column pass gives a column P consecutive
-// lanes (4, 8 or 16), lane q holding levels [q MB, (q + 1) MB), MB = 3 or 4
+// copies of E, E_prev, f_E and omega, in which level k of a run of columns is
+// contiguous (LmCol below).  The column pass gives a column P consecutive
+// lanes (4, 8 or 16), lane q holding levels [q MB, (q + 1) MB), MB = 3 to 8
 // (levels from nz on are identity rows), and solves the column's tridiagonal
 // Newton system by a partitioned Thomas algorithm: each lane eliminates its
 // block down to two rows coupling the block's first and last unknowns to the
 // neighbouring blocks', the first rows are eliminated into one row per lane
 // in the blocks' last unknowns, which cyclic reduction across the P lanes
 // solves, and each lane substitutes back.  Neighbouring lanes exchange values
-// through DPP row shifts, not LDS.  The layer pass and the residual take one
-// thread per column and stream up the levels.  The rows are level_row's, with
+// through DPP row shifts, not LDS.  The layer pass takes a few levels of a tile
+// per wavefront; the residual one thread per column, streaming up the levels.  The rows are level_row's, with
 // the terms that do not depend on the column's own enthalpy (the previous
 // enthalpy, the forcing and the neighbouring columns' advection) gathered
 // into one value per level.
@@ -1570,10 +1590,23 @@ __device__ __forceinline__ double from_above(double x) {  // lane i + S
     return dpp_f64<0x100 + S>(x);
 }
 
-constexpr int kLmCols = 64;  // columns per block of the layout transposes
+// The sweep's layout: tiles of kLmCols consecutive columns, a tile's levels
+// one after another (the last tile as narrow as the columns left, so the planes
+// hold exactly ny nx nz values).  A wavefront's levels then lie within 64 nz
+// values; as whole (nz, ny nx) planes they lay one plane apart, at 512 x 512
+// columns 2 MiB: a page and the same memory channel each, and the column pass
+// waited for memory in four cycles of five at a quarter of its bandwidth.
+constexpr int kLmCols = 64;
+struct LmCol {
+    long base;   // level 0 of the column
+    int stride;  // from a level to the next
+};
+__device__ __forceinline__ LmCol lm_col(long col, long ncol, int nz) {
+    const long c0 = col / kLmCols * kLmCols;
+    return {c0 * nz + (col - c0), (int)min((long)kLmCols, ncol - c0)};
+}
 
-// (ny nx, nz) -> (nz, ny nx) (to_lm) or back, kLmCols columns per block
-// through LDS; both sides are read and written in contiguous runs.
+// (ny nx, nz) -> tiles (to_lm) or back, one tile per block through LDS.
 template <typename T>
 __global__ __launch_bounds__(256) void k_enth_lm_layout(const T* __restrict__ src, T* __restrict__ dst, long ncol,
                                                         int nz, int to_lm) {
@@ -1585,12 +1618,12 @@ __global__ __launch_bounds__(256) void k_enth_lm_layout(const T* __restrict__ sr
         __syncthreads();
         for (int q = threadIdx.x; q < kLmCols * nz; q += blockDim.x) {
             const int k = q / kLmCols, c = q % kLmCols;
-            if (c < nc) dst[(long)k * ncol + c0 + c] = s[c * 65 + k];
+            if (c < nc) dst[c0 * nz + k * nc + c] = s[c * 65 + k];
         }
     } else {
         for (int q = threadIdx.x; q < kLmCols * nz; q += blockDim.x) {
             const int k = q / kLmCols, c = q % kLmCols;
-            if (c < nc) s[c * 65 + k] = src[(long)k * ncol + c0 + c];
+            if (c < nc) s[c * 65 + k] = src[c0 * nz + k * nc + c];
         }
         __syncthreads();
         for (int q = threadIdx.x; q < nc * nz; q += blockDim.x) dst[c0 * nz + q] = s[(q / nz) * 65 + q % nz];
@@ -1605,35 +1638,52 @@ template <typename T>
 struct LmHoriz {
     T self, xp, xm, ym, yp;
 };
+// The loads are unconditional (clamped on the domain edge, whose fluxes are
+// zero): branches around them would wait for each facet's in turn.
 template <typename T>
 __device__ __forceinline__ LmHoriz<T> lm_horiz(const EnthArgs<T>& A, int i, int j) {
-    LmHoriz<T> c{T(0), T(0), T(0), T(0), T(0)};
-    if (!(A.flags & 1)) return c;
-    const Horiz<T> hz = face_fluxes(A, i, j, 0);
+    const int ny = A.ny, nx = A.nx;
+    const long row = (long)i * nx, c = row + j;
+    const T H = A.H[c], Hl = A.H[row + max(j - 1, 0)], Hr = A.H[row + min(j + 1, nx - 1)];
+    const T Ht = A.H[(long)max(i - 1, 0) * nx + j], Hb = A.H[(long)min(i + 1, ny - 1) * nx + j];
+    const T rd = T(1) / A.vel_div;
+    const T ul = A.u2d[c + i] * rd, ur = A.u2d[c + i + 1] * rd, vt = A.v2d[c] * rd, vb = A.v2d[c + nx] * rd;
+    const bool on = A.flags & 1;
+    auto flux = [&](T w, T HA, T HB, bool in) {
+        const T s = w * w + T(kMassFluxReg);
+        const T f = T(0.5) * (HA + HB) * w - T(0.5) * (s * fast_rsqrt(s)) * (HB - HA);
+        return on && in ? f : T(0);
+    };
+    const T Ul = flux(ul, Hl, H, j > 0), Ur = flux(ur, H, Hr, j < nx - 1);
+    const T Vt = flux(vt, H, Ht, i > 0), Vb = flux(vb, Hb, H, i < ny - 1);
     const T sq = A.lf_sq, f = T(kRhoI) * A.dxi;
     auto dl = [&](T U) { return T(0.5) * (U + fabs(U) * sq); };
     auto dr = [&](T U) { return T(0.5) * (U - fabs(U) * sq); };
-    c.self = f * ((dl(hz.Hu_r) - dr(hz.Hu_l)) + (dl(hz.Hv_t) - dr(hz.Hv_b)));
-    c.xp = f * dr(hz.Hu_r);
-    c.xm = -f * dl(hz.Hu_l);
-    c.ym = f * dr(hz.Hv_t);
-    c.yp = -f * dl(hz.Hv_b);
-    return c;
+    return {f * ((dl(Ur) - dr(Ul)) + (dl(Vt) - dr(Vb))), f * dr(Ur), -f * dl(Ul), f * dr(Vt), -f * dl(Vb)};
 }
 
-// The E-independent part of level k's row on the (nz, ny nx) planes:
-// -rho H_prev E_prev / dt - f_E plus the neighbours' horizontal advection.
+// A column and its four neighbours (itself on the domain edge) in the tiles.
+struct LmStencil {
+    LmCol c, xp, xm, ym, yp;
+};
 template <typename T>
-__device__ __forceinline__ T lm_constant(const EnthArgs<T>& A, const LmHoriz<T>& hc, long ncol, long col, int k, int i,
-                                         int j, T hp, T invdt) {
-    const long o = (long)k * ncol;
-    T g = -(T(kRhoI) * hp * A.E_prev[o + col] * invdt) - A.f_E[o + col];
+__device__ __forceinline__ LmStencil lm_stencil(const EnthArgs<T>& A, long ncol, int i, int j) {
+    const int nx = A.nx, im = max(i - 1, 0), ip = min(i + 1, A.ny - 1), jm = max(j - 1, 0), jp = min(j + 1, nx - 1);
+    const long row = (long)i * nx;
+    return {lm_col(row + j, ncol, A.nz), lm_col(row + jp, ncol, A.nz), lm_col(row + jm, ncol, A.nz),
+            lm_col((long)im * nx + j, ncol, A.nz), lm_col((long)ip * nx + j, ncol, A.nz)};
+}
+
+// The E-independent part of level k's row on the tiles: -rho H_prev E_prev / dt
+// - f_E plus the neighbours' horizontal advection.
+template <typename T>
+__device__ __forceinline__ T lm_constant(const EnthArgs<T>& A, const LmHoriz<T>& hc, const LmStencil& n, int k, T hp,
+                                         T invdt) {
+    const long o = n.c.base + (long)k * n.c.stride;
+    T g = -(T(kRhoI) * hp * A.E_prev[o] * invdt) - A.f_E[o];
     if (A.flags & 1) {
-        const int nx = A.nx, im = max(i - 1, 0), ip = min(i + 1, A.ny - 1), jm = max(j - 1, 0),
-                  jp = min(j + 1, nx - 1);
-        const T* E = A.E + o;
-        g += (hc.xp * E[(long)i * nx + jp] + hc.xm * E[(long)i * nx + jm]) +
-             (hc.ym * E[(long)im * nx + j] + hc.yp * E[(long)ip * nx + j]);
+        auto E = [&](const LmCol& q) { return A.E[q.base + (long)k * q.stride]; };
+        g += (hc.xp * E(n.xp) + hc.xm * E(n.xm)) + (hc.ym * E(n.ym) + hc.yp * E(n.yp));
     }
     return g;
 }
@@ -1656,18 +1706,24 @@ __device__ __forceinline__ void pcr_stage(T& a, T& b, T& c, T& d) {
     c = nc;
 }
 
-// Column Newton smoother on the level-major planes (A.E etc. in (nz, ny nx)
-// layout): W = E + omega_relax (E_col - E), and with rmax the max |r| of the
-// starting state (first Newton iteration's rows) folded into the slots as
-// k_enth_column_smooth does.  P lanes per column (4 or 8, consecutive lanes
-// of one 16-lane row), MB >= 3 levels per lane, P MB >= nz.  Left at the
-// compiler's register allocation (143 VGPRs, 3 waves per SIMD, no spills):
-// held to 4 or 5 waves per SIMD the spills cost more (at 512 x 512 x 41 a
-// sweep measured 425 us unconstrained, 503 us at 4 waves, 807 us at 5).
+// Column Newton smoother on the tiles: W = E + omega_relax (E_col - E), and with
+// rmax the max |r| of the starting state (first Newton iteration's rows) folded
+// into the slots as k_enth_column_smooth does.  P lanes per column (consecutive
+// lanes of one 16-lane row), MB >= 3 levels per lane, P MB >= nz.
+//
+// A sweep's column pass at 512 x 512 x 41 took 400 us: it waited for memory in
+// four cycles of five, through a chain of six dependent loads ahead of the first
+// row, and its 142 million wave instructions took 230 us to issue.  Now every
+// load is issued at once from the tiles, cold rows take no exponentials, and six
+// levels a lane need half the reduction stages of three: 277 us, 77 million
+// instructions (126 us to issue; the values read and written once: 88 us).
+// 182 VGPRs at six levels (2 waves per SIMD); held to 168 the spills cost more
+// (349 us).
 template <typename T, int P, int MB>
-__global__ __launch_bounds__(256) void k_enth_column_lm(EnthArgs<T> A, T* __restrict__ W, T omega_relax,
+__global__ __launch_bounds__(256, 2) void k_enth_column_lm(EnthArgs<T> A, T* __restrict__ W, T omega_relax,
                                                         int n_newton, T relaxation,
-                                                        unsigned long long* __restrict__ rmax) {
+                                                        unsigned long long* __restrict__ rmax,
+                                                        ColdValues<T> cold) {
     static_assert(MB >= 3, "the partitioned solve needs three levels per lane");
     static_assert(P == 4 || P == 8 || P == 16, "4, 8 or 16 lanes per column (within a 16-lane DPP row)");
     constexpr int kCols = 256 / P;  // columns per block
@@ -1682,9 +1738,46 @@ __global__ __launch_bounds__(256) void k_enth_column_lm(EnthArgs<T> A, T* __rest
     const int i = (int)(cc / nx), j = (int)(cc % nx);
     const T h = A.H[cc], Es = A.E_surface[cc];
     const T dsig = T(1) / T(nz - 1);
+    const LmStencil n = lm_stencil(A, ncol, i, j);
+    // every load of the column at once (levels beyond it read its last one):
+    // E, and the E-independent part of the rows (lm_constant)
+    // the pass's starting E, the constants and omega stay in LDS (each thread
+    // reads its own), which leaves the registers to the rows and the elimination
+    __shared__ T s_E[MB][256], s_G[MB][256], s_om[MB][256];
+    const int tid = threadIdx.x;
     T El[MB];
+    int kk[MB];
 #pragma unroll
-    for (int m = 0; m < MB; ++m) El[m] = (k0 + m < nz) ? A.E[(long)(k0 + m) * ncol + cc] : T(0);
+    for (int m = 0; m < MB; ++m) kk[m] = min(k0 + m, nz - 1);
+    auto at = [](const LmCol& q, int k) { return q.base + (long)(k * q.stride); };
+    const T hp = A.H_prev[cc], invdt = A.invdt;
+    const bool adv = A.flags & 1, has_om = A.omega;
+    const T* __restrict__ omp = has_om ? A.omega : A.E;
+    T Ex[MB][4], fE[MB], Ep[MB], om[MB];
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+        El[m] = A.E[at(n.c, kk[m])];
+        Ep[m] = A.E_prev[at(n.c, kk[m])];
+        fE[m] = A.f_E[at(n.c, kk[m])];
+        om[m] = omp[at(n.c, kk[m])];
+        Ex[m][0] = A.E[at(n.xp, kk[m])];
+        Ex[m][1] = A.E[at(n.xm, kk[m])];
+        Ex[m][2] = A.E[at(n.ym, kk[m])];
+        Ex[m][3] = A.E[at(n.yp, kk[m])];
+    }
+    // omega one level below and above the block (clamped)
+    T om_lo = omp[at(n.c, min(max(k0 - 1, 0), nz - 1))], om_hi = omp[at(n.c, min(k0 + MB, nz - 1))];
+    const LmHoriz<T> hc = lm_horiz(A, i, j);
+    om_lo = has_om ? om_lo : T(0);
+    om_hi = has_om ? om_hi : T(0);
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+        const T adv_m = (hc.xp * Ex[m][0] + hc.xm * Ex[m][1]) + (hc.ym * Ex[m][2] + hc.yp * Ex[m][3]);
+        s_G[m][tid] = -(T(kRhoI) * hp * Ep[m] * invdt) - fE[m] + (adv ? adv_m : T(0));
+        s_om[m][tid] = has_om ? om[m] : T(0);
+        s_E[m][tid] = El[m];
+        if (k0 + m >= nz) El[m] = T(0);
+    }
     double r_first = 0.0;
     if (h < A.h_thin) {
 #pragma unroll
@@ -1692,19 +1785,7 @@ __global__ __launch_bounds__(256) void k_enth_column_lm(EnthArgs<T> A, T* __rest
             if (k0 + m < nz) El[m] = fmin(Es, e_pmp(T(k0 + m) * dsig, h));
     } else {
         const ColConst<T> cst = col_const(A, h);
-        const T hp = A.H_prev[cc], invdt = cst.invdt;
-        const LmHoriz<T> hc = lm_horiz(A, i, j);
-        const T B0 = T(kRhoI) * h * invdt + hc.self;
-        T G[MB], om[MB];
-#pragma unroll
-        for (int m = 0; m < MB; ++m) {
-            const int k = k0 + m;
-            G[m] = (k < nz - 1) ? lm_constant(A, hc, ncol, cc, k, i, j, hp, invdt) : T(0);
-            om[m] = (A.omega && k < nz) ? A.omega[(long)k * ncol + cc] : T(0);
-        }
-        // omega one level below and above the block (clamped as the column kernel's)
-        const T om_lo = (A.omega && k0 < nz) ? A.omega[(long)max(k0 - 1, 0) * ncol + cc] : T(0);
-        const T om_hi = A.omega ? A.omega[(long)min(k0 + MB, nz - 1) * ncol + cc] : T(0);
+        const T B0 = T(kRhoI) * h * cst.invdt + hc.self;
         for (int it = 0; it < n_newton; ++it) {
             // The per-level terms that do not change between iterations
             // (pressure-melting enthalpies, advection coefficients) are formed
@@ -1712,24 +1793,20 @@ __global__ __launch_bounds__(256) void k_enth_column_lm(EnthArgs<T> A, T* __rest
             // registers than the rows and the elimination together.  The empty
             // statements only hide these inputs' values from that hoisting.
             T hh = h;
-            asm volatile("" : "+v"(hh));
-#pragma unroll
-            for (int m = 0; m < MB; ++m) asm volatile("" : "+v"(om[m]));
+            asm volatile("" : "+v"(hh) : : "memory");
+            T om_m = om_lo, om_k = s_om[0][tid];
             const T Eb = from_below<1>(El[MB - 1]);  // level k0 - 1
             const T Ea = from_above<1>(El[0]);       // level k0 + MB
-            // interface diffusivities above the block's levels; the one below
-            // level k0 is the lane below's last
-            T Ku[MB];
-#pragma unroll
-            for (int m = 0; m < MB; ++m) {
+            // interface diffusivity above level k0 + m; the one below level k0
+            // is the lane below's last
+            auto K_above = [&](int m) {
                 const int k = k0 + m;
-                Ku[m] = T(0);
-                if (k < nz - 1) {
-                    const T Ep_k = e_pmp(T(k) * dsig, hh), Ep_p = e_pmp(T(k + 1) * dsig, hh);
-                    Ku[m] = diffusivity(T(0.5) * (El[m] + (m < MB - 1 ? El[m + 1] : Ea)), T(0.5) * (Ep_k + Ep_p));
-                }
-            }
-            const T Kl0 = from_below<1>(Ku[MB - 1]);
+                const T Ep_k = e_pmp(T(k) * dsig, hh), Ep_p = e_pmp(T(k + 1) * dsig, hh);
+                return diffusivity<T, true>(T(0.5) * (El[m] + (m < MB - 1 ? El[m + 1] : Ea)), T(0.5) * (Ep_k + Ep_p),
+                                            cold.K);
+            };
+            const T K_last = k0 + MB - 1 < nz - 1 ? K_above(MB - 1) : T(0);
+            T Kl = from_below<1>(K_last);
             // rows and forward elimination: row m becomes
             // Ac[m] x_0 + x_m + Cc[m] x_{m+1} = Dc[m] (row 0: Ac[0] multiplies
             // the lane below's last unknown)
@@ -1741,9 +1818,13 @@ __global__ __launch_bounds__(256) void k_enth_column_lm(EnthArgs<T> A, T* __rest
                 const T Ekp1 = m < MB - 1 ? El[m + 1] : Ea;
                 T a = T(0), b = T(1), c = T(0), d = T(0);
                 if (k < nz - 1) {
-                    Row<T> w{B0 * El[m] + G[m], T(0), B0, T(0)};
-                    column_terms(A, cst, k, hh, El[m], Ekm1, Ekp1, m > 0 ? om[m - 1] : om_lo, om[m],
-                                 m < MB - 1 ? om[m + 1] : om_hi, Ku[m], m > 0 ? Ku[m - 1] : Kl0, w);
+                    const T Ku = m == MB - 1 ? K_last : K_above(m);
+                    Row<T> w{B0 * El[m] + s_G[m][tid], T(0), B0, T(0)};
+                    const T om_p = m < MB - 1 ? s_om[m + 1][tid] : om_hi;
+                    column_terms<T, true>(A, cst, k, hh, El[m], Ekm1, Ekp1, om_m, om_k, om_p, Ku, Kl, w, &cold);
+                    Kl = Ku;
+                    om_m = om_k;
+                    om_k = om_p;
                     a = k == 0 ? T(0) : w.a;
                     b = w.b;
                     c = w.c;
@@ -1801,8 +1882,8 @@ __global__ __launch_bounds__(256) void k_enth_column_lm(EnthArgs<T> A, T* __rest
         for (int m = 0; m < MB; ++m) {
             const int k = k0 + m;
             if (k < nz) {
-                const long o = (long)k * ncol + cc;
-                const T E0 = A.E[o];
+                const long o = at(n.c, k);
+                const T E0 = s_E[m][tid];
                 W[o] = E0 + omega_relax * (El[m] - E0);
             }
         }
@@ -1816,59 +1897,112 @@ __global__ __launch_bounds__(256) void k_enth_column_lm(EnthArgs<T> A, T* __rest
     }
 }
 
-// One column's rows on the level-major planes, streamed up the levels:
+// One column's rows on the tiles, streamed up the levels:
 // calls f(k, w) with level k's row (residual with forcing in w.r) for
 // k = 0 .. nz - 2 of a thick column.
 template <typename T, typename F>
 __device__ __forceinline__ void lm_stream_rows(const EnthArgs<T>& A, long ncol, long col, F&& f) {
     const int nz = A.nz, nx = A.nx, i = (int)(col / nx), j = (int)(col % nx);
+    const LmStencil n = lm_stencil(A, ncol, i, j);
+    const long step = n.c.stride;
     const T h = A.H[col], hp = A.H_prev[col];
     const ColConst<T> cst = col_const(A, h);
     const T invdt = cst.invdt, dsig = cst.dsig;
     const LmHoriz<T> hc = lm_horiz(A, i, j);
     const T B0 = T(kRhoI) * h * invdt + hc.self;
-    const T* E = A.E;
-    const T* om = A.omega;
-    T Em = E[col], Ek = E[col], Ep = E[ncol + col];
-    T om_m = om ? om[col] : T(0), om_k = om_m, om_p = om ? om[(long)min(1, nz - 1) * ncol + col] : T(0);
+    const T* E = A.E + n.c.base;
+    const T* om = A.omega ? A.omega + n.c.base : nullptr;
+    T Em = E[0], Ek = E[0], Ep = E[step];
+    T om_m = om ? om[0] : T(0), om_k = om_m, om_p = om ? om[min(1, nz - 1) * step] : T(0);
     T Kl = T(0);
     for (int k = 0; k < nz - 1; ++k) {
         const T Ep_k = e_pmp(T(k) * dsig, h), Ep_p = e_pmp(T(k + 1) * dsig, h);
         const T Ku = diffusivity(T(0.5) * (Ek + Ep), T(0.5) * (Ep_k + Ep_p));
-        Row<T> w{B0 * Ek + lm_constant(A, hc, ncol, col, k, i, j, hp, invdt), T(0), B0, T(0)};
+        Row<T> w{B0 * Ek + lm_constant(A, hc, n, k, hp, invdt), T(0), B0, T(0)};
         column_terms(A, cst, k, h, Ek, Em, Ep, om_m, om_k, om_p, Ku, Kl, w);
         f(k, Ek, w);
         Kl = Ku;
         Em = Ek;
         Ek = Ep;
-        Ep = (k + 2 < nz) ? E[(long)(k + 2) * ncol + col] : T(0);
+        Ep = (k + 2 < nz) ? E[(k + 2) * step] : T(0);
         om_m = om_k;
         om_k = om_p;
-        om_p = om ? om[(long)min(k + 2, nz - 1) * ncol + col] : T(0);
+        om_p = om ? om[min(k + 2, nz - 1) * step] : T(0);
     }
 }
 
-// Pointwise Jacobi layer smoother on the level-major planes:
+// Pointwise Jacobi layer smoother on the tiles:
 // E_out = E + omega_relax (-r / J_kk), E_out = E on surface rows and thin columns.
+// A wavefront takes kLayerLevels levels of a tile, all loads at once: one thread
+// per column streaming up all of them kept two levels in flight (127 us at 512 x
+// 512 x 41, and 28 us at 48 x 48 x 41).
+constexpr int kLayerLevels = 6;
 template <typename T>
-__global__ __launch_bounds__(256) void k_enth_layer_lm(EnthArgs<T> A, T* __restrict__ E_out, T omega_relax) {
+__global__ __launch_bounds__(256) void k_enth_layer_lm(EnthArgs<T> A, T* __restrict__ E_out, T omega_relax,
+                                                       ColdValues<T> cold) {
     if (skipped(A.skip)) return;
-    const long ncol = (long)A.ny * A.nx, nvb = (ncol + 255) / 256;
-    const long col = xcd_block(blockIdx.x, nvb) * 256 + threadIdx.x;
-    if (col >= ncol) return;
-    const int nz = A.nz;
-    if (A.H[col] < A.h_thin) {
-        for (int k = 0; k < nz; ++k) E_out[(long)k * ncol + col] = A.E[(long)k * ncol + col];
-        return;
+    constexpr int CH = kLayerLevels;
+    const int nz = A.nz, nch = (nz + CH - 1) / CH;
+    const long ncol = (long)A.ny * A.nx, items = (ncol + kLmCols - 1) / kLmCols * nch;
+    const long item = xcd_block(blockIdx.x, (items + 3) / 4) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (item >= items) return;
+    const int kb = (int)(item % nch) * CH;
+    const long col = item / nch * kLmCols + (threadIdx.x & 63), cc = min(col, ncol - 1);
+    const int i = (int)(cc / A.nx), j = (int)(cc % A.nx);
+    const LmStencil n = lm_stencil(A, ncol, i, j);
+    const T h = A.H[cc], hp = A.H_prev[cc];
+    const bool adv = A.flags & 1, has_om = A.omega;
+    const T* __restrict__ omp = has_om ? A.omega : A.E;
+    auto at = [](const LmCol& q, int k) { return q.base + (long)(k * q.stride); };
+    // q = 0: the level below the first, q = CH + 1: the one above the last
+    T E[CH + 2], om[CH + 2], Ep[CH], fE[CH], Ex[CH][4];
+#pragma unroll
+    for (int q = 0; q < CH + 2; ++q) {
+        const int k = min(max(kb + q - 1, 0), nz - 1);
+        E[q] = A.E[at(n.c, k)];
+        om[q] = omp[at(n.c, k)];
     }
-    lm_stream_rows(A, ncol, col, [&](int k, T Ek, const Row<T>& w) {
-        const T out = (fabs(w.b) > T(1e-30)) ? -w.r / w.b : T(0);
-        E_out[(long)k * ncol + col] = Ek + omega_relax * out;
-    });
-    E_out[(long)(nz - 1) * ncol + col] = A.E[(long)(nz - 1) * ncol + col];
+#pragma unroll
+    for (int m = 0; m < CH; ++m) {
+        const int k = min(kb + m, nz - 1);
+        Ep[m] = A.E_prev[at(n.c, k)];
+        fE[m] = A.f_E[at(n.c, k)];
+        Ex[m][0] = A.E[at(n.xp, k)];
+        Ex[m][1] = A.E[at(n.xm, k)];
+        Ex[m][2] = A.E[at(n.ym, k)];
+        Ex[m][3] = A.E[at(n.yp, k)];
+    }
+    const LmHoriz<T> hc = lm_horiz(A, i, j);
+    const ColConst<T> cst = col_const(A, h);
+    const T B0 = T(kRhoI) * h * cst.invdt + hc.self;
+    const bool thin = h < A.h_thin, valid = col < ncol;
+#pragma unroll
+    for (int q = 0; q < CH + 2; ++q) om[q] = has_om ? om[q] : T(0);
+    T Epm_lo = e_pmp(T(max(kb - 1, 0)) * cst.dsig, h), Epm = e_pmp(T(kb) * cst.dsig, h);
+    T Kl = T(0);
+    if (kb > 0) Kl = diffusivity<T, true>(T(0.5) * (E[0] + E[1]), T(0.5) * (Epm_lo + Epm), cold.K);
+#pragma unroll
+    for (int m = 0; m < CH; ++m) {
+        const int k = kb + m;
+        if (k >= nz) break;
+        T out = T(0);
+        if (k < nz - 1) {
+            const T Epm_up = e_pmp(T(k + 1) * cst.dsig, h);
+            const T Ku = diffusivity<T, true>(T(0.5) * (E[m + 1] + E[m + 2]), T(0.5) * (Epm + Epm_up), cold.K);
+            const T adv_m = (hc.xp * Ex[m][0] + hc.xm * Ex[m][1]) + (hc.ym * Ex[m][2] + hc.yp * Ex[m][3]);
+            const T G = -(T(kRhoI) * hp * Ep[m] * cst.invdt) - fE[m] + (adv ? adv_m : T(0));
+            Row<T> w{B0 * E[m + 1] + G, T(0), B0, T(0)};
+            column_terms<T, true>(A, cst, k, h, E[m + 1], E[m], E[m + 2], om[m], om[m + 1], om[m + 2], Ku, Kl, w,
+                                  &cold);
+            if (fabs(w.b) > T(1e-30)) out = -w.r / w.b;
+            Kl = Ku;
+            Epm = Epm_up;
+        }
+        if (valid) E_out[at(n.c, k)] = (thin || k == nz - 1) ? E[m + 1] : E[m + 1] + omega_relax * out;
+    }
 }
 
-// Residual (with forcing) on the level-major planes: per-block max |r| into
+// Residual (with forcing) on the tiles: per-block max |r| into
 // partials[blockIdx.x] (grid-stride over columns) and, when r_out is given,
 // r written in the (ny, nx, nz) layout (zero on surface rows and thin columns).
 template <typename T>
@@ -2097,20 +2231,32 @@ hipError_t launch_enth_column_lm(const EnthArgs<T>& A, T* W, T omega_relax, int 
                                  unsigned long long* rmax, hipStream_t st) {
     if (!enth_lm_supported(A.nz) || !A.u2d) return hipErrorInvalidValue;
     const long ncol = (long)A.ny * A.nx;
-    // three or four levels per lane: 4 lanes per column up to 16 levels, 8 up
-    // to 32, 16 above (measured at 41 levels: 16 lanes 6% faster than 8)
-    const int P = A.nz <= 16 ? 4 : A.nz <= 32 ? 8 : 16, mb = (A.nz + P - 1) / P;
+    // Up to eight levels per lane where the columns fill the chip (2 wavefronts
+    // per SIMD), else three or four, whose chain is shorter.  A whole sweep at
+    // 512 x 512 with 4 / 8 lanes for 21 levels 205 / 212 us, with 8 / 16 for 41
+    // 416 / 432 us; at 48 x 48 49 / 45 us and 76 / 68 us; equal at 128 x 128.
+    const bool fills = ncol >= 32768;
+    const int P = A.nz <= 16 ? 4 : A.nz <= 32 ? (fills ? 4 : 8) : (fills ? 8 : 16), mb = (A.nz + P - 1) / P;
     const unsigned nb = (unsigned)((ncol + 256 / P - 1) / (256 / P));
+    const ColdValues<T> cold = cold_values<T>();
     TimedLaunch tl(kTimeEnthColumn, ncol * A.nz, st);
 #define GLIDE_LM_COLUMN(PP, MB)                                                                                   \
     if (P == PP && mb == MB) {                                                                                    \
-        k_enth_column_lm<T, PP, MB><<<nb, 256, 0, st>>>(A, W, omega_relax, n_newton, relaxation, rmax);           \
+        k_enth_column_lm<T, PP, MB><<<nb, 256, 0, st>>>(A, W, omega_relax, n_newton, relaxation, rmax, cold);     \
         return hipGetLastError();                                                                                 \
     }
     GLIDE_LM_COLUMN(4, 3)
     GLIDE_LM_COLUMN(4, 4)
+    GLIDE_LM_COLUMN(4, 5)
+    GLIDE_LM_COLUMN(4, 6)
+    GLIDE_LM_COLUMN(4, 7)
+    GLIDE_LM_COLUMN(4, 8)
     GLIDE_LM_COLUMN(8, 3)
     GLIDE_LM_COLUMN(8, 4)
+    GLIDE_LM_COLUMN(8, 5)
+    GLIDE_LM_COLUMN(8, 6)
+    GLIDE_LM_COLUMN(8, 7)
+    GLIDE_LM_COLUMN(8, 8)
     GLIDE_LM_COLUMN(16, 3)
     GLIDE_LM_COLUMN(16, 4)
 #undef GLIDE_LM_COLUMN
@@ -2121,7 +2267,8 @@ hipError_t launch_enth_layer_lm(const EnthArgs<T>& A, T* E_out, T omega_relax, h
     if (!enth_lm_supported(A.nz) || !A.u2d) return hipErrorInvalidValue;
     const long ncol = (long)A.ny * A.nx;
     TimedLaunch tl(kTimeEnthLayer, ncol * A.nz, st);
-    k_enth_layer_lm<T><<<(unsigned)((ncol + 255) / 256), 256, 0, st>>>(A, E_out, omega_relax);
+    const long items = (ncol + kLmCols - 1) / kLmCols * ((A.nz + kLayerLevels - 1) / kLayerLevels);
+    k_enth_layer_lm<T><<<(unsigned)((items + 3) / 4), 256, 0, st>>>(A, E_out, omega_relax, cold_values<T>());
     return hipGetLastError();
 }
 template <typename T>

@@ -21,6 +21,16 @@ struct EnthArgs {
     // broadcast u3d[k] holds, read from one (ny, nx+1) / (ny+1, nx) plane.
     const T *u2d, *v2d;
     T vel_div;
+    // Functions of nz and dt the rows multiply by (ColConst).
+    T dsig, di, hdi, d2, idd, invdt;
+    void set_constants() {
+        dsig = T(1) / T(nz - 1);
+        di = T(1) / dsig;
+        hdi = T(1) / (T(0.5) * dsig);
+        d2 = T(1) / (dsig * dsig);
+        idd = T(1) / (dsig * (T(0.5) * dsig));
+        invdt = T(1) / dt;
+    }
 };
 
 // Device record of a fused column sweep (EnthalpyOperators.column_sweep).
@@ -153,11 +163,11 @@ hipError_t launch_thermal_vjp(const EnthArgs<T>& A, const ThermalVjpArgs<T>& V, 
 // exp and log as the enthalpy rows compute them, over n values (for tests).
 hipError_t launch_enth_elementary(const double* x, long n, double* e_out, double* l_out, hipStream_t st);
 
-// Level-major form of the fused alternating sweep (thermal step with a
+// Tiled form of the fused alternating sweep (thermal step with a
 // depth-constant velocity, A.u2d set, 9 <= nz <= 64): A.E, A.E_prev, A.f_E and
-// A.omega point to (nz, ny nx) planes.
+// A.omega point to the tiled copies (LmCol in enthalpy_kernels.hip).
 bool enth_lm_supported(int nz);
-// (ny nx, nz) -> (nz, ny nx) when to_lm, else back.
+// (ny nx, nz) -> tiles when to_lm, else back.
 template <typename T>
 hipError_t launch_enth_lm_layout(const T* src, T* dst, long ncol, int nz, bool to_lm, hipStream_t st);
 // Column Newton smoother: W = E + omega_relax (E_col - E), with rmax as

@@ -152,7 +152,7 @@ class EnthalpyOperators:
         self.f_E = z3()
         self.delta_E = z3()
         self._E_work = z3()
-        # level-major copies of E, E_prev, f_E and omega for the fused sweep of the thermal step
+        # tiled copies of E, E_prev, f_E and omega for the fused sweep of the thermal step
         self._sweep_work = grid.zeros((4, nz, ny, nx))
         self._dh_dt = z2()
         self.smoother_config = ColumnSmootherConfig()

@@ -293,6 +293,31 @@ def test_red_black_column_sweep_reaches_the_same_fixed_point():
     assert out[1][2] <= n0
 
 
+@pytest.mark.parametrize("n,nz", [(9, 9), (13, 16), (10, 17), (12, 24), (8, 32), (9, 33), (16, 40), (11, 48), (10, 64),
+                                  (182, 20), (182, 21), (182, 28), (182, 32), (182, 33), (182, 41), (182, 50),
+                                  (182, 64)])
+def test_tiled_sweep_matches_column_wavefronts(n, nz):
+    """The thermal step's sweep on its tiled copies, at every levels-per-lane
+    split of the column pass (small maps and maps of 32768 columns or more),
+    with a narrow last tile and ragged chunks of the layer pass, against the
+    same sweep on the (ny, nx, nz) arrays (the bar of whole sweeps)."""
+    print(f"tiled sweep n={n} nz={nz}", flush=True)
+    out = []
+    for tiled in (True, False):
+        F, g, tm, _ = _thermal_pair(n, nz, 8, strain=True)
+        tm.n_smooth = 4
+        tm.ops.smoother_config.absolute_tolerance = tm.ops.smoother_config.relative_tolerance = 0.0
+        if not tiled:
+            tm.ops._sweep_work = None
+        rep = tm.step(DT, report=True)
+        out.append((N(tm.ops.enthalpy_state.E), N(tm.ops.r_E), [rep.norms[k] for k in range(rep.sweeps)], rep.r0))
+    (E0, r0, n0, a0), (E1, r1, n1, a1) = out
+    assert len(n0) == len(n1) == 4
+    assert rel_err(E0, E1) < STOL
+    assert np.abs(r0 - r1).max() <= 1e-8 * a1
+    assert abs(a0 - a1) <= 1e-8 * a1 and np.allclose(n0, n1, rtol=1e-7, atol=1e-8 * a1)
+
+
 def test_thermal_step_host_path_matches_fused():
     print("thermal_step host path", flush=True)
     F, g, tm, th = _thermal_pair(16, 11, 4, strain=True)
