@@ -52,7 +52,7 @@ struct EnthScratch {
     double* partials = nullptr;   // kEnthResBlocks
     double* max_out = nullptr;    // 1
     unsigned long long* acc = nullptr;  // adjoint passes' maximum and block count, kept zero between uses
-    unsigned long long* rmax = nullptr;  // kEnthRmaxSlots: the column pass's max-|r| accumulators
+    unsigned long long* rmax = nullptr;  // kEnthSlotWords: the column pass's max-|r| accumulators
     EnthStatus* status = nullptr;
     EnthStatus* host = nullptr;   // pinned mirror
 };
@@ -72,7 +72,7 @@ int scratch(EnthScratch** out) {
         HIP_TRY(hipMalloc(&s.acc, 2 * sizeof(unsigned long long)), "hipMalloc(enthalpy accumulator)");
         HIP_TRY(hipMemset(s.acc, 0, 2 * sizeof(unsigned long long)), "hipMemset(enthalpy accumulator)");
         HIP_TRY(hipMalloc(&s.status, sizeof(EnthStatus)), "hipMalloc(enthalpy status)");
-        HIP_TRY(hipMalloc(&s.rmax, sizeof(unsigned long long) * kEnthRmaxSlots), "hipMalloc(enthalpy max slots)");
+        HIP_TRY(hipMalloc(&s.rmax, sizeof(unsigned long long) * kEnthSlotWords), "hipMalloc(enthalpy max slots)");
         HIP_TRY(hipHostMalloc(&s.host, sizeof(EnthStatus), hipHostMallocDefault), "hipHostMalloc(enthalpy status)");
     }
     *out = &s;
@@ -196,6 +196,11 @@ int sweep_core(const glide_enth_column* C, double dt, int n_iter, const glide_en
         EnthArgs<R> Lw = L;
         Lw.E = Wlm;
         HIP_TRY(launch_enth_reduce_slots(rmax, status, 0, rtol, atol, st), "enthalpy max slots");
+        if (enth_sweeps_fit(C->ny, C->nx, nz)) {
+            HIP_TRY(launch_enth_sweeps<R>(L, Elm, Wlm, cfg->omega, cfg->n_newton, cfg->relaxation, rmax, status, rtol,
+                                          atol, n_iter, st),
+                    "enthalpy sweeps");
+        } else
         for (int it = 0; it < n_iter; ++it) {
             HIP_TRY(launch_enth_column_lm<R>(L, Wlm, cfg->omega, cfg->n_newton, cfg->relaxation,
                                              it > 0 ? rmax : nullptr, st),

@@ -421,6 +421,13 @@ __global__ __launch_bounds__(256) void k_enth_residual(EnthArgs<T> A, T* __restr
     if (threadIdx.x == 0) partials[blockIdx.x] = nan_max(nan_max(smax[0], smax[1]), nan_max(smax[2], smax[3]));
 }
 
+// The stopping test; a NaN norm (now or at the start) never stops the sweep.
+__device__ __forceinline__ bool sweep_stops(double r, double r0, double rtol, double atol) {
+    if (!(r == r && r0 == r0)) return false;
+    const double rel = r0 > 0.0 ? r / r0 : 0.0;
+    return rel < rtol || r < atol;
+}
+
 // Sweep bookkeeping: mode 0 starts a sweep (r0, zero count, clear the skip
 // flag); mode 1 closes one sweep iteration (count, norm, stopping test of
 // glide/enthalpy.py:426-471).
@@ -436,11 +443,7 @@ __device__ __forceinline__ void record_sweep(EnthStatus* status, int mode, doubl
         status->sweeps = it + 1;
         status->r = r;
         const double r0 = status->r0;
-        // a NaN norm (now or at the start) never stops the sweep
-        if (r == r && r0 == r0) {
-            const double rel = r0 > 0.0 ? r / r0 : 0.0;
-            if (rel < rtol || r < atol) status->done = 1;
-        }
+        if (sweep_stops(r, r0, rtol, atol)) status->done = 1;
     }
 }
 
@@ -465,17 +468,20 @@ __global__ __launch_bounds__(256) void k_enth_reduce(const double* __restrict__ 
 
 // Maximum over the column pass's max-|r| slots (bit patterns of
 // non-negative doubles, or NaN), zeroing them; mode 1 closes one sweep
-// iteration as k_enth_reduce does, mode 0 only zeroes.
+// iteration as k_enth_reduce does, mode 0 only zeroes (every word of the buffer).
 __global__ __launch_bounds__(256) void k_enth_reduce_slots(unsigned long long* __restrict__ slots, EnthStatus* status,
                                                            int mode, double rtol, double atol) {
     __shared__ double sh[4];
     if (status && mode == 1 && status->done) return;
+    if (mode != 1) {
+        for (int q = threadIdx.x; q < kEnthSlotWords; q += blockDim.x) slots[q] = 0ull;
+        return;
+    }
     double m = 0.0;
     for (int q = threadIdx.x; q < kEnthRmaxSlots; q += blockDim.x) {
         m = nan_max(m, __longlong_as_double((long long)slots[q]));
         slots[q] = 0ull;
     }
-    if (mode != 1) return;
     for (int off = 32; off > 0; off >>= 1) m = nan_max(m, __shfl_down(m, off, 64));
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
     __syncthreads();
@@ -1720,18 +1726,14 @@ __device__ __forceinline__ void pcr_stage(T& a, T& b, T& c, T& d) {
 // 182 VGPRs at six levels (2 waves per SIMD); held to 168 the spills cost more
 // (349 us).
 template <typename T, int P, int MB>
-__global__ __launch_bounds__(256, 2) void k_enth_column_lm(EnthArgs<T> A, T* __restrict__ W, T omega_relax,
-                                                        int n_newton, T relaxation,
-                                                        unsigned long long* __restrict__ rmax,
-                                                        ColdValues<T> cold) {
+__device__ __forceinline__ void column_lm_body(long vb, const EnthArgs<T>& A, T* W, T omega_relax, int n_newton,
+                                               T relaxation, unsigned long long* rmax, const ColdValues<T>& cold) {
     static_assert(MB >= 3, "the partitioned solve needs three levels per lane");
     static_assert(P == 4 || P == 8 || P == 16, "4, 8 or 16 lanes per column (within a 16-lane DPP row)");
     constexpr int kCols = 256 / P;  // columns per block
-    if (skipped(A.skip)) return;
     const int nz = A.nz, nx = A.nx;
     const long ncol = (long)A.ny * nx;
-    const long nvb = (ncol + kCols - 1) / kCols;
-    const long col = xcd_block(blockIdx.x, nvb) * kCols + (threadIdx.x / P);
+    const long col = vb * kCols + (threadIdx.x / P);
     const bool valid = col < ncol;  // the same for the P lanes of a column
     const long cc = valid ? col : ncol - 1;
     const int q = threadIdx.x % P, k0 = q * MB;
@@ -1752,7 +1754,7 @@ __global__ __launch_bounds__(256, 2) void k_enth_column_lm(EnthArgs<T> A, T* __r
     auto at = [](const LmCol& q, int k) { return q.base + (long)(k * q.stride); };
     const T hp = A.H_prev[cc], invdt = A.invdt;
     const bool adv = A.flags & 1, has_om = A.omega;
-    const T* __restrict__ omp = has_om ? A.omega : A.E;
+    const T* omp = has_om ? A.omega : A.E;
     T Ex[MB][4], fE[MB], Ep[MB], om[MB];
 #pragma unroll
     for (int m = 0; m < MB; ++m) {
@@ -1892,9 +1894,18 @@ __global__ __launch_bounds__(256, 2) void k_enth_column_lm(EnthArgs<T> A, T* __r
         double mx = valid ? r_first : 0.0;
         for (int off = 32; off > 0; off >>= 1) mx = nan_max(mx, __shfl_down(mx, off, 64));
         if ((threadIdx.x & 63) == 0)
-            atomicMax(rmax + (((long)blockIdx.x * 4 + (threadIdx.x >> 6)) & (kEnthRmaxSlots - 1)),
+            atomicMax(rmax + ((vb * 4 + (threadIdx.x >> 6)) & (kEnthRmaxSlots - 1)),
                       (unsigned long long)__double_as_longlong(mx));
     }
+}
+
+template <typename T, int P, int MB>
+__global__ __launch_bounds__(256, 2) void k_enth_column_lm(EnthArgs<T> A, T* __restrict__ W, T omega_relax,
+                                                           int n_newton, T relaxation,
+                                                           unsigned long long* __restrict__ rmax,
+                                                           ColdValues<T> cold) {
+    if (skipped(A.skip)) return;
+    column_lm_body<T, P, MB>(xcd_block(blockIdx.x, gridDim.x), A, W, omega_relax, n_newton, relaxation, rmax, cold);
 }
 
 // One column's rows on the tiles, streamed up the levels:
@@ -1938,13 +1949,12 @@ __device__ __forceinline__ void lm_stream_rows(const EnthArgs<T>& A, long ncol, 
 // 512 x 41, and 28 us at 48 x 48 x 41).
 constexpr int kLayerLevels = 6;
 template <typename T>
-__global__ __launch_bounds__(256) void k_enth_layer_lm(EnthArgs<T> A, T* __restrict__ E_out, T omega_relax,
-                                                       ColdValues<T> cold) {
-    if (skipped(A.skip)) return;
+__device__ __forceinline__ void layer_lm_body(long vb, const EnthArgs<T>& A, T* E_out, T omega_relax,
+                                              const ColdValues<T>& cold) {
     constexpr int CH = kLayerLevels;
     const int nz = A.nz, nch = (nz + CH - 1) / CH;
     const long ncol = (long)A.ny * A.nx, items = (ncol + kLmCols - 1) / kLmCols * nch;
-    const long item = xcd_block(blockIdx.x, (items + 3) / 4) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long item = vb * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (item >= items) return;
     const int kb = (int)(item % nch) * CH;
     const long col = item / nch * kLmCols + (threadIdx.x & 63), cc = min(col, ncol - 1);
@@ -1952,7 +1962,7 @@ __global__ __launch_bounds__(256) void k_enth_layer_lm(EnthArgs<T> A, T* __restr
     const LmStencil n = lm_stencil(A, ncol, i, j);
     const T h = A.H[cc], hp = A.H_prev[cc];
     const bool adv = A.flags & 1, has_om = A.omega;
-    const T* __restrict__ omp = has_om ? A.omega : A.E;
+    const T* omp = has_om ? A.omega : A.E;
     auto at = [](const LmCol& q, int k) { return q.base + (long)(k * q.stride); };
     // q = 0: the level below the first, q = CH + 1: the one above the last
     T E[CH + 2], om[CH + 2], Ep[CH], fE[CH], Ex[CH][4];
@@ -1999,6 +2009,139 @@ __global__ __launch_bounds__(256) void k_enth_layer_lm(EnthArgs<T> A, T* __restr
             Epm = Epm_up;
         }
         if (valid) E_out[at(n.c, k)] = (thin || k == nz - 1) ? E[m + 1] : E[m + 1] + omega_relax * out;
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_enth_layer_lm(EnthArgs<T> A, T* __restrict__ E_out, T omega_relax,
+                                                       ColdValues<T> cold) {
+    if (skipped(A.skip)) return;
+    layer_lm_body<T>(xcd_block(blockIdx.x, gridDim.x), A, E_out, omega_relax, cold);
+}
+static inline long layer_blocks(int ny, int nx, int nz) {
+    return (((long)ny * nx + kLmCols - 1) / kLmCols * ((nz + kLayerLevels - 1) / kLayerLevels) + 3) / 4;
+}
+
+// Barrier of the workgroups of a persistent launch, all resident (at most
+// kSweepBlocks, with room for several on a CU).  They span XCDs, whose L2s have
+// to be written back and invalidated; an L2 takes about a microsecond for it, so
+// only the last workgroup to arrive on an XCD does, for all of them (each
+// workgroup's own fences: 40 us a sweep at 48 x 48 x 41, four fifths of it in
+// the two barriers).  words (zeroed before the launch): all arrivals, the XCDs'
+// arrivals, the timeout flag, then per XCD its workgroups, arrivals and
+// releases.  Every wait is bounded: after kSweepPolls polls, or when another
+// workgroup gave up, the barrier returns false.
+constexpr int kSweepBlocks = 256, kSweepPolls = 1 << 20;
+struct SweepBarrier {
+    unsigned long long* w;
+    unsigned long long xcd, here, xcds, gen;
+
+    __device__ __forceinline__ static unsigned long long peek(unsigned long long* p) {
+        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ bool wait(unsigned long long* p, unsigned long long target) {
+        int spins = 0;
+        while (peek(p) < target && !peek(w + 2)) {
+            if (++spins > kSweepPolls) atomicExch(w + 2, 1ull);
+            __builtin_amdgcn_s_sleep(1);
+        }
+        return peek(w + 2) == 0;
+    }
+    // counts the workgroups of each XCD; thread 0 only holds the counts
+    __device__ __forceinline__ bool start(unsigned long long* words) {
+        __shared__ int s_ok;
+        w = words;
+        gen = 0;
+        if (threadIdx.x == 0) {
+            xcd = xcc_id();
+            atomicAdd(w + 3 + xcd, 1ull);
+            __threadfence();
+            atomicAdd(w, 1ull);
+            s_ok = wait(w, gridDim.x);
+            __threadfence();
+            here = peek(w + 3 + xcd);
+            xcds = 0;
+            for (int q = 0; q < kSweepXcds; ++q) xcds += peek(w + 3 + q) != 0;
+        }
+        __syncthreads();
+        return s_ok != 0;
+    }
+    __device__ __forceinline__ bool sync() {
+        __shared__ int s_ok;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's stores are in the L2
+        __syncthreads();
+        ++gen;
+        if (threadIdx.x == 0) {
+            unsigned long long* arrive = w + 3 + kSweepXcds + xcd;
+            unsigned long long* release = w + 3 + 2 * kSweepXcds + xcd;
+            bool ok;
+            if (atomicAdd(arrive, 1ull) + 1 == here * gen) {
+                __threadfence();
+                atomicAdd(w + 1, 1ull);
+                ok = wait(w + 1, xcds * gen);
+                __threadfence();
+                __hip_atomic_store(release, gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            } else {
+                ok = wait(release, gen);
+            }
+            s_ok = ok;
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // this CU's own cache
+        }
+        __syncthreads();
+        return s_ok != 0;
+    }
+};
+
+// All sweeps of a small map in one launch: the column pass (A.E = E into W), the
+// norm of the state it started from and the stopping test, the layer pass (W
+// into E), with a barrier after each pass.  A step mostly converges in a few of
+// its n_iter sweeps, and the launches of the others, three each, were most of a
+// small map's step (40 x 56 x 21 with 100 sweeps: 1020 us, three sweeps run).
+// slots: two sets of kEnthRmaxSlots, zero on entry.  If a barrier timed out, E
+// is filled with NaN, which the sweep's report and the residual then show.
+template <typename T, int P, int MB>
+__global__ __launch_bounds__(256, 2) void k_enth_sweeps(EnthArgs<T> A, T* E, T* W, T omega_relax, int n_newton,
+                                                        T relaxation, unsigned long long* slots,
+                                                        unsigned long long* sync, EnthStatus* status, double rtol,
+                                                        double atol, int n_iter, long col_blocks, long lay_blocks,
+                                                        ColdValues<T> cold) {
+    __shared__ double sh[4];
+    const long nb = gridDim.x;
+    const int tid = threadIdx.x;
+    EnthArgs<T> Aw = A;
+    Aw.E = W;
+    SweepBarrier bar;
+    bool ok = bar.start(sync);
+#pragma unroll 1
+    for (int it = 0; ok && it < n_iter; ++it) {
+        unsigned long long* set = slots + (it & 1) * kEnthRmaxSlots;
+#pragma unroll 1
+        for (long vb = blockIdx.x; vb < col_blocks; vb += nb)
+            column_lm_body<T, P, MB>(vb, A, W, omega_relax, n_newton, relaxation, it > 0 ? set : nullptr, cold);
+        ok = bar.sync();
+        if (!ok) break;
+        if (it > 0) {  // every workgroup comes to the same decision
+            double m = __longlong_as_double(
+                (long long)__hip_atomic_load(set + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            for (int off = 32; off > 0; off >>= 1) m = nan_max(m, __shfl_down(m, off, 64));
+            if ((tid & 63) == 0) sh[tid >> 6] = m;
+            __syncthreads();
+            const double r = nan_max(nan_max(sh[0], sh[1]), nan_max(sh[2], sh[3]));
+            const bool stop = sweep_stops(r, status->r0, rtol, atol);
+            if (blockIdx.x == 0 && tid == 0) record_sweep(status, 1, r, rtol, atol);
+            if (stop) return;
+        }
+#pragma unroll 1
+        for (long vb = blockIdx.x; vb < lay_blocks; vb += nb) layer_lm_body<T>(vb, Aw, E, omega_relax, cold);
+        ok = bar.sync();
+        if (!ok) break;
+        // read by all before the barrier, used again two sweeps later
+        if (blockIdx.x == 0)
+            __hip_atomic_store(set + tid, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (!ok) {
+        const long n = (long)A.ny * A.nx * A.nz;
+        for (long q = (long)blockIdx.x * 256 + tid; q < n; q += nb * 256) E[q] = __longlong_as_double(0x7ff8000000000000ll);
     }
 }
 
@@ -2226,17 +2369,52 @@ hipError_t launch_enth_lm_layout(const T* src, T* dst, long ncol, int nz, bool t
     return hipGetLastError();
 }
 bool enth_lm_supported(int nz) { return nz >= 9 && nz <= 64; }
+// Lanes per column: up to eight levels per lane where the columns fill the chip
+// (2 wavefronts per SIMD), else three or four, whose chain is shorter.  A whole
+// sweep at 512 x 512 with 4 / 8 lanes for 21 levels 205 / 212 us, with 8 / 16
+// for 41 416 / 432 us; at 48 x 48 49 / 45 us and 76 / 68 us; equal at 128 x 128.
+static inline int lm_lanes(long ncol, int nz) {
+    const bool fills = ncol >= 32768;
+    return nz <= 16 ? 4 : nz <= 32 ? (fills ? 4 : 8) : (fills ? 8 : 16);
+}
+// The whole sweep in one launch: maps whose column pass has at most kSweepBlocks
+// workgroups, all of which then run at once.
+bool enth_sweeps_fit(int ny, int nx, int nz) {
+    const long ncol = (long)ny * nx, cols = 256 / lm_lanes(ncol, nz);
+    return (ncol + cols - 1) / cols <= kSweepBlocks;
+}
+template <typename T>
+hipError_t launch_enth_sweeps(const EnthArgs<T>& A, T* E, T* W, T omega_relax, int n_newton, T relaxation,
+                              unsigned long long* slots, EnthStatus* status, double rtol, double atol, int n_iter,
+                              hipStream_t st) {
+    if (!enth_lm_supported(A.nz) || !A.u2d || !enth_sweeps_fit(A.ny, A.nx, A.nz)) return hipErrorInvalidValue;
+    const long ncol = (long)A.ny * A.nx;
+    const int P = lm_lanes(ncol, A.nz), mb = (A.nz + P - 1) / P;
+    const long cb = (ncol + 256 / P - 1) / (256 / P), lb = layer_blocks(A.ny, A.nx, A.nz);
+    const ColdValues<T> cold = cold_values<T>();
+    TimedLaunch tl(kTimeEnthColumn, ncol * A.nz, st);
+#define GLIDE_LM_SWEEPS(PP, MB)                                                                                    \
+    if (P == PP && mb == MB) {                                                                                    \
+        k_enth_sweeps<T, PP, MB><<<(unsigned)cb, 256, 0, st>>>(A, E, W, omega_relax, n_newton, relaxation, slots, \
+                                                               slots + 2 * kEnthRmaxSlots, status, rtol, atol,    \
+                                                               n_iter, cb, lb, cold);                             \
+        return hipGetLastError();                                                                                 \
+    }
+    GLIDE_LM_SWEEPS(4, 3)
+    GLIDE_LM_SWEEPS(4, 4)
+    GLIDE_LM_SWEEPS(8, 3)
+    GLIDE_LM_SWEEPS(8, 4)
+    GLIDE_LM_SWEEPS(16, 3)
+    GLIDE_LM_SWEEPS(16, 4)
+#undef GLIDE_LM_SWEEPS
+    return hipErrorInvalidValue;
+}
 template <typename T>
 hipError_t launch_enth_column_lm(const EnthArgs<T>& A, T* W, T omega_relax, int n_newton, T relaxation,
                                  unsigned long long* rmax, hipStream_t st) {
     if (!enth_lm_supported(A.nz) || !A.u2d) return hipErrorInvalidValue;
     const long ncol = (long)A.ny * A.nx;
-    // Up to eight levels per lane where the columns fill the chip (2 wavefronts
-    // per SIMD), else three or four, whose chain is shorter.  A whole sweep at
-    // 512 x 512 with 4 / 8 lanes for 21 levels 205 / 212 us, with 8 / 16 for 41
-    // 416 / 432 us; at 48 x 48 49 / 45 us and 76 / 68 us; equal at 128 x 128.
-    const bool fills = ncol >= 32768;
-    const int P = A.nz <= 16 ? 4 : A.nz <= 32 ? (fills ? 4 : 8) : (fills ? 8 : 16), mb = (A.nz + P - 1) / P;
+    const int P = lm_lanes(ncol, A.nz), mb = (A.nz + P - 1) / P;
     const unsigned nb = (unsigned)((ncol + 256 / P - 1) / (256 / P));
     const ColdValues<T> cold = cold_values<T>();
     TimedLaunch tl(kTimeEnthColumn, ncol * A.nz, st);
@@ -2267,8 +2445,7 @@ hipError_t launch_enth_layer_lm(const EnthArgs<T>& A, T* E_out, T omega_relax, h
     if (!enth_lm_supported(A.nz) || !A.u2d) return hipErrorInvalidValue;
     const long ncol = (long)A.ny * A.nx;
     TimedLaunch tl(kTimeEnthLayer, ncol * A.nz, st);
-    const long items = (ncol + kLmCols - 1) / kLmCols * ((A.nz + kLayerLevels - 1) / kLayerLevels);
-    k_enth_layer_lm<T><<<(unsigned)((items + 3) / 4), 256, 0, st>>>(A, E_out, omega_relax, cold_values<T>());
+    k_enth_layer_lm<T><<<(unsigned)layer_blocks(A.ny, A.nx, A.nz), 256, 0, st>>>(A, E_out, omega_relax, cold_values<T>());
     return hipGetLastError();
 }
 template <typename T>
@@ -2317,6 +2494,8 @@ hipError_t launch_enth_residual_lm(const EnthArgs<T>& A, T* r_out, double* parti
     template hipError_t launch_enth_column_lm<T>(const EnthArgs<T>&, T*, T, int, T, unsigned long long*,            \
                                                  hipStream_t);                                                       \
     template hipError_t launch_enth_layer_lm<T>(const EnthArgs<T>&, T*, T, hipStream_t);                             \
+    template hipError_t launch_enth_sweeps<T>(const EnthArgs<T>&, T*, T*, T, int, T, unsigned long long*,            \
+                                              EnthStatus*, double, double, int, hipStream_t);                        \
     template hipError_t launch_enth_residual_lm<T>(const EnthArgs<T>&, T*, double*, EnthStatus*, int, double, double, \
                                                    hipStream_t);
 INST(double)

@@ -43,6 +43,10 @@ struct EnthStatus {
 
 constexpr int kEnthResBlocks = 2048;  // residual grid (grid-stride over columns)
 constexpr int kEnthRmaxSlots = 256;   // max-|r| accumulators of the column pass (bit patterns of doubles)
+// The accumulators' buffer: two sets, and the barrier's words of the one-launch
+// sweep (three counters, then the workgroups, arrivals and releases of 16 XCDs).
+constexpr int kSweepXcds = 16;
+constexpr int kEnthSlotWords = 2 * kEnthRmaxSlots + 3 + 3 * kSweepXcds;
 
 // max |r| of the residual over the grid, into `max_out` (device), or, with
 // `status`, the sweep bookkeeping: mode 0 starts a sweep (r0), mode 1 ends an
@@ -175,6 +179,13 @@ hipError_t launch_enth_lm_layout(const T* src, T* dst, long ncol, int nz, bool t
 template <typename T>
 hipError_t launch_enth_column_lm(const EnthArgs<T>& A, T* W, T omega_relax, int n_newton, T relaxation,
                                  unsigned long long* rmax, hipStream_t st);
+// n_iter sweeps (column and layer passes, norms, stopping test) of a small map
+// in one launch, from E (= A.E) through W; slots of kEnthSlotWords, zero on entry.
+bool enth_sweeps_fit(int ny, int nx, int nz);
+template <typename T>
+hipError_t launch_enth_sweeps(const EnthArgs<T>& A, T* E, T* W, T omega_relax, int n_newton, T relaxation,
+                              unsigned long long* slots, EnthStatus* status, double rtol, double atol, int n_iter,
+                              hipStream_t st);
 // Layer smoother: E_out = E + omega_relax delta.
 template <typename T>
 hipError_t launch_enth_layer_lm(const EnthArgs<T>& A, T* E_out, T omega_relax, hipStream_t st);

@@ -61,6 +61,13 @@ __device__ __forceinline__ long offC(int i, int j, int ny, int nx) {
     return (long)clampi(i, 0, ny - 1) * nx + clampi(j, 0, nx - 1);
 }
 
+// The XCC (XCD) the calling wave runs on.
+__device__ __forceinline__ unsigned xcc_id() {
+    unsigned v;
+    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(v));
+    return v & 0xf;
+}
+
 template <typename T>
 __device__ __forceinline__ T grounded_fraction(T H, T bed, T c) {
     T z = c * (bed + T(0.917) * H);

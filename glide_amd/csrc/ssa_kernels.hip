@@ -316,13 +316,6 @@ __device__ __forceinline__ void grid_barrier(const PersistentCtl& ctl, unsigned 
     __syncthreads();
 }
 
-// The XCC (XCD) the calling wave runs on.
-__device__ __forceinline__ unsigned xcc_id() {
-    unsigned v;
-    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(v));
-    return v & 0xf;
-}
-
 // Workgroups of a launch are dispatched to the XCDs in turn, so the
 // persistent kernels launch kXcds times the workgroups they need and work in
 // every kXcds-th one only, which puts the working set on one XCD.

@@ -293,7 +293,7 @@ def test_red_black_column_sweep_reaches_the_same_fixed_point():
     assert out[1][2] <= n0
 
 
-@pytest.mark.parametrize("n,nz", [(9, 9), (13, 16), (10, 17), (12, 24), (8, 32), (9, 33), (16, 40), (11, 48), (10, 64),
+@pytest.mark.parametrize("n,nz", [(9, 9), (13, 16), (10, 17), (12, 24), (8, 32), (9, 33), (16, 40), (11, 48), (10, 64), (64, 21), (60, 41),
                                   (182, 20), (182, 21), (182, 28), (182, 32), (182, 33), (182, 41), (182, 50),
                                   (182, 64)])
 def test_tiled_sweep_matches_column_wavefronts(n, nz):
