@@ -164,6 +164,146 @@ __global__ __launch_bounds__(kRowLanes* NW) void k_tab_adj_pass(const TabAdjPass
                                    J.fu, J.fv, J.fH, J.cr, J.omega, colour);
 }
 
+// All cached additive adjoint passes of a level of at most 16 x 16 cells, in one
+// workgroup: 16 lanes a row, four rows a wavefront, one wavefront per SIMD.
+// Everything a pass reads besides the multipliers (stress and flux
+// coefficients, forcing, the patch's 25 factors) is the same in each of them and
+// stays in registers; the multipliers and the rows' exchanges are in LDS.  A pass
+// is then a chain of about 200 instructions and four barriers: at 14 x 14 0.75 us
+// (6.6 us in the workgroup of k_adjoint_coarse, which reads them all again).  Lanes and rows
+// beyond the level compute along on clamped loads; what they hand to a
+// neighbour is zero, as beyond the domain's edge.
+constexpr int kTinySide = 16;
+__global__ __launch_bounds__(kTinySide* kTinySide) void k_adjoint_tiny(
+    SsaArgs<double> a, const double* __restrict__ cache, double* __restrict__ plu, double* __restrict__ plv,
+    double* __restrict__ plH, const double* __restrict__ fu, const double* __restrict__ fv,
+    const double* __restrict__ fH, double calving_rate, double omega, int n_iter) {
+    using T = double;
+    constexpr int N = kTinySide;
+    // multipliers of the facets and cells with a frame of one, and the planes
+    // handed to the row below (edH, Lyy, lH (1 - mask), d3) and above (Lxy, tA, rv)
+    __shared__ T s_lu[N + 2][N + 2], s_lv[N + 2][N + 2], s_dn[4][N + 1][N], s_up[3][N + 1][N];
+    const int ny = a.ny, nx = a.nx, n = ny * nx;
+    const int j = threadIdx.x & (N - 1), i = threadIdx.x >> 4;
+    const int ic = min(i, ny - 1), jc = min(j, nx - 1), ju = min(j, nx), iv = min(i, ny);
+    const int it_ = max(ic - 1, 0), ib = min(ic + 1, ny - 1), jl = max(jc - 1, 0);
+    auto U = [&](const T* p, int r, int c) { return p[r * (nx + 1) + c]; };
+    auto C = [&](const T* p, int r, int c) { return p[r * nx + c]; };
+    const bool cell = i < ny && j < nx, jin = j > 0 && j < nx;
+    const bool vt_in = jin && i > 0 && i < ny, vb_in = jin && i + 1 < ny;
+    const T D = a.dxi, hD = T(0.5) * D;
+
+    // the state's part, once
+    const T u = U(a.u, ic, ju), ur = U(a.u, ic, min(j + 1, nx)), ut = U(a.u, it_, ju), ub = U(a.u, ib, ju);
+    const T v = C(a.v, iv, jc), vb = C(a.v, min(i + 1, ny), jc), vl = C(a.v, iv, jl), vbl = C(a.v, min(i + 1, ny), jl);
+    const T et = vt_in ? hD * ((ut - u) + (v - vl)) : T(0), eb = vb_in ? hD * ((u - ub) + (vb - vbl)) : T(0);
+    const T exx = (ur - u) * D, eyy = (v - vb) * D, qs = et * et + eb * eb;
+    const T sx = T(2) * exx + eyy, sy = exx + T(2) * eyy;
+    const T e2 = exx * exx + eyy * eyy + exx * eyy + T(0.25) * (qs + lane16_right(qs)) + a.P.eps_reg;
+    const T* eta_c = cache + (long)kAdjointCacheEta * n;
+    auto eH_at = [&](int r, int c) { return C(eta_c, r, c) * C(a.H, r, c); };
+    auto g_at = [&](int r, int c) { return T(1) - (T(1) - C(a.phi, r, c)) * T(0.917); };
+    auto S_at = [&](int r, int c) { return C(a.phi, r, c) * C(a.bed, r, c) + g_at(r, c) * C(a.H, r, c); };
+    auto bp_at = [&](int r, int c) { return C(a.beta, r, c) * C(a.phi, r, c); };
+    const T H = C(a.H, ic, jc), Hl = C(a.H, ic, jl), Ht = C(a.H, it_, jc), eta = C(eta_c, ic, jc), eH = eta * H;
+    const T pe = eH * a.P.glen_p * row_rcp(e2);  // edH = pe de2
+    const T eHv = T(0.25) * ((eH + eH_at(it_, jc)) + (eH_at(ic, jl) + eH_at(it_, jl)));
+    const T S = S_at(ic, jc), g = g_at(ic, jc), bp = bp_at(ic, jc);
+    const T dwu = -(T(0.5) * (bp_at(ic, jl) + bp) + a.P.water_drag);
+    const T dwv = -(T(0.5) * (bp_at(it_, jc) + bp) + a.P.water_drag);
+    T fdu, cAx, cBx, kAx, kBx, fdv, cAy, cBy, kAy, kBy;
+    {
+        const T sp = u * u + T(10), rs = row_rsqrt(sp), al = sp * rs, Hm = T(0.5) * (Hl + H);
+        const T dS = T(0.5) * (S - S_at(ic, jl)) * D, HD = Hm * D;
+        fdu = Hm - T(0.5) * (u * rs) * (H - Hl);
+        cAx = T(0.5) * (u + al); cBx = T(0.5) * (u - al);
+        kAx = dS - HD * g_at(ic, jl); kBx = dS + HD * g;
+    }
+    {
+        const T sp = v * v + T(10), rs = row_rsqrt(sp), al = sp * rs, Hm = T(0.5) * (Ht + H);
+        const T dS = T(0.5) * (S_at(it_, jc) - S) * D, HD = Hm * D;
+        fdv = Hm - T(0.5) * (v * rs) * (Ht - H);
+        cAy = T(0.5) * (v - al); cBy = T(0.5) * (v + al);
+        kAy = dS + HD * g_at(it_, jc); kBy = dS - HD * g;
+    }
+    const T mk = C(a.mask, ic, jc), keep = T(1) - mk;
+    T kH = row_rcp(a.dt);
+    if (calving_rate != T(0)) {
+        const int jr = min(jc + 1, nx - 1);
+        const T k = (T(1) - C(a.phi, ic, jc)) * ((T(1) - C(a.phi, ic, jl)) + (T(1) - C(a.phi, ic, jr)) +
+                                                 (T(1) - C(a.phi, it_, jc)) + (T(1) - C(a.phi, ib, jc)));
+        kH += k * calving_rate * D;
+    }
+    const T gu = fu ? U(fu, ic, ju) : T(0), gv = fv ? C(fv, iv, jc) : T(0), gH = fH ? C(fH, ic, jc) : T(0);
+    T A[25];
+#pragma unroll
+    for (int q = 0; q < 25; ++q) A[q] = C(cache + (long)q * n, ic, jc);
+
+    T lu = U(plu, ic, ju), lv = C(plv, iv, jc), lH = C(plH, ic, jc);
+    const T lu_edge = U(plu, ic, nx);  // Dirichlet facets: no pass changes them
+    const T lv_edge = C(plv, ny, jc);
+    s_lu[i + 1][j + 1] = lu;
+    s_lv[i + 1][j + 1] = lv;
+    if (i == ny - 1) s_lv[ny + 1][j + 1] = lv_edge;
+    if (threadIdx.x < 4 * N) s_dn[threadIdx.x >> 4][0][j] = T(0);
+    if (threadIdx.x < 3 * N) s_up[threadIdx.x >> 4][N][j] = T(0);
+    __syncthreads();
+    const bool iin = i > 0 && i < ny;
+#pragma unroll 1
+    for (int it = 0; it < n_iter; ++it) {
+        const T lut = s_lu[max(i, 1)][j + 1], lub = s_lu[i + 2 > N ? N : i + 2][j + 1], lvb = s_lv[i + 2][j + 1];
+        const T lvl = lane16_left(lv), lvbl = lane16_left(lvb), lr = lane16_right(lu);
+        const T lur = j == nx - 1 ? lu_edge : lr, lHm = lH * keep;
+        const T dt_ = vt_in ? hD * ((lut - lu) + (lv - lvl)) : T(0);
+        const T db = vb_in ? hD * ((lu - lub) + (lvb - lvbl)) : T(0);
+        const T dxx = (lur - lu) * D, dyy = (lv - lvb) * D;
+        const T ws = et * dt_ + eb * db;
+        const T de2 = sx * dxx + sy * dyy + T(0.5) * (ws + lane16_right(ws));
+        const T edH = pe * de2;
+        const T Lxx = T(2) * (eH * (T(2) * dxx + dyy) + sx * edH), Lyy = T(2) * (eH * (dxx + T(2) * dyy) + sy * edH);
+        s_dn[0][i + 1][j] = edH;
+        s_dn[1][i + 1][j] = Lyy;
+        s_dn[2][i + 1][j] = lHm;
+        const T dx_ = (lane16_left(lHm) - lHm) * D, Lxl = lane16_left(Lxx);
+        T ru = (Lxx - Lxl) * D + lu * dwu + fdu * dx_ - gu;
+        const T tAx = jin ? cAx * dx_ - lu * kAx : T(0), tBx = jin ? cBx * dx_ - lu * kBx : T(0);
+        __syncthreads();
+        const T edHs = edH + s_dn[0][i][j], dy_ = (lHm - s_dn[2][i][j]) * D;
+        const T edHl = lane16_left(edHs);
+        const T Lxy = vt_in ? T(2) * (eHv * dt_ + et * (T(0.25) * (edHs + edHl))) : T(0);
+        const T Lxr = lane16_right(Lxy);
+        const T rv = iin ? (s_dn[1][i][j] - Lyy) * D + (Lxr - Lxy) * D + lv * dwv + fdv * dy_ - gv : T(0);
+        const T tAy = iin ? cAy * dy_ - lv * kAy : T(0), tBy = iin ? cBy * dy_ - lv * kBy : T(0);
+        s_up[0][i][j] = Lxy;
+        s_up[1][i][j] = tAy;
+        s_up[2][i][j] = rv;
+        __syncthreads();
+        ru += (Lxy - s_up[0][i + 1][j]) * D;
+        if (!jin) ru = T(0);
+        const T rr = lane16_right(ru), tAr = lane16_right(tAx);
+        T rH = lHm * kH + tBx + tAr + tBy + s_up[1][i + 1][j] - T(2) * eta * de2 - gH;
+        if (mk > T(0)) rH = T(0);
+        const T b[5] = {ru, j == nx - 1 ? T(0) : rr, rv, s_up[2][i + 1][j], rH};
+        T d[5];
+        solve_cached(A, b, d);
+        if (!cell) d[0] = d[1] = d[2] = d[3] = d[4] = T(0);
+        s_dn[3][i + 1][j] = d[3];
+        const T d1l = lane16_left(d[1]);
+        lH += omega * d[4];
+        lu += omega * (T(0.5) * d[0] + (j > 0 ? T(0.5) * d1l : T(0)));
+        __syncthreads();
+        lv += omega * (T(0.5) * d[2] + T(0.5) * s_dn[3][i][j]);
+        s_lu[i + 1][j + 1] = lu;
+        if (i < ny) s_lv[i + 1][j + 1] = lv;
+        __syncthreads();
+    }
+    if (cell) {
+        plu[i * (nx + 1) + j] = lu;
+        plv[i * nx + j] = lv;
+        plH[i * nx + j] = lH;
+    }
+}
+
 constexpr int kVjpWaves = 8;
 constexpr int kVjpCols = kRowLanes - 4, kVjpOutRows = kVjpWaves - 2;
 
@@ -300,6 +440,18 @@ hipError_t launch_adjoint_pass_fused(const SsaArgs<T>& a, const T* cache, const 
     TimedLaunch tl(kTimeAdjointCell, (long)a.ny * a.nx, st);
     k_adjoint_rows<T, kAdjWaves, false><<<adjoint_grid<T, kAdjWaves, false>(a.ny, a.nx), dim3(kRowLanes, kAdjWaves), 0, st>>>(
         a, cache, lu, lv, lH, lu_dst, lv_dst, lH_dst, fu, fv, fH, calving_rate, -omega, -1);
+    return hipGetLastError();
+}
+
+bool adjoint_tiny_fits(const SsaArgs<double>& a) {
+    return a.P.linear_drag && a.ny >= 2 && a.nx >= 2 && a.ny <= kTinySide && a.nx <= kTinySide;
+}
+hipError_t launch_adjoint_tiny(const SsaArgs<double>& a, const double* cache, double* lu, double* lv, double* lH,
+                               const double* fu, const double* fv, const double* fH, double calving_rate,
+                               double omega, int n_iter, hipStream_t st) {
+    if (!adjoint_tiny_fits(a)) return hipErrorInvalidValue;
+    TimedLaunch tl(kTimeAdjointCell, (long)a.ny * a.nx * n_iter, st);
+    k_adjoint_tiny<<<1, kTinySide * kTinySide, 0, st>>>(a, cache, lu, lv, lH, fu, fv, fH, calving_rate, -omega, n_iter);
     return hipGetLastError();
 }
 

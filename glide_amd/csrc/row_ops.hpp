@@ -37,6 +37,16 @@ __device__ __forceinline__ double lane_right(double x) {
     return __hiloint2double(dpp_right(__double2hiint(x)), dpp_right(__double2loint(x)));
 }
 
+// The same within each row of 16 lanes.
+__device__ __forceinline__ int dpp16_left(int x) { return __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true); }
+__device__ __forceinline__ int dpp16_right(int x) { return __builtin_amdgcn_update_dpp(0, x, 0x101, 0xf, 0xf, true); }
+__device__ __forceinline__ double lane16_left(double x) {
+    return __hiloint2double(dpp16_left(__double2hiint(x)), dpp16_left(__double2loint(x)));
+}
+__device__ __forceinline__ double lane16_right(double x) {
+    return __hiloint2double(dpp16_right(__double2hiint(x)), dpp16_right(__double2loint(x)));
+}
+
 // 1/a and 1/sqrt(a) to about an ulp: the hardware estimates, refined in FP32 by
 // one step as fast_rcp and fast_rsqrt refine the FP64 ones by two.
 __device__ __forceinline__ double row_rcp(double a) { return fast_rcp(a); }

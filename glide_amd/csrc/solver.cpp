@@ -329,6 +329,12 @@ int vanka_adjoint_sweeps(const glide_level& L, double dt, int n_iter, const glid
     const R* cache = adj_cache(L, prepared);
     if (cache && g_coarse_adjoint && n_iter > 0) {
         SsaArgs<R> a = make_args(L, dt, true);
+        if (adjoint_tiny_fits(a)) {
+            HIP_TRY(launch_adjoint_tiny(a, cache, P(L.lambda_u), P(L.lambda_v), P(L.lambda_H), CP(L.af_u), CP(L.af_v),
+                                        CP(L.af_H), vk.calving_rate, vc.omega, n_iter, st),
+                    "adjoint passes in registers");
+            return GLIDE_OK;
+        }
         if (adjoint_coarse_fits<R>(a)) {
             HIP_TRY(launch_adjoint_coarse<R>(a, cache, P(L.lambda_u), P(L.lambda_v), P(L.lambda_H), CP(L.af_u),
                                              CP(L.af_v), CP(L.af_H), vk.calving_rate, vc.omega, n_iter, st),

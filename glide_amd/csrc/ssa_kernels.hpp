@@ -178,6 +178,12 @@ hipError_t launch_adjoint_persistent(const SsaArgs<T>& a, const T* cache, T* lu,
 constexpr long kAdjointCoarseMaxCells = 512;
 template <typename T>
 bool adjoint_coarse_fits(const SsaArgs<T>& a);
+// The same for levels of at most 16 x 16 cells, whose state and factors fit the
+// workgroup's registers (row_kernels.hip).
+bool adjoint_tiny_fits(const SsaArgs<double>& a);
+hipError_t launch_adjoint_tiny(const SsaArgs<double>& a, const double* cache, double* lu, double* lv, double* lH,
+                               const double* fu, const double* fv, const double* fH, double calving_rate,
+                               double omega, int n_iter, hipStream_t st);
 template <typename T>
 hipError_t launch_adjoint_coarse(const SsaArgs<T>& a, const T* cache, T* lu, T* lv, T* lH, const T* fu, const T* fv,
                                  const T* fH, T calving_rate, T omega, int n_iter, hipStream_t st);

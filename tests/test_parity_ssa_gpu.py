@@ -460,6 +460,13 @@ def test_adjoint_coarse_workgroup_matches_launches(shape):
         assert rel_err(x, y) < 1e-13
 
 
+@pytest.mark.parametrize("shape", [(2, 2), (3, 16), (16, 16), (14, 14), (8, 15), (15, 16), (16, 5), (8, 8), (17, 16)])
+def test_adjoint_tiny_level_matches_launches(shape):
+    """Levels of at most 16 x 16 cells, whose passes run in one workgroup's
+    registers, and the first beyond them: the same comparison and bar."""
+    test_adjoint_coarse_workgroup_matches_launches(shape)
+
+
 @pytest.mark.parametrize("shape", [(36, 52), (70, 130), (17, 29), (1030, 200)])
 def test_adjoint_pass_fused_matches_launches(shape):
     """A cached adjoint pass as one launch (transpose operator, patch solves
