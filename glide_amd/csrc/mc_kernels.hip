@@ -63,6 +63,76 @@ struct McCentre {
     }
 };
 
+// The folded system of the cell at LDS row rr, column c (grid cell (i, j)) for
+// the state in LDS; its viscosity comes back in e_c.  EDGE: the cell may lie on
+// the domain edge.
+template <typename T, bool LINEAR, bool EDGE, class L>
+__device__ __forceinline__ void mc_cell_sys(CellSys<T>& cs, const L& s, const SsaArgs<T>& a, const McCentre<T>& q,
+                                            const VankaArgs<T>& vk, int rr, int c, int i, int j, T& e_c) {
+    const int ny = a.ny, nx = a.nx, k = rr - 1;
+    const bool il = !EDGE || j > 0, ir = !EDGE || j + 1 < nx, it_ = !EDGE || i > 0, ib = !EDGE || i + 1 < ny;
+    const T D = a.dxi, D2 = D * D;
+    const T e_l = s.eH[k][c - 1], e_r = s.eH[k][c + 1], e_t = s.eH[k - 1][c], e_b = s.eH[k + 1][c];
+    e_c = s.eta[k][c];
+    cs.D = D;
+    cs.hD = T(0.5) * D;
+    cs.H_l = s.H[k][c - 1]; cs.H_r = s.H[k][c + 1]; cs.H_t = s.H[k - 1][c]; cs.H_b = s.H[k + 1][c];
+    cs.dL = il ? D : T(0); cs.dR = ir ? D : T(0); cs.dT = it_ ? D : T(0); cs.dB = ib ? D : T(0);
+    const T p_c = s.phi[k][c];
+    T kcal = T(0);
+    if (vk.calving_rate != T(0))
+        kcal = (T(1) - p_c) * vk.calving_rate *
+               ((T(1) - s.phi[k][c - 1]) + (T(1) - s.phi[k][c + 1]) + (T(1) - s.phi[k - 1][c]) +
+                (T(1) - s.phi[k + 1][c]));
+    cs.r4h = T(1) / a.dt + kcal * D;
+    cs.j24c = cs.r4h + vk.mc_damping;
+    cs.f4 = q.f[4];
+    cs.kH = T(2) * e_c * D2;
+    const T qc = T(0.25) * e_c;
+    const bool vtl = it_ && il, vtr = it_ && ir, vbl = ib && il, vbr = ib && ir;
+    cs.C_tl = vtl ? T(0.25) * (s.eH[k - 1][c - 1] + e_t + e_l) : T(0);
+    cs.C_tr = vtr ? T(0.25) * (e_t + s.eH[k - 1][c + 1] + e_r) : T(0);
+    cs.C_bl = vbl ? T(0.25) * (e_l + s.eH[k + 1][c - 1] + e_b) : T(0);
+    cs.C_br = vbr ? T(0.25) * (e_r + e_b + s.eH[k + 1][c + 1]) : T(0);
+    cs.q_tl = vtl ? qc : T(0); cs.q_tr = vtr ? qc : T(0); cs.q_bl = vbl ? qc : T(0); cs.q_br = vbr ? qc : T(0);
+    cs.u_tl = s.u[rr - 1][c]; cs.u_tr = s.u[rr - 1][c + 1];
+    cs.u_bl = s.u[rr + 1][c]; cs.u_br = s.u[rr + 1][c + 1];
+    cs.v_lt = s.v[rr][c - 1]; cs.v_lb = s.v[rr + 1][c - 1];
+    cs.v_rt = s.v[rr][c + 1]; cs.v_rb = s.v[rr + 1][c + 1];
+    cs.s_tl = cs.hD * (cs.u_tl - cs.v_lt);
+    cs.s_tr = cs.hD * (cs.u_tr + cs.v_rt);
+    cs.s_bl = -cs.hD * (cs.u_bl + cs.v_lb);
+    cs.s_br = cs.hD * (cs.v_rb - cs.u_br);
+    const T nl = il ? T(2) * e_l * D2 : T(0), nr = ir ? T(2) * e_r * D2 : T(0);
+    const T nt = it_ ? T(2) * e_t * D2 : T(0), nb = ib ? T(2) * e_b * D2 : T(0);
+    cs.c0 = -nl * (cs.v_lt - cs.v_lb - T(2) * s.u[rr][c - 1]) - q.f[0];
+    cs.c1 = nr * (T(2) * s.u[rr][c + 2] + cs.v_rt - cs.v_rb) - q.f[1];
+    cs.c2 = nt * (cs.u_tr - cs.u_tl + T(2) * s.v[rr - 1][c]) - q.f[2];
+    cs.c3 = -nb * (cs.u_br - cs.u_bl - T(2) * s.v[rr + 2][c]) - q.f[3];
+    const T b_c = s.bp[k][c];
+    cs.be_l = T(0.5) * (s.bp[k][c - 1] + b_c);
+    cs.be_r = T(0.5) * (b_c + s.bp[k][c + 1]);
+    cs.be_t = T(0.5) * (s.bp[k - 1][c] + b_c);
+    cs.be_b = T(0.5) * (b_c + s.bp[k + 1][c]);
+    const T lin = LINEAR ? T(1) : T(0), wd = a.P.water_drag;
+    cs.o0 = -T(2) * nl - lin * (cs.be_l + wd);
+    cs.o1 = -T(2) * nr - lin * (cs.be_r + wd);
+    cs.o2 = -T(2) * nt - lin * (cs.be_t + wd);
+    cs.o3 = -T(2) * nb - lin * (cs.be_b + wd);
+    cs.a0 = cs.o0 - (cs.C_tl + cs.C_bl) * D2 - vk.ssa_damping;
+    cs.a1 = cs.o1 - (cs.C_tr + cs.C_br) * D2 - vk.ssa_damping;
+    cs.a2 = cs.o2 - (cs.C_tl + cs.C_tr) * D2 - vk.ssa_damping;
+    cs.a3 = cs.o3 - (cs.C_bl + cs.C_br) * D2 - vk.ssa_damping;
+    cs.h0 = -(cs.q_tl + cs.q_bl) * D2;
+    cs.h1 = -(cs.q_tr + cs.q_br) * D2;
+    cs.h2 = -(cs.q_tl + cs.q_tr) * D2;
+    cs.h3 = -(cs.q_bl + cs.q_br) * D2;
+    cs.eD = T(2) * e_c * D;
+    cs.S_l = s.S[k][c - 1]; cs.S_r = s.S[k][c + 1]; cs.S_t = s.S[k - 1][c]; cs.S_b = s.S[k + 1][c];
+    cs.Zc = p_c * q.bed;
+    cs.gc = T(1) - (T(1) - p_c) * T(0.917);
+}
+
 // Local Newton iteration of the cell at LDS row rr, column c (grid cell (i, j))
 // against the state in LDS: the new unknowns x, the active-set flag, and the
 // cell's viscosity and surface coefficients.  EDGE: the cell may lie on the
@@ -72,70 +142,10 @@ __device__ __forceinline__ void mc_newton(const McLds<T, NW>& s, const SsaArgs<T
                                           const VankaArgs<T>& vk, bool solves, int rr, int c, int i, int j, T x[5],
                                           T& masked, T& e_c, T& Zc, T& gc) {
     const int ny = a.ny, nx = a.nx, k = rr - 1;
-    const bool il = !EDGE || j > 0, ir = !EDGE || j + 1 < nx, it_ = !EDGE || i > 0, ib = !EDGE || i + 1 < ny;
-    const T D = a.dxi, D2 = D * D;
     CellSys<T> cs;
-    {
-        const T e_l = s.eH[k][c - 1], e_r = s.eH[k][c + 1], e_t = s.eH[k - 1][c], e_b = s.eH[k + 1][c];
-        e_c = s.eta[k][c];
-        cs.D = D;
-        cs.hD = T(0.5) * D;
-        cs.H_l = s.H[k][c - 1]; cs.H_r = s.H[k][c + 1]; cs.H_t = s.H[k - 1][c]; cs.H_b = s.H[k + 1][c];
-        cs.dL = il ? D : T(0); cs.dR = ir ? D : T(0); cs.dT = it_ ? D : T(0); cs.dB = ib ? D : T(0);
-        const T p_c = s.phi[k][c];
-        T kcal = T(0);
-        if (vk.calving_rate != T(0))
-            kcal = (T(1) - p_c) * vk.calving_rate *
-                   ((T(1) - s.phi[k][c - 1]) + (T(1) - s.phi[k][c + 1]) + (T(1) - s.phi[k - 1][c]) +
-                    (T(1) - s.phi[k + 1][c]));
-        cs.r4h = T(1) / a.dt + kcal * D;
-        cs.j24c = cs.r4h + vk.mc_damping;
-        cs.f4 = q.f[4];
-        cs.kH = T(2) * e_c * D2;
-        const T qc = T(0.25) * e_c;
-        const bool vtl = it_ && il, vtr = it_ && ir, vbl = ib && il, vbr = ib && ir;
-        cs.C_tl = vtl ? T(0.25) * (s.eH[k - 1][c - 1] + e_t + e_l) : T(0);
-        cs.C_tr = vtr ? T(0.25) * (e_t + s.eH[k - 1][c + 1] + e_r) : T(0);
-        cs.C_bl = vbl ? T(0.25) * (e_l + s.eH[k + 1][c - 1] + e_b) : T(0);
-        cs.C_br = vbr ? T(0.25) * (e_r + e_b + s.eH[k + 1][c + 1]) : T(0);
-        cs.q_tl = vtl ? qc : T(0); cs.q_tr = vtr ? qc : T(0); cs.q_bl = vbl ? qc : T(0); cs.q_br = vbr ? qc : T(0);
-        cs.u_tl = s.u[rr - 1][c]; cs.u_tr = s.u[rr - 1][c + 1];
-        cs.u_bl = s.u[rr + 1][c]; cs.u_br = s.u[rr + 1][c + 1];
-        cs.v_lt = s.v[rr][c - 1]; cs.v_lb = s.v[rr + 1][c - 1];
-        cs.v_rt = s.v[rr][c + 1]; cs.v_rb = s.v[rr + 1][c + 1];
-        cs.s_tl = cs.hD * (cs.u_tl - cs.v_lt);
-        cs.s_tr = cs.hD * (cs.u_tr + cs.v_rt);
-        cs.s_bl = -cs.hD * (cs.u_bl + cs.v_lb);
-        cs.s_br = cs.hD * (cs.v_rb - cs.u_br);
-        const T nl = il ? T(2) * e_l * D2 : T(0), nr = ir ? T(2) * e_r * D2 : T(0);
-        const T nt = it_ ? T(2) * e_t * D2 : T(0), nb = ib ? T(2) * e_b * D2 : T(0);
-        cs.c0 = -nl * (cs.v_lt - cs.v_lb - T(2) * s.u[rr][c - 1]) - q.f[0];
-        cs.c1 = nr * (T(2) * s.u[rr][c + 2] + cs.v_rt - cs.v_rb) - q.f[1];
-        cs.c2 = nt * (cs.u_tr - cs.u_tl + T(2) * s.v[rr - 1][c]) - q.f[2];
-        cs.c3 = -nb * (cs.u_br - cs.u_bl - T(2) * s.v[rr + 2][c]) - q.f[3];
-        const T b_c = s.bp[k][c];
-        cs.be_l = T(0.5) * (s.bp[k][c - 1] + b_c);
-        cs.be_r = T(0.5) * (b_c + s.bp[k][c + 1]);
-        cs.be_t = T(0.5) * (s.bp[k - 1][c] + b_c);
-        cs.be_b = T(0.5) * (b_c + s.bp[k + 1][c]);
-        const T lin = LINEAR ? T(1) : T(0), wd = a.P.water_drag;
-        cs.o0 = -T(2) * nl - lin * (cs.be_l + wd);
-        cs.o1 = -T(2) * nr - lin * (cs.be_r + wd);
-        cs.o2 = -T(2) * nt - lin * (cs.be_t + wd);
-        cs.o3 = -T(2) * nb - lin * (cs.be_b + wd);
-        cs.a0 = cs.o0 - (cs.C_tl + cs.C_bl) * D2 - vk.ssa_damping;
-        cs.a1 = cs.o1 - (cs.C_tr + cs.C_br) * D2 - vk.ssa_damping;
-        cs.a2 = cs.o2 - (cs.C_tl + cs.C_tr) * D2 - vk.ssa_damping;
-        cs.a3 = cs.o3 - (cs.C_bl + cs.C_br) * D2 - vk.ssa_damping;
-        cs.h0 = -(cs.q_tl + cs.q_bl) * D2;
-        cs.h1 = -(cs.q_tr + cs.q_br) * D2;
-        cs.h2 = -(cs.q_tl + cs.q_tr) * D2;
-        cs.h3 = -(cs.q_bl + cs.q_br) * D2;
-        cs.eD = T(2) * e_c * D;
-        cs.S_l = s.S[k][c - 1]; cs.S_r = s.S[k][c + 1]; cs.S_t = s.S[k - 1][c]; cs.S_b = s.S[k + 1][c];
-        cs.Zc = Zc = p_c * q.bed;
-        cs.gc = gc = T(1) - (T(1) - p_c) * T(0.917);
-    }
+    mc_cell_sys<T, LINEAR, EDGE>(cs, s, a, q, vk, rr, c, i, j, e_c);
+    Zc = cs.Zc;
+    gc = cs.gc;
     const T thk = q.thk;
     x[0] = s.u[rr][c];
     x[1] = s.u[rr][c + 1];
@@ -317,6 +327,135 @@ __global__ __launch_bounds__(kRowLanes* NW) void k_mc_pass(SsaArgs<T> a, T* __re
     mc_pass_body<T, NW, LINEAR>(b % gx, b / gx, a, u_dst, v_dst, H_dst, mask, phi_dst, vk);
 }
 
+// All additive forward passes of a level of at most 16 x 16 cells in one
+// workgroup, the state in LDS: 16 lanes a row, four rows a wavefront, one
+// wavefront per SIMD.  A pass of k_vanka_persistent reads the level's state and
+// parameters through the L2 twice (viscosity, then patches) and meets other
+// workgroups at a barrier; most passes of the coarsest level run one or two
+// Newton iterations, so that this was most of a pass (14 x 14: 5.9 us, here 3.5).
+constexpr int kTinySide = 16;
+template <typename T>
+struct TinyLds {  // the planes of McLds for one tile of 16 x 16
+    static constexpr int kF = kTinySide + 6, kC = kTinySide + 4;
+    T u[kF][kF], v[kF][kF];
+    T H[kC][kF], eH[kC][kF], eta[kC][kF], S[kC][kF], bp[kC][kF], phi[kC][kF];
+    T w3[kTinySide + 1][kTinySide];  // bottom-facet increments of row r at r + 1
+};
+template <bool LINEAR>
+__global__ __launch_bounds__(kTinySide* kTinySide, 1) void k_vanka_tiny(SsaArgs<double> a, double* __restrict__ pu,
+                                                                        double* __restrict__ pv,
+                                                                        double* __restrict__ pH,
+                                                                        double* __restrict__ mask,
+                                                                        VankaArgs<double> vk, double omega,
+                                                                        int n_iter) {
+    using T = double;
+    using L = TinyLds<T>;
+    __shared__ L s;
+    const int ny = a.ny, nx = a.nx, tid = threadIdx.x;
+    const int j = tid & (kTinySide - 1), i = tid >> 4, rr = i + 3, c = j + 3, k = rr - 1;
+    const bool cell = i < ny && j < nx;
+    for (int q = tid; q < L::kF * L::kF; q += kTinySide * kTinySide) {
+        const int r = q / L::kF, l = q % L::kF;
+        const int ri = clampi(r - 3, 0, ny - 1), lj = clampi(l - 3, 0, nx - 1);
+        s.u[r][l] = pu[ri * (nx + 1) + clampi(l - 3, 0, nx)];
+        s.v[r][l] = pv[clampi(r - 3, 0, ny) * nx + lj];
+        if (r >= 1 && r <= L::kC) {
+            const int o = ri * nx + lj;
+            const T H = pH[o], p = a.phi[o];
+            s.H[r - 1][l] = H;
+            s.phi[r - 1][l] = p;
+            s.S[r - 1][l] = p * a.bed[o] - (T(1) - p) * T(0.917) * H + H;
+            s.bp[r - 1][l] = a.beta[o] * p;
+            s.eH[r - 1][l] = T(0);
+            s.eta[r - 1][l] = T(0);
+        }
+    }
+    if (tid < kTinySide) s.w3[0][tid] = T(0);
+    const int ic = min(i, ny - 1), jc = min(j, nx - 1);
+    McCentre<T> q{};
+    q.load(a, ic, jc);
+    const T B = a.B[ic * nx + jc];
+    T masked = mask[ic * nx + jc];
+    const bool jin = j > 0 && j < nx, vt_in = jin && i > 0 && i < ny, vb_in = jin && i + 1 < ny;
+    const bool pin0 = j == 0, pin1 = j == nx - 1, pin2 = i == 0, pin3 = i == ny - 1;
+    const T D = a.dxi, hD = T(0.5) * D, tol = T(1e-6);
+    __syncthreads();
+#pragma unroll 1
+    for (int pass = 0; pass < n_iter; ++pass) {
+        {
+            const T u = s.u[rr][c], v = s.v[rr][c], vb = s.v[rr + 1][c];
+            const T et = vt_in ? hD * ((s.u[rr - 1][c] - u) + (v - s.v[rr][c - 1])) : T(0);
+            const T eb = vb_in ? hD * ((u - s.u[rr + 1][c]) + (vb - s.v[rr + 1][c - 1])) : T(0);
+            const T qs = et * et + eb * eb, exx = (s.u[rr][c + 1] - u) * D, eyy = (v - vb) * D;
+            const T e2 = exx * exx + eyy * eyy + exx * eyy + T(0.25) * (qs + lane16_right(qs)) + a.P.eps_reg;
+            const T eta = T(0.5) * B * glen_power(e2, a.P);
+            if (cell) {
+                s.eta[k][c] = eta;
+                s.eH[k][c] = eta * s.H[k][c];
+            }
+        }
+        __syncthreads();
+        const T x0[5] = {s.u[rr][c], s.u[rr][c + 1], s.v[rr][c], s.v[rr + 1][c], s.H[k][c]};
+        T x[5] = {x0[0], x0[1], x0[2], x0[3], x0[4]}, cmp[5] = {T(0), T(0), T(0), T(0), T(0)};
+        CellSys<T> cs;
+        T e_c;
+        mc_cell_sys<T, LINEAR, true>(cs, s, a, q, vk, rr, c, i, j, e_c);
+        bool go = cell && vk.newton_steps > 0;
+        int it = 0;
+        while (__any(go)) {  // as cell_newton
+            T J[25], r[5], d[5];
+            cell_system<T, T, LINEAR>(cs, cs, x, J, r, a.P);
+            if (pin0) { pin_row(J, 0); r[0] = x[0]; }
+            if (pin1) { pin_row(J, 1); r[1] = x[1]; }
+            if (pin2) { pin_row(J, 2); r[2] = x[2]; }
+            if (pin3) { pin_row(J, 3); r[3] = x[3]; }
+            const bool pin4 = (x[4] - a.dt * r[4]) <= q.thk;
+            if (pin4) {
+                pin_row(J, 4);
+                r[4] = x[4] - q.thk;
+            }
+            masked = go ? (pin4 ? T(1) : T(0)) : masked;
+            lu5_solve_rcp(J, r, d);
+            const T rnorm = r[0] * r[0] + r[1] * r[1] + r[2] * r[2] + r[3] * r[3] + r[4] * r[4];
+#pragma unroll
+            for (int m = 0; m < 5; ++m) {  // compensated relaxed update, local relaxation 0.5
+                const T y = T(-0.5) * d[m] - cmp[m];
+                T t = x[m] + y;
+                const T e = (t - x[m]) - y;
+                if (m == 4) t = fmax(t, q.thk);
+                cmp[m] = go ? e : cmp[m];
+                x[m] = go ? t : x[m];
+            }
+            it += go ? 1 : 0;
+            go = go && it < vk.newton_steps && rnorm > tol;
+        }
+        const T w0 = T(0.5) * (x[0] - x0[0]), w1 = cell ? T(0.5) * (x[1] - x0[1]) : T(0);
+        const T w2 = T(0.5) * (x[2] - x0[2]), w3 = cell ? T(0.5) * (x[3] - x0[3]) : T(0);
+        s.w3[i + 1][j] = w3;
+        const T w1l = lane16_left(w1);
+        __syncthreads();
+        if (cell) {
+            s.u[rr][c] = x0[0] + omega * (w0 + w1l);
+            if (pin1) s.u[rr][c + 1] = x0[1] + omega * w1;
+            s.v[rr][c] = x0[2] + omega * (w2 + s.w3[i][j]);
+            if (pin3) s.v[rr + 1][c] = x0[3] + omega * w3;
+            const T H = x0[4] + omega * (x[4] - x0[4]);
+            s.H[k][c] = H;
+            s.S[k][c] = cs.Zc + cs.gc * H;
+        }
+        __syncthreads();
+    }
+    if (cell) {
+        const int o = i * nx + j;
+        pu[o + i] = s.u[rr][c];
+        if (pin1) pu[o + i + 1] = s.u[rr][c + 1];
+        pv[o] = s.v[rr][c];
+        if (pin3) pv[o + nx] = s.v[rr + 1][c];
+        pH[o] = s.H[k][c];
+        mask[o] = masked;
+    }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void k_pin_rows(T* __restrict__ du, T* __restrict__ dv, T* __restrict__ dH,
                                                   const T* __restrict__ mask, int ny, int nx) {
@@ -330,6 +469,24 @@ __global__ __launch_bounds__(256) void k_pin_rows(T* __restrict__ du, T* __restr
 }
 
 }  // namespace
+
+// The coarsest level's calls (200 passes), whose passes mostly take one or two
+// Newton iterations: per pass at 14 x 14 in 200 passes 3.5 against 5.9 us.  The ten
+// or twenty passes of another level are bound by their thirty iterations a cell,
+// the same in both forms.  With four rows or fewer one wavefront holds the level.
+bool vanka_tiny_fits(int ny, int nx, int n_iter) {
+    return n_iter >= 32 && ny > 4 && ny <= kTinySide && nx >= 2 && nx <= kTinySide;
+}
+hipError_t launch_vanka_tiny(const SsaArgs<double>& a, double* u, double* v, double* H, double* mask,
+                             const VankaArgs<double>& vk, double omega, int n_iter, hipStream_t st) {
+    if (!vanka_tiny_fits(a.ny, a.nx, n_iter) || vk.local_fp32) return hipErrorInvalidValue;
+    TimedLaunch tl(kTimeVankaCell, (long)a.ny * a.nx * n_iter, st);
+    if (a.P.linear_drag)
+        k_vanka_tiny<true><<<1, kTinySide * kTinySide, 0, st>>>(a, u, v, H, mask, vk, omega, n_iter);
+    else
+        k_vanka_tiny<false><<<1, kTinySide * kTinySide, 0, st>>>(a, u, v, H, mask, vk, omega, n_iter);
+    return hipGetLastError();
+}
 
 template <typename T>
 hipError_t launch_pin_rows(T* du, T* dv, T* dH, const T* mask, int ny, int nx, hipStream_t st) {

@@ -245,6 +245,12 @@ int vanka_sweeps(const glide_level& L, double dt, int n_iter, const glide_vanka_
         R* alt_u = P(L.work);
         R* alt_v = alt_u + nU(L);
         R* alt_H = alt_v + nV(L);
+        if (g_persistent_forward && !vk.local_fp32 && vanka_tiny_fits(L.ny, L.nx, n_iter)) {
+            HIP_TRY(launch_vanka_tiny(make_args(L, dt, false), P(L.u), P(L.v), P(L.H), P(L.mask), vk, vc.omega, n_iter,
+                                      st),
+                    "vanka passes in one workgroup");
+            return GLIDE_OK;
+        }
         if (g_persistent_forward && n_iter > 1 && vanka_persistent_fits(L.ny, L.nx)) {
             PersistentCtl ctl;
             GLIDE_TRY(persistent_ctl(L, &ctl));

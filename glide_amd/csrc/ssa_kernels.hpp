@@ -113,6 +113,11 @@ constexpr int kPersistentRows = GLIDE_PERSISTENT_ROWS;
 #define GLIDE_PERSISTENT_MAX_BLOCKS 32
 #endif
 constexpr int kPersistentMaxBlocks = GLIDE_PERSISTENT_MAX_BLOCKS;
+// Forward smoothing passes of levels of at most 16 x 16 cells in one workgroup,
+// in place (mc_kernels.hip); not the mixed form.
+bool vanka_tiny_fits(int ny, int nx, int n_iter);
+hipError_t launch_vanka_tiny(const SsaArgs<double>& a, double* u, double* v, double* H, double* mask,
+                             const VankaArgs<double>& vk, double omega, int n_iter, hipStream_t st);
 bool vanka_persistent_fits(int ny, int nx);
 // Control words of a persistent launch: sync holds three 64-bit words the
 // launch zeroes first (arrival counter, timeout flag, XCD mask); a timed-out

@@ -268,6 +268,31 @@ def test_vanka_persistent_passes_match_fused_launches(shape, n_pass, m):
         assert np.array_equal(x, y)
 
 
+@pytest.mark.parametrize("shape", [(5, 16), (16, 16), (14, 14), (8, 8), (13, 7), (16, 2), (6, 15)])
+@pytest.mark.parametrize("n_pass,m", [(33, 1.0), (32, 1.0 / 3.0)])
+def test_vanka_tiny_level_matches_launches(shape, n_pass, m):
+    """Levels of at most 16 x 16 cells, whose passes run in one workgroup with
+    the state in LDS: one launch per pass gives the same state (the bar of a few
+    passes against the oracle) and active set."""
+    from glide_amd import _lib
+    ny, nx = shape
+    print(f"vanka tiny shape={shape} passes={n_pass} m={m:.3f}", flush=True)
+    F = dome_fields(ny=ny, nx=nx, seed=47, mask_frac=0.1)
+    out = []
+    for one in (True, False):
+        _lib.forward_persistent_enable(one)
+        g = grid_from(F)
+        g.sliding.m.set(m)
+        g.calving.calving_rate.set(0.2)
+        g.forward_operators.vanka_sweep(10.0, n_pass, freeze_phi=True)
+        torch.cuda.synchronize()
+        out.append([N(t.data) for t in (g.state.u, g.state.v, g.state.H, g.state.mask)])
+    _lib.forward_persistent_enable(True)
+    for x, y in zip(out[0][:3], out[1][:3]):
+        assert rel_err(x, y) < 1e-11
+    assert np.array_equal(out[0][3], out[1][3])
+
+
 @pytest.mark.parametrize("shape,n_pass", [((32, 32), 30), ((64, 64), 5), ((128, 128), 3), ((17, 29), 4)])
 def test_vanka_mixed_one_launch_forms_match_two_launch_passes(shape, n_pass):
     """The mixed form (FP32 patch Jacobian and LU) through the one-launch
