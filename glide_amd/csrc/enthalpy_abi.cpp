@@ -195,9 +195,13 @@ int sweep_core(const glide_enth_column* C, double dt, int n_iter, const glide_en
         L.skip = &status->done;
         EnthArgs<R> Lw = L;
         Lw.E = Wlm;
-        HIP_TRY(launch_enth_reduce_slots(rmax, status, 0, rtol, atol, st), "enthalpy max slots");
-        if (enth_sweeps_fit(C->ny, C->nx, nz)) {
-            HIP_TRY(launch_enth_sweeps<R>(L, Elm, Wlm, cfg->omega, cfg->n_newton, cfg->relaxation, rmax, status, rtol,
+        // the one-launch form keeps its norms and barrier in r_E, which only the
+        // final residual below fills: each column's own, on whatever stream
+        const bool one_launch = enth_sweeps_fit(C->ny, C->nx, nz) && plane >= kEnthSlotWords;
+        unsigned long long* slots = one_launch ? reinterpret_cast<unsigned long long*>(C->r_E) : rmax;
+        HIP_TRY(launch_enth_reduce_slots(slots, status, 0, rtol, atol, st), "enthalpy max slots");
+        if (one_launch) {
+            HIP_TRY(launch_enth_sweeps<R>(L, Elm, Wlm, cfg->omega, cfg->n_newton, cfg->relaxation, slots, status, rtol,
                                           atol, n_iter, st),
                     "enthalpy sweeps");
         } else
