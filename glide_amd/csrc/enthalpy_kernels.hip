@@ -1570,8 +1570,8 @@ hipError_t launch_enth_elementary(const double* x, long n, double* e_out, double
 // neighbouring blocks', the first rows are eliminated into one row per lane
 // in the blocks' last unknowns, which cyclic reduction across the P lanes
 // solves, and each lane substitutes back.  Neighbouring lanes exchange values
-// through DPP row shifts, not LDS.  The layer pass takes a few levels of a tile
-// per wavefront; the residual one thread per column, streaming up the levels.  The rows are level_row's, with
+// through DPP row shifts, not LDS.  The layer pass and the residual take a few
+// levels of a tile per wavefront.  The rows are level_row's, with
 // the terms that do not depend on the column's own enthalpy (the previous
 // enthalpy, the forcing and the neighbouring columns' advection) gathered
 // into one value per level.
@@ -1680,20 +1680,6 @@ __device__ __forceinline__ LmStencil lm_stencil(const EnthArgs<T>& A, long ncol,
             lm_col((long)im * nx + j, ncol, A.nz), lm_col((long)ip * nx + j, ncol, A.nz)};
 }
 
-// The E-independent part of level k's row on the tiles: -rho H_prev E_prev / dt
-// - f_E plus the neighbours' horizontal advection.
-template <typename T>
-__device__ __forceinline__ T lm_constant(const EnthArgs<T>& A, const LmHoriz<T>& hc, const LmStencil& n, int k, T hp,
-                                         T invdt) {
-    const long o = n.c.base + (long)k * n.c.stride;
-    T g = -(T(kRhoI) * hp * A.E_prev[o] * invdt) - A.f_E[o];
-    if (A.flags & 1) {
-        auto E = [&](const LmCol& q) { return A.E[q.base + (long)k * q.stride]; };
-        g += (hc.xp * E(n.xp) + hc.xm * E(n.xm)) + (hc.ym * E(n.ym) + hc.yp * E(n.yp));
-    }
-    return g;
-}
-
 // One stage of parallel cyclic reduction over the P lanes of a column
 // group, one row a z_{q-1} + b z_q + c z_{q+1} = d per lane: a = 0 on the
 // group's first S lanes and c = 0 on its last S lanes (true of the initial
@@ -1742,7 +1728,8 @@ __device__ __forceinline__ void column_lm_body(long vb, const EnthArgs<T>& A, T*
     const T dsig = T(1) / T(nz - 1);
     const LmStencil n = lm_stencil(A, ncol, i, j);
     // every load of the column at once (levels beyond it read its last one):
-    // E, and the E-independent part of the rows (lm_constant)
+    // E, and what the E-independent part of the rows takes: -rho H_prev E_prev / dt
+    // - f_E plus the neighbours' horizontal advection
     // the pass's starting E, the constants and omega stay in LDS (each thread
     // reads its own), which leaves the registers to the rows and the elimination
     __shared__ T s_E[MB][256], s_G[MB][256], s_om[MB][256];
@@ -1908,49 +1895,17 @@ __global__ __launch_bounds__(256, 2) void k_enth_column_lm(EnthArgs<T> A, T* __r
     column_lm_body<T, P, MB>(xcd_block(blockIdx.x, gridDim.x), A, W, omega_relax, n_newton, relaxation, rmax, cold);
 }
 
-// One column's rows on the tiles, streamed up the levels:
-// calls f(k, w) with level k's row (residual with forcing in w.r) for
-// k = 0 .. nz - 2 of a thick column.
-template <typename T, typename F>
-__device__ __forceinline__ void lm_stream_rows(const EnthArgs<T>& A, long ncol, long col, F&& f) {
-    const int nz = A.nz, nx = A.nx, i = (int)(col / nx), j = (int)(col % nx);
-    const LmStencil n = lm_stencil(A, ncol, i, j);
-    const long step = n.c.stride;
-    const T h = A.H[col], hp = A.H_prev[col];
-    const ColConst<T> cst = col_const(A, h);
-    const T invdt = cst.invdt, dsig = cst.dsig;
-    const LmHoriz<T> hc = lm_horiz(A, i, j);
-    const T B0 = T(kRhoI) * h * invdt + hc.self;
-    const T* E = A.E + n.c.base;
-    const T* om = A.omega ? A.omega + n.c.base : nullptr;
-    T Em = E[0], Ek = E[0], Ep = E[step];
-    T om_m = om ? om[0] : T(0), om_k = om_m, om_p = om ? om[min(1, nz - 1) * step] : T(0);
-    T Kl = T(0);
-    for (int k = 0; k < nz - 1; ++k) {
-        const T Ep_k = e_pmp(T(k) * dsig, h), Ep_p = e_pmp(T(k + 1) * dsig, h);
-        const T Ku = diffusivity(T(0.5) * (Ek + Ep), T(0.5) * (Ep_k + Ep_p));
-        Row<T> w{B0 * Ek + lm_constant(A, hc, n, k, hp, invdt), T(0), B0, T(0)};
-        column_terms(A, cst, k, h, Ek, Em, Ep, om_m, om_k, om_p, Ku, Kl, w);
-        f(k, Ek, w);
-        Kl = Ku;
-        Em = Ek;
-        Ek = Ep;
-        Ep = (k + 2 < nz) ? E[(k + 2) * step] : T(0);
-        om_m = om_k;
-        om_k = om_p;
-        om_p = om ? om[min(k + 2, nz - 1) * step] : T(0);
-    }
-}
-
 // Pointwise Jacobi layer smoother on the tiles:
 // E_out = E + omega_relax (-r / J_kk), E_out = E on surface rows and thin columns.
 // A wavefront takes kLayerLevels levels of a tile, all loads at once: one thread
 // per column streaming up all of them kept two levels in flight (127 us at 512 x
 // 512 x 41, and 28 us at 48 x 48 x 41).
 constexpr int kLayerLevels = 6;
-template <typename T>
-__device__ __forceinline__ void layer_lm_body(long vb, const EnthArgs<T>& A, T* E_out, T omega_relax,
-                                              const ColdValues<T>& cold) {
+// f(column, level, position in the tiles, E, row, active) for each level of the
+// wavefront's chunk; active: the row is one of the system's (neither a surface
+// row nor a thin column).
+template <typename T, typename F>
+__device__ __forceinline__ void lm_chunk_rows(long vb, const EnthArgs<T>& A, const ColdValues<T>& cold, F&& f) {
     constexpr int CH = kLayerLevels;
     const int nz = A.nz, nch = (nz + CH - 1) / CH;
     const long ncol = (long)A.ny * A.nx, items = (ncol + kLmCols - 1) / kLmCols * nch;
@@ -1995,21 +1950,29 @@ __device__ __forceinline__ void layer_lm_body(long vb, const EnthArgs<T>& A, T* 
     for (int m = 0; m < CH; ++m) {
         const int k = kb + m;
         if (k >= nz) break;
-        T out = T(0);
+        Row<T> w{T(0), T(0), T(1), T(0)};
         if (k < nz - 1) {
             const T Epm_up = e_pmp(T(k + 1) * cst.dsig, h);
             const T Ku = diffusivity<T, true>(T(0.5) * (E[m + 1] + E[m + 2]), T(0.5) * (Epm + Epm_up), cold.K);
             const T adv_m = (hc.xp * Ex[m][0] + hc.xm * Ex[m][1]) + (hc.ym * Ex[m][2] + hc.yp * Ex[m][3]);
             const T G = -(T(kRhoI) * hp * Ep[m] * cst.invdt) - fE[m] + (adv ? adv_m : T(0));
-            Row<T> w{B0 * E[m + 1] + G, T(0), B0, T(0)};
+            w = {B0 * E[m + 1] + G, T(0), B0, T(0)};
             column_terms<T, true>(A, cst, k, h, E[m + 1], E[m], E[m + 2], om[m], om[m + 1], om[m + 2], Ku, Kl, w,
                                   &cold);
-            if (fabs(w.b) > T(1e-30)) out = -w.r / w.b;
             Kl = Ku;
             Epm = Epm_up;
         }
-        if (valid) E_out[at(n.c, k)] = (thin || k == nz - 1) ? E[m + 1] : E[m + 1] + omega_relax * out;
+        if (valid) f(col, k, at(n.c, k), E[m + 1], w, !thin && k < nz - 1);
     }
+}
+
+template <typename T>
+__device__ __forceinline__ void layer_lm_body(long vb, const EnthArgs<T>& A, T* E_out, T omega_relax,
+                                              const ColdValues<T>& cold) {
+    lm_chunk_rows(vb, A, cold, [&](long, int, long o, T E, const Row<T>& w, bool active) {
+        const T out = (fabs(w.b) > T(1e-30)) ? -w.r / w.b : T(0);
+        E_out[o] = active ? E + omega_relax * out : E;
+    });
 }
 
 template <typename T>
@@ -2146,29 +2109,23 @@ __global__ __launch_bounds__(256, 2) void k_enth_sweeps(EnthArgs<T> A, T* E, T* 
 }
 
 // Residual (with forcing) on the tiles: per-block max |r| into
-// partials[blockIdx.x] (grid-stride over columns) and, when r_out is given,
+// partials[blockIdx.x] (grid-stride over chunks) and, when r_out is given,
 // r written in the (ny, nx, nz) layout (zero on surface rows and thin columns).
+// Chunks of levels as the layer pass (one thread per column streaming up them:
+// 240 us with r_out at 512 x 512 x 41, here 164; 28 and 8 us at 40 x 56 x 21).
 template <typename T>
 __global__ __launch_bounds__(256) void k_enth_residual_lm(EnthArgs<T> A, T* __restrict__ r_out,
-                                                          double* __restrict__ partials) {
+                                                          double* __restrict__ partials, long blocks,
+                                                          ColdValues<T> cold) {
     __shared__ double smax[4];
     if (skipped(A.skip)) return;
-    const int nz = A.nz;
-    const long ncol = (long)A.ny * A.nx;
     double mx = 0.0;
-    for (long col = (long)blockIdx.x * 256 + threadIdx.x; col < ncol; col += (long)gridDim.x * 256) {
-        const long base = col * nz;
-        if (A.H[col] < A.h_thin) {
-            if (r_out)
-                for (int k = 0; k < nz; ++k) r_out[base + k] = T(0);
-            continue;
-        }
-        lm_stream_rows(A, ncol, col, [&](int k, T, const Row<T>& w) {
-            if (r_out) r_out[base + k] = w.r;
-            mx = nan_max(mx, fabs((double)w.r));
+    for (long vb = blockIdx.x; vb < blocks; vb += gridDim.x)
+        lm_chunk_rows(vb, A, cold, [&](long col, int k, long, T, const Row<T>& w, bool active) {
+            const T r = active ? w.r : T(0);
+            if (r_out) r_out[col * A.nz + k] = r;
+            mx = nan_max(mx, fabs((double)r));
         });
-        if (r_out) r_out[base + nz - 1] = T(0);
-    }
     for (int off = 32; off > 0; off >>= 1) mx = nan_max(mx, __shfl_down(mx, off, 64));
     if ((threadIdx.x & 63) == 0) smax[threadIdx.x >> 6] = mx;
     __syncthreads();
@@ -2453,11 +2410,10 @@ hipError_t launch_enth_residual_lm(const EnthArgs<T>& A, T* r_out, double* parti
                                    int status_mode, double rtol, double atol, hipStream_t st) {
     if (!enth_lm_supported(A.nz) || !A.u2d) return hipErrorInvalidValue;
     const long ncol = (long)A.ny * A.nx;
-    long g = (ncol + 255) / 256;
-    if (g > kEnthResBlocks) g = kEnthResBlocks;
+    const long blocks = layer_blocks(A.ny, A.nx, A.nz), g = blocks < kEnthResBlocks ? blocks : kEnthResBlocks;
     {
         TimedLaunch tl(kTimeEnthResidual, ncol * A.nz, st);
-        k_enth_residual_lm<T><<<(unsigned)g, 256, 0, st>>>(A, r_out, partials);
+        k_enth_residual_lm<T><<<(unsigned)g, 256, 0, st>>>(A, r_out, partials, blocks, cold_values<T>());
     }
     k_enth_reduce<<<1, 256, 0, st>>>(partials, (int)g, nullptr, status, status_mode, rtol, atol);
     return hipGetLastError();
