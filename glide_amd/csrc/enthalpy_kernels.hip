@@ -635,62 +635,65 @@ __global__ __launch_bounds__(256) void k_enth_apply(const int* __restrict__ skip
 // equation (glide/cuda/enthalpy.cu:1276-1372): lanes form the per-level
 // flux divergence, lane 0 integrates in level order; the result is divided
 // by out_div.
+// The once-a-step kernels below take kBlockCols columns a block: what is the same
+// for a whole column (its sums, powers and divisions) one thread per column, the
+// (ny, nx, nz) values in contiguous runs.  A wavefront per column formed the
+// column's part in all or in one of its lanes, and took about 175 us each at
+// 512 x 512 x 41; here the strain heating takes 22, omega 35 and the forcing 39 us
+// (20 to 35 us for the values read and written).
+constexpr int kBlockCols = 64;
 template <typename T>
 __global__ __launch_bounds__(256) void k_enth_omega(EnthArgs<T> A, const T* __restrict__ dhdt,
                                                     const T* __restrict__ bmb, T out_div, T* __restrict__ omega) {
-    __shared__ T sdiv[kColsPerBlock][64];
-    const long ncol = (long)A.ny * A.nx;
-    const ColIdx q = col_index(wave_column(), A.nx, ncol);
-    if (!q.valid) return;
-    const int nz = A.nz, k = q.k, w = threadIdx.x >> 6;
-    const int ny = A.ny, nx = A.nx, i = q.i, j = q.j;
-    const long base = q.col * nz;
-    const T h = A.H[q.col];
-    if (h < T(1e-3)) {
-        if (k < nz) omega[base + k] = T(0);
-        return;
-    }
-    if (k < nz) {
+    __shared__ T s[kBlockCols * 65];
+    const long ncol = (long)A.ny * A.nx, c0 = (long)blockIdx.x * kBlockCols;
+    const int nc = (int)min((long)kBlockCols, ncol - c0), nz = A.nz, ny = A.ny, nx = A.nx;
+    auto divergence = [&](long col, int k) {
+        const int i = (int)(col / nx), j = (int)(col % nx);
+        const T h = A.H[col];
         const T* u = A.u2d ? A.u2d : A.u3d + (long)k * ny * (nx + 1);
         const T* v = A.u2d ? A.v2d : A.v3d + (long)k * (ny + 1) * nx;
         T fr = 0, fl = 0, fb = 0, ft = 0;
         if (j < nx - 1) {
-            T ur = u[(long)i * (nx + 1) + j + 1], Hp = A.H[q.col + 1];
+            T ur = u[(long)i * (nx + 1) + j + 1], Hp = A.H[col + 1];
             fr = T(0.5) * (h + Hp) * ur - T(0.5) * sqrt(ur * ur + T(kMassFluxRegYr)) * (Hp - h);
         }
         if (j > 0) {
-            T ul = u[(long)i * (nx + 1) + j], Hm = A.H[q.col - 1];
+            T ul = u[(long)i * (nx + 1) + j], Hm = A.H[col - 1];
             fl = T(0.5) * (Hm + h) * ul - T(0.5) * sqrt(ul * ul + T(kMassFluxRegYr)) * (h - Hm);
         }
         if (i < ny - 1) {
-            T vb = v[(long)(i + 1) * nx + j], Hp = A.H[q.col + nx];
+            T vb = v[(long)(i + 1) * nx + j], Hp = A.H[col + nx];
             fb = T(0.5) * (h + Hp) * vb - T(0.5) * sqrt(vb * vb + T(kMassFluxRegYr)) * (h - Hp);
         }
         if (i > 0) {
-            T vt = v[(long)i * nx + j], Hm = A.H[q.col - nx];
+            T vt = v[(long)i * nx + j], Hm = A.H[col - nx];
             ft = T(0.5) * (Hm + h) * vt - T(0.5) * sqrt(vt * vt + T(kMassFluxRegYr)) * (Hm - h);
         }
-        sdiv[w][k] = (fr - fl + ft - fb) * A.dxi;
+        return (fr - fl + ft - fb) * A.dxi;
+    };
+    if (!A.u2d) {
+        for (int q = threadIdx.x; q < nc * nz; q += blockDim.x) s[(q / nz) * 65 + q % nz] = divergence(c0 + q / nz, q % nz);
+        __syncthreads();
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (k == 0) {  // the upward sum in level order, in place over the divergences
-        const T dsig = T(1) / T(nz - 1), dh = dhdt[q.col];
-        T o = bmb ? -bmb[q.col] : T(0);
-        T prev = sdiv[w][0];
-        sdiv[w][0] = o;
+    if ((int)threadIdx.x < nc) {  // the upward sum in level order, in place over the divergences
+        const long col = c0 + threadIdx.x;
+        T* d = s + threadIdx.x * 65;
+        const T dsig = T(1) / T(nz - 1), dh = dhdt[col];
+        const bool thin = A.H[col] < T(1e-3);
+        const T flat = A.u2d ? divergence(col, 0) : T(0);
+        T o = bmb ? -bmb[col] : T(0);
+        T prev = A.u2d ? flat : d[0];
+        d[0] = thin ? T(0) : o;
         for (int m = 1; m < nz; ++m) {
-            const T cur = sdiv[w][m];
+            const T cur = A.u2d ? flat : d[m];
             o = o - dsig * (dh + T(0.5) * (prev + cur));
-            sdiv[w][m] = o;
+            d[m] = thin ? T(0) : o;
             prev = cur;
         }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (k < nz) omega[base + k] = sdiv[w][k] / out_div;
+    __syncthreads();
+    for (int q = threadIdx.x; q < nc * nz; q += blockDim.x) omega[c0 * nz + q] = s[(q / nz) * 65 + q % nz] / out_div;
 }
 
 template <typename T>
@@ -714,31 +717,40 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_enth_rhs(EnthArgs<T> A, const T* __restrict__ beta, T m, T u_reg,
                                                   int frictional, T* __restrict__ Q_fh, T* __restrict__ f_E) {
     // frictional: Q_fh from the velocities (else read); f_E == nullptr: Q_fh only.
-    const long ncol = (long)A.ny * A.nx;
-    const ColIdx q = col_index(wave_column(), A.nx, ncol);
-    if (!q.valid) return;
-    const int nz = A.nz, k = q.k, nx = A.nx;
-    const long base = q.col * nz;
-    T qfh;
-    if (frictional) {
-        const T* ub = A.u2d ? A.u2d : A.u3d;
-        const T* vb = A.u2d ? A.v2d : A.v3d;
-        const T div = A.u2d ? A.vel_div : T(1);
-        T uc = T(0.5) * (ub[(long)q.i * (nx + 1) + q.j + 1] / div + ub[(long)q.i * (nx + 1) + q.j] / div);
-        T vc = T(0.5) * (vb[(long)(q.i + 1) * nx + q.j] / div + vb[(long)q.i * nx + q.j] / div);
-        T speed = sqrt(uc * uc + vc * vc + u_reg * u_reg);
-        qfh = beta[q.col] * pow(speed, m + T(1));
-        if (k == 0) Q_fh[q.col] = qfh;
-    } else {
-        qfh = Q_fh[q.col];
+    __shared__ T s_h[kBlockCols], s_bed[kBlockCols];
+    const long ncol = (long)A.ny * A.nx, c0 = (long)blockIdx.x * kBlockCols;
+    const int nc = (int)min((long)kBlockCols, ncol - c0), nz = A.nz, nx = A.nx;
+    if ((int)threadIdx.x < nc) {
+        const long col = c0 + threadIdx.x;
+        const int i = (int)(col / nx), j = (int)(col % nx);
+        T qfh;
+        if (frictional) {
+            const T* ub = A.u2d ? A.u2d : A.u3d;
+            const T* vb = A.u2d ? A.v2d : A.v3d;
+            const T div = A.u2d ? A.vel_div : T(1);
+            T uc = T(0.5) * (ub[(long)i * (nx + 1) + j + 1] / div + ub[(long)i * (nx + 1) + j] / div);
+            T vc = T(0.5) * (vb[(long)(i + 1) * nx + j] / div + vb[(long)i * nx + j] / div);
+            T speed = sqrt(uc * uc + vc * vc + u_reg * u_reg);
+            qfh = beta[col] * pow(speed, m + T(1));
+            Q_fh[col] = qfh;
+        } else {
+            qfh = Q_fh[col];
+        }
+        if (f_E) {
+            const T dsig_half = T(0.5) * (T(1) / T(nz - 1));
+            s_h[threadIdx.x] = A.H[col];
+            s_bed[threadIdx.x] = (A.Q_geo[col] + qfh) / (dsig_half * T(kEScale));
+        }
     }
-    if (k >= nz || !f_E) return;
-    const T h = A.H[q.col];
-    const T dsig_half = T(0.5) * (T(1) / T(nz - 1));
-    T f = A.phi_strain ? h * A.phi_strain[base + k] / T(kEScale) : T(0);
-    if (k == 0) f += (A.Q_geo[q.col] + qfh) / (dsig_half * T(kEScale));
-    if (k == nz - 1) f = T(0);
-    f_E[base + k] = f;
+    if (!f_E) return;
+    __syncthreads();
+    for (int q = threadIdx.x; q < nc * nz; q += blockDim.x) {
+        const int c = q / nz, k = q % nz;
+        T f = A.phi_strain ? s_h[c] * A.phi_strain[c0 * nz + q] / T(kEScale) : T(0);
+        if (k == 0) f += s_bed[c];
+        if (k == nz - 1) f = T(0);
+        f_E[c0 * nz + q] = f;
+    }
 }
 
 // SSA strain heating, uniform over the column (no counterpart in the
@@ -750,13 +762,19 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_enth_strain_heating(const T* __restrict__ u, const T* __restrict__ v,
                                                              const T* __restrict__ B, int ny, int nx, int nz, T dxi,
                                                              T glen_p, T eps_reg, T rho_g, T* __restrict__ phi) {
-    const long ncol = (long)ny * nx;
-    const ColIdx q = col_index(wave_column(), nx, ncol);
-    if (!q.valid || q.k >= nz) return;
-    const CellVel<T> c = load_cell_vel(u, v, q.i, q.j, ny, nx);
-    const T e2 = strain_invariant(c, q.i, q.j, ny, nx, dxi, T(0));
-    const T eta = T(0.5) * B[q.col] * pow(e2 + eps_reg, glen_p);
-    phi[q.col * nz + q.k] = T(4) * eta * e2 * rho_g / T(kSecPerYr);
+    __shared__ T s[kBlockCols];
+    const long ncol = (long)ny * nx, c0 = (long)blockIdx.x * kBlockCols;
+    const int nc = (int)min((long)kBlockCols, ncol - c0);
+    if ((int)threadIdx.x < nc) {
+        const long col = c0 + threadIdx.x;
+        const int i = (int)(col / nx), j = (int)(col % nx);
+        const CellVel<T> c = load_cell_vel(u, v, i, j, ny, nx);
+        const T e2 = strain_invariant(c, i, j, ny, nx, dxi, T(0));
+        const T eta = T(0.5) * B[col] * pow(e2 + eps_reg, glen_p);
+        s[threadIdx.x] = T(4) * eta * e2 * rho_g / T(kSecPerYr);
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < nc * nz; q += blockDim.x) phi[c0 * nz + q] = s[q / nz];
 }
 
 // Paterson-Budd rate factor A(T) (1 + 181.25 w) averaged over the levels and
@@ -764,24 +782,26 @@ __global__ __launch_bounds__(256) void k_enth_strain_heating(const T* __restrict
 // glide/model.py:209-213).
 template <typename T>
 __global__ __launch_bounds__(256) void k_enth_arrhenius(EnthArgs<T> A, T n_glen, T scale, T* __restrict__ B) {
-    const long ncol = (long)A.ny * A.nx;
-    const ColIdx q = col_index(wave_column(), A.nx, ncol);
-    if (!q.valid) return;
-    const int nz = A.nz, k = q.k;
-    T val = T(0);
-    if (k < nz) {
-        const T h = A.H[q.col];
-        const T Tp = t_pmp(T(k) * (T(1) / T(nz - 1)), h);
-        const T Ek = A.E[q.col * nz + k];
+    __shared__ T s[kBlockCols * 65];
+    const long ncol = (long)A.ny * A.nx, c0 = (long)blockIdx.x * kBlockCols;
+    const int nc = (int)min((long)kBlockCols, ncol - c0), nz = A.nz;
+    for (int q = threadIdx.x; q < nc * nz; q += blockDim.x) {
+        const int c = q / nz, k = q % nz;
+        const T Tp = t_pmp(T(k) * (T(1) / T(nz - 1)), A.H[c0 + c]);
+        const T Ek = A.E[c0 * nz + q];
         const T Tk = fmin(Ek * T(kEScale) / T(kCI) + T(kTRef), Tp);
         const T Af = Tk < T(263.15) ? T(3.985e-13) : T(1.916e3);
         const T Qf = Tk < T(263.15) ? T(60e3) : T(139e3);
         const T Ak = Af * exp(-Qf / (T(8.314) * fmax(Tk, T(1))));
         const T wk = fmax(Ek * T(kEScale) - T(kCI) * (Tp - T(kTRef)), T(0)) / T(kLHeat);
-        val = Ak * (T(1) + T(181.25) * wk);
+        s[c * 65 + k] = Ak * (T(1) + T(181.25) * wk);
     }
-    for (int off = 32; off > 0; off >>= 1) val += __shfl_down(val, off, 64);
-    if (k == 0) B[q.col] = pow(val / T(nz), T(-1) / n_glen) / scale;
+    __syncthreads();
+    if ((int)threadIdx.x < nc) {
+        T val = T(0);
+        for (int k = 0; k < nz; ++k) val += s[threadIdx.x * 65 + k];
+        B[c0 + threadIdx.x] = pow(val / T(nz), T(-1) / n_glen) / scale;
+    }
 }
 
 // Temperature min(E E_SCALE / C_I + T_REF, T_pmp) and water content
@@ -2136,6 +2156,9 @@ __global__ __launch_bounds__(256) void k_enth_residual_lm(EnthArgs<T> A, T* __re
 static inline unsigned col_blocks(int ny, int nx) {
     return (unsigned)(((long)ny * nx + kColsPerBlock - 1) / kColsPerBlock);
 }
+static inline unsigned block_columns(int ny, int nx) {
+    return (unsigned)(((long)ny * nx + kBlockCols - 1) / kBlockCols);
+}
 static inline unsigned flat_blocks(long n) {
     long b = (n + 255) / 256;
     return (unsigned)(b < 8192 ? (b > 0 ? b : 1) : 8192);
@@ -2187,7 +2210,7 @@ hipError_t launch_enth_apply(const EnthArgs<T>& A, T* E, const T* delta, T omega
 }
 template <typename T>
 hipError_t launch_enth_omega(const EnthArgs<T>& A, const T* dhdt, const T* bmb, T out_div, T* omega, hipStream_t st) {
-    k_enth_omega<T><<<col_blocks(A.ny, A.nx), 256, 0, st>>>(A, dhdt, bmb, out_div, omega);
+    k_enth_omega<T><<<block_columns(A.ny, A.nx), 256, 0, st>>>(A, dhdt, bmb, out_div, omega);
     return hipGetLastError();
 }
 template <typename T>
@@ -2204,19 +2227,19 @@ hipError_t launch_enth_tendency(const T* a, const T* b, T div, T* out, long n, h
 template <typename T>
 hipError_t launch_enth_rhs(const EnthArgs<T>& A, const T* beta, T m, T u_reg, int frictional, T* Q_fh, T* f_E,
                            hipStream_t st) {
-    k_enth_rhs<T><<<col_blocks(A.ny, A.nx), 256, 0, st>>>(A, beta, m, u_reg, frictional, Q_fh, f_E);
+    k_enth_rhs<T><<<block_columns(A.ny, A.nx), 256, 0, st>>>(A, beta, m, u_reg, frictional, Q_fh, f_E);
     return hipGetLastError();
 }
 template <typename T>
 hipError_t launch_enth_strain_heating(const T* u, const T* v, const T* B, int ny, int nx, int nz, T dxi, T n_glen,
                                      T eps_reg, T rho_g, T* phi, hipStream_t st) {
     const T glen_p = (T(1) - n_glen) / (T(2) * n_glen);
-    k_enth_strain_heating<T><<<col_blocks(ny, nx), 256, 0, st>>>(u, v, B, ny, nx, nz, dxi, glen_p, eps_reg, rho_g, phi);
+    k_enth_strain_heating<T><<<block_columns(ny, nx), 256, 0, st>>>(u, v, B, ny, nx, nz, dxi, glen_p, eps_reg, rho_g, phi);
     return hipGetLastError();
 }
 template <typename T>
 hipError_t launch_enth_arrhenius(const EnthArgs<T>& A, T n_glen, T scale, T* B, hipStream_t st) {
-    k_enth_arrhenius<T><<<col_blocks(A.ny, A.nx), 256, 0, st>>>(A, n_glen, scale, B);
+    k_enth_arrhenius<T><<<block_columns(A.ny, A.nx), 256, 0, st>>>(A, n_glen, scale, B);
     return hipGetLastError();
 }
 template <typename T>

@@ -191,7 +191,7 @@ class Ensemble:
         self._handle = h
 
     def set_tiles(self, rows: Sequence[int]) -> None:
-        """Rows of cell pairs per block of the batched red-black phases: one
+        """Tile setting (1, 2, 4 or 8) of the batched red-black passes: one
         entry per level (the most levels of any domain) and one for the
         coarsest-level passes (glide_ensemble_set_tiles).  The results do not
         depend on them."""
