@@ -191,15 +191,19 @@ int sweep_core(const glide_enth_column* C, double dt, int n_iter, const glide_en
             HIP_TRY(launch_enth_lm_layout<R>(A.omega, omlm, ncol, nz, true, st), "enthalpy tiled copy");
             L.omega = omlm;
         }
-        HIP_TRY(launch_enth_residual_lm<R>(L, nullptr, partials, status, 0, rtol, atol, st), "enthalpy residual");
+        // What the one-launch form's result depends on (norms, starting norm,
+        // barrier words) is in this call's own r_E and E_work, so that steps on
+        // several streams give what they give alone: r_E is free until the final
+        // residual below, E_work while a residual is taken.
+        const bool one_launch = enth_sweeps_fit(C->ny, C->nx, nz) && plane >= kEnthSlotWords;
+        unsigned long long* slots = one_launch ? reinterpret_cast<unsigned long long*>(C->r_E) : rmax;
+        double* own_r0 = one_launch ? reinterpret_cast<double*>(slots + 2 * kEnthRmaxSlots + kSweepR0) : nullptr;
+        double* parts = one_launch ? Wlm : partials;
+        HIP_TRY(launch_enth_reduce_slots(slots, status, 0, rtol, atol, st), "enthalpy max slots");
+        HIP_TRY(launch_enth_residual_lm<R>(L, nullptr, parts, own_r0, status, 0, rtol, atol, st), "enthalpy residual");
         L.skip = &status->done;
         EnthArgs<R> Lw = L;
         Lw.E = Wlm;
-        // the one-launch form keeps its norms and barrier in r_E, which only the
-        // final residual below fills: each column's own, on whatever stream
-        const bool one_launch = enth_sweeps_fit(C->ny, C->nx, nz) && plane >= kEnthSlotWords;
-        unsigned long long* slots = one_launch ? reinterpret_cast<unsigned long long*>(C->r_E) : rmax;
-        HIP_TRY(launch_enth_reduce_slots(slots, status, 0, rtol, atol, st), "enthalpy max slots");
         if (one_launch) {
             HIP_TRY(launch_enth_sweeps<R>(L, Elm, Wlm, cfg->omega, cfg->n_newton, cfg->relaxation, slots, status, rtol,
                                           atol, n_iter, st),
@@ -216,7 +220,7 @@ int sweep_core(const glide_enth_column* C, double dt, int n_iter, const glide_en
         // early (the bookkeeping closes nothing then)
         EnthArgs<R> Lf = L;
         Lf.skip = nullptr;
-        HIP_TRY(launch_enth_residual_lm<R>(Lf, P(C->r_E), partials, status, 1, rtol, atol, st), "enthalpy residual");
+        HIP_TRY(launch_enth_residual_lm<R>(Lf, P(C->r_E), parts, nullptr, status, 1, rtol, atol, st), "enthalpy residual");
         HIP_TRY(launch_enth_lm_layout<R>(Elm, P(C->E), ncol, nz, false, st), "enthalpy layout");
     } else {
         HIP_TRY(launch_enth_residual<R>(A, P(C->r_E), 1, partials, nullptr, status, 0, rtol, atol, st),

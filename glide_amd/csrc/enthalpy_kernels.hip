@@ -2011,8 +2011,8 @@ static inline long layer_blocks(int ny, int nx, int nz) {
 // only the last workgroup to arrive on an XCD does, for all of them (each
 // workgroup's own fences: 40 us a sweep at 48 x 48 x 41, four fifths of it in
 // the two barriers).  words (zeroed before the launch): all arrivals, the XCDs'
-// arrivals, the timeout flag, then per XCD its workgroups, arrivals and
-// releases.  Every wait is bounded: after kSweepPolls polls, or when another
+// arrivals, the timeout flag, the sweep's starting norm, then (from kSweepHead)
+// per XCD its workgroups, arrivals and releases.  Every wait is bounded: after kSweepPolls polls, or when another
 // workgroup gave up, the barrier returns false.
 constexpr int kSweepBlocks = 256, kSweepPolls = 1 << 20;
 struct SweepBarrier {
@@ -2037,14 +2037,14 @@ struct SweepBarrier {
         gen = 0;
         if (threadIdx.x == 0) {
             xcd = xcc_id();
-            atomicAdd(w + 3 + xcd, 1ull);
+            atomicAdd(w + kSweepHead + xcd, 1ull);
             __threadfence();
             atomicAdd(w, 1ull);
             s_ok = wait(w, gridDim.x);
             __threadfence();
-            here = peek(w + 3 + xcd);
+            here = peek(w + kSweepHead + xcd);
             xcds = 0;
-            for (int q = 0; q < kSweepXcds; ++q) xcds += peek(w + 3 + q) != 0;
+            for (int q = 0; q < kSweepXcds; ++q) xcds += peek(w + kSweepHead + q) != 0;
         }
         __syncthreads();
         return s_ok != 0;
@@ -2055,8 +2055,8 @@ struct SweepBarrier {
         __syncthreads();
         ++gen;
         if (threadIdx.x == 0) {
-            unsigned long long* arrive = w + 3 + kSweepXcds + xcd;
-            unsigned long long* release = w + 3 + 2 * kSweepXcds + xcd;
+            unsigned long long* arrive = w + kSweepHead + kSweepXcds + xcd;
+            unsigned long long* release = w + kSweepHead + 2 * kSweepXcds + xcd;
             bool ok;
             if (atomicAdd(arrive, 1ull) + 1 == here * gen) {
                 __threadfence();
@@ -2080,7 +2080,10 @@ struct SweepBarrier {
 // into E), with a barrier after each pass.  A step mostly converges in a few of
 // its n_iter sweeps, and the launches of the others, three each, were most of a
 // small map's step (40 x 56 x 21 with 100 sweeps: 1020 us, three sweeps run).
-// slots: two sets of kEnthRmaxSlots, zero on entry.  If a barrier timed out, E
+// slots: two sets of kEnthRmaxSlots, zero on entry.  Every workgroup decides for
+// itself whether to stop, so what it decides by (norms, starting norm) is in the
+// call's own words: `status` is the device's one record, which a step on another
+// stream may rewrite meanwhile, and only takes the norms for the report.  If a barrier timed out, E
 // is filled with NaN, which the sweep's report and the residual then show.
 template <typename T, int P, int MB>
 __global__ __launch_bounds__(256, 2) void k_enth_sweeps(EnthArgs<T> A, T* E, T* W, T omega_relax, int n_newton,
@@ -2095,6 +2098,7 @@ __global__ __launch_bounds__(256, 2) void k_enth_sweeps(EnthArgs<T> A, T* E, T* 
     Aw.E = W;
     SweepBarrier bar;
     bool ok = bar.start(sync);
+    const double r0 = __longlong_as_double((long long)SweepBarrier::peek(sync + kSweepR0));
 #pragma unroll 1
     for (int it = 0; ok && it < n_iter; ++it) {
         unsigned long long* set = slots + (it & 1) * kEnthRmaxSlots;
@@ -2110,7 +2114,7 @@ __global__ __launch_bounds__(256, 2) void k_enth_sweeps(EnthArgs<T> A, T* E, T* 
             if ((tid & 63) == 0) sh[tid >> 6] = m;
             __syncthreads();
             const double r = nan_max(nan_max(sh[0], sh[1]), nan_max(sh[2], sh[3]));
-            const bool stop = sweep_stops(r, status->r0, rtol, atol);
+            const bool stop = sweep_stops(r, r0, rtol, atol);
             if (blockIdx.x == 0 && tid == 0) record_sweep(status, 1, r, rtol, atol);
             if (stop) return;
         }
@@ -2429,8 +2433,8 @@ hipError_t launch_enth_layer_lm(const EnthArgs<T>& A, T* E_out, T omega_relax, h
     return hipGetLastError();
 }
 template <typename T>
-hipError_t launch_enth_residual_lm(const EnthArgs<T>& A, T* r_out, double* partials, EnthStatus* status,
-                                   int status_mode, double rtol, double atol, hipStream_t st) {
+hipError_t launch_enth_residual_lm(const EnthArgs<T>& A, T* r_out, double* partials, double* max_out,
+                                   EnthStatus* status, int status_mode, double rtol, double atol, hipStream_t st) {
     if (!enth_lm_supported(A.nz) || !A.u2d) return hipErrorInvalidValue;
     const long ncol = (long)A.ny * A.nx;
     const long blocks = layer_blocks(A.ny, A.nx, A.nz), g = blocks < kEnthResBlocks ? blocks : kEnthResBlocks;
@@ -2438,7 +2442,7 @@ hipError_t launch_enth_residual_lm(const EnthArgs<T>& A, T* r_out, double* parti
         TimedLaunch tl(kTimeEnthResidual, ncol * A.nz, st);
         k_enth_residual_lm<T><<<(unsigned)g, 256, 0, st>>>(A, r_out, partials, blocks, cold_values<T>());
     }
-    k_enth_reduce<<<1, 256, 0, st>>>(partials, (int)g, nullptr, status, status_mode, rtol, atol);
+    k_enth_reduce<<<1, 256, 0, st>>>(partials, (int)g, max_out, status, status_mode, rtol, atol);
     return hipGetLastError();
 }
 
@@ -2475,8 +2479,8 @@ hipError_t launch_enth_residual_lm(const EnthArgs<T>& A, T* r_out, double* parti
     template hipError_t launch_enth_layer_lm<T>(const EnthArgs<T>&, T*, T, hipStream_t);                             \
     template hipError_t launch_enth_sweeps<T>(const EnthArgs<T>&, T*, T*, T, int, T, unsigned long long*,            \
                                               EnthStatus*, double, double, int, hipStream_t);                        \
-    template hipError_t launch_enth_residual_lm<T>(const EnthArgs<T>&, T*, double*, EnthStatus*, int, double, double, \
-                                                   hipStream_t);
+    template hipError_t launch_enth_residual_lm<T>(const EnthArgs<T>&, T*, double*, double*, EnthStatus*, int,      \
+                                                   double, double, hipStream_t);
 INST(double)
 #undef INST
 

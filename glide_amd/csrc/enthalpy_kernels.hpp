@@ -43,10 +43,11 @@ struct EnthStatus {
 
 constexpr int kEnthResBlocks = 2048;  // residual grid (grid-stride over columns)
 constexpr int kEnthRmaxSlots = 256;   // max-|r| accumulators of the column pass (bit patterns of doubles)
-// The accumulators' buffer: two sets, and the barrier's words of the one-launch
-// sweep (three counters, then the workgroups, arrivals and releases of 16 XCDs).
-constexpr int kSweepXcds = 16;
-constexpr int kEnthSlotWords = 2 * kEnthRmaxSlots + 3 + 3 * kSweepXcds;
+// The accumulators' buffer: two sets, and the words of the one-launch sweep (the
+// barrier's three counters, the starting norm, then the workgroups, arrivals and
+// releases of 16 XCDs).
+constexpr int kSweepXcds = 16, kSweepHead = 4, kSweepR0 = 3;
+constexpr int kEnthSlotWords = 2 * kEnthRmaxSlots + kSweepHead + 3 * kSweepXcds;
 
 // max |r| of the residual over the grid, into `max_out` (device), or, with
 // `status`, the sweep bookkeeping: mode 0 starts a sweep (r0), mode 1 ends an
@@ -180,7 +181,8 @@ template <typename T>
 hipError_t launch_enth_column_lm(const EnthArgs<T>& A, T* W, T omega_relax, int n_newton, T relaxation,
                                  unsigned long long* rmax, hipStream_t st);
 // n_iter sweeps (column and layer passes, norms, stopping test) of a small map
-// in one launch, from E (= A.E) through W; slots of kEnthSlotWords, zero on entry.
+// in one launch, from E (= A.E) through W; slots of kEnthSlotWords, zero on entry
+// but for the starting norm at 2 kEnthRmaxSlots + kSweepR0.
 bool enth_sweeps_fit(int ny, int nx, int nz);
 template <typename T>
 hipError_t launch_enth_sweeps(const EnthArgs<T>& A, T* E, T* W, T omega_relax, int n_newton, T relaxation,
@@ -190,10 +192,10 @@ hipError_t launch_enth_sweeps(const EnthArgs<T>& A, T* E, T* W, T omega_relax, i
 template <typename T>
 hipError_t launch_enth_layer_lm(const EnthArgs<T>& A, T* E_out, T omega_relax, hipStream_t st);
 // Residual with forcing into the sweep bookkeeping (status mode as
-// launch_enth_residual's) and, when r_out is given, written in the
-// (ny, nx, nz) layout.
+// launch_enth_residual's) and, when given, its norm into max_out (device) and
+// its values into r_out, in the (ny, nx, nz) layout.
 template <typename T>
-hipError_t launch_enth_residual_lm(const EnthArgs<T>& A, T* r_out, double* partials, EnthStatus* status,
-                                   int status_mode, double rtol, double atol, hipStream_t st);
+hipError_t launch_enth_residual_lm(const EnthArgs<T>& A, T* r_out, double* partials, double* max_out,
+                                   EnthStatus* status, int status_mode, double rtol, double atol, hipStream_t st);
 
 }  // namespace glide

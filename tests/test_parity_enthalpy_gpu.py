@@ -318,6 +318,43 @@ def test_tiled_sweep_matches_column_wavefronts(n, nz):
     assert abs(a0 - a1) <= 1e-8 * a1 and np.allclose(n0, n1, rtol=1e-7, atol=1e-8 * a1)
 
 
+def test_thermal_steps_on_two_streams_match_steps_alone():
+    """Steps of two small maps enqueued on two streams give, bitwise, what each
+    gives alone: what a sweep stops by is its own, not the device's one record.
+    The maps' starting norms and stopping sweeps differ."""
+    print("thermal steps on two streams", flush=True)
+
+    def pair():
+        tms = [_thermal_pair(n, nz, seed, strain=True)[2] for n, nz, seed in ((24, 21, 3), (33, 33, 8))]
+        for tm in tms:
+            tm.n_smooth = 60
+            tm.ops.smoother_config.relative_tolerance, tm.ops.smoother_config.absolute_tolerance = 1e-9, 0.0
+        return tms
+
+    ref = []
+    for tm in pair():
+        ref.append([])
+        for _ in range(4):
+            rep = tm.step(DT, report=True)
+            ref[-1].append((N(tm.ops.enthalpy_state.E), rep.sweeps))
+            tm.pre_momentum()
+    assert max(s for _, s in ref[0]) < min(s for _, s in ref[1]) < 60  # they stop at different sweeps
+    tms = pair()
+    streams = [torch.cuda.Stream() for _ in tms]
+    got = [[], []]
+    torch.cuda.synchronize()
+    for _ in range(4):
+        for tm, st, out in zip(tms, streams, got):
+            with torch.cuda.stream(st):
+                tm.step(DT)
+                out.append(tm.ops.enthalpy_state.E.clone())
+                tm.pre_momentum()
+    torch.cuda.synchronize()
+    for g, r in zip(got, ref):
+        for E, (E0, _) in zip(g, r):
+            assert np.array_equal(N(E), E0)
+
+
 def test_thermal_step_host_path_matches_fused():
     print("thermal_step host path", flush=True)
     F, g, tm, th = _thermal_pair(16, 11, 4, strain=True)
