@@ -22,6 +22,7 @@
 
 namespace glide {
 void set_last_error(const std::string& msg);
+int persistent_spin_limit();
 }
 
 using namespace glide;
@@ -206,7 +207,7 @@ int sweep_core(const glide_enth_column* C, double dt, int n_iter, const glide_en
         Lw.E = Wlm;
         if (one_launch) {
             HIP_TRY(launch_enth_sweeps<R>(L, Elm, Wlm, cfg->omega, cfg->n_newton, cfg->relaxation, slots, status, rtol,
-                                          atol, n_iter, st),
+                                          atol, n_iter, persistent_spin_limit(), st),
                     "enthalpy sweeps");
         } else
         for (int it = 0; it < n_iter; ++it) {

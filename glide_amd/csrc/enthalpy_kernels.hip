@@ -2005,46 +2005,63 @@ static inline long layer_blocks(int ny, int nx, int nz) {
     return (((long)ny * nx + kLmCols - 1) / kLmCols * ((nz + kLayerLevels - 1) / kLayerLevels) + 3) / 4;
 }
 
-// Barrier of the workgroups of a persistent launch, all resident (at most
-// kSweepBlocks, with room for several on a CU).  They span XCDs, whose L2s have
-// to be written back and invalidated; an L2 takes about a microsecond for it, so
-// only the last workgroup to arrive on an XCD does, for all of them (each
-// workgroup's own fences: 40 us a sweep at 48 x 48 x 41, four fifths of it in
-// the two barriers).  words (zeroed before the launch): all arrivals, the XCDs'
-// arrivals, the timeout flag, the sweep's starting norm, then (from kSweepHead)
-// per XCD its workgroups, arrivals and releases.  Every wait is bounded: after kSweepPolls polls, or when another
-// workgroup gave up, the barrier returns false.
-constexpr int kSweepBlocks = 256, kSweepPolls = 1 << 20;
+// Barrier of the workgroups of a persistent launch (at most kSweepBlocks).  They
+// span XCDs, whose L2s have to be written back and invalidated; an L2 takes about
+// a microsecond for it, so only the last workgroup to arrive on an XCD does, for
+// all of them (each workgroup's own fences: 40 us a sweep at 48 x 48 x 41, four
+// fifths of it in the two barriers).  One workgroup's fence may stand for the
+// others' stores because they are all in the L2 that it writes back: the CUs of
+// an XCD share one L2, their caches write through to it, and each wavefront waits
+// for the acknowledgement of its stores (s_waitcnt) before its workgroup
+// arrives.  Likewise the fence after the wait empties that L2 before any of them
+// is released, and each then empties its own CU's cache.
+//
+// words (zeroed before the launch): all arrivals, the XCDs' arrivals, the flag
+// that one gave up, the sweep's starting norm, the workgroups that have left, how
+// far the first to give up had come, the norms recorded, then (from kSweepHead)
+// per XCD its workgroups, arrivals and releases.  Every wait is bounded: after
+// spin_limit polls (at once if negative), or when another workgroup gave up, the
+// barrier returns false, and the last workgroup to leave does the rest alone.
+constexpr int kSweepBlocks = 256;
 struct SweepBarrier {
     unsigned long long* w;
-    unsigned long long xcd, here, xcds, gen;
+    int spin_limit;
+    unsigned* own;  // in LDS: this workgroup's XCD, the workgroups on it, the XCDs in use
+    unsigned gen;
+    bool alone;
 
     __device__ __forceinline__ static unsigned long long peek(unsigned long long* p) {
         return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __device__ __forceinline__ bool wait(unsigned long long* p, unsigned long long target) {
+        if (spin_limit < 0) atomicExch(w + 2, 1ull);
         int spins = 0;
         while (peek(p) < target && !peek(w + 2)) {
-            if (++spins > kSweepPolls) atomicExch(w + 2, 1ull);
+            if (++spins > spin_limit) atomicExch(w + 2, 1ull);
             __builtin_amdgcn_s_sleep(1);
         }
         return peek(w + 2) == 0;
     }
-    // counts the workgroups of each XCD; thread 0 only holds the counts
-    __device__ __forceinline__ bool start(unsigned long long* words) {
+    // counts the workgroups of each XCD
+    __device__ __forceinline__ bool start(unsigned long long* words, int limit) {
         __shared__ int s_ok;
+        __shared__ unsigned s_own[3];
         w = words;
+        own = s_own;
+        spin_limit = limit;
         gen = 0;
+        alone = false;
         if (threadIdx.x == 0) {
-            xcd = xcc_id();
+            const unsigned xcd = own[0] = xcc_id();
             atomicAdd(w + kSweepHead + xcd, 1ull);
             __threadfence();
             atomicAdd(w, 1ull);
             s_ok = wait(w, gridDim.x);
             __threadfence();
-            here = peek(w + kSweepHead + xcd);
-            xcds = 0;
+            own[1] = (unsigned)peek(w + kSweepHead + xcd);
+            unsigned xcds = 0;
             for (int q = 0; q < kSweepXcds; ++q) xcds += peek(w + kSweepHead + q) != 0;
+            own[2] = xcds;
         }
         __syncthreads();
         return s_ok != 0;
@@ -2055,13 +2072,15 @@ struct SweepBarrier {
         __syncthreads();
         ++gen;
         if (threadIdx.x == 0) {
-            unsigned long long* arrive = w + kSweepHead + kSweepXcds + xcd;
-            unsigned long long* release = w + kSweepHead + 2 * kSweepXcds + xcd;
+            unsigned long long* arrive = w + kSweepHead + kSweepXcds + own[0];
+            unsigned long long* release = arrive + kSweepXcds;
             bool ok;
-            if (atomicAdd(arrive, 1ull) + 1 == here * gen) {
+            if (alone) {
+                ok = true;
+            } else if (atomicAdd(arrive, 1ull) + 1 == (unsigned long long)own[1] * gen) {
                 __threadfence();
                 atomicAdd(w + 1, 1ull);
-                ok = wait(w + 1, xcds * gen);
+                ok = wait(w + 1, (unsigned long long)own[2] * gen);
                 __threadfence();
                 __hip_atomic_store(release, gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             } else {
@@ -2073,6 +2092,34 @@ struct SweepBarrier {
         __syncthreads();
         return s_ok != 0;
     }
+    // The workgroup leaves, having given up (after `passes` of `total`) or not.
+    // Returns -1, or in the last one to leave, if any gave up, the passes that all
+    // have done; it then works alone.
+    __device__ __forceinline__ int leave(bool gave_up, int passes, int total) {
+        __shared__ int s_from;
+        if (alone) return -1;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            if (gave_up) {  // no barrier has published its last pass
+                __threadfence();
+                atomicMax(w + 5, (unsigned long long)(total - passes + 1));
+                __threadfence();
+            }
+            int from = -1;
+            if (atomicAdd(w + 4, 1ull) + 1 == gridDim.x) {
+                const int behind = (int)peek(w + 5);
+                if (behind) {
+                    from = total + 1 - behind;
+                    __threadfence();
+                }
+            }
+            s_from = from;
+        }
+        __syncthreads();
+        alone = true;
+        return s_from;
+    }
 };
 
 // All sweeps of a small map in one launch: the column pass (A.E = E into W), the
@@ -2083,52 +2130,70 @@ struct SweepBarrier {
 // slots: two sets of kEnthRmaxSlots, zero on entry.  Every workgroup decides for
 // itself whether to stop, so what it decides by (norms, starting norm) is in the
 // call's own words: `status` is the device's one record, which a step on another
-// stream may rewrite meanwhile, and only takes the norms for the report.  If a barrier timed out, E
-// is filled with NaN, which the sweep's report and the residual then show.
+// stream may rewrite meanwhile, and only takes the norms for the report.
+//
+// Nothing says that the workgroups run at the same time: other streams' work may
+// hold the CUs.  A workgroup whose wait gives up leaves, and the last to leave
+// goes on by itself from the first pass that not all have done.  That pass can be
+// done again: it reads what the one before it wrote and writes the other of E and
+// W (nobody is further than that pass, whose barrier needs all), and a norm is a
+// maximum.  The results are bitwise those of a launch whose waits end.
 template <typename T, int P, int MB>
 __global__ __launch_bounds__(256, 2) void k_enth_sweeps(EnthArgs<T> A, T* E, T* W, T omega_relax, int n_newton,
                                                         T relaxation, unsigned long long* slots,
                                                         unsigned long long* sync, EnthStatus* status, double rtol,
-                                                        double atol, int n_iter, long col_blocks, long lay_blocks,
-                                                        ColdValues<T> cold) {
+                                                        double atol, int n_iter, int col_blocks, int lay_blocks,
+                                                        int spin_limit, ColdValues<T> cold) {
     __shared__ double sh[4];
-    const long nb = gridDim.x;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, total = 2 * n_iter;
+    int first = blockIdx.x, step = gridDim.x;
     EnthArgs<T> Aw = A;
     Aw.E = W;
     SweepBarrier bar;
-    bool ok = bar.start(sync);
+    bool ok = bar.start(sync, spin_limit);
     const double r0 = __longlong_as_double((long long)SweepBarrier::peek(sync + kSweepR0));
+    auto clear = [&](int it) {  // the norms of sweep it, for sweep it + 2
+        if (first == 0)
+            __hip_atomic_store(slots + (it & 1) * kEnthRmaxSlots + tid, 0ull, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    };
+    int p = 0;  // passes done: of sweep p / 2 the column pass (even), the layer pass
+    for (;;) {
 #pragma unroll 1
-    for (int it = 0; ok && it < n_iter; ++it) {
-        unsigned long long* set = slots + (it & 1) * kEnthRmaxSlots;
+        while (ok && p < total) {
+            const int it = p >> 1;
+            unsigned long long* set = slots + (it & 1) * kEnthRmaxSlots;
+            if (!(p & 1)) {
 #pragma unroll 1
-        for (long vb = blockIdx.x; vb < col_blocks; vb += nb)
-            column_lm_body<T, P, MB>(vb, A, W, omega_relax, n_newton, relaxation, it > 0 ? set : nullptr, cold);
-        ok = bar.sync();
-        if (!ok) break;
-        if (it > 0) {  // every workgroup comes to the same decision
-            double m = __longlong_as_double(
-                (long long)__hip_atomic_load(set + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-            for (int off = 32; off > 0; off >>= 1) m = nan_max(m, __shfl_down(m, off, 64));
-            if ((tid & 63) == 0) sh[tid >> 6] = m;
-            __syncthreads();
-            const double r = nan_max(nan_max(sh[0], sh[1]), nan_max(sh[2], sh[3]));
-            const bool stop = sweep_stops(r, r0, rtol, atol);
-            if (blockIdx.x == 0 && tid == 0) record_sweep(status, 1, r, rtol, atol);
-            if (stop) return;
+                for (int vb = first; vb < col_blocks; vb += step)
+                    column_lm_body<T, P, MB>(vb, A, W, omega_relax, n_newton, relaxation, it > 0 ? set : nullptr, cold);
+            } else {
+                if (it > 0) {  // every workgroup comes to the same decision
+                    double m = __longlong_as_double((long long)SweepBarrier::peek(set + tid));
+                    for (int off = 32; off > 0; off >>= 1) m = nan_max(m, __shfl_down(m, off, 64));
+                    if ((tid & 63) == 0) sh[tid >> 6] = m;
+                    __syncthreads();
+                    const double r = nan_max(nan_max(sh[0], sh[1]), nan_max(sh[2], sh[3]));
+                    if (first == 0 && tid == 0 && (int)SweepBarrier::peek(sync + 6) < it) {
+                        record_sweep(status, 1, r, rtol, atol);
+                        __hip_atomic_store(sync + 6, (unsigned long long)it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                    if (sweep_stops(r, r0, rtol, atol)) break;
+                }
+#pragma unroll 1
+                for (int vb = first; vb < lay_blocks; vb += step) layer_lm_body<T>(vb, Aw, E, omega_relax, cold);
+            }
+            ++p;
+            ok = bar.sync();
+            if (ok && !(p & 1)) clear(it);  // read by all before the barrier
         }
-#pragma unroll 1
-        for (long vb = blockIdx.x; vb < lay_blocks; vb += nb) layer_lm_body<T>(vb, Aw, E, omega_relax, cold);
-        ok = bar.sync();
-        if (!ok) break;
-        // read by all before the barrier, used again two sweeps later
-        if (blockIdx.x == 0)
-            __hip_atomic_store(set + tid, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (!ok) {
-        const long n = (long)A.ny * A.nx * A.nz;
-        for (long q = (long)blockIdx.x * 256 + tid; q < n; q += nb * 256) E[q] = __longlong_as_double(0x7ff8000000000000ll);
+        p = bar.leave(!ok, p, total);
+        if (p < 0) return;
+        first = 0;
+        step = 1;
+        ok = true;
+        if (p > 0 && !(p & 1)) clear((p >> 1) - 1);  // block 0 may have left before it
+        __syncthreads();
     }
 }
 
@@ -2370,7 +2435,7 @@ bool enth_sweeps_fit(int ny, int nx, int nz) {
 template <typename T>
 hipError_t launch_enth_sweeps(const EnthArgs<T>& A, T* E, T* W, T omega_relax, int n_newton, T relaxation,
                               unsigned long long* slots, EnthStatus* status, double rtol, double atol, int n_iter,
-                              hipStream_t st) {
+                              int spin_limit, hipStream_t st) {
     if (!enth_lm_supported(A.nz) || !A.u2d || !enth_sweeps_fit(A.ny, A.nx, A.nz)) return hipErrorInvalidValue;
     const long ncol = (long)A.ny * A.nx;
     const int P = lm_lanes(ncol, A.nz), mb = (A.nz + P - 1) / P;
@@ -2381,7 +2446,7 @@ hipError_t launch_enth_sweeps(const EnthArgs<T>& A, T* E, T* W, T omega_relax, i
     if (P == PP && mb == MB) {                                                                                    \
         k_enth_sweeps<T, PP, MB><<<(unsigned)cb, 256, 0, st>>>(A, E, W, omega_relax, n_newton, relaxation, slots, \
                                                                slots + 2 * kEnthRmaxSlots, status, rtol, atol,    \
-                                                               n_iter, cb, lb, cold);                             \
+                                                               n_iter, (int)cb, (int)lb, spin_limit, cold);       \
         return hipGetLastError();                                                                                 \
     }
     GLIDE_LM_SWEEPS(4, 3)
@@ -2478,7 +2543,7 @@ hipError_t launch_enth_residual_lm(const EnthArgs<T>& A, T* r_out, double* parti
                                                  hipStream_t);                                                       \
     template hipError_t launch_enth_layer_lm<T>(const EnthArgs<T>&, T*, T, hipStream_t);                             \
     template hipError_t launch_enth_sweeps<T>(const EnthArgs<T>&, T*, T*, T, int, T, unsigned long long*,            \
-                                              EnthStatus*, double, double, int, hipStream_t);                        \
+                                              EnthStatus*, double, double, int, int, hipStream_t);                   \
     template hipError_t launch_enth_residual_lm<T>(const EnthArgs<T>&, T*, double*, double*, EnthStatus*, int,      \
                                                    double, double, hipStream_t);
 INST(double)

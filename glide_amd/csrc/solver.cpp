@@ -2586,6 +2586,7 @@ int ensemble_enqueue(glide_ensemble* e, hipStream_t st) {
 
 namespace glide {
 void set_last_error(const std::string& msg) { g_last_error = msg; }
+int persistent_spin_limit() { return g_spin_limit; }
 int noalloc_setup();
 }  // namespace glide
 

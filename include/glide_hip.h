@@ -147,7 +147,9 @@ int glide_init(void);
 /* Synchronises `stream` and reports (then clears) the failure latch: GLIDE_OK,
  * or GLIDE_ERR_TIMEOUT if a persistent launch's barrier wait gave up since
  * the last check (its solve's results are NaN).  Solves that synchronise for
- * a report check the latch themselves (no counterpart in the reference). */
+ * a report check the latch themselves (no counterpart in the reference).  The
+ * thermal step's one-launch sweep is not reported: when a wait of it gives up,
+ * its last workgroup finishes the sweeps alone, with the same results. */
 int glide_check_status(void* stream);
 /* Copies the calling thread's last error message into buf (NUL-terminated);
  * returns its full length. */
@@ -366,7 +368,8 @@ int glide_persistent_fenced_enable(int on);
 /* Polls a persistent barrier wait makes before it gives up (default 2^20);
  * a negative value gives up at the first barrier, which exercises the
  * failure path (NaN results, GLIDE_ERR_TIMEOUT from the next synchronising
- * call) without any kernel waiting (testing switch; no counterpart in the
+ * call; in a thermal step's one-launch sweep, one workgroup doing the sweeps)
+ * without any kernel waiting (testing switch; no counterpart in the
  * reference). */
 int glide_persistent_spin_limit(int polls);
 

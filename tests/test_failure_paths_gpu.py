@@ -5,7 +5,8 @@ The reference lets NaNs propagate silently (CuPy norms, glide/operators.py:126,
 glide/enthalpy.py:364).  Here a NaN reaches every reported norm, a sweep with a
 NaN residual never passes its stopping test, and a synchronising call returns
 GLIDE_ERR_NONFINITE (-4).  A persistent launch whose barrier gives up latches a
-status word that the next synchronising call reports as GLIDE_ERR_TIMEOUT (-5).
+status word that the next synchronising call reports as GLIDE_ERR_TIMEOUT (-5);
+the thermal step's one-launch sweep instead lets its last workgroup finish alone.
 The timeout is forced from the host (a negative spin limit gives up at the
 first barrier without waiting), so every kernel still exits normally.
 """
@@ -49,6 +50,36 @@ def test_nan_adjoint_seed_reaches_the_adjoint_report():
     seed[2, 2, 3] = float("nan")
     with pytest.raises(GlideError, match=r"\(-4\)"):
         ops.adjoint_solve(DT, seed, n_iter=5, relative_tolerance=1e-12, report=True)
+
+
+@pytest.mark.parametrize("n,nz,rel,n_smooth", [(9, 9, 1e-9, 30), (24, 21, 1e-9, 30), (24, 21, 0.0, 1),
+                                               (24, 21, 0.0, 4), (33, 33, 1e-5, 30), (48, 41, 1e-5, 7)])
+@pytest.mark.parametrize("limit", [-1, 0, 1, 3, 10, 30, 100])
+def test_enthalpy_sweep_whose_waits_give_up_gives_the_same_results(n, nz, rel, n_smooth, limit):
+    """The one-launch sweep of a small map with waits that give up at once
+    (negative: one workgroup does everything) or after a few polls (somewhere
+    between two passes): E, the residual, the sweeps run and every norm are
+    bitwise those of a launch whose waits end, and nothing is reported."""
+    from glide_amd import _lib
+    from tests.test_parity_enthalpy_gpu import _thermal_pair
+    print(f"sweep give-up n={n} nz={nz} rel={rel} n_smooth={n_smooth} limit={limit}", flush=True)
+    out = []
+    try:
+        for spins in (1 << 20, limit):
+            tm = _thermal_pair(n, nz, 5, strain=True)[2]
+            tm.n_smooth = n_smooth
+            tm.ops.smoother_config.relative_tolerance, tm.ops.smoother_config.absolute_tolerance = rel, 0.0
+            torch.cuda.synchronize()
+            _lib.persistent_spin_limit(spins)
+            rep = tm.step(DT, report=True)
+            _lib.check_status()
+            out.append((tm.ops.enthalpy_state.E.cpu().numpy(), tm.ops.r_E.cpu().numpy(), rep.r0,
+                        [rep.norms[k] for k in range(rep.sweeps)]))
+    finally:
+        _lib.persistent_spin_limit(1 << 20)
+    assert 1 <= len(out[0][3]) <= n_smooth
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
 
 
 def _model(n=32, L=3, seed=0):
