@@ -56,6 +56,7 @@ struct EnthScratch {
     unsigned long long* rmax = nullptr;  // kEnthSlotWords: the column pass's max-|r| accumulators
     EnthStatus* status = nullptr;
     EnthStatus* host = nullptr;   // pinned mirror
+    int cus = 0, sweeps_per_cu = 0;     // the device's CUs, workgroups of the one-launch sweep on each
 };
 
 std::mutex g_mutex;
@@ -75,9 +76,24 @@ int scratch(EnthScratch** out) {
         HIP_TRY(hipMalloc(&s.status, sizeof(EnthStatus)), "hipMalloc(enthalpy status)");
         HIP_TRY(hipMalloc(&s.rmax, sizeof(unsigned long long) * kEnthSlotWords), "hipMalloc(enthalpy max slots)");
         HIP_TRY(hipHostMalloc(&s.host, sizeof(EnthStatus), hipHostMallocDefault), "hipHostMalloc(enthalpy status)");
+        HIP_TRY(hipDeviceGetAttribute(&s.cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute");
+        HIP_TRY(enth_sweeps_per_cu(&s.sweeps_per_cu), "occupancy of the enthalpy sweep");
     }
     *out = &s;
     return GLIDE_OK;
+}
+
+// Workgroups of the one-launch sweep that can run at once on the CUs the stream
+// may use.
+int sweep_residents(const EnthScratch& s, hipStream_t st) {
+    uint32_t mask[32] = {};
+    int cus = 0;
+    if (hipExtStreamGetCUMask(st, 32, mask) == hipSuccess) {
+        for (uint32_t m : mask) cus += __builtin_popcount(m);
+    } else {
+        (void)hipGetLastError();
+    }
+    return s.sweeps_per_cu * (cus > 0 && cus < s.cus ? cus : s.cus);
 }
 
 // A reported sweep whose residual norm went non-finite (NaN propagates through
@@ -156,10 +172,10 @@ int make_args(const glide_enth_column* C, double dt, bool needs_state, EnthArgs<
 // The fused sweep with its reduction partials (kEnthResBlocks values) and
 // status record in caller-chosen device memory; `host` is a pinned mirror of
 // the record for the report, or nullptr (then the report is read through a
-// stack copy).
+// stack copy).  residents: sweep_residents for the one-launch form, 0 without it.
 int sweep_core(const glide_enth_column* C, double dt, int n_iter, const glide_enth_sweep_config* cfg,
                glide_enth_report* report, hipStream_t st, double* partials, EnthStatus* status, EnthStatus* host,
-               const R* u2d, const R* v2d, double vel_div, unsigned long long* rmax = nullptr) {
+               const R* u2d, const R* v2d, double vel_div, unsigned long long* rmax = nullptr, int residents = 0) {
     if (!cfg) return fail(GLIDE_ERR_INVALID_ARG, "sweep config is NULL");
     if (n_iter < 0 || n_iter > GLIDE_ENTH_MAX_SWEEPS)
         return fail(GLIDE_ERR_INVALID_ARG, "n_iter must be in [0, GLIDE_ENTH_MAX_SWEEPS]");
@@ -196,7 +212,8 @@ int sweep_core(const glide_enth_column* C, double dt, int n_iter, const glide_en
         // barrier words) is in this call's own r_E and E_work, so that steps on
         // several streams give what they give alone: r_E is free until the final
         // residual below, E_work while a residual is taken.
-        const bool one_launch = enth_sweeps_fit(C->ny, C->nx, nz) && plane >= kEnthSlotWords;
+        const int sweep_blocks = plane >= kEnthSlotWords ? enth_sweeps_blocks(C->ny, C->nx, nz, residents) : 0;
+        const bool one_launch = sweep_blocks > 0;
         unsigned long long* slots = one_launch ? reinterpret_cast<unsigned long long*>(C->r_E) : rmax;
         double* own_r0 = one_launch ? reinterpret_cast<double*>(slots + 2 * kEnthRmaxSlots + kSweepR0) : nullptr;
         double* parts = one_launch ? Wlm : partials;
@@ -207,7 +224,7 @@ int sweep_core(const glide_enth_column* C, double dt, int n_iter, const glide_en
         Lw.E = Wlm;
         if (one_launch) {
             HIP_TRY(launch_enth_sweeps<R>(L, Elm, Wlm, cfg->omega, cfg->n_newton, cfg->relaxation, slots, status, rtol,
-                                          atol, n_iter, persistent_spin_limit(), st),
+                                          atol, n_iter, persistent_spin_limit(), sweep_blocks, st),
                     "enthalpy sweeps");
         } else
         for (int it = 0; it < n_iter; ++it) {
@@ -307,7 +324,8 @@ int sweep_impl(const glide_enth_column* C, double dt, int n_iter, const glide_en
         return fail(GLIDE_ERR_INVALID_ARG, "n_iter must be in [0, GLIDE_ENTH_MAX_SWEEPS]");
     EnthScratch* s = nullptr;
     GLIDE_TRY(scratch(&s));
-    return sweep_core(C, dt, n_iter, cfg, report, st, s->partials, s->status, s->host, u2d, v2d, vel_div, s->rmax);
+    return sweep_core(C, dt, n_iter, cfg, report, st, s->partials, s->status, s->host, u2d, v2d, vel_div, s->rmax,
+                      sweep_residents(*s, st));
 }
 
 }  // namespace

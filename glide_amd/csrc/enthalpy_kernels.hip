@@ -2016,19 +2016,28 @@ static inline long layer_blocks(int ny, int nx, int nz) {
 // arrives.  Likewise the fence after the wait empties that L2 before any of them
 // is released, and each then empties its own CU's cache.
 //
-// words (zeroed before the launch): all arrivals, the XCDs' arrivals, the flag
-// that one gave up, the sweep's starting norm, the workgroups that have left, how
-// far the first to give up had come, the norms recorded, then (from kSweepHead)
-// per XCD its workgroups, arrivals and releases.  Every wait is bounded: after
+// Who takes part is counted, not assumed: other streams may hold the CUs, and two
+// launches that each wait for workgroups the other keeps out would never end.  The
+// first workgroup to run closes the launch when all have come, or when none has
+// for quiet_polls polls (about a millisecond); those that come later leave, and
+// the others, all of them running, share the work.
+//
+// words (zeroed before the launch): tickets and the closed bit, the XCDs'
+// arrivals, the flag that one gave up, the sweep's starting norm, the workgroups
+// that have left, how far the first to give up had come, the norms recorded, the
+// workgroups that have started, how many take part, then (from kSweepHead) per
+// XCD its workgroups, arrivals and releases.  Every wait is bounded: after
 // spin_limit polls (at once if negative), or when another workgroup gave up, the
 // barrier returns false, and the last workgroup to leave does the rest alone.
-constexpr int kSweepBlocks = 256;
+constexpr int kSweepBlocks = 256, kSweepQuietShift = 10;  // quiet_polls = spin_limit / 1024
+constexpr unsigned long long kSweepClosed = 1ull << 32;
 struct SweepBarrier {
     unsigned long long* w;
     int spin_limit;
     unsigned* own;  // in LDS: this workgroup's XCD, the workgroups on it, the XCDs in use
     unsigned gen;
     bool alone;
+    int rank, size;  // among those that take part
 
     __device__ __forceinline__ static unsigned long long peek(unsigned long long* p) {
         return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2042,9 +2051,9 @@ struct SweepBarrier {
         }
         return peek(w + 2) == 0;
     }
-    // counts the workgroups of each XCD
-    __device__ __forceinline__ bool start(unsigned long long* words, int limit) {
-        __shared__ int s_ok;
+    // 1: takes part, with the workgroups of each XCD counted; 0: gave up; -1: came late
+    __device__ __forceinline__ int start(unsigned long long* words, int limit) {
+        __shared__ int s_out[3];
         __shared__ unsigned s_own[3];
         w = words;
         own = s_own;
@@ -2052,19 +2061,42 @@ struct SweepBarrier {
         gen = 0;
         alone = false;
         if (threadIdx.x == 0) {
-            const unsigned xcd = own[0] = xcc_id();
-            atomicAdd(w + kSweepHead + xcd, 1ull);
-            __threadfence();
-            atomicAdd(w, 1ull);
-            s_ok = wait(w, gridDim.x);
-            __threadfence();
-            own[1] = (unsigned)peek(w + kSweepHead + xcd);
-            unsigned xcds = 0;
-            for (int q = 0; q < kSweepXcds; ++q) xcds += peek(w + kSweepHead + q) != 0;
-            own[2] = xcds;
+            const unsigned long long ticket = atomicAdd(w, 1ull);
+            int state = -1;
+            if (ticket < kSweepClosed) {
+                const unsigned xcd = own[0] = xcc_id();
+                atomicAdd(w + kSweepHead + xcd, 1ull);
+                __threadfence();
+                atomicAdd(w + 7, 1ull);
+                if (ticket == 0) {
+                    const int quiet = spin_limit >> kSweepQuietShift;
+                    unsigned long long n = peek(w);
+                    for (int idle = 0; n < gridDim.x && idle < quiet;) {
+                        __builtin_amdgcn_s_sleep(1);
+                        const unsigned long long m = peek(w);
+                        idle = m == n ? idle + 1 : 0;
+                        n = m;
+                    }
+                    n = atomicOr(w, kSweepClosed);
+                    state = wait(w + 7, n);  // theirs are under way
+                    if (state) __hip_atomic_store(w + 8, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                } else {
+                    state = wait(w + 8, 1);
+                }
+                __threadfence();
+                s_out[2] = (int)peek(w + 8);
+                own[1] = (unsigned)peek(w + kSweepHead + xcd);
+                unsigned xcds = 0;
+                for (int q = 0; q < kSweepXcds; ++q) xcds += peek(w + kSweepHead + q) != 0;
+                own[2] = xcds;
+            }
+            s_out[0] = state;
+            s_out[1] = (int)ticket;
         }
         __syncthreads();
-        return s_ok != 0;
+        rank = __builtin_amdgcn_readfirstlane(s_out[1]);
+        size = __builtin_amdgcn_readfirstlane(s_out[2]);
+        return __builtin_amdgcn_readfirstlane(s_out[0]);
     }
     __device__ __forceinline__ bool sync() {
         __shared__ int s_ok;
@@ -2132,12 +2164,12 @@ struct SweepBarrier {
 // call's own words: `status` is the device's one record, which a step on another
 // stream may rewrite meanwhile, and only takes the norms for the report.
 //
-// Nothing says that the workgroups run at the same time: other streams' work may
-// hold the CUs.  A workgroup whose wait gives up leaves, and the last to leave
-// goes on by itself from the first pass that not all have done.  That pass can be
-// done again: it reads what the one before it wrote and writes the other of E and
-// W (nobody is further than that pass, whose barrier needs all), and a norm is a
-// maximum.  The results are bitwise those of a launch whose waits end.
+// A workgroup whose wait gives up leaves, and the last to leave goes on by itself
+// from the first pass that not all have done.  That pass can be done again: it
+// reads what the one before it wrote and writes the other of E and W (nobody is
+// further than that pass, whose barrier needs all), and a norm is a maximum.  The
+// results are bitwise those of a launch whose waits end, and do not depend on how
+// many take part.
 template <typename T, int P, int MB>
 __global__ __launch_bounds__(256, 2) void k_enth_sweeps(EnthArgs<T> A, T* E, T* W, T omega_relax, int n_newton,
                                                         T relaxation, unsigned long long* slots,
@@ -2146,11 +2178,12 @@ __global__ __launch_bounds__(256, 2) void k_enth_sweeps(EnthArgs<T> A, T* E, T* 
                                                         int spin_limit, ColdValues<T> cold) {
     __shared__ double sh[4];
     const int tid = threadIdx.x, total = 2 * n_iter;
-    int first = blockIdx.x, step = gridDim.x;
     EnthArgs<T> Aw = A;
     Aw.E = W;
     SweepBarrier bar;
-    bool ok = bar.start(sync, spin_limit);
+    const int state = bar.start(sync, spin_limit);
+    int first = bar.rank, step = bar.size;
+    bool ok = state > 0;
     const double r0 = __longlong_as_double((long long)SweepBarrier::peek(sync + kSweepR0));
     auto clear = [&](int it) {  // the norms of sweep it, for sweep it + 2
         if (first == 0)
@@ -2187,12 +2220,12 @@ __global__ __launch_bounds__(256, 2) void k_enth_sweeps(EnthArgs<T> A, T* E, T* 
             ok = bar.sync();
             if (ok && !(p & 1)) clear(it);  // read by all before the barrier
         }
-        p = bar.leave(!ok, p, total);
+        p = bar.leave(state >= 0 && !ok, p, total);
         if (p < 0) return;
         first = 0;
         step = 1;
         ok = true;
-        if (p > 0 && !(p & 1)) clear((p >> 1) - 1);  // block 0 may have left before it
+        if (p > 0 && !(p & 1)) clear((p >> 1) - 1);  // the first may have left before it
         __syncthreads();
     }
 }
@@ -2427,16 +2460,36 @@ static inline int lm_lanes(long ncol, int nz) {
     return nz <= 16 ? 4 : nz <= 32 ? (fills ? 4 : 8) : (fills ? 8 : 16);
 }
 // The whole sweep in one launch: maps whose column pass has at most kSweepBlocks
-// workgroups, all of which then run at once.
-bool enth_sweeps_fit(int ny, int nx, int nz) {
-    const long ncol = (long)ny * nx, cols = 256 / lm_lanes(ncol, nz);
-    return (ncol + cols - 1) / cols <= kSweepBlocks;
+// workgroups, which a whole device holds at once (two a CU).  resident: how many
+// it holds of this kernel (of a partition's CUs, or those its stream may use);
+// with fewer than the passes have blocks each does several, as it would in
+// launches of their own.
+int enth_sweeps_blocks(int ny, int nx, int nz, int resident) {
+    if (!enth_lm_supported(nz)) return 0;
+    const long ncol = (long)ny * nx, cols = 256 / lm_lanes(ncol, nz), blocks = (ncol + cols - 1) / cols;
+    if (blocks > kSweepBlocks) return 0;
+    return (int)(blocks < resident ? blocks : resident);
+}
+#define GLIDE_LM_SWEEP_SPLITS(F) F(4, 3) F(4, 4) F(8, 3) F(8, 4) F(16, 3) F(16, 4)
+hipError_t enth_sweeps_per_cu(int* workgroups) {
+    int least = 1 << 20;
+    hipError_t e = hipSuccess;
+#define GLIDE_LM_OCC(PP, MB)                                                                              \
+    if (e == hipSuccess) {                                                                                \
+        int n = 0;                                                                                        \
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_enth_sweeps<double, PP, MB>, 256, 0);      \
+        least = n < least ? n : least;                                                                    \
+    }
+    GLIDE_LM_SWEEP_SPLITS(GLIDE_LM_OCC)
+#undef GLIDE_LM_OCC
+    *workgroups = least;
+    return e;
 }
 template <typename T>
 hipError_t launch_enth_sweeps(const EnthArgs<T>& A, T* E, T* W, T omega_relax, int n_newton, T relaxation,
                               unsigned long long* slots, EnthStatus* status, double rtol, double atol, int n_iter,
-                              int spin_limit, hipStream_t st) {
-    if (!enth_lm_supported(A.nz) || !A.u2d || !enth_sweeps_fit(A.ny, A.nx, A.nz)) return hipErrorInvalidValue;
+                              int spin_limit, int blocks, hipStream_t st) {
+    if (!enth_lm_supported(A.nz) || !A.u2d || blocks < 1) return hipErrorInvalidValue;
     const long ncol = (long)A.ny * A.nx;
     const int P = lm_lanes(ncol, A.nz), mb = (A.nz + P - 1) / P;
     const long cb = (ncol + 256 / P - 1) / (256 / P), lb = layer_blocks(A.ny, A.nx, A.nz);
@@ -2444,17 +2497,13 @@ hipError_t launch_enth_sweeps(const EnthArgs<T>& A, T* E, T* W, T omega_relax, i
     TimedLaunch tl(kTimeEnthColumn, ncol * A.nz, st);
 #define GLIDE_LM_SWEEPS(PP, MB)                                                                                    \
     if (P == PP && mb == MB) {                                                                                    \
-        k_enth_sweeps<T, PP, MB><<<(unsigned)cb, 256, 0, st>>>(A, E, W, omega_relax, n_newton, relaxation, slots, \
-                                                               slots + 2 * kEnthRmaxSlots, status, rtol, atol,    \
-                                                               n_iter, (int)cb, (int)lb, spin_limit, cold);       \
+        k_enth_sweeps<T, PP, MB><<<(unsigned)blocks, 256, 0, st>>>(A, E, W, omega_relax, n_newton, relaxation,    \
+                                                                   slots, slots + 2 * kEnthRmaxSlots, status,     \
+                                                                   rtol, atol, n_iter, (int)cb, (int)lb,          \
+                                                                   spin_limit, cold);                             \
         return hipGetLastError();                                                                                 \
     }
-    GLIDE_LM_SWEEPS(4, 3)
-    GLIDE_LM_SWEEPS(4, 4)
-    GLIDE_LM_SWEEPS(8, 3)
-    GLIDE_LM_SWEEPS(8, 4)
-    GLIDE_LM_SWEEPS(16, 3)
-    GLIDE_LM_SWEEPS(16, 4)
+    GLIDE_LM_SWEEP_SPLITS(GLIDE_LM_SWEEPS)
 #undef GLIDE_LM_SWEEPS
     return hipErrorInvalidValue;
 }
@@ -2543,7 +2592,7 @@ hipError_t launch_enth_residual_lm(const EnthArgs<T>& A, T* r_out, double* parti
                                                  hipStream_t);                                                       \
     template hipError_t launch_enth_layer_lm<T>(const EnthArgs<T>&, T*, T, hipStream_t);                             \
     template hipError_t launch_enth_sweeps<T>(const EnthArgs<T>&, T*, T*, T, int, T, unsigned long long*,            \
-                                              EnthStatus*, double, double, int, int, hipStream_t);                   \
+                                              EnthStatus*, double, double, int, int, int, hipStream_t);              \
     template hipError_t launch_enth_residual_lm<T>(const EnthArgs<T>&, T*, double*, double*, EnthStatus*, int,      \
                                                    double, double, hipStream_t);
 INST(double)

@@ -45,7 +45,7 @@ constexpr int kEnthResBlocks = 2048;  // residual grid (grid-stride over columns
 constexpr int kEnthRmaxSlots = 256;   // max-|r| accumulators of the column pass (bit patterns of doubles)
 // The accumulators' buffer: two sets, and the words of the one-launch sweep
 // (SweepBarrier; the starting norm is word kSweepR0 of them).
-constexpr int kSweepXcds = 16, kSweepHead = 7, kSweepR0 = 3;
+constexpr int kSweepXcds = 16, kSweepHead = 9, kSweepR0 = 3;
 constexpr int kEnthSlotWords = 2 * kEnthRmaxSlots + kSweepHead + 3 * kSweepXcds;
 
 // max |r| of the residual over the grid, into `max_out` (device), or, with
@@ -184,11 +184,14 @@ hipError_t launch_enth_column_lm(const EnthArgs<T>& A, T* W, T omega_relax, int 
 // but for the starting norm at 2 kEnthRmaxSlots + kSweepR0.  spin_limit bounds the
 // waits between its workgroups (polls; negative gives up at once); the results do
 // not depend on it.
-bool enth_sweeps_fit(int ny, int nx, int nz);
+// enth_sweeps_blocks: the launch's workgroups, or 0 where it does not apply, on a
+// device that holds `resident` of them (enth_sweeps_per_cu for each CU).
+int enth_sweeps_blocks(int ny, int nx, int nz, int resident);
+hipError_t enth_sweeps_per_cu(int* workgroups);
 template <typename T>
 hipError_t launch_enth_sweeps(const EnthArgs<T>& A, T* E, T* W, T omega_relax, int n_newton, T relaxation,
                               unsigned long long* slots, EnthStatus* status, double rtol, double atol, int n_iter,
-                              int spin_limit, hipStream_t st);
+                              int spin_limit, int blocks, hipStream_t st);
 // Layer smoother: E_out = E + omega_relax delta.
 template <typename T>
 hipError_t launch_enth_layer_lm(const EnthArgs<T>& A, T* E_out, T omega_relax, hipStream_t st);

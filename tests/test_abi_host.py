@@ -26,6 +26,18 @@ def test_library_exports_every_declared_symbol():
     assert not missing, missing
 
 
+@pytest.mark.parametrize("ny,nx,nz,resident,blocks", [
+    (40, 56, 21, 512, 70), (40, 56, 21, 64, 64), (40, 56, 21, 0, 0),  # the device, a partition, not known
+    (60, 60, 41, 512, 225), (60, 60, 41, 128, 128), (64, 64, 41, 512, 256), (65, 64, 41, 512, 0),
+    (1, 1, 9, 512, 1), (8, 8, 8, 512, 0), (8, 8, 65, 512, 0)])
+def test_enthalpy_sweep_workgroups_follow_the_device(ny, nx, nz, resident, blocks):
+    """The one-launch sweep never asks for more workgroups than the device (its
+    partition, or the CUs its stream may use) holds at once."""
+    lib = ctypes.CDLL(str(ROOT / "glide_amd" / "libglide_hip.so"))
+    f = lib._ZN5glide18enth_sweeps_blocksEiiii  # glide::enth_sweeps_blocks(int, int, int, int)
+    assert f(ny, nx, nz, resident) == blocks
+
+
 def test_python_binding_covers_header():
     from glide_amd import _lib
     assert set(declared_symbols()) == set(_lib.SIGNATURES)

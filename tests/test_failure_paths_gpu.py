@@ -54,12 +54,14 @@ def test_nan_adjoint_seed_reaches_the_adjoint_report():
 
 @pytest.mark.parametrize("n,nz,rel,n_smooth", [(9, 9, 1e-9, 30), (24, 21, 1e-9, 30), (24, 21, 0.0, 1),
                                                (24, 21, 0.0, 4), (33, 33, 1e-5, 30), (48, 41, 1e-5, 7)])
-@pytest.mark.parametrize("limit", [-1, 0, 1, 3, 10, 30, 100])
+@pytest.mark.parametrize("limit", [-1, 0, 1, 3, 10, 30, 100, 1000, 5000])
 def test_enthalpy_sweep_whose_waits_give_up_gives_the_same_results(n, nz, rel, n_smooth, limit):
     """The one-launch sweep of a small map with waits that give up at once
     (negative: one workgroup does everything) or after a few polls (somewhere
-    between two passes): E, the residual, the sweeps run and every norm are
-    bitwise those of a launch whose waits end, and nothing is reported."""
+    between two passes), or whose first workgroup hardly waits for the others to
+    come (1000, 5000: those that come later leave): E, the residual, the sweeps
+    run and every norm are bitwise those of an undisturbed launch, and nothing is
+    reported."""
     from glide_amd import _lib
     from tests.test_parity_enthalpy_gpu import _thermal_pair
     print(f"sweep give-up n={n} nz={nz} rel={rel} n_smooth={n_smooth} limit={limit}", flush=True)

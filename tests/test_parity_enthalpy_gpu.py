@@ -318,14 +318,16 @@ def test_tiled_sweep_matches_column_wavefronts(n, nz):
     assert abs(a0 - a1) <= 1e-8 * a1 and np.allclose(n0, n1, rtol=1e-7, atol=1e-8 * a1)
 
 
-def test_thermal_steps_on_two_streams_match_steps_alone():
-    """Steps of two small maps enqueued on two streams give, bitwise, what each
-    gives alone: what a sweep stops by is its own, not the device's one record.
-    The maps' starting norms and stopping sweeps differ."""
-    print("thermal steps on two streams", flush=True)
+@pytest.mark.parametrize("maps", [((24, 21, 3), (33, 33, 8)), ((24, 21, 3), (60, 41, 8), (59, 41, 9), (64, 41, 7))])
+def test_thermal_steps_on_several_streams_match_steps_alone(maps):
+    """Steps of small maps enqueued on a stream each give, bitwise, what each
+    gives alone: what a sweep stops by is its own, not the device's one record,
+    and launches that do not all fit on the device at once (the larger maps') do
+    not wait for each other.  The maps' starting norms and stopping sweeps differ."""
+    print(f"thermal steps on {len(maps)} streams", flush=True)
 
     def pair():
-        tms = [_thermal_pair(n, nz, seed, strain=True)[2] for n, nz, seed in ((24, 21, 3), (33, 33, 8))]
+        tms = [_thermal_pair(n, nz, seed, strain=True)[2] for n, nz, seed in maps]
         for tm in tms:
             tm.n_smooth = 60
             tm.ops.smoother_config.relative_tolerance, tm.ops.smoother_config.absolute_tolerance = 1e-9, 0.0
@@ -341,7 +343,7 @@ def test_thermal_steps_on_two_streams_match_steps_alone():
     assert max(s for _, s in ref[0]) < min(s for _, s in ref[1]) < 60  # they stop at different sweeps
     tms = pair()
     streams = [torch.cuda.Stream() for _ in tms]
-    got = [[], []]
+    got = [[] for _ in tms]
     torch.cuda.synchronize()
     for _ in range(4):
         for tm, st, out in zip(tms, streams, got):
