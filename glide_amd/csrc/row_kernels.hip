@@ -227,7 +227,7 @@ __global__ __launch_bounds__(kTinySide* kTinySide) void k_adjoint_tiny(
         kAy = dS + HD * g_at(it_, jc); kBy = dS - HD * g;
     }
     const T mk = C(a.mask, ic, jc), keep = T(1) - mk;
-    T kH = row_rcp(a.dt);
+    T kH = T(1) / a.dt;
     if (calving_rate != T(0)) {
         const int jr = min(jc + 1, nx - 1);
         const T k = (T(1) - C(a.phi, ic, jc)) * ((T(1) - C(a.phi, ic, jl)) + (T(1) - C(a.phi, ic, jr)) +

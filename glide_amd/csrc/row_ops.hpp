@@ -48,7 +48,9 @@ __device__ __forceinline__ double lane16_right(double x) {
 }
 
 // 1/a and 1/sqrt(a) to about an ulp: the hardware estimates, refined in FP32 by
-// one step as fast_rcp and fast_rsqrt refine the FP64 ones by two.
+// one step as fast_rcp and fast_rsqrt refine the FP64 ones by two.  For values
+// that the kernels form themselves: of an infinite argument the refinement makes
+// a NaN (a caller may give an infinite step, which drops the time term).
 __device__ __forceinline__ double row_rcp(double a) { return fast_rcp(a); }
 __device__ __forceinline__ float row_rcp(float a) {
     const float y = __builtin_amdgcn_rcpf(a);
@@ -241,7 +243,7 @@ struct TransposeRows {
                 ru += u * (ms + lane_left(ms));
             }
             rvb = q[2][lane];
-            T acc = lHm * row_rcp(a.dt) + tB_x + lane_right(tA_x) + tB_y + q[1][lane] - T(2) * eta * de2 - gH;
+            T acc = lHm * (T(1) / a.dt) + tB_x + lane_right(tA_x) + tB_y + q[1][lane] - T(2) * eta * de2 - gH;
             if (calving_rate != T(0)) {
                 const long rt = (long)clampi(ic - 1, 0, ny - 1) * nx, rb = (long)clampi(ic + 1, 0, ny - 1) * nx;
                 const int jl = clampi(jc - 1, 0, nx - 1), jr = clampi(jc + 1, 0, nx - 1);

@@ -134,6 +134,43 @@ def test_row_operators_at_tile_edges(orc, shape, m):
             assert rel_err(N(a), b) < KTOL
 
 
+@pytest.mark.parametrize("shape", [(14, 14), (17, 61)])
+@pytest.mark.parametrize("m", [1.0, 1.0 / 3.0])
+def test_adjoint_operators_without_a_time_term(orc, shape, m):
+    """An infinite step drops the time term (a steady state's adjoint): J^T lambda
+    against the oracle, and an adjoint pass in its forms (one workgroup, one
+    launch, two launches) finite and equal."""
+    from glide_amd import _lib
+    print(f"infinite step shape={shape} m={m:.3f}", flush=True)
+    ny, nx = shape
+    F = dome_fields(ny=ny, nx=nx, seed=45, mask_frac=0.2)
+    P = orc.phys(m=m, calving_rate=0.3)
+    lam = _lam(F, 46)
+    out = []
+    try:
+        for on in (True, False):
+            _lib.adjoint_coarse_enable(on)
+            _lib.adjoint_pass_fused_enable(on)
+            g = grid_from(F)
+            g.sliding.m.set(m)
+            g.calving.calving_rate.set(0.3)
+            for t, x in zip((g.adjoint.lambda_u, g.adjoint.lambda_v, g.adjoint.lambda_H), lam):
+                t.set(x)
+            ao = g.adjoint_operators
+            ao.use_cache = True
+            ao.compute_vjp(float("inf"))
+            ao.vanka_sweep(float("inf"), 1)
+            torch.cuda.synchronize()
+            for a, b in zip((ao.vjp_u, ao.vjp_v, ao.vjp_H), orc.vjp(F, *lam, P, 1500.0, float("inf"))):
+                assert rel_err(N(a), b) < KTOL
+            out.append([N(t.data) for t in (g.adjoint.lambda_u, g.adjoint.lambda_v, g.adjoint.lambda_H)])
+    finally:
+        _lib.adjoint_coarse_enable(True)
+        _lib.adjoint_pass_fused_enable(True)
+    for x, y in zip(*out):
+        assert np.isfinite(x).all() and rel_err(x, y) < 1e-11
+
+
 def test_jvp_freeze_calving_and_phi_refresh(orc):
     """freeze_calving drops the calving term; without freeze_phi the grounded
     fraction is recomputed from H and bed first."""
