@@ -82,12 +82,18 @@ __device__ __forceinline__ void fill_eta_tile(T (*s_eta)[TX + 2], const SsaArgs<
 // returns the increments w = ((u_l, u_r, v_t, v_b) change / 2, H change) and
 // the active-set flag.  edge: the calling wave may hold cells on the domain's
 // edge (the loop then tests the Dirichlet pins; interior waves carry no pin
-// code).  The wave-uniform edge test keeps one loop copy per wave.  Every lane
-// of the wavefront calls it (those without a cell to solve with the indices of
-// another one and solves = false) and iterates as long as any of them does:
-// with about ten lanes or fewer in its execution mask a wavefront issues these
-// instructions at a third of the rate, and the last iterations of a pass belong
-// to a few cells.
+// code).  The wave-uniform edge test keeps one loop copy per wave.
+//
+// Every lane of the wavefront calls it (those without a cell to solve with the
+// indices of another one and solves = false).  With ten lanes or so in its
+// execution mask a wavefront issues these instructions at a third of the rate, so
+// once kFewLanes or fewer iterate, the others compute along and keep their values
+// by selects; while more do, the lanes that are done drop out, which spares the
+// selects (a tenth of an iteration).  Ten passes at 200 x 200 (last tile 8 columns)
+// / 64 x 64 / 512 x 512, the last two with 64 columns a tile: 870 / 292 / 1030 us
+// with dropping out alone, 345 / 322 / 1070 with computing along alone, 347 / 303 /
+// 1041 with both.
+constexpr int kFewLanes = 32;
 template <typename T, bool LINEAR, typename TJ, int W, class Ld = LdPlain>
 __device__ __forceinline__ void cell_newton(const SsaArgs<T>& a, const T (*s_eta)[W], int li, int lj, int i, int j,
                                             const VankaArgs<T>& vk, bool solves, bool edge, T w[5], T& masked,
@@ -117,40 +123,46 @@ __device__ __forceinline__ void cell_newton(const SsaArgs<T>& a, const T (*s_eta
     const bool pin0 = j == 0, pin1 = j == nx - 1, pin2 = i == 0, pin3 = i == ny - 1;
     int it = 0;
     bool go = solves && vk.newton_steps > 0;
-    auto newton = [&](auto edge_tag) {
-        constexpr bool EDGE = decltype(edge_tag)::value;
-        while (__any(go)) {
-            TJ J[25];
-            T r[5];
-            cell_system<T, TJ, LINEAR>(cs, *cq, x, J, r, a.P);
-            if constexpr (EDGE) {
-                if (pin0) { pin_row(J, 0); r[0] = x[0]; }
-                if (pin1) { pin_row(J, 1); r[1] = x[1]; }
-                if (pin2) { pin_row(J, 2); r[2] = x[2]; }
-                if (pin3) { pin_row(J, 3); r[3] = x[3]; }
-            }
-            const bool pin4 = (x[4] - a.dt * r[4]) <= thk;
-            if (pin4) {
-                pin_row(J, 4);
-                r[4] = x[4] - thk;
-            }
-            masked = go ? (pin4 ? T(1) : T(0)) : masked;
-            TJ rj[5] = {TJ(r[0]), TJ(r[1]), TJ(r[2]), TJ(r[3]), TJ(r[4])};
-            TJ d[5];
-            lu5_solve_rcp(J, rj, d);
-            const T rnorm = r[0] * r[0] + r[1] * r[1] + r[2] * r[2] + r[3] * r[3] + r[4] * r[4];
-#pragma unroll
-            for (int k = 0; k < 5; ++k) {  // compensated relaxed update, local relaxation 0.5
-                const T y = T(-0.5) * T(d[k]) - cmp[k];
-                T t = x[k] + y;
-                const T e = (t - x[k]) - y;
-                if (k == 4) t = fmax(t, thk);
-                cmp[k] = go ? e : cmp[k];
-                x[k] = go ? t : x[k];
-            }
-            it += go ? 1 : 0;
-            go = go && it < vk.newton_steps && rnorm > tol;
+    // ALIVE: lanes that are done (go false) compute along and keep their values
+    auto step = [&](auto edge_tag, auto alive_tag) {
+        constexpr bool EDGE = decltype(edge_tag)::value, ALIVE = decltype(alive_tag)::value;
+        TJ J[25];
+        T r[5];
+        cell_system<T, TJ, LINEAR>(cs, *cq, x, J, r, a.P);
+        if constexpr (EDGE) {
+            if (pin0) { pin_row(J, 0); r[0] = x[0]; }
+            if (pin1) { pin_row(J, 1); r[1] = x[1]; }
+            if (pin2) { pin_row(J, 2); r[2] = x[2]; }
+            if (pin3) { pin_row(J, 3); r[3] = x[3]; }
         }
+        const bool pin4 = (x[4] - a.dt * r[4]) <= thk;
+        if (pin4) {
+            if constexpr (!ALIVE) masked = T(1);
+            pin_row(J, 4);
+            r[4] = x[4] - thk;
+        } else {
+            if constexpr (!ALIVE) masked = T(0);
+        }
+        if constexpr (ALIVE) masked = go ? (pin4 ? T(1) : T(0)) : masked;
+        TJ rj[5] = {TJ(r[0]), TJ(r[1]), TJ(r[2]), TJ(r[3]), TJ(r[4])};
+        TJ d[5];
+        lu5_solve_rcp(J, rj, d);
+        const T rnorm = r[0] * r[0] + r[1] * r[1] + r[2] * r[2] + r[3] * r[3] + r[4] * r[4];
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {  // compensated relaxed update, local relaxation 0.5
+            const T y = T(-0.5) * T(d[k]) - cmp[k];
+            T t = x[k] + y;
+            const T e = (t - x[k]) - y;
+            if (k == 4) t = fmax(t, thk);
+            cmp[k] = !ALIVE || go ? e : cmp[k];
+            x[k] = !ALIVE || go ? t : x[k];
+        }
+        it += !ALIVE || go ? 1 : 0;
+        go = go && it < vk.newton_steps && rnorm > tol;
+    };
+    auto newton = [&](auto edge_tag) {
+        while (go && __popcll(__ballot(true)) > kFewLanes) step(edge_tag, std::false_type{});
+        while (__any(go)) step(edge_tag, std::true_type{});
     };
     if (edge) newton(std::true_type{});
     else newton(std::false_type{});

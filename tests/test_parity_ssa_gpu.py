@@ -225,6 +225,24 @@ def test_vanka_single_pass(orc, shape):
     assert np.array_equal(N(g.state.mask.data), mask)
 
 
+@pytest.mark.parametrize("shape", [(5, 32), (5, 33), (4, 95), (4, 97), (3, 65)])
+@pytest.mark.parametrize("freeze", [False, True])
+def test_vanka_pass_with_few_columns_in_a_wavefront(orc, shape, freeze):
+    """Widths whose last wavefront holds 1, 31, 32 or 33 columns, where the local
+    iterations go over from lanes that drop out to lanes that compute along: one
+    pass against the oracle (the pass bar)."""
+    ny, nx = shape
+    print(f"vanka pass shape={shape} freeze={freeze}", flush=True)
+    F = dome_fields(ny=ny, nx=nx, seed=6, mask_frac=0.1)
+    g = grid_from(F)
+    g.forward_operators.vanka_sweep(10.0, 1, freeze_phi=freeze)
+    Fo = F if freeze else dict(F, phi=orc.grounded(F["H"], F["bed"], 0.1))
+    u, v, H, mask, _ = orc.vanka_sweep(Fo, orc.phys(), 1500.0, 10.0)
+    for a, b in ((g.state.u, u), (g.state.v, v), (g.state.H, H)):
+        assert rel_err(N(a.data), b) < KTOL
+    assert np.array_equal(N(g.state.mask.data), mask)
+
+
 @pytest.mark.parametrize("shape", SHAPES[:2])
 def test_vanka_single_pass_nonlinear_drag_calving(orc, shape):
     ny, nx = shape
