@@ -327,6 +327,106 @@ __global__ __launch_bounds__(kRowLanes* NW) void k_mc_pass(SsaArgs<T> a, T* __re
     mc_pass_body<T, NW, LINEAR>(b % gx, b / gx, a, u_dst, v_dst, H_dst, mask, phi_dst, vk);
 }
 
+// The pass in three launches, for levels that fill the device with heavy local
+// solves (mc_phases_faster): the viscosity, then a launch per colour, from one
+// buffer set into the other.  A lane owns a cell of the colour and the other cell
+// beside it, so a wavefront covers 128 columns and no cell is solved twice: the
+// one-launch form solves 8 rows of red cells for every 6 and leaves 3 lanes of 32
+// and a wavefront of 4 idle in turn.
+template <typename T>
+__global__ __launch_bounds__(256) void k_cell_eta(SsaArgs<T> a, T* __restrict__ eta) {
+    const int j = blockIdx.x * 256 + threadIdx.x, i = blockIdx.y;
+    if (j >= a.nx) return;
+    const CellVel<T> c = load_cell_vel<T>(a.u, a.v, i, j, a.ny, a.nx);
+    const T e2 = strain_invariant(c, i, j, a.ny, a.nx, a.dxi, a.P.eps_reg);
+    eta[(long)i * a.nx + j] = T(0.5) * a.B[(long)i * a.nx + j] * glen_power(e2, a.P);
+}
+
+// Local Newton iteration of cell (i, j) against the state in a; returns the
+// new unknowns x and the active-set flag.  EDGE: the cell may lie on the
+// domain edge (the Dirichlet pins are tested).
+template <typename T, bool LINEAR, bool EDGE>
+__device__ __forceinline__ void phase_newton(const SsaArgs<T>& a, const T* __restrict__ eta, int i, int j,
+                                             const VankaArgs<T>& vk, T x[5], T& masked) {
+    const int ny = a.ny, nx = a.nx;
+    CellSys<T> cs;
+    T thk;
+    {
+        Patch<T> p;
+        load_patch_with<T>(p, a, [&](int di, int dj) { return eta[offC(i + di, j + dj, ny, nx)]; }, i, j, a.f_u, a.f_v,
+                           a.f_H, a.phi);
+        make_cell_sys(cs, p, a.P, vk.calving_rate, a.dxi, a.dt, vk.ssa_damping, vk.mc_damping);
+        thk = p.gam;
+    }
+    const long c = (long)i * nx + j;
+    x[0] = a.u[(long)i * (nx + 1) + j];
+    x[1] = a.u[(long)i * (nx + 1) + j + 1];
+    x[2] = a.v[c];
+    x[3] = a.v[c + nx];
+    x[4] = a.H[c];
+    const bool pin0 = j == 0, pin1 = j == nx - 1, pin2 = i == 0, pin3 = i == ny - 1;
+    T rnorm = T(1e30);
+    for (int it = 0; it < vk.newton_steps && rnorm > vk.tol; ++it) {
+        T J[25], r[5];
+        cell_system<T, T, LINEAR>(cs, cs, x, J, r, a.P);
+        if constexpr (EDGE) {
+            if (pin0) { pin_row(J, 0); r[0] = x[0]; }
+            if (pin1) { pin_row(J, 1); r[1] = x[1]; }
+            if (pin2) { pin_row(J, 2); r[2] = x[2]; }
+            if (pin3) { pin_row(J, 3); r[3] = x[3]; }
+        }
+        if ((x[4] - a.dt * r[4]) <= thk) {
+            masked = T(1);
+            pin_row(J, 4);
+            r[4] = x[4] - thk;
+        } else {
+            masked = T(0);
+        }
+        T d[5];
+        lu5_solve_rcp(J, r, d);
+        rnorm = r[0] * r[0] + r[1] * r[1] + r[2] * r[2] + r[3] * r[3] + r[4] * r[4];
+#pragma unroll
+        for (int k = 0; k < 5; ++k) x[k] -= vk.relax * d[k];
+        x[4] = fmax(x[4], thk);
+    }
+}
+
+constexpr int kPhaseRows = 4;  // rows per block
+template <typename T, bool LINEAR>
+__global__ __launch_bounds__(kRowLanes* kPhaseRows) void k_mc_phase(SsaArgs<T> a, const T* __restrict__ eta,
+                                                                    T* __restrict__ u_dst, T* __restrict__ v_dst,
+                                                                    T* __restrict__ H_dst, T* __restrict__ mask,
+                                                                    VankaArgs<T> vk, int colour) {
+    const int ny = a.ny, nx = a.nx;
+    const int bx = blockIdx.x, i = blockIdx.y * kPhaseRows + threadIdx.y;
+    if (i >= ny) return;
+    const int pair = bx * kRowLanes + threadIdx.x;
+    const int p = (i + colour) & 1;
+    const int j = 2 * pair + p;       // the lane's cell of the colour
+    const int jo = 2 * pair + 1 - p;  // and the other one beside it
+    if (j < nx) {
+        const long c = (long)i * nx + j;
+        T x[5], masked = mask[c];
+        const bool edge = i == 0 || i == ny - 1 || bx == 0 || 2 * (bx + 1) * kRowLanes >= nx;
+        if (edge) phase_newton<T, LINEAR, true>(a, eta, i, j, vk, x, masked);
+        else phase_newton<T, LINEAR, false>(a, eta, i, j, vk, x, masked);
+        u_dst[(long)i * (nx + 1) + j] = x[0];
+        u_dst[(long)i * (nx + 1) + j + 1] = x[1];
+        v_dst[c] = x[2];
+        v_dst[c + nx] = x[3];
+        H_dst[c] = x[4];
+        mask[c] = masked;
+    }
+    if (jo < nx) {
+        const long c = (long)i * nx + jo;
+        H_dst[c] = a.H[c];
+        if (jo == 0) u_dst[(long)i * (nx + 1)] = a.u[(long)i * (nx + 1)];
+        if (jo == nx - 1) u_dst[(long)i * (nx + 1) + nx] = a.u[(long)i * (nx + 1) + nx];
+        if (i == 0) v_dst[jo] = a.v[jo];
+        if (i == ny - 1) v_dst[(long)ny * nx + jo] = a.v[(long)ny * nx + jo];
+    }
+}
+
 // All additive forward passes of a level of at most 16 x 16 cells in one
 // workgroup, the state in LDS: 16 lanes a row, four rows a wavefront, one
 // wavefront per SIMD.  A pass of k_vanka_persistent reads the level's state and
@@ -524,6 +624,42 @@ hipError_t launch_vanka_mc(const SsaArgs<T>& a, T* u_dst, T* v_dst, T* H_dst, T*
     return hipGetLastError();
 }
 
+// Heavy local solves, a nonlinear drag law or five Newton steps and more, are bound
+// by instructions, of which the one-launch form has up to 1.5 times as many; it
+// wins where its workgroups fit the 256 CUs in as many rounds (fewer launches, less
+// traffic), and where the solves are light.  Four passes, one launch / phases, us:
+//   linear drag, 3 / 6 / 30 steps      256 x 256: 62/86, 81/104, 229/246;
+//     512 x 512: 133/133, 191/167, 658/429;  1024 x 1024: 342/337, 515/422, 1908/1447
+//   Weertman drag (m = 1/3), 1 / 3 / 30 steps      256 x 256: 83/104, 149/171, 1036/1065;
+//     320 x 320: 138/115, 263/182, 1960/1078;  384 x 384: 145/175, 275/300, 2043/2001;
+//     512 x 512: 253/197, 495/328, 3765/2119;  1024 x 1024: 751/583, 1535/1110, 12136/8276
+bool mc_phases_faster(int ny, int nx, int newton_steps, bool linear) {
+    constexpr long kCus = 256;
+    int gx;
+    const long one = mc_blocks(ny, nx, kMcWaves, &gx);
+    const long phase = (((long)nx + 1) / 2 + kRowLanes - 1) / kRowLanes * (((long)ny + kPhaseRows - 1) / kPhaseRows);
+    return (!linear || newton_steps >= 5) && (phase + kCus - 1) / kCus < (one + kCus - 1) / kCus;
+}
+
+template <typename T>
+hipError_t launch_mc_phases(const SsaArgs<T>& a, T* eta, T* u, T* v, T* H, T* u_alt, T* v_alt, T* H_alt, T* mask,
+                            const VankaArgs<T>& vk, hipStream_t st) {
+    TimedLaunch tl(std::is_same<T, float>::value ? kTimeVankaMc32 : kTimeVankaMc64, (long)a.ny * a.nx, st);
+    k_cell_eta<T><<<dim3((a.nx + 255) / 256, a.ny), 256, 0, st>>>(a, eta);
+    const int pairs = (a.nx + 1) / 2;
+    const dim3 g((pairs + kRowLanes - 1) / kRowLanes, (a.ny + kPhaseRows - 1) / kPhaseRows), b(kRowLanes, kPhaseRows);
+    SsaArgs<T> black = a;
+    black.u = u_alt; black.v = v_alt; black.H = H_alt;
+    if (a.P.linear_drag) {
+        k_mc_phase<T, true><<<g, b, 0, st>>>(a, eta, u_alt, v_alt, H_alt, mask, vk, 0);
+        k_mc_phase<T, true><<<g, b, 0, st>>>(black, eta, u, v, H, mask, vk, 1);
+    } else {
+        k_mc_phase<T, false><<<g, b, 0, st>>>(a, eta, u_alt, v_alt, H_alt, mask, vk, 0);
+        k_mc_phase<T, false><<<g, b, 0, st>>>(black, eta, u, v, H, mask, vk, 1);
+    }
+    return hipGetLastError();
+}
+
 // ------------------------------------------------------------ domain tables
 namespace {
 template <typename T, int NW, bool LINEAR>
@@ -684,7 +820,9 @@ hipError_t launch_krylov_axpy(double* out, const double* V, long ld, long n, int
 
 #define GLIDE_MC_INSTANTIATE(T)                                                                                     \
     template hipError_t launch_pin_rows<T>(T*, T*, T*, const T*, int, int, hipStream_t);                           \
-    template hipError_t launch_vanka_mc<T>(const SsaArgs<T>&, T*, T*, T*, T*, T*, const VankaArgs<T>&, hipStream_t);
+    template hipError_t launch_vanka_mc<T>(const SsaArgs<T>&, T*, T*, T*, T*, T*, const VankaArgs<T>&, hipStream_t); \
+    template hipError_t launch_mc_phases<T>(const SsaArgs<T>&, T*, T*, T*, T*, T*, T*, T*, T*, const VankaArgs<T>&, \
+                                            hipStream_t);
 
 GLIDE_MC_INSTANTIATE(double)
 GLIDE_MC_INSTANTIATE(float)

@@ -223,11 +223,12 @@ int persistent_ctl(const glide_level& L, PersistentCtl* ctl) {
 }
 
 template <typename T>
-int mc_sweeps_t(const glide_level& L, double dt, int n_iter, const glide_vanka_config& vc, int flags, hipStream_t st);
+int mc_sweeps_t(const glide_level& L, double dt, int n_iter, const glide_vanka_config& vc, int flags, hipStream_t st,
+                bool mixed);
 
 int vanka_sweeps(const glide_level& L, double dt, int n_iter, const glide_vanka_config& vc, int flags,
                  hipStream_t st) {
-    if (vc.multicolour) return mc_sweeps_t<R>(L, dt, n_iter, vc, flags, st);
+    if (vc.multicolour) return mc_sweeps_t<R>(L, dt, n_iter, vc, flags, st, false);
     const bool freeze_phi = (flags & GLIDE_FREEZE_PHI) != 0;
     VankaArgs<R> vk;
     vk.newton_steps = vc.newton_steps;
@@ -873,10 +874,13 @@ int residual_t(const glide_level& L, double dt, int flags, T* ou, T* ov, T* oH, 
 // type T, one launch each, alternating between the level's state and the
 // workspace; an odd count copies the state back at the end.  The pass itself
 // refreshes the grounded fraction unless frozen or relaxed (a workgroup would
-// then read the old fraction of cells that another one rewrites).
+// then read the old fraction of cells that another one rewrites).  Heavy local
+// solves on large levels go in three launches a pass; in the mixed solves (mixed)
+// only those of a nonlinear drag law, since a batched ensemble, whose drag is
+// linear, gives bitwise what they do.
 template <typename T>
 int mc_sweeps_t(const glide_level& L, double dt, int n_iter, const glide_vanka_config& vc, int flags,
-                hipStream_t st) {
+                hipStream_t st, bool mixed) {
     const bool freeze_phi = (flags & GLIDE_FREEZE_PHI) != 0, relaxed = T(vc.relax_phi) != T(0);
     VankaArgs<T> vk;
     vk.newton_steps = vc.newton_steps;
@@ -889,6 +893,19 @@ int mc_sweeps_t(const glide_level& L, double dt, int n_iter, const glide_vanka_c
     vk.tol = T(vc.newton_tol);
     T* own[3] = {PT<T>(L.u), PT<T>(L.v), PT<T>(L.H)};
     T* alt[3] = {PT<T>(L.work), PT<T>(L.work) + nU(L), PT<T>(L.work) + nU(L) + nV(L)};
+    if (mc_phases_faster(L.ny, L.nx, mixed ? 0 : vk.newton_steps, make_phys(L.phys).linear_drag)) {
+        for (int it = 0; it < n_iter; ++it) {
+            const SsaArgs<T> a = make_args_t<T>(L, dt, false);
+            if (!freeze_phi)
+                HIP_TRY(launch_grounded<T>(PT<T>(L.phi), a.H, CPT<T>(L.bed), T(L.phys.flotation_reg_driving),
+                                           T(vc.relax_phi), (long)nC(L), st),
+                        "grounded");
+            HIP_TRY(launch_mc_phases<T>(a, alt[2] + nC(L), own[0], own[1], own[2], alt[0], alt[1], alt[2],
+                                        PT<T>(L.mask), vk, st),
+                    "red-black phases");
+        }
+        return GLIDE_OK;
+    }
     for (int it = 0; it < n_iter; ++it) {
         T* const* src = (it & 1) ? alt : own;
         T* const* dst = (it & 1) ? own : alt;
@@ -944,7 +961,7 @@ int coarsest_fp64(MixedCtx& X, int l, int n_iter, int flags) {
     in.add(kMixTo64, D.f_H, A.f_H, nullptr, (long)nC(A));
     in.add(kMixTo64, D.gamma, A.gamma, nullptr, (long)nC(A));
     GLIDE_TRY(run_mixed(in, X.st));
-    GLIDE_TRY(mc_sweeps_t<double>(D, X.dt, n_iter, X.vc[l], flags, X.st));
+    GLIDE_TRY(mc_sweeps_t<double>(D, X.dt, n_iter, X.vc[l], flags, X.st, true));
     MixedBatch out;
     out.add(kMixTo32, A.u, D.u, nullptr, (long)nU(A));
     out.add(kMixTo32, A.v, D.v, nullptr, (long)nV(A));
@@ -970,7 +987,7 @@ int mixed_vcycle(MixedCtx& X, int l, bool finest) {
     };
     auto smooth = [&](const glide_level& A, int n, int flags) -> int {
         if (n <= 0) return GLIDE_OK;
-        return mc_sweeps_t<F>(A, X.dt, n, X.vc[l], flags, st);
+        return mc_sweeps_t<F>(A, X.dt, n, X.vc[l], flags, st, true);
     };
     if (finest) {
         EwBatch<F> b;

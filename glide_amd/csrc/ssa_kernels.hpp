@@ -226,6 +226,13 @@ hipError_t launch_grad_B(const SsaArgs<T>& a, const T* lu, const T* lv, T* gB, h
 // goes to u_dst / v_dst / H_dst, which must differ from a's buffers, the
 // active-set flag in place.  phi_dst != nullptr: the pass takes the grounded
 // fraction of the state in a (not a.phi) and writes it there.
+// launch_mc_phases: the same pass (to rounding) in a launch for the viscosity,
+// into eta (ny, nx), and one per colour: red into the alternate buffers, black
+// back into u / v / H, which are a's own.
+bool mc_phases_faster(int ny, int nx, int newton_steps, bool linear);
+template <typename T>
+hipError_t launch_mc_phases(const SsaArgs<T>& a, T* eta, T* u, T* v, T* H, T* u_alt, T* v_alt, T* H_alt, T* mask,
+                            const VankaArgs<T>& vk, hipStream_t st);
 // Zero the multipliers / corrections of the rows the patch solves pin: the
 // domain-edge facets and the cells of the active set (mask > 0.5).
 template <typename T>

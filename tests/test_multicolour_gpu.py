@@ -100,6 +100,33 @@ def test_mc_pass_tiles_and_grounded_refresh(orc, shape, relax_phi):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("shape", [(320, 320), (323, 317)])
+@pytest.mark.parametrize("m,steps,relax_phi", [(1.0, 4, 0.0), (1.0, 5, 0.0), (1.0 / 3.0, 3, 0.0), (1.0 / 3.0, 3, 0.3)])
+def test_mc_pass_in_one_and_in_three_launches(orc, shape, m, steps, relax_phi):
+    """Large levels on both sides of the rule for heavy local solves (linear drag
+    up to four steps: one launch a pass; more steps or a nonlinear law: three): a
+    pass that refreshes (or relaxes) the grounded fraction against the oracle."""
+    ny, nx = shape
+    print(f"mc pass forms shape={shape} m={m:.3f} steps={steps} relax_phi={relax_phi}", flush=True)
+    s = dict(MIXED, steps=steps)
+    F = dome_fields(ny=ny, nx=nx, seed=15, mask_frac=0.1)
+    g = grid_from(F)
+    g.sliding.m.set(m)
+    fo = g.forward_operators
+    _configure(fo.vanka_config, s)
+    fo.vanka_config.relax_phi = relax_phi
+    phi = (1.0 - relax_phi) * orc.grounded(F["H"], F["bed"], 0.1) + relax_phi * F["phi"]
+    for k in range(2):
+        fo.vanka_sweep(10.0, 1, freeze_phi=k > 0)
+        torch.cuda.synchronize()
+        u, v, H, mask, _ = orc.mc_sweep(dict(F, phi=phi), orc.phys(m=m), 1500.0, 10.0, **_oracle_kw(s))
+        F.update(u=u, v=v, H=H, mask=mask)
+        assert rel_err(N(g.state.phi.data), phi) < 1e-12
+        for a, b in ((g.state.u, u), (g.state.v, v), (g.state.H, H)):
+            assert rel_err(N(a.data), b) < (1e-12 if k == 0 else 1e-11), k
+        assert np.array_equal(N(g.state.mask.data), mask), k
+
+
 def _warm_models(orc, n, L, warm=2, ny=None, compat=True):
     """GPU model and oracle hierarchy after `warm` additive V-cycles (matching
     to 1e-10), then H_prev = H (the start of a next time step)."""
