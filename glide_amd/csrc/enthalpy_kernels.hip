@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <type_traits>
 
 #include "enthalpy_kernels.hpp"
 #include "ssa_device.hpp"
@@ -631,23 +632,30 @@ __global__ __launch_bounds__(256) void k_enth_apply(const int* __restrict__ skip
         E[q] += omega_relax * delta[q];
 }
 
-// omega = H sigma_dot by upward integration of the sigma-space continuity
-// equation (glide/cuda/enthalpy.cu:1276-1372): lanes form the per-level
-// flux divergence, lane 0 integrates in level order; the result is divided
-// by out_div.
-// The once-a-step kernels below take kBlockCols columns a block: what is the same
-// for a whole column (its sums, powers and divisions) one thread per column, the
-// (ny, nx, nz) values in contiguous runs.  A wavefront per column formed the
-// column's part in all or in one of its lanes, and took about 175 us each at
-// 512 x 512 x 41; here the strain heating takes 22, omega 35 and the forcing 39 us
-// (20 to 35 us for the values read and written).
+// The once-a-step kernels (omega, forcing, strain heating, rate factor) take COLS
+// columns a block (by_block_columns): what is the same for a whole column (its
+// sums, powers and divisions) one thread per column, the (ny, nx, nz) values in
+// contiguous runs.  A wavefront per column formed the column's part in all or in
+// one of its lanes: at 512 x 512 x 41 strain heating 159 us, here 17 (86 MB written:
+// 5 TB/s), the forcing 48 and 28, omega of a depth-varying velocity 186 and 96.
 constexpr int kBlockCols = 64;
-template <typename T>
+// q / nz for q < kBlockCols * 64 (nz >= 2): a multiplication, the division done once
+struct ByLevels {
+    unsigned m;
+    __device__ __forceinline__ explicit ByLevels(int nz) : m(0xffffffffu / (unsigned)nz + 1u) {}
+    __device__ __forceinline__ int operator()(int q) const { return (int)__umulhi((unsigned)q, m); }
+};
+// omega = H sigma_dot by upward integration of the sigma-space continuity
+// equation (glide/cuda/enthalpy.cu:1276-1372): the levels' flux divergences (one
+// for all where the velocity is the same on every level), then each column's sum
+// in level order; the result is divided by out_div.
+template <typename T, int COLS>
 __global__ __launch_bounds__(256) void k_enth_omega(EnthArgs<T> A, const T* __restrict__ dhdt,
                                                     const T* __restrict__ bmb, T out_div, T* __restrict__ omega) {
-    __shared__ T s[kBlockCols * 65];
-    const long ncol = (long)A.ny * A.nx, c0 = (long)blockIdx.x * kBlockCols;
-    const int nc = (int)min((long)kBlockCols, ncol - c0), nz = A.nz, ny = A.ny, nx = A.nx;
+    __shared__ T s[COLS * 65];
+    const long ncol = (long)A.ny * A.nx, c0 = (long)blockIdx.x * COLS;
+    const int nc = (int)min((long)COLS, ncol - c0), nz = A.nz, ny = A.ny, nx = A.nx;
+    const ByLevels by_nz(nz);
     auto divergence = [&](long col, int k) {
         const int i = (int)(col / nx), j = (int)(col % nx);
         const T h = A.H[col];
@@ -673,7 +681,11 @@ __global__ __launch_bounds__(256) void k_enth_omega(EnthArgs<T> A, const T* __re
         return (fr - fl + ft - fb) * A.dxi;
     };
     if (!A.u2d) {
-        for (int q = threadIdx.x; q < nc * nz; q += blockDim.x) s[(q / nz) * 65 + q % nz] = divergence(c0 + q / nz, q % nz);
+        // a run of columns at a time: the velocities' planes are read along it
+        for (int q = threadIdx.x; q < COLS * nz; q += blockDim.x) {
+            const int k = q / COLS, c = q % COLS;
+            if (c < nc) s[c * 65 + k] = divergence(c0 + c, k);
+        }
         __syncthreads();
     }
     if ((int)threadIdx.x < nc) {  // the upward sum in level order, in place over the divergences
@@ -693,7 +705,10 @@ __global__ __launch_bounds__(256) void k_enth_omega(EnthArgs<T> A, const T* __re
         }
     }
     __syncthreads();
-    for (int q = threadIdx.x; q < nc * nz; q += blockDim.x) omega[c0 * nz + q] = s[(q / nz) * 65 + q % nz] / out_div;
+    for (int q = threadIdx.x; q < nc * nz; q += blockDim.x) {
+        const int c = by_nz(q);
+        omega[c0 * nz + q] = s[c * 65 + q - c * nz] / out_div;
+    }
 }
 
 template <typename T>
@@ -713,13 +728,14 @@ __global__ __launch_bounds__(256) void k_enth_tendency(const T* __restrict__ a, 
 // Basal frictional heating Q_fh = beta |u_b|^(m+1) from the bed-layer
 // velocities averaged to cell centres (glide/model.py:215-228), then the
 // forcing f_E of glide/enthalpy.py:473-519.
-template <typename T>
+template <typename T, int COLS>
 __global__ __launch_bounds__(256) void k_enth_rhs(EnthArgs<T> A, const T* __restrict__ beta, T m, T u_reg,
                                                   int frictional, T* __restrict__ Q_fh, T* __restrict__ f_E) {
     // frictional: Q_fh from the velocities (else read); f_E == nullptr: Q_fh only.
-    __shared__ T s_h[kBlockCols], s_bed[kBlockCols];
-    const long ncol = (long)A.ny * A.nx, c0 = (long)blockIdx.x * kBlockCols;
-    const int nc = (int)min((long)kBlockCols, ncol - c0), nz = A.nz, nx = A.nx;
+    __shared__ T s_h[COLS], s_bed[COLS];
+    const long ncol = (long)A.ny * A.nx, c0 = (long)blockIdx.x * COLS;
+    const int nc = (int)min((long)COLS, ncol - c0), nz = A.nz, nx = A.nx;
+    const ByLevels by_nz(nz);
     if ((int)threadIdx.x < nc) {
         const long col = c0 + threadIdx.x;
         const int i = (int)(col / nx), j = (int)(col % nx);
@@ -745,7 +761,7 @@ __global__ __launch_bounds__(256) void k_enth_rhs(EnthArgs<T> A, const T* __rest
     if (!f_E) return;
     __syncthreads();
     for (int q = threadIdx.x; q < nc * nz; q += blockDim.x) {
-        const int c = q / nz, k = q % nz;
+        const int c = by_nz(q), k = q - c * nz;
         T f = A.phi_strain ? s_h[c] * A.phi_strain[c0 * nz + q] / T(kEScale) : T(0);
         if (k == 0) f += s_bed[c];
         if (k == nz - 1) f = T(0);
@@ -758,13 +774,14 @@ __global__ __launch_bounds__(256) void k_enth_rhs(EnthArgs<T> A, const T* __rest
 // SEC_PER_YR in W/m^3, with eps_e^2 the momentum solver's cell strain-rate
 // invariant of the velocities (m/a) and eta = B/2 (eps_e^2 + eps_reg)^p its
 // Glen viscosity (B in head units).
-template <typename T>
+template <typename T, int COLS>
 __global__ __launch_bounds__(256) void k_enth_strain_heating(const T* __restrict__ u, const T* __restrict__ v,
                                                              const T* __restrict__ B, int ny, int nx, int nz, T dxi,
                                                              T glen_p, T eps_reg, T rho_g, T* __restrict__ phi) {
-    __shared__ T s[kBlockCols];
-    const long ncol = (long)ny * nx, c0 = (long)blockIdx.x * kBlockCols;
-    const int nc = (int)min((long)kBlockCols, ncol - c0);
+    __shared__ T s[COLS];
+    const long ncol = (long)ny * nx, c0 = (long)blockIdx.x * COLS;
+    const int nc = (int)min((long)COLS, ncol - c0);
+    const ByLevels by_nz(nz);
     if ((int)threadIdx.x < nc) {
         const long col = c0 + threadIdx.x;
         const int i = (int)(col / nx), j = (int)(col % nx);
@@ -774,19 +791,20 @@ __global__ __launch_bounds__(256) void k_enth_strain_heating(const T* __restrict
         s[threadIdx.x] = T(4) * eta * e2 * rho_g / T(kSecPerYr);
     }
     __syncthreads();
-    for (int q = threadIdx.x; q < nc * nz; q += blockDim.x) phi[c0 * nz + q] = s[q / nz];
+    for (int q = threadIdx.x; q < nc * nz; q += blockDim.x) phi[c0 * nz + q] = s[by_nz(q)];
 }
 
 // Paterson-Budd rate factor A(T) (1 + 181.25 w) averaged over the levels and
 // returned as B = <A>^(-1/n) / scale (glide/enthalpy.py:600-643,
 // glide/model.py:209-213).
-template <typename T>
+template <typename T, int COLS>
 __global__ __launch_bounds__(256) void k_enth_arrhenius(EnthArgs<T> A, T n_glen, T scale, T* __restrict__ B) {
-    __shared__ T s[kBlockCols * 65];
-    const long ncol = (long)A.ny * A.nx, c0 = (long)blockIdx.x * kBlockCols;
-    const int nc = (int)min((long)kBlockCols, ncol - c0), nz = A.nz;
+    __shared__ T s[COLS * 65];
+    const long ncol = (long)A.ny * A.nx, c0 = (long)blockIdx.x * COLS;
+    const int nc = (int)min((long)COLS, ncol - c0), nz = A.nz;
+    const ByLevels by_nz(nz);
     for (int q = threadIdx.x; q < nc * nz; q += blockDim.x) {
-        const int c = q / nz, k = q % nz;
+        const int c = by_nz(q), k = q - c * nz;
         const T Tp = t_pmp(T(k) * (T(1) / T(nz - 1)), A.H[c0 + c]);
         const T Ek = A.E[c0 * nz + q];
         const T Tk = fmin(Ek * T(kEScale) / T(kCI) + T(kTRef), Tp);
@@ -2258,8 +2276,20 @@ __global__ __launch_bounds__(256) void k_enth_residual_lm(EnthArgs<T> A, T* __re
 static inline unsigned col_blocks(int ny, int nx) {
     return (unsigned)(((long)ny * nx + kColsPerBlock - 1) / kColsPerBlock);
 }
-static inline unsigned block_columns(int ny, int nx) {
-    return (unsigned)(((long)ny * nx + kBlockCols - 1) / kBlockCols);
+// f(blocks, columns of a block as a constant).  MOST: on maps of 32768 columns and
+// more, which fill the device at 64; 16 and 8 below, whose blocks would be few and
+// their loops over the levels long.  8 / 16 / 64 columns (a wavefront per column),
+// us: omega at 40 x 56 x 21 4.4 / 5.4 / 9.5 (4.3), at 128 x 128 x 41 11.3 / 10.4 / 19.6
+// (18.6), at 512 x 512 x 41 134 / 96 / 110 (186), hence 16 at most for omega; forcing
+// 2.4 / 2.6 / 3.7 (2.5), 4.0 / 3.8 / 5.7 (4.8), 35 / 28 / 28 (48); strain heating 3.2 /
+// 2.9 / 2.8 (3.8), 4.5 / 3.8 / 3.6 (12.2), 38 / 23 / 17 (159).
+template <int MOST, typename F>
+static inline void by_block_columns(int ny, int nx, F&& f) {
+    const long ncol = (long)ny * nx;
+    auto with = [&](auto cols) { f((unsigned)((ncol + decltype(cols)::value - 1) / decltype(cols)::value), cols); };
+    if (ncol < 5000) with(std::integral_constant<int, 8>());
+    else if (ncol < 32768) with(std::integral_constant<int, 16>());
+    else with(std::integral_constant<int, MOST>());
 }
 static inline unsigned flat_blocks(long n) {
     long b = (n + 255) / 256;
@@ -2312,7 +2342,9 @@ hipError_t launch_enth_apply(const EnthArgs<T>& A, T* E, const T* delta, T omega
 }
 template <typename T>
 hipError_t launch_enth_omega(const EnthArgs<T>& A, const T* dhdt, const T* bmb, T out_div, T* omega, hipStream_t st) {
-    k_enth_omega<T><<<block_columns(A.ny, A.nx), 256, 0, st>>>(A, dhdt, bmb, out_div, omega);
+    by_block_columns<16>(A.ny, A.nx, [&](unsigned nb, auto cols) {
+        k_enth_omega<T, decltype(cols)::value><<<nb, 256, 0, st>>>(A, dhdt, bmb, out_div, omega);
+    });
     return hipGetLastError();
 }
 template <typename T>
@@ -2329,19 +2361,26 @@ hipError_t launch_enth_tendency(const T* a, const T* b, T div, T* out, long n, h
 template <typename T>
 hipError_t launch_enth_rhs(const EnthArgs<T>& A, const T* beta, T m, T u_reg, int frictional, T* Q_fh, T* f_E,
                            hipStream_t st) {
-    k_enth_rhs<T><<<block_columns(A.ny, A.nx), 256, 0, st>>>(A, beta, m, u_reg, frictional, Q_fh, f_E);
+    by_block_columns<kBlockCols>(A.ny, A.nx, [&](unsigned nb, auto cols) {
+        k_enth_rhs<T, decltype(cols)::value><<<nb, 256, 0, st>>>(A, beta, m, u_reg, frictional, Q_fh, f_E);
+    });
     return hipGetLastError();
 }
 template <typename T>
 hipError_t launch_enth_strain_heating(const T* u, const T* v, const T* B, int ny, int nx, int nz, T dxi, T n_glen,
                                      T eps_reg, T rho_g, T* phi, hipStream_t st) {
     const T glen_p = (T(1) - n_glen) / (T(2) * n_glen);
-    k_enth_strain_heating<T><<<block_columns(ny, nx), 256, 0, st>>>(u, v, B, ny, nx, nz, dxi, glen_p, eps_reg, rho_g, phi);
+    by_block_columns<kBlockCols>(ny, nx, [&](unsigned nb, auto cols) {
+        k_enth_strain_heating<T, decltype(cols)::value><<<nb, 256, 0, st>>>(u, v, B, ny, nx, nz, dxi, glen_p, eps_reg,
+                                                                           rho_g, phi);
+    });
     return hipGetLastError();
 }
 template <typename T>
 hipError_t launch_enth_arrhenius(const EnthArgs<T>& A, T n_glen, T scale, T* B, hipStream_t st) {
-    k_enth_arrhenius<T><<<block_columns(A.ny, A.nx), 256, 0, st>>>(A, n_glen, scale, B);
+    by_block_columns<kBlockCols>(A.ny, A.nx, [&](unsigned nb, auto cols) {
+        k_enth_arrhenius<T, decltype(cols)::value><<<nb, 256, 0, st>>>(A, n_glen, scale, B);
+    });
     return hipGetLastError();
 }
 template <typename T>

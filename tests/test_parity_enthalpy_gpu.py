@@ -70,6 +70,31 @@ def test_set_rhs(ny, nx, nz, seed):
     assert rel_err(N(ops.f_E), th.f_E) < KTOL
 
 
+@pytest.mark.parametrize("ny,nx,nz", [(7, 9, 64), (68, 73, 9), (70, 72, 33), (180, 181, 2), (181, 183, 21)])
+def test_once_a_step_kernels_at_block_edges(ny, nx, nz):
+    """Forcing, omega, rate factor and strain heating on maps on both sides of the
+    rule for the columns of a block (5000 and 32768 columns) with ragged last
+    blocks, against the oracle."""
+    print(f"once-a-step kernels {ny}x{nx}x{nz}", flush=True)
+    from oracle.oracle import SEC_PER_YR, strain_heating
+    from tests.util import dome_fields
+    th, ops = make_pair(enth_case(ny, nx, nz, 12), nz)
+    assert rel_err(N(ops.f_E), th.f_E) < KTOL
+    dh = 0.5 * np.random.default_rng(13).standard_normal((ny, nx))
+    for a in (ops.enthalpy_velocity.u3d, ops.enthalpy_velocity.v3d):
+        a.mul_(SEC_PER_YR)
+    th.u3d, th.v3d = (np.ascontiguousarray(N(a)) for a in (ops.enthalpy_velocity.u3d, ops.enthalpy_velocity.v3d))
+    ops.compute_omega(T(dh))
+    assert rel_err(N(ops.enthalpy_velocity.omega), th.compute_omega(dh)) < KTOL
+    assert rel_err(N(ops.get_arrhenius_factor()), th.get_arrhenius_factor(3.0)) < KTOL
+    F = dome_fields(ny=ny, nx=nx, seed=14)
+    for k, dst in (("u", ops.grid.state.u), ("v", ops.grid.state.v), ("B", ops.grid.rheology.B)):
+        dst.set(T(F[k]))
+    ops.compute_strain_heating()
+    ref = strain_heating(F["u"], F["v"], F["B"], 3.0, float(ops.grid.rheology.eps_reg.value), DX, 917.0)
+    assert rel_err(N(ops.enthalpy_forcing.phi_strain), np.repeat(ref[:, :, None], nz, axis=2)) < KTOL
+
+
 @pytest.mark.parametrize("flags", [7, 6, 5, 3, 1, 0])
 @pytest.mark.parametrize("ny,nx,nz,seed", CASES)
 def test_residual(ny, nx, nz, seed, flags):
