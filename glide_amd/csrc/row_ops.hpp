@@ -341,7 +341,7 @@ struct ForwardRows {
             const T Hl = lane_left(H), Sl = lane_left(S), Sxl = lane_left(Sxx), be = T(0.5) * (lane_left(bp) + bp);
             const T sp = u * u + T(10), rs = row_rsqrt(sp), al = sp * rs, Hm = T(0.5) * (Hl + H);
             T pw = T(1), dpw = T(0);
-            if constexpr (DRAG) {
+            if (DRAG && w > 0 && w < NW - 1) {  // the halo rows need no drag
                 const T z = u * u + T(0.25) * (vl * vl + v * v + vbl * vbl + vb * vb) + a.P.u_reg;
                 pw = pow(z, a.P.drag_q);
                 if constexpr (JVP) dpw = a.P.drag_q * pow(z, a.P.drag_q - T(1));
@@ -375,7 +375,7 @@ struct ForwardRows {
             const T sp = v * v + T(10), rs = row_rsqrt(sp), al = sp * rs, Hm = T(0.5) * (Ht + H);
             const bool iin = i > 0 && i < ny;
             T pw = T(1), dpw = T(0);
-            if constexpr (DRAG) {
+            if (DRAG && w < NW - 1) {
                 const T utr = lane_right(ut);
                 const T z = v * v + T(0.25) * (ut * ut + utr * utr + u * u + ur * ur) + a.P.u_reg;
                 pw = pow(z, a.P.drag_q);
