@@ -170,6 +170,7 @@ SIGNATURES = {
     "glide_ensemble_destroy": (_I, [_P]),
     "glide_ssa_vjp": (_I, [_LP, _D, _I, _P, _P, _P, _P, _P, _P, _P]),
     "glide_vanka_adjoint_sweeps": (_I, [_LP, _D, _I, ctypes.POINTER(VankaConfigC), _I, _P]),
+    "glide_red_black_sweeps": (_I, [_LP, _I, _I, _D, _I, ctypes.POINTER(VankaConfigC), _I, _P]),
     "glide_fas_adjoint_solve": (_I, [_LP, _I, _I, _D, ctypes.POINTER(FasConfigC), ctypes.POINTER(VankaConfigC),
                                      ctypes.POINTER(SolveReport), _P]),
     "glide_fas_adjoint_vcycle": (_I, [_LP, _I, _I, _I, _D, ctypes.POINTER(FasConfigC),

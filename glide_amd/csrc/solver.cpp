@@ -2803,6 +2803,30 @@ int glide_vanka_adjoint_sweeps(const glide_level* L, double dt, int n_iter, cons
     return vanka_adjoint_sweeps(*L, dt, n_iter, *vc, flags, (hipStream_t)stream, true);
 }
 
+int glide_red_black_sweeps(const glide_level* L, int fp32, int adjoint, double dt, int n_iter,
+                           const glide_vanka_config* vc, int flags, void* stream) {
+    GLIDE_TRY(check_level(L));
+    GLIDE_TRY(check_ssa_inputs(*L));
+    if (!vc) return fail(GLIDE_ERR_INVALID_ARG, "vc is NULL");
+    if (n_iter < 0) return fail(GLIDE_ERR_INVALID_ARG, "n_iter must be non-negative");
+    if (!(dt > 0.0)) return fail(GLIDE_ERR_INVALID_ARG, "dt must be positive");
+    REQ(L->work);
+    hipStream_t st = (hipStream_t)stream;
+    if (!adjoint) {
+        REQ(L->f_u); REQ(L->f_v); REQ(L->f_H); REQ(L->gamma);
+        return fp32 ? mc_sweeps_t<float>(*L, dt, n_iter, *vc, flags, st, false)
+                    : mc_sweeps_t<double>(*L, dt, n_iter, *vc, flags, st, false);
+    }
+    REQ(L->lambda_u); REQ(L->lambda_v); REQ(L->lambda_H); REQ(L->af_u); REQ(L->af_v); REQ(L->af_H);
+    REQ(L->adj_cache);
+    if (fp32) {
+        GLIDE_TRY(adjoint_prepare_t<float>(*L, dt, *vc, st));
+        return mc_adjoint_sweeps_t<float>(*L, dt, n_iter, *vc, st);
+    }
+    GLIDE_TRY(adjoint_prepare_t<double>(*L, dt, *vc, st));
+    return mc_adjoint_sweeps_t<double>(*L, dt, n_iter, *vc, st);
+}
+
 int glide_fas_adjoint_solve(const glide_level* levels, int n_levels, int start_level, double dt,
                             const glide_fas_config* cfg, const glide_vanka_config* vc, glide_solve_report* report,
                             void* stream) {

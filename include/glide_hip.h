@@ -282,6 +282,12 @@ int glide_ssa_vjp(const glide_level* L, double dt, int flags, const void* lambda
                   const void* lambda_H, void* out_u, void* out_v, void* out_H, void* stream);
 int glide_vanka_adjoint_sweeps(const glide_level* L, double dt, int n_iter, const glide_vanka_config* vc, int flags,
                                void* stream);
+/* Red-black passes of one level as the mixed solves run them, for tests of a
+ * single pass (no counterpart in the reference): forward (flags as for
+ * glide_vanka_sweeps) or adjoint (linear drag; the patch factors are taken
+ * first), fp32 != 0 on a level whose buffers hold floats. */
+int glide_red_black_sweeps(const glide_level* L, int fp32, int adjoint, double dt, int n_iter,
+                           const glide_vanka_config* vc, int flags, void* stream);
 int glide_fas_adjoint_solve(const glide_level* levels, int n_levels, int start_level, double dt,
                             const glide_fas_config* cfg, const glide_vanka_config* vc, glide_solve_report* report,
                             void* stream);

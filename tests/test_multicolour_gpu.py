@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 import torch
 
-from tests.test_parity_ssa_gpu import N, grid_from
+from tests.test_parity_ssa_gpu import N, T, grid_from
 from tests.util import dome_fields, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -125,6 +125,104 @@ def test_mc_pass_in_one_and_in_three_launches(orc, shape, m, steps, relax_phi):
         for a, b in ((g.state.u, u), (g.state.v, v), (g.state.H, H)):
             assert rel_err(N(a.data), b) < (1e-12 if k == 0 else 1e-11), k
         assert np.array_equal(N(g.state.mask.data), mask), k
+
+
+# Shapes at the edges of the passes' tiles (6 rows; 58 columns forward, 60
+# adjoint) and of the factor cache's even / odd split (odd widths).
+EDGES = [(2, 2), (5, 3), (6, 58), (6, 60), (7, 61), (12, 59), (13, 121), (17, 300)]
+
+
+def _mirror32(g, F, lam=None, af=None):
+    """An FP32 level holding the fields rounded once, and those fields in FP64."""
+    from glide_amd.mixed import Level32
+    L = Level32(g, lam is not None)
+    named = dict(F)
+    if lam is not None:
+        named.update(zip(("lambda_u", "lambda_v", "lambda_H"), lam))
+        named.update(zip(("af_u", "af_v", "af_H"), af))
+    out = {}
+    for k, a in named.items():
+        if k in L.buf:
+            L.buf[k].copy_(T(a))
+            out[k] = N(L.buf[k].double())
+    return L, dict(F, **out)
+
+
+def _sweeps(level, fp32, adjoint, n, vc, flags=0):
+    import ctypes
+    from glide_amd import _lib
+    _lib.call("glide_red_black_sweeps", ctypes.byref(level), int(fp32), int(adjoint), 10.0, n, ctypes.byref(vc), flags,
+              _lib.stream_handle(torch.device("cuda")))
+    torch.cuda.synchronize()
+
+
+def _vanka_c(omega=0.85, steps=3, relaxation=0.5):
+    from glide_amd import _lib
+    return _lib.VankaConfigC(omega=omega, relax_phi=0.0, newton_steps=steps, relaxation=relaxation, ssa_damping=0.0,
+                             mc_damping=0.0, local_fp32=0, multicolour=1, newton_tol=0.0)
+
+
+# An FP32 pass against the FP64 oracle on the same (rounded) inputs.  Adjoint: the
+# rounding 2^-24 of about thirty terms that a multiplier's increment sums.  Forward:
+# times the terms' ratio to the residual they cancel to, up to 1e3 together on the
+# smallest grids; a wrong column, facet or factor is off by whole increments.
+FP32_ADJOINT, FP32_FORWARD = 2.0 ** -24 * 32, 2.0 ** -24 * 1e3
+
+
+@pytest.mark.parametrize("shape", EDGES)
+@pytest.mark.parametrize("fp32", [False, True])
+def test_red_black_adjoint_passes_match_oracle(orc, shape, fp32):
+    """One and then two more passes of both colour phases on row wavefronts with
+    the split factor cache, mask and calving on."""
+    ny, nx = shape
+    print(f"red-black adjoint shape={shape} fp32={fp32}", flush=True)
+    F = dome_fields(ny=ny, nx=nx, seed=61, mask_frac=0.15)
+    P = orc.phys(calving_rate=0.3)
+    rng = np.random.default_rng(62)
+    shapes = ((ny, nx + 1), (ny + 1, nx), (ny, nx))
+    lam, af = (tuple(rng.standard_normal(q) for q in shapes) for _ in range(2))
+    g = grid_from(F)
+    g.calving.calving_rate.set(0.3)
+    names = ("lambda_u", "lambda_v", "lambda_H")
+    if fp32:
+        L, F = _mirror32(g, F, lam, af)
+        lam, af = (tuple(F[k] for k in q) for q in (names, ("af_u", "af_v", "af_H")))
+        level, got = L.struct(), [L.buf[k] for k in names]
+    else:
+        ao = g.adjoint_operators
+        ao.use_cache = True
+        for dst, x in zip((g.adjoint.lambda_u, g.adjoint.lambda_v, g.adjoint.lambda_H), lam):
+            dst.set(T(x))
+        for dst, x in zip((ao.f_u, ao.f_v, ao.f_H), af):
+            dst.copy_(T(x))
+        level, got = g.level_struct(), [getattr(g.adjoint, k).data for k in names]
+    for n in (1, 2):
+        _sweeps(level, fp32, True, n, _vanka_c())
+        for _ in range(n):
+            lam = orc.mc_adjoint_sweep(F, lam, af, P, 1500.0, 10.0, omega=0.85)
+        err = [rel_err(N(a.double()), b) for a, b in zip(got, lam)]
+        print("  ", n, err, flush=True)
+        assert max(err) < (FP32_ADJOINT if fp32 else 1e-13)
+
+
+@pytest.mark.parametrize("shape", EDGES)
+@pytest.mark.parametrize("m", [1.0, 1.0 / 3.0])
+def test_red_black_fp32_passes_match_oracle(orc, shape, m):
+    """The FP32 instances of the forward pass, with the mixed solver's settings."""
+    ny, nx = shape
+    print(f"red-black fp32 shape={shape} m={m:.3f}", flush=True)
+    F = dome_fields(ny=ny, nx=nx, seed=63, mask_frac=0.1)
+    P = orc.phys(m=m, calving_rate=0.2)
+    g = grid_from(F)
+    g.sliding.m.set(m)
+    g.calving.calving_rate.set(0.2)
+    L, F = _mirror32(g, F)
+    from glide_amd.operators import FREEZE_PHI
+    _sweeps(L.struct(), True, False, 1, _vanka_c(), FREEZE_PHI)
+    u, v, H, _, _ = orc.mc_sweep(F, P, 1500.0, 10.0, **_oracle_kw(MIXED))
+    err = [rel_err(N(L.buf[k].double()), b) for k, b in (("u", u), ("v", v), ("H", H))]
+    print("  ", err, flush=True)
+    assert max(err) < FP32_FORWARD
 
 
 def _warm_models(orc, n, L, warm=2, ny=None, compat=True):
