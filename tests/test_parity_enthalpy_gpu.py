@@ -343,6 +343,33 @@ def test_tiled_sweep_matches_column_wavefronts(n, nz):
     assert abs(a0 - a1) <= 1e-8 * a1 and np.allclose(n0, n1, rtol=1e-7, atol=1e-8 * a1)
 
 
+@pytest.mark.parametrize("n,nz,seed", [(16, 11, 3), (24, 21, 3), (33, 33, 8), (40, 21, 3), (9, 9, 8), (60, 41, 8)])
+@pytest.mark.parametrize("rel,n_smooth", [(None, 100), (1e-5, 100), (1e-8, 100), (1e-9, 100), (1e-5, 8), (1e-5, 1)])
+def test_one_launch_sweep_stops_where_the_launches_stop(n, nz, seed, rel, n_smooth):
+    """The stopping branch of the sweep that small maps run in one launch: the
+    sweeps run, every norm, E and the residual of the form on the (ny, nx, nz)
+    arrays, with the default tolerances (a stop at the first sweep), at sweeps of
+    both parities and where the count ends it."""
+    print(f"sweep stop n={n} nz={nz} rel={rel} n_smooth={n_smooth}", flush=True)
+    out = []
+    for one in (True, False):
+        tm = _thermal_pair(n, nz, seed, strain=True)[2]
+        tm.n_smooth = n_smooth
+        if rel is not None:
+            tm.ops.smoother_config.relative_tolerance, tm.ops.smoother_config.absolute_tolerance = rel, 0.0
+        if not one:
+            tm.ops._sweep_work = None
+        rep = tm.step(DT, report=True)
+        out.append((rep.sweeps, [rep.norms[k] for k in range(rep.sweeps)], N(tm.ops.enthalpy_state.E),
+                    N(tm.ops.r_E), rep.r0, rep.r))
+    (s0, n0, E0, r0, a0, e0), (s1, n1, E1, r1, a1, e1) = out
+    print("   sweeps", s0, flush=True)
+    assert s0 == s1
+    assert np.allclose(n0, n1, rtol=1e-7, atol=1e-12 * a1) and np.isclose(e0, e1, rtol=1e-7, atol=1e-12 * a1)
+    assert rel_err(E0, E1) < STOL
+    assert abs(a0 - a1) <= 1e-8 * a1 and np.abs(r0 - r1).max() <= 1e-8 * a1
+
+
 @pytest.mark.parametrize("maps", [((24, 21, 3), (33, 33, 8)), ((24, 21, 3), (60, 41, 8), (59, 41, 9), (64, 41, 7))])
 def test_thermal_steps_on_several_streams_match_steps_alone(maps):
     """Steps of small maps enqueued on a stream each give, bitwise, what each
