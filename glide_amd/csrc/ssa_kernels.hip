@@ -137,13 +137,10 @@ __device__ __forceinline__ void cell_newton(const SsaArgs<T>& a, const T (*s_eta
         }
         const bool pin4 = (x[4] - a.dt * r[4]) <= thk;
         if (pin4) {
-            if constexpr (!ALIVE) masked = T(1);
             pin_row(J, 4);
             r[4] = x[4] - thk;
-        } else {
-            if constexpr (!ALIVE) masked = T(0);
         }
-        if constexpr (ALIVE) masked = go ? (pin4 ? T(1) : T(0)) : masked;
+        masked = !ALIVE || go ? (pin4 ? T(1) : T(0)) : masked;
         TJ rj[5] = {TJ(r[0]), TJ(r[1]), TJ(r[2]), TJ(r[3]), TJ(r[4])};
         TJ d[5];
         lu5_solve_rcp(J, rj, d);
