@@ -950,14 +950,6 @@ __device__ __forceinline__ long cb_base(int c, int i, int t, int ny, int nz, int
     return ((long)c * nz * ny + i) * hw + t;
 }
 
-// Virtual block vb of nvb: blocks go round-robin over the eight XCDs, so each
-// XCD is given one contiguous range of rows and finds the neighbouring rows a
-// pass rereads in its own L2.
-__device__ __forceinline__ long xcd_block(long vb, long nvb) {
-    const long q = nvb / 8, r = nvb % 8, x = vb % 8, l = vb / 8;
-    return x * q + (x < r ? x : r) + l;
-}
-
 // Transposed horizontal couplings of node (i, j): the coefficient the
 // neighbour's row holds for this node's enthalpy (its xp / xm / yp / ym in
 // exact_row), from the shared facet's flux, which the node's own face_fluxes
@@ -2481,7 +2473,7 @@ hipError_t launch_thermal_vjp(const EnthArgs<T>& A, const ThermalVjpArgs<T>& V, 
     return hipGetLastError();
 }
 
-// Level-major sweep launchers.
+// Tiled sweep launchers.
 template <typename T>
 hipError_t launch_enth_lm_layout(const T* src, T* dst, long ncol, int nz, bool to_lm, hipStream_t st) {
     if (nz > 64) return hipErrorInvalidValue;

@@ -19,6 +19,9 @@
 // Newton iteration runs the folded cell system of the additive smoother
 // (cell_system, refined hardware reciprocals), without compensated updates and
 // with the caller's relaxation and stopping threshold.
+//
+// k_cell_eta, k_mc_phase: the same pass as a launch for the viscosity and one per
+// colour, for heavy local solves on large levels (mc_phases_faster).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -321,9 +324,8 @@ template <typename T, int NW, bool LINEAR>
 __global__ __launch_bounds__(kRowLanes* NW) void k_mc_pass(SsaArgs<T> a, T* __restrict__ u_dst,
                                                            T* __restrict__ v_dst, T* __restrict__ H_dst,
                                                            T* __restrict__ mask, T* __restrict__ phi_dst,
-                                                           VankaArgs<T> vk, int gx, int blocks) {
-    const int b = xcd_block(blockIdx.x, gridDim.x);
-    if (b >= blocks) return;
+                                                           VankaArgs<T> vk, int gx) {
+    const int b = (int)xcd_block(blockIdx.x, gridDim.x);
     mc_pass_body<T, NW, LINEAR>(b % gx, b / gx, a, u_dst, v_dst, H_dst, mask, phi_dst, vk);
 }
 
@@ -616,11 +618,10 @@ hipError_t launch_vanka_mc(const SsaArgs<T>& a, T* u_dst, T* v_dst, T* H_dst, T*
     int gx;
     const int blocks = mc_blocks(a.ny, a.nx, NW, &gx);
     const dim3 b(kRowLanes, NW);
-    const int g = (blocks + kXcdCount - 1) / kXcdCount * kXcdCount;
     if (a.P.linear_drag)
-        k_mc_pass<T, NW, true><<<g, b, 0, st>>>(a, u_dst, v_dst, H_dst, mask, phi_dst, vk, gx, blocks);
+        k_mc_pass<T, NW, true><<<blocks, b, 0, st>>>(a, u_dst, v_dst, H_dst, mask, phi_dst, vk, gx);
     else
-        k_mc_pass<T, NW, false><<<g, b, 0, st>>>(a, u_dst, v_dst, H_dst, mask, phi_dst, vk, gx, blocks);
+        k_mc_pass<T, NW, false><<<blocks, b, 0, st>>>(a, u_dst, v_dst, H_dst, mask, phi_dst, vk, gx);
     return hipGetLastError();
 }
 

@@ -65,14 +65,6 @@ __device__ __forceinline__ float row_rsqrt(float a) {
 // The row of a wavefront as a scalar, so that row pointers live in SGPRs.
 __device__ __forceinline__ int wave_row(int r) { return __builtin_amdgcn_readfirstlane(r); }
 
-// Workgroups are dispatched to the eight XCDs in turn; workgroup b of a grid of
-// n (a multiple of kXcdCount) takes this tile, so that an XCD's tiles are
-// neighbours and their halos meet in its L2.
-constexpr int kXcdCount = 8;
-__device__ __forceinline__ int xcd_block(int b, int n) {
-    return (b % kXcdCount) * (n / kXcdCount) + b / kXcdCount;
-}
-
 // Position of cell (i, j) in a plane of the patch-factor cache.  split: the even
 // columns of a row first, then the odd ones, so that the cells a colour phase
 // solves in a row are contiguous.

@@ -61,6 +61,14 @@ __device__ __forceinline__ long offC(int i, int j, int ny, int nx) {
     return (long)clampi(i, 0, ny - 1) * nx + clampi(j, 0, nx - 1);
 }
 
+// Workgroups are dispatched to the eight XCDs in turn, each with an L2 of its own;
+// workgroup vb of nvb (any number) takes this tile, so that an XCD is given one
+// contiguous range of them and finds in its L2 what neighbouring tiles reread.
+__device__ __forceinline__ long xcd_block(long vb, long nvb) {
+    const long q = nvb / 8, r = nvb % 8, x = vb % 8, l = vb / 8;
+    return x * q + (x < r ? x : r) + l;
+}
+
 // The XCC (XCD) the calling wave runs on.
 __device__ __forceinline__ unsigned xcc_id() {
     unsigned v;

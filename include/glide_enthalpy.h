@@ -70,9 +70,11 @@ typedef struct glide_enth_column {
     /* Optional (no counterpart in the reference), NULL for none: 4 nz ny nx
      * doubles of workspace.  With it, a fused alternating sweep with a
      * depth-constant velocity (glide_thermal_step) and 9 <= nz <= 64 runs on
-     * level-major copies of E, E_prev, f_E and omega (E_work then holds the
-     * column pass's output in that layout); results equal the column-major
-     * sweep's to rounding. */
+     * copies of E, E_prev, f_E and omega in tiles of 64 columns, a tile's levels
+     * one after another (E_work then holds the column pass's output in that
+     * layout); small maps run all sweeps in one launch, which keeps its norms
+     * and barrier in r_E.  Results equal the column-major sweep's to rounding.
+     * The record of the last sweep, for `report`, is one per device. */
     void *sweep_work;
 } glide_enth_column;
 

@@ -341,14 +341,15 @@ int glide_forward_fused_enable(int on);
  * all passes of one call as one persistent launch of one workgroup per three
  * rows, a device-wide barrier between passes (it uses the last two values of
  * the level's workspace as its arrival counter and timeout flag; a timed-out
- * barrier leaves NaN thicknesses); 0 launches each pass as above.  Both give
- * the same state. */
+ * barrier leaves NaN thicknesses), and calls of 32 passes or more of levels of 5 to
+ * 16 rows and at most 16 columns in one workgroup (FP64 local solves; the same to
+ * rounding); 0 launches each pass as above.  Both give the same state. */
 int glide_forward_persistent_enable(int on);
 /* Cached adjoint smoothing of levels of at most 512 cells with linear drag
  * (no counterpart in the reference): 1 (default) runs all passes of one call
  * in a single workgroup (transpose operator, patch solves and update per pass,
- * separated by workgroup barriers), when the device's LDS per block holds the
- * level; 0 launches the transpose operator and the adjoint pass per pass.
+ * separated by workgroup barriers; levels up to 16 x 16 cells in its registers),
+ * when the device's LDS per block holds the level; 0 launches the transpose operator and the adjoint pass per pass.
  * Both give the same multipliers. */
 int glide_adjoint_coarse_enable(int on);
 /* Cached adjoint passes of levels of at most 512 x 512 cells with linear drag
@@ -384,7 +385,7 @@ int glide_persistent_spin_limit(int polls);
  * (0 forward patch solve, 1 patch increment apply, 2 adjoint patch solve,
  * 3 transpose operator, 4 residual, 5 adjoint increment apply, 6 enthalpy
  * column smoother, 7 enthalpy layer smoother, 8 enthalpy residual, 9 adjoint
- * patch factorisation into the cache, 10 / 11 one colour phase of the
+ * patch factorisation into the cache, 10 / 11 one pass (both colours) of the
  * red-black smoother in FP32 / FP64, 12 / 13 one colour phase of the red-black
  * adjoint pass in FP32 / FP64; the red-black launches count every cell).
  * glide_timing_read synchronises those events and returns the launch count,
@@ -426,9 +427,9 @@ int glide_ensemble_create(int32_t n_domains, const int32_t* n_levels, const glid
                           glide_ensemble** out);
 int glide_ensemble_step(glide_ensemble* e, double dt, void* stream);
 int32_t glide_ensemble_launches(const glide_ensemble* e);
-/* Tile shapes of the red-black smoothing phases (no counterpart in the
- * reference): rows[l] cell-pair rows per block (1, 2, 4 or 8; default 4) for
- * the stages of level l, l < glide_ensemble_levels(e) (the most levels of any
+/* Tile shapes of the red-black smoothing passes (no counterpart in the
+ * reference): rows[l] a setting of 1, 2, 4 or 8 (2, 2, 6 or 14 rows of cells a
+ * block; default 4) for the stages of level l, l < glide_ensemble_levels(e) (the most levels of any
  * domain), and rows[levels] for the coarsest-level passes; n = levels + 1.
  * The results do not depend on the tiles (each cell's arithmetic is the
  * same); the tables are recorded again at the next step.  Chosen by
