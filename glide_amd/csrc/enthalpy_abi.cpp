@@ -88,9 +88,9 @@ int scratch(EnthScratch** out) {
 int sweep_residents(const EnthScratch& s, hipStream_t st) {
     uint32_t mask[32] = {};
     int cus = 0;
-    if (hipExtStreamGetCUMask(st, 32, mask) == hipSuccess) {
+    if (st && hipExtStreamGetCUMask(st, 32, mask) == hipSuccess) {
         for (uint32_t m : mask) cus += __builtin_popcount(m);
-    } else {
+    } else if (st) {
         (void)hipGetLastError();
     }
     return s.sweeps_per_cu * (cus > 0 && cus < s.cus ? cus : s.cus);

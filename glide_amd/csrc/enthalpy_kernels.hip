@@ -1078,7 +1078,7 @@ __global__ __launch_bounds__(256) void k_enth_adj_pass(const int* __restrict__ s
     const T* __restrict__ rW = rows + P;
     const T* __restrict__ rC = rows + 2 * P;
     double m = 0.0;
-    const long w = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+    const long w = (long)xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
     const int i = (int)(w / hw), t = (int)(w % hw);
     const int j = 2 * t + ((i + color) & 1);
     if (w < n && j < nx) {

@@ -325,7 +325,7 @@ __global__ __launch_bounds__(kRowLanes* NW) void k_mc_pass(SsaArgs<T> a, T* __re
                                                            T* __restrict__ v_dst, T* __restrict__ H_dst,
                                                            T* __restrict__ mask, T* __restrict__ phi_dst,
                                                            VankaArgs<T> vk, int gx) {
-    const int b = (int)xcd_block(blockIdx.x, gridDim.x);
+    const int b = xcd_block(blockIdx.x, gridDim.x);
     mc_pass_body<T, NW, LINEAR>(b % gx, b / gx, a, u_dst, v_dst, H_dst, mask, phi_dst, vk);
 }
 

@@ -64,9 +64,9 @@ __device__ __forceinline__ long offC(int i, int j, int ny, int nx) {
 // Workgroups are dispatched to the eight XCDs in turn, each with an L2 of its own;
 // workgroup vb of nvb (any number) takes this tile, so that an XCD is given one
 // contiguous range of them and finds in its L2 what neighbouring tiles reread.
-__device__ __forceinline__ long xcd_block(long vb, long nvb) {
-    const long q = nvb / 8, r = nvb % 8, x = vb % 8, l = vb / 8;
-    return x * q + (x < r ? x : r) + l;
+__device__ __forceinline__ int xcd_block(unsigned vb, unsigned nvb) {
+    const unsigned q = nvb / 8, r = nvb % 8, x = vb % 8, l = vb / 8;
+    return (int)(x * q + (x < r ? x : r) + l);
 }
 
 // The XCC (XCD) the calling wave runs on.
